@@ -434,8 +434,10 @@ int adamas_decode_layer_step(const void* qkv, const float* cos_table, const floa
  * Causal attention of n_new prompt tokens over the paged cache of one sequence that already holds them:
  * q, out [n_new][num_heads][128], query token i sees tokens 0 .. past_len + i; page_table points at the
  * sequence's first entry.  Replaces the prefill kernel behind
- * prefill_forward of the reference (adamas/utils/__init__.py:159-201).  fp32 online softmax, 16-bit probabilities in the value
- * product.  flags: ADAMAS_F_BF16, ADAMAS_F_HND.  workspace: adamas_prefill_workspace_bytes() bytes, 16-byte
+ * prefill_forward of the reference (adamas/utils/__init__.py:159-201).  fp32 online softmax; in the value
+ * product the probabilities are two 16-bit values where query heads share a key/value head and past_len
+ * is not 0 (an error as with fp32 probabilities), one 16-bit value relative to the largest otherwise.
+ * flags: ADAMAS_F_BF16, ADAMAS_F_HND.  workspace: adamas_prefill_workspace_bytes() bytes, 16-byte
  * aligned, contents irrelevant before and after (0 bytes: may be NULL).
  */
 size_t adamas_prefill_workspace_bytes(uint32_t n_new, uint32_t past_len, uint32_t num_heads,

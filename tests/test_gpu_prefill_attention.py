@@ -79,3 +79,37 @@ def test_prefill_attention_of_a_misaligned_view(gpu_device):
     flat = torch.empty(q.numel() + 1, dtype=q.dtype, device=gpu_device)
     flat[1:] = q.reshape(-1)
     assert torch.equal(U.prefill_forward(flat[1:].view(q.shape), ctrl, 0), U.prefill_forward(q, ctrl, 0))
+
+
+def _rms(x):
+    return float(x.double().pow(2).mean().sqrt())
+
+
+@pytest.mark.parametrize("n,past,kv_heads,dtype,sharpness", [
+    (300, 900, 8, torch.float16, 1.0),     # grouped heads behind a cache, token ranges merged
+    (300, 900, 8, torch.bfloat16, 1.0),
+    (1200, 300, 4, torch.bfloat16, 3.0),
+    (777, 0, 32, torch.float16, 3.0),      # one weight near 1, the maximum found late
+    (777, 0, 8, torch.bfloat16, 3.0),
+    (400, 1100, 32, torch.bfloat16, 1.0),
+])
+def test_prefill_attention_error_is_that_of_its_roundings(gpu_device, n, past, kv_heads, dtype, sharpness):
+    """rms error against float64.  Grouped heads behind a cache: the rounding of the output and nothing
+    else (weights of 22 or 16 significant bits add less than 1e-4 of it).  The other calls: the weights
+    are rounded to 16 bits too, relative to the largest.  More than 10^6 values: the rms of two
+    realisations of the same roundings differs by about 0.1 %, 2 % are allowed."""
+    ctrl, q, k, v = _cache(gpu_device, n, past, kv_heads, 16, dtype, 0, False, n + past)
+    q = (q * sharpness).to(dtype)
+    ref, _ = _reference(q, k, v, past)
+    best = ref
+    if past == 0 or kv_heads == 32:
+        best = torch.empty_like(ref)
+        hidden = (torch.arange(n + past, device=gpu_device)[None] >
+                  (past + torch.arange(n, device=gpu_device))[:, None])
+        for h in range(32):
+            kh, vh = (x[:, h // (32 // kv_heads)].double() for x in (k, v))
+            s = (q[:, h].double() @ kh.T / math.sqrt(128)).masked_fill(hidden, -math.inf)
+            w = torch.exp(s - s.amax(-1, keepdim=True))
+            best[:, h] = (w.to(dtype).double() @ vh) / w.sum(-1, keepdim=True)
+    err = _rms(U.prefill_forward(q, ctrl, 0).double() - ref)
+    assert err <= 1.02 * _rms(best.to(dtype).double() - ref)
