@@ -694,7 +694,9 @@ __global__ __launch_bounds__(kDenseThreads) void dense_decode_gqa_kernel(
 // run as 16x16x32 MFMA tiles with the query heads in the N dimension (2 kG of the 16 columns are used:
 // the matrix cores have throughput to spare, what matters is that the products leave the vector ALU).
 // Columns 0 .. kG-1 carry the softmax weights rounded to 16 bits, columns kG .. 2kG-1 what that rounding
-// left over: the weights keep at least 16 significant bits at no further matrix instruction.
+// left over: the weights keep 16 significant bits in bf16 and 22 in fp16 (there down to 2^-40 of the
+// largest: they are shifted up by kGqaShift ahead of the rounding, as what is left over ends at 2^-25) at no
+// further matrix instruction.
 //
 //   loads    a wave owns a tile of 32 tokens of one key/value head.  A load instruction covers four
 //            whole rows (lane / 16 = row, lane % 16 = 16-byte piece: 256 contiguous bytes per row); the
@@ -727,6 +729,8 @@ typedef uint32_t mfma_uint4 __attribute__((ext_vector_type(4)));  // (arrays of 
 
 constexpr uint32_t kGqaTile = 32;      // tokens of a tile
 constexpr uint32_t kGqaRowBytes = 256;
+template <bool kBf16>
+constexpr float kGqaShift = kBf16 ? 0.f : 15.f;   // weights of up to 2^15 are finite in fp16
 
 template <bool kBf16>
 __device__ __forceinline__ mfma_float4 mfma_16x16x32(const uint4& a, const uint4& b, mfma_float4 c) {
@@ -852,10 +856,11 @@ __global__ __launch_bounds__(kDenseThreads) void dense_decode_gqa_mfma_kernel(
     tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
     const float m_new = fmaxf(m_run, tmax);
     const float alpha = exp2_raw(m_run - m_new);
+    const float m_shift = m_new - kGqaShift<kBf16>;
     float p[8], psum = 0.f;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      p[i] = exp2_raw(s[i] - m_new);  // (the tile holds at least one token: a masked score gives zero)
+      p[i] = exp2_raw(s[i] - m_shift);  // (the tile holds at least one token: a masked score gives zero)
       psum += p[i];
     }
     l_run = l_run * alpha + psum;

@@ -51,3 +51,33 @@ def test_dense_attention_of_ragged_batches(gpu_device, lens, kv_heads, page, dty
         # left of an fp16 weight may be denormal: 2^-25 absolute against a sum of weights of at least 1
         bound = u * ref.abs() + 2.0 ** -14 * mag + 2.0 ** -25 * v.abs().sum(1)
         assert bool(((o[b].double() - ref).abs() <= bound).all()), (b, n)
+
+
+@pytest.mark.parametrize("lens,kv_heads,dtype", [
+    ([2000, 1777], 8, torch.float16), ([2000, 1777], 4, torch.float16), ([1900] * 4, 16, torch.float16),
+    ([2000, 1777], 8, torch.bfloat16), ([9000], 8, torch.float16)])
+def test_dense_attention_of_many_small_weights(gpu_device, lens, kv_heads, dtype):
+    """One key outweighs each of the others by 2^20.35, but its value is zero: the output is the sum of the
+    small weights, which are below the smallest normal number of fp16."""
+    dev = gpu_device
+    ctrl = U.InferenceController(1, 32, 128, 16, 1 << 20, max(lens), dtype, dev, batch_size=len(lens),
+                                 num_kv_heads=kv_heads)
+    ctrl.prepare_hadamard(lens)
+    q = torch.zeros(len(lens), 32, 128, device=dev, dtype=dtype)
+    q[:, :, 0] = 8.0
+    for b, n in enumerate(lens):
+        k = torch.zeros(n, kv_heads, 128, device=dev, dtype=dtype)
+        k[n // 3, :, 0] = 20.35 / math.log2(math.e) * math.sqrt(128) / 8.0
+        v = torch.ones_like(k)
+        v[n // 3] = 0
+        U.append_kvh(k, v, None, ctrl, 0, seq_idx=b)
+    top = 8.0 * float(torch.tensor(20.35 / math.log2(math.e) * math.sqrt(128) / 8.0).to(dtype)) / math.sqrt(128)
+    ctrl.begin_forward(1)
+    o = U.decode_sparse_attn(q, ctrl, 0, U.ALL_PAST_TOKENS).double()
+    for b, n in enumerate(lens):
+        rest = (n - 1) * math.exp(-top)
+        ref = rest / (1.0 + rest)
+        # 2^-16 of a weight's rounding in bf16 (2^-22 in fp16), fp32 scores of about 2^4 (2^-19 in the
+        # exponent), fp32 sums: below 2^-14; the result rounded once (fp16: normal above 2^-14)
+        bound = (2.0 ** -14 + 2.0 ** (-11 if dtype == torch.float16 else -8)) * ref
+        assert float((o[b] - ref).abs().max()) <= bound, (b, n)
