@@ -849,7 +849,7 @@ __global__ __launch_bounds__(kDenseThreads) void dense_decode_gqa_mfma_kernel(
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const bool ok = base + 16u * (i >> 2) + 4u * qt + (i & 3) < row_end;
-      s[i] = ok ? sc[i >> 2][i & 3] * scale_log2 : kNegBig;
+      s[i] = ok ? sc[i >> 2][i & 3] * scale_log2 : -INFINITY;  // (a weight of zero under every maximum)
       tmax = fmaxf(tmax, s[i]);
     }
     tmax = fmaxf(tmax, __shfl_xor(tmax, 16));
@@ -860,7 +860,7 @@ __global__ __launch_bounds__(kDenseThreads) void dense_decode_gqa_mfma_kernel(
     float p[8], psum = 0.f;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      p[i] = exp2_raw(s[i] - m_shift);  // (the tile holds at least one token: a masked score gives zero)
+      p[i] = exp2_raw(s[i] - m_shift);
       psum += p[i];
     }
     l_run = l_run * alpha + psum;

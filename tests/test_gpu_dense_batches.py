@@ -81,3 +81,30 @@ def test_dense_attention_of_many_small_weights(gpu_device, lens, kv_heads, dtype
         # exponent), fp32 sums: below 2^-14; the result rounded once (fp16: normal above 2^-14)
         bound = (2.0 ** -14 + 2.0 ** (-11 if dtype == torch.float16 else -8)) * ref
         assert float((o[b] - ref).abs().max()) <= bound, (b, n)
+
+
+SHORT = [1500, 1333, 40, 1201]
+
+
+def _short_batch(dev, kv_heads, dtype):
+    ctrl = U.InferenceController(1, 32, 128, 16, 1 << 20, max(SHORT), dtype, dev, batch_size=len(SHORT),
+                                 num_kv_heads=kv_heads)
+    ctrl.prepare_hadamard(SHORT)
+    q = torch.zeros(len(SHORT), 32, 128, device=dev, dtype=dtype)
+    k = torch.zeros(max(SHORT), kv_heads, 128, device=dev, dtype=dtype)
+    g = torch.Generator(device=dev).manual_seed(kv_heads)
+    v = [torch.randn(n, kv_heads, 128, generator=g, device=dev).to(dtype) for n in SHORT]
+    return ctrl, q, k, v
+
+
+@pytest.mark.parametrize("kv_heads", [32, 16, 8, 4])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_dense_attention_with_every_score_at_minus_infinity(gpu_device, kv_heads, dtype):
+    """No token has a weight: zeros, whatever the slots past the end of a tile hold."""
+    ctrl, q, k, v = _short_batch(gpu_device, kv_heads, dtype)
+    q[:, :, 3] = 1.0
+    k[:, :, 3] = -math.inf
+    for b, n in enumerate(SHORT):
+        U.append_kvh(k[:n].contiguous(), v[b], None, ctrl, 0, seq_idx=b)
+    ctrl.begin_forward(1)
+    assert not U.decode_sparse_attn(q, ctrl, 0, U.ALL_PAST_TOKENS).any()
