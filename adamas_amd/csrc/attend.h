@@ -172,6 +172,13 @@ __device__ __forceinline__ void attend_rows(const HeadKV& kv, const float (&qf)[
         vr[i] = *reinterpret_cast<const uint4*>(kp + kv.v_delta);
       }
     }
+    if (kLoadAlways && !kRowIndex && base + kGroups * kTile > row_end) {
+      // (uniform) the last token's value stands in for what is past the end: its weight there is zero,
+      // but zero times an infinity is NaN
+#pragma unroll
+      for (int i = 0; i < kTile; ++i)
+        if (!valid[i]) vr[i] = make_uint4(0, 0, 0, 0);
+    }
     float s[kTile];
     float m_new = st.m;
 #pragma unroll

@@ -138,7 +138,7 @@ __device__ __forceinline__ void merge_splits(const float* __restrict__ partial, 
     float m[16], l[16], a[16];
 #pragma unroll
     for (int u = 0; u < 16; ++u) {
-      // past the end: a duplicate of the last split, weighted zero below
+      // past the end: a duplicate of the last split, left out below
       const uint32_t s2 = min(s0 + u * kMergeGroups, n_split - 1);
       const float* p = base + static_cast<size_t>(s2) * kPartialFloats;
       m[u] = p[0];
@@ -156,7 +156,7 @@ __device__ __forceinline__ void merge_splits(const float* __restrict__ partial, 
     for (int u = 0; u < 16; ++u) {
       const float w = s0 + u * kMergeGroups < n_split ? exp2_raw(m[u] - m_new) : 0.f;
       L += l[u] * w;
-      A += a[u] * w;
+      A += (s0 + u * kMergeGroups < n_split ? a[u] : 0.f) * w;  // (zero times an infinity is NaN)
     }
     M = m_new;
   }
@@ -822,8 +822,14 @@ __global__ __launch_bounds__(kDenseThreads) void dense_decode_gqa_mfma_kernel(
       vr[i] = __builtin_nontemporal_load(reinterpret_cast<const mfma_uint4*>(kp + kvl.v_delta));
     }
   };
-  // row 4i + qt: K piece t16 at t16 ^ (row % 16), V piece at its 64-byte group ^ (row % 4)
-  auto store_tile = [&]() __attribute__((always_inline)) {
+  // row 4i + qt: K piece t16 at t16 ^ (row % 16), V piece at its 64-byte group ^ (row % 4).  Values past
+  // the end of the sequence are stored as zeros: their weight is zero, but zero times an infinity is NaN.
+  auto store_tile = [&](uint32_t base) __attribute__((always_inline)) {
+    if (base + kGqaTile > row_end) {  // (uniform)
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        if (base + 4u * i + qt >= row_end) vr[i] = mfma_uint4{0u, 0u, 0u, 0u};
+    }
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const uint32_t row = 4u * i + qt;
@@ -903,7 +909,7 @@ __global__ __launch_bounds__(kDenseThreads) void dense_decode_gqa_mfma_kernel(
     load_pages(first + kStep);
     for (uint32_t t = 0; t < n_tiles; ++t) {
       const uint32_t base = first + t * kStep;
-      store_tile();
+      store_tile(base);
       if (t + 1 < n_tiles) {
         load_tile(base + kStep);
         load_pages(base + 2 * kStep);
@@ -913,11 +919,15 @@ __global__ __launch_bounds__(kDenseThreads) void dense_decode_gqa_mfma_kernel(
   }
 
   // ---- the slices of the workgroup, then the splits: as in dense_decode_gqa_kernel ------------------
-  // what the columns kG .. 2kG-1 hold belongs to the heads of the first kG
+  // what the columns kG .. 2kG-1 hold belongs to the heads of the first kG (not where these are infinite:
+  // what a rounding leaves over can be zero or negative, and makes NaN of an infinite value)
 #pragma unroll
   for (int ct = 0; ct < 8; ++ct)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) acc[ct][i] += __shfl_xor(acc[ct][i], kG);
+    for (int i = 0; i < 4; ++i) {
+      const float rest = __shfl_xor(acc[ct][i], kG);
+      acc[ct][i] = fabsf(acc[ct][i]) < INFINITY ? acc[ct][i] + rest : acc[ct][i];
+    }
   __syncthreads();  // every wave is done with its V tile: the same LDS now takes the slice states
   float l_tot = l_run;  // the four lanes of a head hold the denominators of their own tokens
   l_tot += __shfl_xor(l_tot, 16);

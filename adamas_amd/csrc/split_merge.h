@@ -55,7 +55,7 @@ __device__ __forceinline__ void merge_partials(const float* base, uint32_t n_spl
     float m[kBatch], l[kBatch], a[kBatch][kVec];
 #pragma unroll
     for (int u = 0; u < kBatch; ++u) {
-      const uint32_t s2 = min(s0 + u, n_split - 1);  // past the end: a duplicate, weighted zero below
+      const uint32_t s2 = min(s0 + u, n_split - 1);  // past the end: a duplicate, left out below
       const float* p = base + static_cast<size_t>(s2) * kPartialFloats;
       m[u] = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       l[u] = __hip_atomic_load(p + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -75,7 +75,7 @@ __device__ __forceinline__ void merge_partials(const float* base, uint32_t n_spl
       const float w = s0 + u < n_split ? exp2_raw(m[u] - m_new) : 0.f;
       L += l[u] * w;
 #pragma unroll
-      for (int e = 0; e < kVec; ++e) A[e] += a[u][e] * w;
+      for (int e = 0; e < kVec; ++e) A[e] += (s0 + u < n_split ? a[u][e] : 0.f) * w;  // (0 * infinity is NaN)
     }
     M = m_new;
   }
@@ -99,7 +99,7 @@ __device__ __forceinline__ void merge_partial_pairs(const float* base, uint32_t 
     uint64_t ml[kBatch], aa[kBatch];
 #pragma unroll
     for (int u = 0; u < kBatch; ++u) {
-      const uint32_t s2 = min(s0 + u, n_split - 1);  // past the end: a duplicate, weighted zero below
+      const uint32_t s2 = min(s0 + u, n_split - 1);  // past the end: a duplicate, left out below
       const uint64_t* p =
           reinterpret_cast<const uint64_t*>(base + static_cast<size_t>(s2) * kPartialFloats);
       ml[u] = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -119,6 +119,7 @@ __device__ __forceinline__ void merge_partial_pairs(const float* base, uint32_t 
                           ? exp2_raw(__uint_as_float(static_cast<uint32_t>(ml[u])) - m_new)
                           : 0.f;
       L += __uint_as_float(static_cast<uint32_t>(ml[u] >> 32)) * w;
+      if (s0 + u >= n_split) aa[u] = 0;  // (zero times an infinity is NaN)
       A[0] += __uint_as_float(static_cast<uint32_t>(aa[u])) * w;
       A[1] += __uint_as_float(static_cast<uint32_t>(aa[u] >> 32)) * w;
     }

@@ -108,3 +108,20 @@ def test_dense_attention_with_every_score_at_minus_infinity(gpu_device, kv_heads
         U.append_kvh(k[:n].contiguous(), v[b], None, ctrl, 0, seq_idx=b)
     ctrl.begin_forward(1)
     assert not U.decode_sparse_attn(q, ctrl, 0, U.ALL_PAST_TOKENS).any()
+
+
+@pytest.mark.parametrize("kv_heads", [32, 16, 8, 4])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_dense_attention_of_infinite_values(gpu_device, kv_heads, dtype):
+    """Equal weights (exact in 16 bits: nothing is left over); an infinite channel of the value of one token,
+    the last one among them, is infinite in the sum, with its sign, and no other channel sees it."""
+    ctrl, q, k, v = _short_batch(gpu_device, kv_heads, dtype)
+    for b, n in enumerate(SHORT):
+        v[b][n // 2, :, 5] = math.inf
+        v[b][n - 1, :, 70] = -math.inf
+        U.append_kvh(k[:n].contiguous(), v[b], None, ctrl, 0, seq_idx=b)
+    ctrl.begin_forward(1)
+    o = U.decode_sparse_attn(q, ctrl, 0, U.ALL_PAST_TOKENS)
+    want = torch.zeros_like(o)
+    want[:, :, 5], want[:, :, 70] = math.inf, -math.inf
+    assert not o.isnan().any() and torch.equal(torch.where(o.isinf(), o, 0), want)
