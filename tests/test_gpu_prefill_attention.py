@@ -113,3 +113,27 @@ def test_prefill_attention_error_is_that_of_its_roundings(gpu_device, n, past, k
             best[:, h] = (w.to(dtype).double() @ vh) / w.sum(-1, keepdim=True)
     err = _rms(U.prefill_forward(q, ctrl, 0).double() - ref)
     assert err <= 1.02 * _rms(best.to(dtype).double() - ref)
+
+
+@pytest.mark.parametrize("n,past,kv_heads,dtype", [
+    (70, 0, 32, torch.float16), (200, 41, 8, torch.bfloat16), (200, 41, 8, torch.float16),
+    (90, 5000, 8, torch.float16), (90, 5000, 32, torch.bfloat16)])
+def test_prefill_attention_of_infinite_values(gpu_device, n, past, kv_heads, dtype):
+    """Equal weights; an infinite channel of a value is infinite, with its sign, for the query tokens that see
+    it, does not reach the tiles of tokens before it, and no other channel sees it.  (For the queries of its
+    own tile that do not see it, zero times an infinity is NaN, as in any product with a masked matrix.)"""
+    ctrl, q, k, v = _cache(gpu_device, n, past, kv_heads, 16, dtype, 0, False, n)
+    mid, last = past + n // 2, past + n - 1
+    v[mid, :, 5] = math.inf
+    v[last, :, 70] = -math.inf
+    ctrl.clean_states()
+    ctrl.prepare_hadamard(past + n)
+    U.append_kvh(k, v, None, ctrl, 0)
+    o = U.prefill_forward(torch.zeros_like(q), ctrl, 0)
+    assert bool((o[n // 2:, :, 5] == math.inf).all()) and bool((o[n - 1, :, 70] == -math.inf).all())
+    rest = torch.ones(128, dtype=torch.bool, device=gpu_device)
+    rest[[5, 70]] = False
+    assert bool(o[:, :, rest].isfinite().all())
+    # queries whose last 256-row block of stacked rows ends before the tile of the token
+    blocks = (max(0, (mid // 64 * 64) - past) * 32 // kv_heads) // 256
+    assert bool(o[:blocks * 256 * kv_heads // 32, :, 5].isfinite().all())
