@@ -31,7 +31,7 @@ def _cache(dev, n, past, kv_heads, page, dtype, layout, growing, seed):
     return ctrl, q, k, v
 
 
-def _reference(q, k, v, past):
+def _reference(q, k, v, past, scale=1 / math.sqrt(128)):
     """(attention, sum of weights * |v|) in float64."""
     n, hq, _ = q.shape
     group = hq // k.shape[1]
@@ -39,7 +39,7 @@ def _reference(q, k, v, past):
     mag = torch.empty_like(out)
     hidden = torch.arange(k.shape[0], device=q.device)[None] > (past + torch.arange(n, device=q.device))[:, None]
     for h in range(hq):
-        s = q[:, h].double() @ k[:, h // group].double().T / math.sqrt(128)
+        s = q[:, h].double() @ k[:, h // group].double().T * scale
         w = s.masked_fill(hidden, -math.inf).softmax(-1)
         vh = v[:, h // group].double()
         out[:, h], mag[:, h] = w @ vh, w @ vh.abs()
@@ -137,3 +137,22 @@ def test_prefill_attention_of_infinite_values(gpu_device, n, past, kv_heads, dty
     # queries whose last 256-row block of stacked rows ends before the tile of the token
     blocks = (max(0, (mid // 64 * 64) - past) * 32 // kv_heads) // 256
     assert bool(o[:blocks * 256 * kv_heads // 32, :, 5].isfinite().all())
+
+
+@pytest.mark.parametrize("scale", [-0.11, 0.0, -0.0, 1e-30])
+@pytest.mark.parametrize("n,past,kv_heads,dtype", [(90, 0, 32, torch.float16), (130, 77, 8, torch.bfloat16)])
+def test_prefill_attention_of_any_scale(gpu_device, n, past, kv_heads, dtype, scale):
+    """No scale lets a query see a later token or loses the maximum.  Bound as in the test of the edges."""
+    ctrl, q, k, v = _cache(gpu_device, n, past, kv_heads, 16, dtype, 0, False, 5)
+    lib = _lib.load()
+    o = torch.empty_like(q)
+    need = lib.adamas_prefill_workspace_bytes(n, past, 32, kv_heads)
+    ws = torch.empty(max(need, 1), dtype=torch.uint8, device=gpu_device)
+    rc = lib.adamas_prefill_attention(q.data_ptr(), ctrl.kv_cache.buf_layer(0).data_ptr(), ctrl.seqs.table_ptr(0),
+                                      o.data_ptr(), ws.data_ptr(), need, n, past, 32, kv_heads, 128, 16, scale,
+                                      ctrl.kv_flags, _lib.current_stream())
+    assert rc == 0
+    ref, mag = _reference(q, k, v, past, scale)
+    u = 2.0 ** (-11 if dtype == torch.float16 else -8)
+    bound = u * (mag + ref.abs()) + 2.0 ** -14 * mag + 2.0 ** -25 * v.double().abs().sum(0).max()
+    assert bool(((o.double() - ref).abs() <= bound).all())
