@@ -1033,10 +1033,12 @@ static int sparse_decode_impl(const void* q, const void* kv_data, const int32_t*
     const uint32_t part_rows = std::max(128u, (max_seq_len + want - 1) / want);
     const uint32_t part_units = (part_rows + unit - 1) / unit;
     const uint32_t n_equal = (max_seq_len + part_units * unit - 1) / (part_units * unit);
-    if (n_equal > 1 || workspace) {
-      const WorkspaceLayout w = workspace_layout(batch, num_heads, 0, 0);
-      if (!workspace || workspace_bytes < w.dist_off) return ADAMAS_E_WORKSPACE;
-      if (reinterpret_cast<uintptr_t>(workspace) & 255) return ADAMAS_E_ALIGN;
+    const WorkspaceLayout w = workspace_layout(batch, num_heads, 0, 0);
+    const bool enough = workspace && workspace_bytes >= w.dist_off;
+    const bool aligned = (reinterpret_cast<uintptr_t>(workspace) & 255) == 0;
+    if (n_equal > 1 && !enough) return ADAMAS_E_WORKSPACE;
+    if (n_equal > 1 && !aligned) return ADAMAS_E_ALIGN;
+    if (enough && aligned) {  // (without, equal parts need none)
       counters = reinterpret_cast<uint32_t*>(static_cast<char*>(workspace) + w.counters_off);
       partial = reinterpret_cast<float*>(static_cast<char*>(workspace) + w.partial_off);
     }

@@ -7,6 +7,7 @@ import pytest
 import torch
 
 import adamas_amd.utils as U
+from adamas_amd import _lib
 
 pytestmark = pytest.mark.gpu
 
@@ -125,3 +126,39 @@ def test_dense_attention_of_infinite_values(gpu_device, kv_heads, dtype):
     want = torch.zeros_like(o)
     want[:, :, 5], want[:, :, 70] = math.inf, -math.inf
     assert not o.isnan().any() and torch.equal(torch.where(o.isinf(), o, 0), want)
+
+
+@pytest.mark.parametrize("kv_heads,flags", [(32, 0), (8, 0), (8, _lib.F_NO_MFMA)])
+def test_dense_attention_that_needs_no_workspace_takes_any(gpu_device, kv_heads, flags):
+    """70 sequences of up to 500 tokens keep every CU busy without a split: a workspace that is missing, too
+    small or misaligned is not used and refuses nothing.  One sequence is split and wants a whole one."""
+    dev = gpu_device
+    lens = [500 - 7 * i for i in range(70)]
+    ctrl = U.InferenceController(1, 32, 128, 16, 1 << 20, max(lens), torch.float16, dev, batch_size=len(lens),
+                                 num_kv_heads=kv_heads)
+    g = torch.Generator(device=dev).manual_seed(1)
+    ctrl.pool.kv.copy_(torch.randn(ctrl.pool.kv.shape, generator=g, device=dev))
+    ctrl.prepare_hadamard(lens)
+    ctrl.begin_forward(1)
+    q = torch.randn(len(lens), 32, 128, generator=g, device=dev).half()
+    want = U.decode_sparse_attn(q, ctrl, 0, U.ALL_PAST_TOKENS)
+    ws = ctrl.workspace(1)
+    need = _lib.load().adamas_workspace_bytes(len(lens), 32, 1, 1)
+
+    def call(pointer, size, batch=len(lens), longest=max(lens)):
+        o = torch.empty_like(q)
+        rc = _lib.load().adamas_sparse_decode_f(
+            q.data_ptr(), ctrl.pool.kv[0].data_ptr(), ctrl.seqs.table_dev.data_ptr(),
+            ctrl.seqs.indptr_dev.data_ptr(), ctrl.seqs.seq_lens_dev.data_ptr(), None, 0, 0, o.data_ptr(), pointer,
+            size, batch, 32, kv_heads, 128, 16, 1.0 / math.sqrt(128), longest, flags, _lib.current_stream())
+        return rc, o
+
+    assert ws.numel() >= need + 16
+    for pointer, size in ((None, 0), (ws.data_ptr(), 16), (ws.data_ptr() + 16, need)):
+        rc, o = call(pointer, size)
+        assert rc == 0
+        torch.testing.assert_close(o, want, rtol=2e-3, atol=2e-3)   # fp16 results of sums in another order
+    # (the length bound may exceed the lengths: equal parts of the bound, most of them empty)
+    assert call(None, 0, batch=1, longest=8000)[0] == -3
+    assert call(ws.data_ptr(), 16, batch=1, longest=8000)[0] == -3
+    assert call(ws.data_ptr() + 16, need, batch=1, longest=8000)[0] == -4
