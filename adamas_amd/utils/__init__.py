@@ -461,11 +461,41 @@ def apply_rope_in_place(q: torch.Tensor, k: torch.Tensor, past_kv_len: int,
     _lib.check(rc, "adamas_rope_in_place")
 
 
+def _is_traced(t: torch.Tensor) -> bool:
+    """Whether a derivative or a transform follows t, so that a kernel launched on its data would drop it."""
+    return (torch.is_grad_enabled() and t.requires_grad
+            or torch._C._functorch.is_functorch_wrapped_tensor(t)
+            or torch.autograd.forward_ad.unpack_dual(t).tangent is not None)
+
+
+def _prefill_with_torch_operators(q: torch.Tensor, c: InferenceController, layer_idx: int,
+                                  length: int) -> torch.Tensor:
+    """prefill_forward out of torch operators in float32, blocks of 4096 query rows."""
+    n, p = q.shape[0], c.page_size
+    n_pages = (length + p - 1) // p
+    kv = c.kv_cache.buf_layer(layer_idx).index_select(0, c.seqs.table_dev[:n_pages].long())
+    kv = kv.permute(1, 3, 0, 2, 4) if c.layout == TensorLayout.NHD else kv.permute(1, 2, 0, 3, 4)
+    keys, values = kv.reshape(2, c.num_kv_heads, n_pages * p, c.head_dim)[:, :, :length].float()
+    group, past = c.num_heads // c.num_kv_heads, length - n
+    qh = q.float().reshape(n, c.num_kv_heads, group, c.head_dim).permute(1, 2, 0, 3)  # [Hkv, G, N, D]
+    out = []
+    for r0 in range(0, n, 4096):
+        r1 = min(n, r0 + 4096)
+        rows = qh[:, :, r0:r1].reshape(c.num_kv_heads, group * (r1 - r0), c.head_dim)
+        s = rows @ keys[:, :past + r1].transpose(1, 2) / math.sqrt(c.head_dim)
+        hidden = (torch.arange(past + r1, device=q.device)[None] >
+                  past + torch.arange(r0, r1, device=q.device)[:, None])  # query row r sees tokens 0 .. past + r
+        w = s.masked_fill(hidden.repeat(group, 1), -math.inf).softmax(-1)
+        out.append((w @ values[:, :past + r1]).reshape(c.num_heads, r1 - r0, c.head_dim))
+    return torch.cat(out, dim=1).transpose(0, 1).to(c.dtype).contiguous()
+
+
 def prefill_forward(q: torch.Tensor, iController: InferenceController, layer_idx: int,
                     rope_scale: Optional[float] = None, rope_theta: Optional[float] = None) -> torch.Tensor:
     """Causal attention of the last N tokens of the sequence, q [N, Hq, 128], over the K/V already in
     the paged cache of `layer_idx` (adamas/utils/__init__.py:159-201); returns [N, Hq, 128].  The pages
-    are read where they lie, on the matrix cores.  rope_scale and rope_theta are accepted and unused, as
+    are read where they lie, on the matrix cores; a q that carries gradients or is inside a torch.func
+    transform goes through torch operators instead.  rope_scale and rope_theta are accepted and unused, as
     in the reference, whose q and cached k are already rotated.  Single sequence, like the reference."""
     c = iController
     _check_cuda_contig(q, "q", c.dtype, 3)
@@ -476,6 +506,8 @@ def prefill_forward(q: torch.Tensor, iController: InferenceController, layer_idx
         raise RuntimeError("q must be [N, num_heads, head_dim]")
     if n == 0 or n > length:
         raise RuntimeError("q holds %d tokens, the cache %d" % (n, length))
+    if _is_traced(q):
+        return _prefill_with_torch_operators(q, c, layer_idx, length)
     if q.data_ptr() % 16:   # a view into the middle of something: the kernel reads 128 bits at a time
         q = q.clone()
     lib = _lib.load()

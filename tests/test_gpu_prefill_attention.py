@@ -156,3 +156,37 @@ def test_prefill_attention_of_any_scale(gpu_device, n, past, kv_heads, dtype, sc
     u = 2.0 ** (-11 if dtype == torch.float16 else -8)
     bound = u * (mag + ref.abs()) + 2.0 ** -14 * mag + 2.0 ** -25 * v.double().abs().sum(0).max()
     assert bool(((o.double() - ref).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("n,past,kv_heads,layout", [(40, 0, 32, 0), (33, 70, 8, 1)])
+def test_prefill_attention_carries_gradients_and_transforms(gpu_device, n, past, kv_heads, layout):
+    """Gradients of q against float64 autograd, forward mode against the same, vmap against single calls."""
+    ctrl, q, k, v = _cache(gpu_device, n, past, kv_heads, 16, torch.float16, layout, False, 7)
+    g = torch.Generator(device=gpu_device).manual_seed(8)
+    w = torch.randn(q.shape, generator=g, device=gpu_device)
+
+    def reference(x):
+        group = 32 // kv_heads
+        kk, vv = (t.double().repeat_interleave(group, dim=1).transpose(0, 1) for t in (k, v))
+        hidden = (torch.arange(n + past, device=gpu_device)[None] >
+                  past + torch.arange(n, device=gpu_device)[:, None])
+        s = x.transpose(0, 1) @ kk.transpose(1, 2) / math.sqrt(128)
+        return (s.masked_fill(hidden, -math.inf).softmax(-1) @ vv).transpose(0, 1)
+
+    plain = U.prefill_forward(q, ctrl, 0)
+    x = q.clone().requires_grad_()
+    o = U.prefill_forward(x, ctrl, 0)
+    torch.testing.assert_close(o, plain, rtol=2e-3, atol=2e-3)     # both rounded to fp16
+    o.backward(w.half())
+    x64 = q.double().requires_grad_()
+    reference(x64).backward(w.half().double())
+    # fp32 all the way, the gradient rounded to fp16 (2^-11)
+    torch.testing.assert_close(x.grad.double(), x64.grad, rtol=1e-3, atol=1e-4)
+    with torch.no_grad():
+        assert U.prefill_forward(x, ctrl, 0).grad_fn is None and torch.equal(U.prefill_forward(x, ctrl, 0), plain)
+    _, tangent = torch.func.jvp(lambda t: U.prefill_forward(t, ctrl, 0), (q,), (w.half(),))
+    _, want = torch.func.jvp(reference, (q.double(),), (w.half().double(),))
+    torch.testing.assert_close(tangent.double(), want, rtol=1e-3, atol=1e-4)
+    both = torch.func.vmap(lambda t: U.prefill_forward(t, ctrl, 0))(torch.stack([q, -q]))
+    torch.testing.assert_close(both[0], plain, rtol=2e-3, atol=2e-3)
+    torch.testing.assert_close(both[1], U.prefill_forward(-q, ctrl, 0), rtol=2e-3, atol=2e-3)
