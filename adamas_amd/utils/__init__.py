@@ -514,10 +514,11 @@ def prefill_forward(q: torch.Tensor, iController: InferenceController, layer_idx
     o = torch.empty_like(q)
     need = lib.adamas_prefill_workspace_bytes(n, length - n, c.num_heads, c.num_kv_heads)
     ws = torch.empty(need, dtype=torch.uint8, device=q.device) if need else None
-    rc = lib.adamas_prefill_attention(q.data_ptr(), c.kv_cache.buf_layer(layer_idx).data_ptr(),
-                                      c.seqs.table_ptr(0), o.data_ptr(), _lib.ptr(ws), need, n,
-                                      length - n, c.num_heads, c.num_kv_heads, c.head_dim, c.page_size,
-                                      1.0 / math.sqrt(c.head_dim), c.kv_flags, _lib.current_stream())
+    with torch.cuda.device(q.device):  # (its current stream, as torch operators take it)
+        rc = lib.adamas_prefill_attention(
+            q.data_ptr(), c.kv_cache.buf_layer(layer_idx).data_ptr(), c.seqs.table_ptr(0), o.data_ptr(),
+            _lib.ptr(ws), need, n, length - n, c.num_heads, c.num_kv_heads, c.head_dim, c.page_size,
+            1.0 / math.sqrt(c.head_dim), c.kv_flags, _lib.current_stream())
     _lib.check(rc, "adamas_prefill_attention")
     return o
 

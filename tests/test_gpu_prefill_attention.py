@@ -190,3 +190,12 @@ def test_prefill_attention_carries_gradients_and_transforms(gpu_device, n, past,
     both = torch.func.vmap(lambda t: U.prefill_forward(t, ctrl, 0))(torch.stack([q, -q]))
     torch.testing.assert_close(both[0], plain, rtol=2e-3, atol=2e-3)
     torch.testing.assert_close(both[1], U.prefill_forward(-q, ctrl, 0), rtol=2e-3, atol=2e-3)
+
+
+def test_prefill_attention_launches_on_the_device_of_its_tensors(gpu_device, monkeypatch):
+    ctrl, q, _, _ = _cache(gpu_device, 40, 0, 32, 16, torch.float16, 0, False, 3)
+    entered = []
+    enter = torch.cuda.device.__enter__
+    monkeypatch.setattr(torch.cuda.device, "__enter__", lambda self: (entered.append(self.idx), enter(self))[1])
+    U.prefill_forward(q, ctrl, 0)
+    assert entered == [q.device.index]
