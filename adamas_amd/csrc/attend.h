@@ -122,8 +122,9 @@ struct SoftmaxState {
 //                       sequence, all with weight zero: the loads cost less than the branches and
 //                       the zeroed registers they replace.  A sequence without tokens is left
 //                       before the first load.
+//   kStreamed (with kLoadAlways): nobody else reads these rows, the loads leave the caches alone.
 template <int kGroups, int kTile, bool kRowIndex = false, bool kBf16 = false, bool kLoadAlways = false,
-          typename PosFn>
+          bool kStreamed = false, typename PosFn>
 __device__ __forceinline__ void attend_rows(const HeadKV& kv, const float (&qf)[8], uint32_t g,
                                             uint32_t row_begin, uint32_t row_end, PosFn&& pos_of,
                                             SoftmaxState& st) {
@@ -149,9 +150,8 @@ __device__ __forceinline__ void attend_rows(const HeadKV& kv, const float (&qf)[
         const __half* kp = kv.kv_data + static_cast<size_t>(row) * kv.tok_stride + kv.head_off;
         const uint4* k4 = reinterpret_cast<const uint4*>(kp);
         const uint4* v4 = reinterpret_cast<const uint4*>(kp + kv.v_delta);
-        // (dense attention streams every row once; listed rows may be shared by the heads of a group)
-        kr[i] = kRowIndex ? *k4 : load_streamed(k4);
-        vr[i] = kRowIndex ? *v4 : load_streamed(v4);
+        kr[i] = kStreamed ? load_streamed(k4) : *k4;
+        vr[i] = kStreamed ? load_streamed(v4) : *v4;
         continue;
       }
       const int32_t pos = (r < row_end) ? pos_of(r) : -1;

@@ -162,3 +162,39 @@ def test_dense_attention_that_needs_no_workspace_takes_any(gpu_device, kv_heads,
     assert call(None, 0, batch=1, longest=8000)[0] == -3
     assert call(ws.data_ptr(), 16, batch=1, longest=8000)[0] == -3
     assert call(ws.data_ptr() + 16, need, batch=1, longest=8000)[0] == -4
+
+
+@pytest.mark.parametrize("heads,kv_heads,lens,dtype,layout", [
+    (8, 8, [60000, 1], torch.float16, 0),          # one head group: its parts fill every slot for partials
+    (8, 2, [60000, 1, 1], torch.bfloat16, 1),
+    (16, 16, [60000, 1], torch.bfloat16, 0),       # two head groups
+    (16, 4, [60000, 1, 1], torch.float16, 0),
+    (8, 1, [40000, 300], torch.float16, 0),
+    (32, 2, [9001, 128, 1, 4097], torch.float16, 0),   # rows that several workgroups read
+    (24, 8, [9001, 128, 1, 4097], torch.bfloat16, 1),  # a group that is no power of two
+    (40, 8, [5000], torch.float16, 0),
+    (32, 1, [3000], torch.bfloat16, 0),
+    (32, 16, [2600], torch.float16, 0),            # equal parts, two query heads per key/value head
+    (32, 16, [7001], torch.bfloat16, 1),
+])
+def test_dense_attention_of_other_head_counts(gpu_device, heads, kv_heads, lens, dtype, layout):
+    dev = gpu_device
+    g = torch.Generator(device=dev).manual_seed(heads + kv_heads)
+    ctrl = U.InferenceController(1, heads, 128, 16, 1 << 20, max(lens), dtype, dev, batch_size=len(lens),
+                                 num_kv_heads=kv_heads, layout=layout)
+    ctrl.pool.kv.copy_(torch.randn(ctrl.pool.kv.shape, generator=g, device=dev))
+    ctrl.prepare_hadamard(lens)
+    ctrl.inference_page_budget = max(lens)
+    q = torch.randn(len(lens), heads, 128, generator=g, device=dev).to(dtype)
+    o = U.decode_sparse_attn(q, ctrl, 0, U.ALL_PAST_TOKENS)
+    assert torch.equal(o, U.decode_sparse_attn(q, ctrl, 0, U.ALL_PAST_TOKENS))
+    u = 2.0 ** (-11 if dtype == torch.float16 else -8)
+    for b, n in enumerate(lens):
+        kv = ctrl.pool.kv[0][torch.tensor(ctrl.seqs.pages[b], device=dev)]
+        kv = (kv if layout == 0 else kv.transpose(2, 3)).transpose(0, 1).reshape(2, -1, kv_heads, 128)[:, :n]
+        for h in range(heads):
+            k, v = (x[:, h // (heads // kv_heads)].double() for x in kv)
+            w = torch.softmax(k @ q[b, h].double() / math.sqrt(128), dim=-1)
+            ref, mag = w @ v, w @ v.abs()
+            # as above: the result rounded to 16 bits, weights of at least 16 significant bits, fp32 sums
+            assert bool(((o[b, h].double() - ref).abs() <= u * ref.abs() + 2.0 ** -14 * mag).all()), (b, h)
