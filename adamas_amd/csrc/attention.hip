@@ -975,6 +975,33 @@ extern "C" size_t adamas_workspace_bytes(uint32_t batch, uint32_t num_heads, uin
   return workspace_layout(batch, num_heads, max_seq_len, budget).total;
 }
 
+// Whether attention over all tokens goes through the kernel for row lists (sel_idx == nullptr: the rows are
+// the positions 0 .. seq_len - 1) instead of the dense kernels, which take eight heads at once and leave CUs
+// idle where there is little to do.  One sequence: up to 4096 tokens, 2048 where the row kernel would read a
+// row once per query head of a group (32 heads, row / dense kernel in us: 1000 tokens 8.4 / 18.2, 4000 18.9 /
+// 22.6; 32:8 heads, 2000 tokens 11.6 / 14.2).  A batch: by the tokens times heads of all sequences.
+//   - Up to 128 tokens the row kernel needs no split and is the better one wherever rows are not shared (32:32
+//     heads, 64 sequences of 128 tokens 25.5 / 25.0, 32 14.5 / 18.7).  Where they are: 16 sequences of 48 at
+//     32:8 heads 5.3 / 6.4, 32 8.6 / 6.5; with two heads per group, or more than a matrix-core tile takes, 16
+//     of 128 9.9 / 10.4 and 7.6 / 9.2 (32:16, 32:2), 32 14.7 / 13.3 and 11.0 / 9.1.
+//   - Beyond, 32:32 heads: 32 sequences of 160 23.9 / 24.6, 64 50.3 / 36.6, 4 of 1000 19.6 / 20.5, 8 33.4 /
+//     30.1; 32:8 heads: 8 of 256 9.9 / 13.8, 16 18.6 / 15.2, 2 of 1000 10.0 / 13.6, 4 16.8 / 14.8.  A single
+//     group of eight heads fills fewer workgroups: 32 of 1000 32.7 / 37.5 at 8:8, 64 70.9 / 63.3; 16 17.3 /
+//     18.6 at 8:4, 32 29.8 / 20.7.
+static bool dense_as_rows(uint32_t batch, uint32_t num_heads, uint32_t group, uint32_t max_seq_len) {
+  if (max_seq_len > (group == 1 ? 4096u : 2048u)) return false;
+  if (batch == 1) return true;
+  uint64_t limit;
+  if (max_seq_len <= 128) {
+    if (group == 1) return true;
+    limit = group == 2 || group > 8 ? 81920u : 40960u;
+  } else {
+    limit = group == 1 ? 163840u : 81920u;
+    if (num_heads == kDenseHeads && group <= 2) limit *= 2u;
+  }
+  return static_cast<uint64_t>(batch) * max_seq_len * num_heads <= limit;
+}
+
 static int sparse_decode_impl(const void* q, const void* kv_data, const int32_t* page_indices,
                               const int32_t* page_indptr, const int32_t* seq_lens,
                               const int32_t* sel_idx, int64_t sel_stride, uint32_t n_sel, void* out,
@@ -1002,17 +1029,13 @@ static int sparse_decode_impl(const void* q, const void* kv_data, const int32_t*
   // lanes of one group load the same rows (correct, merged by the memory pipeline, but slower)
   const bool gqa_kernel = (gq == 2 || gq == 4 || gq == 8) && num_heads % kDenseHeads == 0;
   const bool gqa_mfma = gqa_kernel && !(flags & ADAMAS_F_NO_MFMA);
-  // Few tokens are attended through the kernel for row lists below (sel_idx == nullptr: the rows are the
-  // positions 0 .. seq_len - 1): the dense kernels take eight heads at once, which leaves most CUs idle
-  // (1024 tokens: 17.5 us against 9.4; 130 tokens: 16.4 against 7.1).  What counts is the tokens of the
-  // whole batch.  Row kernel against dense kernel in us, lengths from half to the maximum given: 32 heads,
-  // one sequence of 3000 tokens 16.9 / 20.5, 4 of 1000 20.7 / 20.7, 16 of 300 22.7 / 24.9, 8 of 1200
-  // 39.6 / 34.2, 4 of 2000 37.4 / 29.5; four query heads per key/value head, whose rows the row kernel
-  // reads four times, one of 1500 11.3 / 14.2, 8 of 300 12.9 / 14.5, 16 of 300 19.6 / 15.1, 4 of 2000
-  // 32.6 / 16.3.
-  const uint64_t batch_tokens = static_cast<uint64_t>(batch) * max_seq_len;
-  const uint64_t dense_rows_limit = (gq == 1 ? 4096u : 2048u) * (batch > 1 ? 5u : 4u) / 4u;
-  if (!sel_idx && num_heads % kDenseHeads == 0 && batch_tokens > dense_rows_limit) {
+  const WorkspaceLayout w = workspace_layout(batch, num_heads, 0, 0);
+  const bool ws_enough = workspace && workspace_bytes >= w.dist_off;
+  const bool ws_aligned = (reinterpret_cast<uintptr_t>(workspace) & 255) == 0;
+  // (the row kernel splits what is longer than 128 tokens, and then wants a workspace)
+  if (!sel_idx && num_heads % kDenseHeads == 0 &&
+      (!dense_as_rows(batch, num_heads, gq, max_seq_len) ||
+       (max_seq_len > 128 && !(ws_enough && ws_aligned)))) {
     const uint32_t hgroups = num_heads / kDenseHeads;
     float* partial = nullptr;
     uint32_t* counters = nullptr;
@@ -1036,17 +1059,18 @@ static int sparse_decode_impl(const void* q, const void* kv_data, const int32_t*
     const uint32_t part_rows = std::max(128u, (max_seq_len + want - 1) / want);
     const uint32_t part_units = (part_rows + unit - 1) / unit;
     const uint32_t n_equal = (max_seq_len + part_units * unit - 1) / (part_units * unit);
-    const WorkspaceLayout w = workspace_layout(batch, num_heads, 0, 0);
-    const bool enough = workspace && workspace_bytes >= w.dist_off;
-    const bool aligned = (reinterpret_cast<uintptr_t>(workspace) & 255) == 0;
-    if (n_equal > 1 && !enough) return ADAMAS_E_WORKSPACE;
-    if (n_equal > 1 && !aligned) return ADAMAS_E_ALIGN;
-    if (enough && aligned) {  // (without, equal parts need none)
+    if (n_equal > 1 && !ws_enough) return ADAMAS_E_WORKSPACE;
+    if (n_equal > 1 && !ws_aligned) return ADAMAS_E_ALIGN;
+    if (ws_enough && ws_aligned) {  // (without, equal parts need none)
       counters = reinterpret_cast<uint32_t*>(static_cast<char*>(workspace) + w.counters_off);
       partial = reinterpret_cast<float*>(static_cast<char*>(workspace) + w.partial_off);
     }
     if (gqa_mfma || !gqa_kernel) {
-      const bool list = batch > 1 && partial;
+      // The list of DenseWalk pays where lengths can differ by much.  Sequences of up to 128 tokens are one
+      // part each either way (256 of 16 tokens at 32:8 heads: list 24.9 us, equal parts 20.1; 32 of 128 at
+      // 32:2 20.7 / 9.1), and with a single group of eight heads that share rows the slots for partials keep
+      // the list from half the CUs (6 of 1000 to 16000 at 8:2 25.3 / 19.6; 8:8 on the list 41.1 / 46.2).
+      const bool list = batch > 1 && partial && max_seq_len > 128 && (hgroups > 1 || gq == 1);
       // no more workgroups than slots for partials: a head group holds 1 / hgroups of the list
       const uint32_t n_wg = list ? std::min(target, (kMaxSplits - 1u) * hgroups) : 0u;
       const dim3 grid = list ? dim3(n_wg) : dim3(n_equal, hgroups, batch);
@@ -1125,9 +1149,8 @@ static int sparse_decode_impl(const void* q, const void* kv_data, const int32_t*
   float* partial = nullptr;
   uint32_t* counters = nullptr;
   if (n_split > 1) {
-    const WorkspaceLayout w = workspace_layout(batch, num_heads, 0, 0);
-    if (!workspace || workspace_bytes < w.dist_off) return ADAMAS_E_WORKSPACE;
-    if (reinterpret_cast<uintptr_t>(workspace) & 255) return ADAMAS_E_ALIGN;
+    if (!ws_enough) return ADAMAS_E_WORKSPACE;
+    if (!ws_aligned) return ADAMAS_E_ALIGN;
     counters = reinterpret_cast<uint32_t*>(static_cast<char*>(workspace) + w.counters_off);
     partial = reinterpret_cast<float*>(static_cast<char*>(workspace) + w.partial_off);
   }

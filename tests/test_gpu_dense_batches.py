@@ -176,6 +176,15 @@ def test_dense_attention_that_needs_no_workspace_takes_any(gpu_device, kv_heads,
     (32, 1, [3000], torch.bfloat16, 0),
     (32, 16, [2600], torch.float16, 0),            # equal parts, two query heads per key/value head
     (32, 16, [7001], torch.bfloat16, 1),
+    # batches of short sequences on both sides of the rule for the row kernel
+    (32, 8, [48 - i for i in range(26)], torch.float16, 0),
+    (32, 8, [48 - i for i in range(27)], torch.float16, 1),
+    (32, 2, [100 - i for i in range(26)], torch.bfloat16, 0),
+    (24, 8, [128 - i for i in range(14)], torch.float16, 0),
+    (8, 4, [129 - i for i in range(128)], torch.float16, 0),
+    (8, 2, [300, 1, 299, 7] * 9, torch.bfloat16, 1),
+    (8, 8, [1300, 1200] * 16, torch.float16, 0),
+    (32, 32, [129, 3, 128, 64] * 10, torch.float16, 0),
 ])
 def test_dense_attention_of_other_head_counts(gpu_device, heads, kv_heads, lens, dtype, layout):
     dev = gpu_device
