@@ -98,6 +98,7 @@ F_CODE_FROM_FP32 = 1
 F_BF16 = 2
 F_HND = 4
 F_NO_MFMA = 8
+F_CODES_CACHED = 16
 STATIC_SCRATCH_BYTES = 24 << 20
 E_SCRATCH = -5
 DIST_FP16, DIST_U16 = 0, 1

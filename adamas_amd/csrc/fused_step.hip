@@ -148,8 +148,9 @@ __device__ __forceinline__ uint32_t wave_query_code(const WaveRopeLoads& r, int 
 // kShare = 4 (grouped queries, groups of a multiple of four heads): a lane scores the codes it loads
 // for the four query heads that share them.  One load instruction then covers 16 tokens instead of
 // four, and the bit planes of a key are made once instead of four times.
+// kStreamCodes: the codes are more than the caches keep from one token to the next, read past them.
 template <int kPage, int kPasses, bool kPartial, bool kHist = false, int kHeads = kFusedHeads,
-          bool kFromQkv = false, int kShare = 1>
+          bool kFromQkv = false, int kShare = 1, bool kStreamCodes = false>
 __global__ __launch_bounds__(kHeads * kWave) void estimate_select_kernel(
     const int32_t* __restrict__ seq_lens, const int32_t* __restrict__ page_indices,
     const unsigned char* __restrict__ code_data, const uint16_t* __restrict__ q_code,
@@ -282,12 +283,8 @@ __global__ __launch_bounds__(kHeads * kWave) void estimate_select_kernel(
     const uint32_t row_bytes = num_kv_heads * 32u;
     const unsigned char* lane_base = code_data + kv_head_of(head, kv_inv16) * 32u + half * 16u;
 
-    // The codes of long sequences (selection mode, eight heads per workgroup) are more than the caches keep
-    // from one token to the next: read past them.  Eight layers of 32768 tokens 148.6 -> 135.1 us, two of
-    // 131072 88.4 -> 79.3.  The other instances also serve codes that do stay there: eight layers of 4096
-    // tokens 99.5 us, 103.2 with it, four of 8 sequences of 1500 to 7000 at 32:8 heads 125.1 and 128.2.
     auto load_codes = [&](const uint4* p) __attribute__((always_inline)) -> uint4 {
-      return kHeads == 8 && !kHist && kShare == 1 ? load_streamed(p) : *p;
+      return kStreamCodes ? load_streamed(p) : *p;
     };
 
     // issues the loads of pass `pass`; tokens past the end of the sequence read some valid slot and
@@ -1214,6 +1211,18 @@ static bool est_share(uint32_t batch, int est_heads, uint32_t num_heads, uint32_
   return num_heads / num_kv_heads % 4 == 0 && (batch > 1 || est_heads == kFusedHeads);
 }
 
+// Whether the wide estimator reads the codes past the caches.  Where the caches cannot keep them until the
+// next step that saves what they evict; where they can, a full chip loses nothing by it, but workgroups that
+// leave CUs idle wait for memory each time.  In us per step with the layers in turn, through / past the
+// caches (the last level holds 256 MB): 32 heads, 65536 tokens, 2 layers (134 MB) 20.2 / 19.3, 8 layers 23.8 /
+// 21.0; 8 heads (64 workgroups), 131072 tokens, 4 layers (134 MB) 20.6 / 22.5, 12 layers 25.3 / 23.4; 16
+// heads, 131072 tokens, 3 layers 23.2 / 24.3, 8 layers 27.6 / 24.9.  The narrow, shared and histogram
+// instances read through the caches.
+static bool est_stream(uint32_t flags, int est_heads, bool share, uint32_t workgroups) {
+  return est_heads == kFusedHeads && !share &&
+         (workgroups >= kStepWorkgroups || !(flags & ADAMAS_F_CODES_CACHED));
+}
+
 static StepGeom geom_of(const StepPlan& p) {
   StepGeom g;
   g.units_q = p.units_q;
@@ -1231,7 +1240,7 @@ static int step_candidates_impl(const void* q_code, const void* code_data,
                                 uint32_t num_kv_heads, uint32_t page_size, uint32_t max_seq_len,
                                 uint32_t page_table_stride, uint32_t flags,
                                 adamas_stream_t stream, const QkvSource* qsrc) {
-  if (flags & ~(ADAMAS_F_BF16 | ADAMAS_F_HND)) return ADAMAS_E_BADARG;
+  if (flags & ~(ADAMAS_F_BF16 | ADAMAS_F_HND | ADAMAS_F_CODES_CACHED)) return ADAMAS_E_BADARG;
   if (qsrc) q_code = qsrc->qkv;  // any valid, aligned pointer: the kernel does not read it
   if (!q_code || !code_data || !page_indices || (!page_indptr && !page_table_stride) ||
       !seq_lens || !workspace ||
@@ -1253,10 +1262,12 @@ static int step_candidates_impl(const void* q_code, const void* code_data,
   const StepPlan& plan = w.plan;
   const int est_heads = static_cast<int>(plan.heads);
   const bool share = est_share(batch, est_heads, num_heads, num_kv_heads);
+  const bool stream_codes = est_stream(flags, est_heads, share, plan.chunks * (num_heads / kFusedHeads));
   const dim3 grid(plan.chunks, num_heads / est_heads, batch);
   hipStream_t s = static_cast<hipStream_t>(stream);
-#define ADAMAS_LAUNCH_ESTSEL_Q(PG, PASSES, PARTIAL, HEADS, FROMQKV, SHARE)                           \
-  hipLaunchKernelGGL((estimate_select_kernel<PG, PASSES, PARTIAL, false, HEADS, FROMQKV, SHARE>),    \
+#define ADAMAS_LAUNCH_ESTSEL_Q(PG, PASSES, PARTIAL, HEADS, FROMQKV, SHARE, STREAM)                   \
+  hipLaunchKernelGGL((estimate_select_kernel<PG, PASSES, PARTIAL, false, HEADS, FROMQKV, SHARE,      \
+                                             STREAM>),                                               \
                      grid, dim3(HEADS * kWave), 0, s, seq_lens, page_indices,                        \
                      static_cast<const unsigned char*>(code_data),                                   \
                      static_cast<const uint16_t*>(q_code), page_table_stride, plan.units_q,          \
@@ -1265,21 +1276,23 @@ static int step_candidates_impl(const void* q_code, const void* code_data,
                      plan.kc, qcode_ws, static_cast<unsigned char*>(nullptr), 0u,                    \
                      static_cast<uint16_t*>(nullptr), static_cast<int64_t>(0),                       \
                      static_cast<uint32_t*>(nullptr), qsrc ? *qsrc : QkvSource())
-#define ADAMAS_LAUNCH_ESTSEL_H(PG, PASSES, PARTIAL, HEADS, SHARE)     \
-  if (qsrc) {                                                         \
-    ADAMAS_LAUNCH_ESTSEL_Q(PG, PASSES, PARTIAL, HEADS, true, SHARE);  \
-  } else {                                                            \
-    ADAMAS_LAUNCH_ESTSEL_Q(PG, PASSES, PARTIAL, HEADS, false, SHARE); \
+#define ADAMAS_LAUNCH_ESTSEL_H(PG, PASSES, PARTIAL, HEADS, SHARE, STREAM)     \
+  if (qsrc) {                                                                 \
+    ADAMAS_LAUNCH_ESTSEL_Q(PG, PASSES, PARTIAL, HEADS, true, SHARE, STREAM);  \
+  } else {                                                                    \
+    ADAMAS_LAUNCH_ESTSEL_Q(PG, PASSES, PARTIAL, HEADS, false, SHARE, STREAM); \
   }
-#define ADAMAS_LAUNCH_ESTSEL(PG, PASSES, PARTIAL)       \
-  if (share && est_heads == 4) {                        \
-    ADAMAS_LAUNCH_ESTSEL_H(PG, PASSES, PARTIAL, 4, 4)   \
-  } else if (share) {                                   \
-    ADAMAS_LAUNCH_ESTSEL_H(PG, PASSES, PARTIAL, 8, 4)   \
-  } else if (est_heads == 4) {                          \
-    ADAMAS_LAUNCH_ESTSEL_H(PG, PASSES, PARTIAL, 4, 1)   \
-  } else {                                              \
-    ADAMAS_LAUNCH_ESTSEL_H(PG, PASSES, PARTIAL, 8, 1)   \
+#define ADAMAS_LAUNCH_ESTSEL(PG, PASSES, PARTIAL)              \
+  if (share && est_heads == 4) {                               \
+    ADAMAS_LAUNCH_ESTSEL_H(PG, PASSES, PARTIAL, 4, 4, false)   \
+  } else if (share) {                                          \
+    ADAMAS_LAUNCH_ESTSEL_H(PG, PASSES, PARTIAL, 8, 4, false)   \
+  } else if (est_heads == 4) {                                 \
+    ADAMAS_LAUNCH_ESTSEL_H(PG, PASSES, PARTIAL, 4, 1, false)   \
+  } else if (stream_codes) {                                   \
+    ADAMAS_LAUNCH_ESTSEL_H(PG, PASSES, PARTIAL, 8, 1, true)    \
+  } else {                                                     \
+    ADAMAS_LAUNCH_ESTSEL_H(PG, PASSES, PARTIAL, 8, 1, false)   \
   }
 #define ADAMAS_LAUNCH_ESTSEL_PAGE(PASSES, PARTIAL)   \
   if (page_size == 16) {                             \
@@ -1345,7 +1358,7 @@ static int step_attend_impl(const void* q, void* kv_data, void* code_data,
                             uint32_t head_dim, uint32_t page_size, float sm_scale,
                             uint32_t max_seq_len, uint32_t page_table_stride, uint32_t flags,
                             adamas_stream_t stream, const QkvSource* qsrc) {
-  if (flags & ~(ADAMAS_F_BF16 | ADAMAS_F_HND)) return ADAMAS_E_BADARG;
+  if (flags & ~(ADAMAS_F_BF16 | ADAMAS_F_HND | ADAMAS_F_CODES_CACHED)) return ADAMAS_E_BADARG;
   if (qsrc) q = qsrc->qkv;
   const bool bf16 = (flags & ADAMAS_F_BF16) != 0;
   const bool hnd = (flags & ADAMAS_F_HND) != 0;
@@ -1446,7 +1459,7 @@ extern "C" int adamas_decode_step_f(const void* q, const void* q_code, const voi
                                     float sm_scale, uint32_t max_seq_len,
                                     uint32_t page_table_stride, uint32_t flags,
                                     adamas_stream_t stream) {
-  if (flags & ~(ADAMAS_F_BF16 | ADAMAS_F_HND)) return ADAMAS_E_BADARG;
+  if (flags & ~(ADAMAS_F_BF16 | ADAMAS_F_HND | ADAMAS_F_CODES_CACHED)) return ADAMAS_E_BADARG;
   if (!q || !q_code || !kv_data || !code_data || !page_indices || !page_indptr || !seq_lens ||
       !out || !workspace || budget == 0 || max_seq_len == 0 || batch == 0 || page_size == 0)
     return ADAMAS_E_BADARG;
@@ -1629,7 +1642,8 @@ extern "C" int adamas_decode_layer_step(const void* qkv, const float* cos_table,
                                         float hadamard_scale, uint32_t flags,
                                         adamas_stream_t stream) {
   if (!qkv || !cos_table || !sin_table || !kv_data || !code_data) return ADAMAS_E_BADARG;
-  if (flags & ~(ADAMAS_F_CODE_FROM_FP32 | ADAMAS_F_BF16 | ADAMAS_F_HND)) return ADAMAS_E_BADARG;
+  if (flags & ~(ADAMAS_F_CODE_FROM_FP32 | ADAMAS_F_BF16 | ADAMAS_F_HND | ADAMAS_F_CODES_CACHED))
+    return ADAMAS_E_BADARG;
   if ((reinterpret_cast<uintptr_t>(qkv) | reinterpret_cast<uintptr_t>(cos_table) |
        reinterpret_cast<uintptr_t>(sin_table)) & 15)
     return ADAMAS_E_ALIGN;
@@ -1639,7 +1653,8 @@ extern "C" int adamas_decode_layer_step(const void* qkv, const float* cos_table,
   src.sin_table = sin_table;
   src.scale = hadamard_scale;
   src.code_flags = flags;
-  const uint32_t kv_flags = flags & (ADAMAS_F_BF16 | ADAMAS_F_HND);  // format and layout of the caches
+  // format and layout of the caches, and the hint about the codes
+  const uint32_t kv_flags = flags & (ADAMAS_F_BF16 | ADAMAS_F_HND | ADAMAS_F_CODES_CACHED);
   int rc = step_candidates_impl(nullptr, code_data, page_indices, page_indptr, seq_lens, budget,
                                 workspace, workspace_bytes, batch, num_heads, num_kv_heads,
                                 page_size, max_seq_len, page_table_stride, kv_flags, stream, &src);

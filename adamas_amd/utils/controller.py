@@ -40,6 +40,10 @@ ALL_PAST_TOKENS = _AllPastTokens()
 ORTHONORMAL_SCALE = 128 ** -0.5
 RAW_SCALE = 1.0
 
+# Code bytes of all layers and sequences up to which the last-level cache (256 MB on an MI355X) keeps them
+# from one token to the next.
+CODES_CACHED_BYTES = 208 << 20
+
 
 class InferenceController:
     def __init__(self, num_layers, num_heads, head_dim, page_size,
@@ -126,6 +130,12 @@ class InferenceController:
     @property
     def min_len_now(self) -> int:
         return min(self.seqs.lengths)
+
+    @property
+    def codes_hint(self) -> int:
+        """F_CODES_CACHED for the decode step where the codes of all layers stay cached between tokens."""
+        code_bytes = self.num_layers * self.batch_size * self.max_len_now * self.num_kv_heads * 2 * CODE_WORDS
+        return _lib.F_CODES_CACHED if code_bytes <= CODES_CACHED_BYTES else 0
 
     def workspace(self, budget: int, max_len: Optional[int] = None) -> torch.Tensor:
         """Workspace of the attention kernel and of the step for this token budget and the length

@@ -106,13 +106,14 @@ def estimator_instance(_lib, page_size: int, heads: int, batch: int, max_seq_len
                        kv_heads: int = 0) -> str:
     """Name of the fused estimator's template instance the library launches for these sizes
     (page size, passes, partial last pass, histogram mode, heads per workgroup, fused projection,
-    query heads that share a lane), from the library's own plan."""
+    query heads that share a lane, codes read past the caches), from the library's own plan."""
     p = _lib.step_plan(batch, heads, max_seq_len, budget)
     flag = lambda v: "true" if v else "false"
     grouped = heads // (kv_heads or heads) % 4 == 0
     share = 4 if grouped and (batch > 1 or p["heads"] == 8) else 1
     return (f"estimate_select_kernel<{16 if page_size == 16 else 0}, {p['passes']}, "
-            f"{flag(p['partial'])}, false, {p['heads']}, false, {share}>")
+            f"{flag(p['partial'])}, false, {p['heads']}, false, {share}, "
+            f"{flag(p['heads'] == 8 and share == 1)}>")
 
 
 def log(msg: str) -> None:

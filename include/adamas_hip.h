@@ -62,6 +62,10 @@ typedef void* adamas_stream_t;
 #define ADAMAS_F_NO_MFMA 8u        /* adamas_sparse_decode_f, dense mode with 2, 4 or 8 query heads per
                                       key/value head: the vector-ALU kernel instead of the matrix-core
                                       one (same results within tolerance; kept for measurement)       */
+#define ADAMAS_F_CODES_CACHED 16u  /* the decode step and its estimator: all code pages read between two
+                                      steps of a layer (every layer, every sequence) stay in the
+                                      last-level cache, so the codes are not read past it.  A hint:
+                                      the results are the same with and without                       */
 
 /* output formats of adamas_estimate / key modes of adamas_topk */
 #define ADAMAS_DIST_FP16 0u /* integer distance stored as fp16 (the reference's output dtype) */

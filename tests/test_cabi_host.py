@@ -350,3 +350,21 @@ def test_prefill_plan_is_quick(args):
         return time.perf_counter() - t
 
     assert min(once() for _ in range(50)) < 150e-6
+
+
+def test_codes_cached_hint():
+    """The controller's hint goes by the codes of all layers and sequences: 32 bytes per token and head."""
+    from adamas_amd.utils.controller import CODES_CACHED_BYTES
+    c = _ctrl(num_layers=3, batch_size=2)
+    c.seqs.lengths[:] = [5, 7]
+    edge = CODES_CACHED_BYTES // (3 * 2 * 32 * 32)
+    c._len_bound = edge
+    assert c.codes_hint == _lib.F_CODES_CACHED
+    c._len_bound = edge + 1
+    assert c.codes_hint == 0
+    lib = _lib.load()    # a hint for the step and its two halves, not for the operators
+    step = [16] * 7 + [8, 16, None, 256, 1 << 40, 1, 32, 32, 64, 16, 1.0, 100, 8]   # head_dim 64: refused later
+    assert lib.adamas_decode_step_f(*step, _lib.F_CODES_CACHED, None) == -2
+    assert lib.adamas_decode_step_f(*step, 2 * _lib.F_CODES_CACHED, None) == -1
+    assert lib.adamas_sparse_decode_f(*[16] * 5, None, 0, 0, 16, None, 0, 1, 32, 32, 64, 16, 1.0, 100,
+                                      _lib.F_CODES_CACHED, None) == -1

@@ -75,3 +75,35 @@ def _check(gpu_device, lens, budget, page, kv_heads, dtype, layout):
     # the same rows in another order of summation: fp32 sums, one rounding to 16 bits each
     ulp = 2.0 ** (-10 if dtype == torch.float16 else -7)
     assert bool(((o.float() - o2.float()).abs() <= ulp * o2.float().abs() + 1e-5).all())
+
+
+@pytest.mark.parametrize("heads,length,page", [(8, 33000, 16), (8, 70001, 1), (16, 40000, 16), (32, 32768, 32)])
+def test_step_reads_codes_through_and_past_the_caches(gpu_device, heads, length, page, monkeypatch):
+    """The hint about cached codes changes no bit: both instances of the wide estimator (fewer workgroups than
+    CUs) and the one that ignores the hint, from the projection and from query codes; selection against the
+    stand-alone operators."""
+    from adamas_amd.utils import controller as C
+    dev = gpu_device
+    g = torch.Generator(device=dev).manual_seed(length)
+    ctrl = U.InferenceController(1, heads, 128, page, 128, length, torch.float16, dev)
+    ctrl.pool.kv.copy_(torch.randn(ctrl.pool.kv.shape, generator=g, device=dev))
+    ctrl.pool.codes.copy_(torch.randint(-32768, 32768, ctrl.pool.codes.shape, generator=g, device=dev))
+    ctrl.prepare_hadamard(length)
+    ctrl.begin_forward(1)
+    qkv = torch.randn(1, 3 * heads, 128, generator=g, device=dev).half()
+    angle = torch.rand(length, 64, generator=g, device=dev)
+    q, k, v = (x.contiguous() for x in qkv.chunk(3, dim=1))
+    q_code = U.append_kvh(k, v, None, ctrl, 0, q=q)
+    got = []
+    for limit in (0, 1 << 40):
+        monkeypatch.setattr(C, "CODES_CACHED_BYTES", limit)
+        o, sel = U.decode_step(q, q_code, ctrl, 0, return_indices=True)
+        got.append((o, sel.clone()))
+        o, sel = U.decode_layer_step(qkv, angle.cos(), angle.sin(), ctrl, 0, return_indices=True)
+        got.append((o, sel.clone()))
+        U.append_kvh(k, v, None, ctrl, 0, q=q)     # (the layer step rotated the new token's row)
+    assert torch.equal(got[0][0], got[2][0]) and torch.equal(got[0][1], got[2][1])
+    assert torch.equal(got[1][0], got[3][0]) and torch.equal(got[1][1], got[3][1])
+    U.decode_topk(U.decode_estimate(q_code, ctrl, 0), ctrl)
+    want = ctrl.topk_dindices_buffer.sort(dim=1).values
+    assert torch.equal(got[0][1].sort(dim=1).values, want)
