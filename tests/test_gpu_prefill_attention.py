@@ -199,3 +199,30 @@ def test_prefill_attention_launches_on_the_device_of_its_tensors(gpu_device, mon
     monkeypatch.setattr(torch.cuda.device, "__enter__", lambda self: (entered.append(self.idx), enter(self))[1])
     U.prefill_forward(q, ctrl, 0)
     assert entered == [q.device.index]
+
+
+@pytest.mark.parametrize("heads,kv_heads,n,past,dtype,page", [
+    (24, 8, 200, 0, torch.float16, 16),      # groups of 3: the heads of a query cross from one 256-row block to the next
+    (24, 8, 86, 2000, torch.bfloat16, 16),   # the same, token ranges merged
+    (40, 8, 257, 63, torch.bfloat16, 12),    # groups of 5
+    (40, 8, 52, 5000, torch.float16, 16),
+    (32, 1, 70, 0, torch.float16, 16),       # one key/value head
+    (32, 1, 33, 3000, torch.bfloat16, 16),
+    (8, 1, 300, 100, torch.float16, 1),
+])
+def test_prefill_attention_of_other_groups(gpu_device, heads, kv_heads, n, past, dtype, page):
+    dev = gpu_device
+    g = torch.Generator(device=dev).manual_seed(heads + n)
+    length = n + past
+    ctrl = U.InferenceController(1, heads, 128, page, 64, length, dtype, dev, num_kv_heads=kv_heads)
+    k, v = (torch.randn(length, kv_heads, 128, generator=g, device=dev).to(dtype) for _ in range(2))
+    q = torch.randn(n, heads, 128, generator=g, device=dev).to(dtype)
+    ctrl.prepare_hadamard(length)
+    U.append_kvh(k, v, None, ctrl, 0)
+    split = _lib.load().adamas_prefill_workspace_bytes(n, past, heads, kv_heads) > 0
+    assert split or past < 2000, "the token ranges are tested where they are meant to be"
+    ref, mag = _reference(q, k, v, past)
+    # as at the edges above
+    u = 2.0 ** (-11 if dtype == torch.float16 else -8)
+    bound = u * (mag + ref.abs()) + 2.0 ** -14 * mag + 2.0 ** -25 * v.double().abs().sum(0).max()
+    assert bool(((U.prefill_forward(q, ctrl, 0).double() - ref).abs() <= bound).all())
