@@ -465,7 +465,8 @@ def _is_traced(t: torch.Tensor) -> bool:
     """Whether a derivative or a transform follows t, so that a kernel launched on its data would drop it."""
     return (torch.is_grad_enabled() and t.requires_grad
             or torch._C._functorch.is_functorch_wrapped_tensor(t)
-            or torch.autograd.forward_ad.unpack_dual(t).tangent is not None)
+            or (torch.autograd.forward_ad._current_level >= 0
+                and torch.autograd.forward_ad.unpack_dual(t).tangent is not None))
 
 
 def _prefill_with_torch_operators(q: torch.Tensor, c: InferenceController, layer_idx: int,
@@ -508,17 +509,25 @@ def prefill_forward(q: torch.Tensor, iController: InferenceController, layer_idx
         raise RuntimeError("q holds %d tokens, the cache %d" % (n, length))
     if _is_traced(q):
         return _prefill_with_torch_operators(q, c, layer_idx, length)
+    if q.device.index != torch.cuda.current_device():  # (launched where the tensors are, as torch operators are)
+        with torch.cuda.device(q.device):
+            return _prefill(q, c, layer_idx, length)
+    return _prefill(q, c, layer_idx, length)
+
+
+def _prefill(q: torch.Tensor, c: InferenceController, layer_idx: int, length: int) -> torch.Tensor:
+    """The kernel behind prefill_forward, on the current device."""
+    n = q.shape[0]
     if q.data_ptr() % 16:   # a view into the middle of something: the kernel reads 128 bits at a time
         q = q.clone()
     lib = _lib.load()
     o = torch.empty_like(q)
     need = lib.adamas_prefill_workspace_bytes(n, length - n, c.num_heads, c.num_kv_heads)
     ws = torch.empty(need, dtype=torch.uint8, device=q.device) if need else None
-    with torch.cuda.device(q.device):  # (its current stream, as torch operators take it)
-        rc = lib.adamas_prefill_attention(
-            q.data_ptr(), c.kv_cache.buf_layer(layer_idx).data_ptr(), c.seqs.table_ptr(0), o.data_ptr(),
-            _lib.ptr(ws), need, n, length - n, c.num_heads, c.num_kv_heads, c.head_dim, c.page_size,
-            1.0 / math.sqrt(c.head_dim), c.kv_flags, _lib.current_stream())
+    rc = lib.adamas_prefill_attention(q.data_ptr(), c.kv_cache.buf_layer(layer_idx).data_ptr(),
+                                      c.seqs.table_ptr(0), o.data_ptr(), _lib.ptr(ws), need, n,
+                                      length - n, c.num_heads, c.num_kv_heads, c.head_dim, c.page_size,
+                                      1.0 / math.sqrt(c.head_dim), c.kv_flags, _lib.current_stream())
     _lib.check(rc, "adamas_prefill_attention")
     return o
 
