@@ -509,14 +509,16 @@ def prefill_forward(q: torch.Tensor, iController: InferenceController, layer_idx
         raise RuntimeError("q holds %d tokens, the cache %d" % (n, length))
     if _is_traced(q):
         return _prefill_with_torch_operators(q, c, layer_idx, length)
-    if q.device.index != torch.cuda.current_device():  # (launched where the tensors are, as torch operators are)
-        with torch.cuda.device(q.device):
-            return _prefill(q, c, layer_idx, length)
-    return _prefill(q, c, layer_idx, length)
+    device = q.get_device()
+    if device == torch._C._cuda_getDevice():
+        return _prefill(q, c, layer_idx, length, device)
+    with torch.cuda.device(device):  # (launched where the tensors are, as torch operators are)
+        return _prefill(q, c, layer_idx, length, device)
 
 
-def _prefill(q: torch.Tensor, c: InferenceController, layer_idx: int, length: int) -> torch.Tensor:
-    """The kernel behind prefill_forward, on the current device."""
+def _prefill(q: torch.Tensor, c: InferenceController, layer_idx: int, length: int,
+             device: int) -> torch.Tensor:
+    """The kernel behind prefill_forward, on q's device, which is the current one."""
     n = q.shape[0]
     if q.data_ptr() % 16:   # a view into the middle of something: the kernel reads 128 bits at a time
         q = q.clone()
@@ -527,7 +529,8 @@ def _prefill(q: torch.Tensor, c: InferenceController, layer_idx: int, length: in
     rc = lib.adamas_prefill_attention(q.data_ptr(), c.kv_cache.buf_layer(layer_idx).data_ptr(),
                                       c.seqs.table_ptr(0), o.data_ptr(), _lib.ptr(ws), need, n,
                                       length - n, c.num_heads, c.num_kv_heads, c.head_dim, c.page_size,
-                                      1.0 / math.sqrt(c.head_dim), c.kv_flags, _lib.current_stream())
+                                      1.0 / math.sqrt(c.head_dim), c.kv_flags,
+                                      torch._C._cuda_getCurrentRawStream(device))
     _lib.check(rc, "adamas_prefill_attention")
     return o
 

@@ -199,9 +199,7 @@ def test_prefill_attention_launches_on_the_device_of_its_tensors(gpu_device, mon
     monkeypatch.setattr(torch.cuda.device, "__enter__", lambda self: (entered.append(self.idx), enter(self))[1])
     U.prefill_forward(q, ctrl, 0)
     assert entered == []
-    answers = iter([q.device.index + 1])           # once another device than q's, then the real one
-    real = torch.cuda.current_device
-    monkeypatch.setattr(torch.cuda, "current_device", lambda: next(answers, None) or real())
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: q.device.index + 1)   # (another one than q's)
     U.prefill_forward(q, ctrl, 0)
     assert entered == [q.device.index]
 
