@@ -331,10 +331,10 @@ __device__ __forceinline__ DensePart dense_part(const DenseList& l, const int32_
 
 // The parts of a workgroup.  kList: its range of the list.  Otherwise grid (parts, head groups, batch)
 // with every sequence cut into equal parts of `grid_units` units, the longest into all of them: for one
-// sequence that is just as even and needs neither the scan nor the divisions (2 us at the start of every
-// workgroup; 32768 tokens 98.9 us with the list, 95.9 without).  In us, equal parts -> list: 32 heads, 3
-// sequences of 700 to 20000 tokens 125 -> 106, 13 of 1000 to 9000 222 -> 200, 16 of 8000 to 32000 997 ->
-// 914 (5.7 TB/s); 32:8 heads, 8 of 3000 to 16384 76 -> 68, 16 of 8000 to 32000 282 -> 251 (5.2 TB/s).
+// sequence that is just as even and needs neither the scan nor the divisions (29869 tokens, 32:8 heads 30.6
+// us with the list, 28.2 without).  In us, equal parts -> list: 32 heads, 3 sequences of 700 to 20000 tokens
+// 117 -> 88, 13 of 1000 to 9000 208 -> 171, 16 of 8000 to 32000 947 -> 788 (6.7 TB/s); 32:8 heads, 8 of 3000
+// to 16384 69 -> 63, 16 of 8000 to 32000 237 -> 214 (6.1 TB/s).
 template <bool kList>
 struct DenseWalk {
   DenseList list;

@@ -94,7 +94,8 @@ int adamas_hadamard(const void* x, void* out, uint64_t n_rows, float scale, adam
  *   ADAMAS_F_BF16 : bfloat16 in place of fp16 wherever it reads or writes float data (q, k, v, h,
  *                   the KV cache, the attention output); codes, distances, selections and all
  *                   arithmetic (fp32) are unchanged;
- *   ADAMAS_F_HND  : the other page layout of the KV cache (see the flag).
+ *   ADAMAS_F_HND  : the other page layout of the KV cache (see the flag);
+ *   ADAMAS_F_CODES_CACHED : a hint for the decode step, its two halves and the layer step (see the flag).
  * The un-suffixed entry points are flags = 0; the append entry points have taken flags all along;
  * estimate and top-k see neither float data nor KV pages.  Flags an entry point does not know give
  * ADAMAS_E_BADARG.  The reference dispatches fp16 only
@@ -225,7 +226,7 @@ size_t adamas_workspace_bytes(uint32_t batch, uint32_t num_heads, uint32_t max_s
  *   sel_idx != NULL : S(b,h) = { sel_idx[(b*num_heads+h)*sel_stride + i], i < n_sel, entry >= 0 }
  *                     united with the current token seq_lens[b]-1 (logical token positions).
  *   sel_idx == NULL : S(b,h) = all tokens 0 .. seq_lens[b]-1 (dense decode attention).
- * q, out [batch][num_heads][128] fp16.
+ * q, out [batch][num_heads][128] fp16.  Sizes that need no split take any workspace, NULL included.
  * Replaces: BatchDecodeWithPagedKVCachePyTorchWrapper::Forward, adamas/ops/csrc/bsk_ops.h:95-124
  * (kernel BatchDecodeWithPagedKVCacheKernel, kernels/include/decode/decode_attn.cuh:482-702, and the
  * BeginForward/EndForward planning of kernels/include/decode/decode_handler.cuh:73-136, which has no
