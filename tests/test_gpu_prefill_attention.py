@@ -74,6 +74,25 @@ def test_prefill_attention_edges(gpu_device, n, past, kv_heads, page, dtype, lay
     assert bool((err <= bound).all()), f"error {float((err - bound).max()):.3e} above the bound"
 
 
+@pytest.mark.parametrize("n,past,kv_heads,page,dtype,layout", [
+    (130, 70, 32, 8, torch.float16, 0),       # the smallest page with one address for a wave's eight rows
+    (130, 70, 8, 4, torch.bfloat16, 1),       # the largest power of two below it
+    (100, 301, 8, 24, torch.float16, 0),      # a multiple of eight that is no power of two
+    (65, 190, 32, 128, torch.bfloat16, 1),    # a page of two tiles, the second tile not begun
+    (4230, 0, 8, 16, torch.float16, 0),       # 67 tiles: the page ids a wave keeps are looked up again
+    (4230, 0, 8, 1, torch.bfloat16, 0),
+])
+def test_prefill_attention_page_sizes(gpu_device, n, past, kv_heads, page, dtype, layout):
+    ctrl, q, k, v = _cache(gpu_device, n, past, kv_heads, page, dtype, layout, False, n + page)
+    if n > 4096:
+        assert _lib.load().adamas_prefill_workspace_bytes(n, past, 32, kv_heads) == 0, "one range of all tiles"
+    ref, mag = _reference(q, k, v, past)
+    # as at the edges above
+    u = 2.0 ** (-11 if dtype == torch.float16 else -8)
+    bound = u * (mag + ref.abs()) + 2.0 ** -14 * mag + 2.0 ** -25 * v.double().abs().sum(0).max()
+    assert bool(((U.prefill_forward(q, ctrl, 0).double() - ref).abs() <= bound).all())
+
+
 def test_prefill_attention_of_a_misaligned_view(gpu_device):
     ctrl, q, k, v = _cache(gpu_device, 40, 0, 32, 16, torch.float16, 0, False, 3)
     flat = torch.empty(q.numel() + 1, dtype=q.dtype, device=gpu_device)
