@@ -148,7 +148,7 @@ __device__ __forceinline__ uint32_t wave_query_code(const WaveRopeLoads& r, int 
 // kShare = 4 (grouped queries, groups of a multiple of four heads): a lane scores the codes it loads
 // for the four query heads that share them.  One load instruction then covers 16 tokens instead of
 // four, and the bit planes of a key are made once instead of four times.
-// kStreamCodes: the codes are more than the caches keep from one token to the next, read past them.
+// kStreamCodes: the codes are more than the caches keep from one token to the next, read past them (est_stream).
 template <int kPage, int kPasses, bool kPartial, bool kHist = false, int kHeads = kFusedHeads,
           bool kFromQkv = false, int kShare = 1, bool kStreamCodes = false>
 __global__ __launch_bounds__(kHeads * kWave) void estimate_select_kernel(
@@ -1211,16 +1211,20 @@ static bool est_share(uint32_t batch, int est_heads, uint32_t num_heads, uint32_
   return num_heads / num_kv_heads % 4 == 0 && (batch > 1 || est_heads == kFusedHeads);
 }
 
-// Whether the wide estimator reads the codes past the caches.  Where the caches cannot keep them until the
-// next step that saves what they evict; where they can, a full chip loses nothing by it, but workgroups that
-// leave CUs idle wait for memory each time.  In us per step with the layers in turn, through / past the
-// caches (the last level holds 256 MB): 32 heads, 65536 tokens, 2 layers (134 MB) 20.2 / 19.3, 8 layers 23.8 /
-// 21.0; 8 heads (64 workgroups), 131072 tokens, 4 layers (134 MB) 20.6 / 22.5, 12 layers 25.3 / 23.4; 16
-// heads, 131072 tokens, 3 layers 23.2 / 24.3, 8 layers 27.6 / 24.9.  The narrow, shared and histogram
-// instances read through the caches.
+// Whether the estimator reads the codes past the caches.  Where the caches cannot keep them until the next
+// step that saves what they evict; where they can (the last level holds 256 MB, the caller says so with
+// ADAMAS_F_CODES_CACHED), workgroups wait for memory each time.  In us per layer with the layers in turn,
+// through / past the caches.  Selection: 32 heads, 16 sequences of 8192 to 32768 tokens, 1 layer (335 MB of codes)
+// 88.2 / 80.1, 2 layers 87.0 / 77.0; 8 of 1500 to 7000, 4 layers (139 MB) 22.8 / 23.0, 8 layers 24.0 / 21.9; one
+// sequence of 4096, 8 layers (34 MB) 12.8 / 12.8, 80 layers 14.0 / 12.9; 8 heads, 131072, 7 layers (235 MB) 23.2 / 25.7, 9
+// layers 27.2 / 25.6.  Histograms, budget 512: 16 of 4000 to 16000, 1 layer (164 MB) 82.6 / 81.9, 2 layers
+// 88.8 / 81.6; 65536 tokens, 4 layers (268 MB) 31.9 / 32.7, 8 layers 32.6 / 31.7.
+// A full chip of wide workgroups loses nothing by it in a step (65536 tokens, 2 layers 20.2 / 19.3).  The
+// shared instances read 128 or 256 bytes per token, lines that other workgroups want too, and always
+// lose: 32:8 heads, 16 of 8192 to 32768, 2 layers 51.0 / 56.9.
 static bool est_stream(uint32_t flags, int est_heads, bool share, uint32_t workgroups) {
-  return est_heads == kFusedHeads && !share &&
-         (workgroups >= kStepWorkgroups || !(flags & ADAMAS_F_CODES_CACHED));
+  return !share && ((est_heads == kFusedHeads && workgroups >= kStepWorkgroups) ||
+                    !(flags & ADAMAS_F_CODES_CACHED));
 }
 
 static StepGeom geom_of(const StepPlan& p) {
@@ -1282,17 +1286,21 @@ static int step_candidates_impl(const void* q_code, const void* code_data,
   } else {                                                                    \
     ADAMAS_LAUNCH_ESTSEL_Q(PG, PASSES, PARTIAL, HEADS, false, SHARE, STREAM); \
   }
-#define ADAMAS_LAUNCH_ESTSEL(PG, PASSES, PARTIAL)              \
-  if (share && est_heads == 4) {                               \
-    ADAMAS_LAUNCH_ESTSEL_H(PG, PASSES, PARTIAL, 4, 4, false)   \
-  } else if (share) {                                          \
-    ADAMAS_LAUNCH_ESTSEL_H(PG, PASSES, PARTIAL, 8, 4, false)   \
-  } else if (est_heads == 4) {                                 \
-    ADAMAS_LAUNCH_ESTSEL_H(PG, PASSES, PARTIAL, 4, 1, false)   \
-  } else if (stream_codes) {                                   \
-    ADAMAS_LAUNCH_ESTSEL_H(PG, PASSES, PARTIAL, 8, 1, true)    \
-  } else {                                                     \
-    ADAMAS_LAUNCH_ESTSEL_H(PG, PASSES, PARTIAL, 8, 1, false)   \
+#define ADAMAS_LAUNCH_ESTSEL_S(PG, PASSES, PARTIAL, HEADS, SHARE)   \
+  if (stream_codes) {                                               \
+    ADAMAS_LAUNCH_ESTSEL_H(PG, PASSES, PARTIAL, HEADS, SHARE, true)  \
+  } else {                                                          \
+    ADAMAS_LAUNCH_ESTSEL_H(PG, PASSES, PARTIAL, HEADS, SHARE, false) \
+  }
+#define ADAMAS_LAUNCH_ESTSEL(PG, PASSES, PARTIAL)            \
+  if (share && est_heads == 4) {                             \
+    ADAMAS_LAUNCH_ESTSEL_H(PG, PASSES, PARTIAL, 4, 4, false) \
+  } else if (share) {                                        \
+    ADAMAS_LAUNCH_ESTSEL_H(PG, PASSES, PARTIAL, 8, 4, false) \
+  } else if (est_heads == 4) {                               \
+    ADAMAS_LAUNCH_ESTSEL_S(PG, PASSES, PARTIAL, 4, 1)        \
+  } else {                                                   \
+    ADAMAS_LAUNCH_ESTSEL_S(PG, PASSES, PARTIAL, 8, 1)        \
   }
 #define ADAMAS_LAUNCH_ESTSEL_PAGE(PASSES, PARTIAL)   \
   if (page_size == 16) {                             \
@@ -1318,6 +1326,7 @@ static int step_candidates_impl(const void* q_code, const void* code_data,
   }
 #undef ADAMAS_LAUNCH_ESTSEL_PAGE
 #undef ADAMAS_LAUNCH_ESTSEL
+#undef ADAMAS_LAUNCH_ESTSEL_S
 #undef ADAMAS_LAUNCH_ESTSEL_H
 #undef ADAMAS_LAUNCH_ESTSEL_Q
   ADAMAS_RETURN_IF_LAUNCH_FAILED();
@@ -1514,6 +1523,7 @@ extern "C" int adamas_decode_step_f(const void* q, const void* q_code, const voi
                                         2 * ((wide + kStepWorkgroups - 1) / kStepWorkgroups);
     const int est_heads = narrow ? 4 : kFusedHeads;
     const bool share = est_share(batch, est_heads, num_heads, num_kv_heads);
+    const bool stream_codes = !share && !(flags & ADAMAS_F_CODES_CACHED);  // (as in est_stream)
     const dim3 grid(n_chunks, num_heads / est_heads, batch);
     StepGeom hist_geom;
     hist_geom.units_q = chunk_tokens / kStepUnit;
@@ -1523,8 +1533,8 @@ extern "C" int adamas_decode_step_f(const void* q, const void* q_code, const voi
     unsigned char* hist = reinterpret_cast<unsigned char*>(ws + w.hist_off);
     hipStream_t s = static_cast<hipStream_t>(stream);
     uint32_t* rowmap = reinterpret_cast<uint32_t*>(ws + w.rowmap_off);
-#define ADAMAS_LAUNCH_ESTHIST_S(PG, PASSES, HEADS, SHARE)                                               \
-  hipLaunchKernelGGL((estimate_select_kernel<PG, PASSES, false, true, HEADS, false, SHARE>),            \
+#define ADAMAS_LAUNCH_ESTHIST_C(PG, PASSES, HEADS, SHARE, STREAM)                                       \
+  hipLaunchKernelGGL((estimate_select_kernel<PG, PASSES, false, true, HEADS, false, SHARE, STREAM>),    \
                      grid, dim3(HEADS * kWave), 0, s, seq_lens, page_indices,                           \
                      static_cast<const unsigned char*>(code_data),                                      \
                      static_cast<const uint16_t*>(q_code), page_table_stride, hist_geom.units_q,        \
@@ -1532,9 +1542,15 @@ extern "C" int adamas_decode_step_f(const void* q, const void* q_code, const voi
                      page_size, rows_per_page_of(flags, page_size, num_kv_heads), page_indptr,          \
                      static_cast<uint64_t*>(nullptr), hist_geom.kc, static_cast<uint16_t*>(nullptr),    \
                      hist, n_chunks, dist, static_cast<int64_t>(w.dist_stride), rowmap)
+#define ADAMAS_LAUNCH_ESTHIST_S(PG, PASSES, HEADS, SHARE)          \
+  if (stream_codes) {                                              \
+    ADAMAS_LAUNCH_ESTHIST_C(PG, PASSES, HEADS, SHARE, true);       \
+  } else {                                                         \
+    ADAMAS_LAUNCH_ESTHIST_C(PG, PASSES, HEADS, SHARE, false);      \
+  }
 #define ADAMAS_LAUNCH_ESTHIST_P(PG, PASSES, HEADS)      \
   if (share) {                                          \
-    ADAMAS_LAUNCH_ESTHIST_S(PG, PASSES, HEADS, 4);      \
+    ADAMAS_LAUNCH_ESTHIST_C(PG, PASSES, HEADS, 4, false); \
   } else {                                              \
     ADAMAS_LAUNCH_ESTHIST_S(PG, PASSES, HEADS, 1);      \
   }

@@ -107,3 +107,33 @@ def test_step_reads_codes_through_and_past_the_caches(gpu_device, heads, length,
     U.decode_topk(U.decode_estimate(q_code, ctrl, 0), ctrl)
     want = ctrl.topk_dindices_buffer.sort(dim=1).values
     assert torch.equal(got[0][1].sort(dim=1).values, want)
+
+
+@pytest.mark.parametrize("lens,budget,page", [
+    ([700, 5000, 1, 513, 2049], 100, 16),     # selection, narrow workgroups of a batch
+    ([9000], 64, 1),                          # selection, narrow workgroups of one sequence
+    ([700, 5000, 1, 513, 2049], 600, 16),     # histograms
+    ([16385], 300, 32),
+])
+def test_step_of_narrow_workgroups_reads_codes_through_and_past_the_caches(gpu_device, lens, budget, page, monkeypatch):
+    """Both instances give the same bits, and the selection of the stand-alone operators."""
+    from adamas_amd.utils import controller as C
+    dev = gpu_device
+    g = torch.Generator(device=dev).manual_seed(sum(lens))
+    n = len(lens)
+    ctrl = U.InferenceController(1, 32, 128, page, budget, max(lens) + 1, torch.float16, dev, batch_size=n)
+    ctrl.pool.kv.copy_(torch.randn(ctrl.pool.kv.shape, generator=g, device=dev))
+    ctrl.pool.codes.copy_(torch.randint(-32768, 32768, ctrl.pool.codes.shape, generator=g, device=dev))
+    ctrl.prepare_hadamard(lens)
+    ctrl.prepare_hadamard(1)
+    ctrl.begin_forward(1)
+    q, k, v = (torch.randn(n, 32, 128, generator=g, device=dev).half() for _ in range(3))
+    q_code = U.append_kvh(k, v, None, ctrl, 0, q=q)
+    got = []
+    for limit in (0, 1 << 40):
+        monkeypatch.setattr(C, "CODES_CACHED_BYTES", limit)
+        o, sel = U.decode_step(q, q_code, ctrl, 0, return_indices=True)
+        got.append((o, sel.clone()))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    U.decode_topk(U.decode_estimate(q_code, ctrl, 0), ctrl)
+    assert torch.equal(got[0][1].sort(dim=1).values, ctrl.topk_dindices_buffer.sort(dim=1).values)
