@@ -160,4 +160,5 @@ def ptr(t) -> int | None:
 
 
 def current_stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    """The current stream of the current device (2.7 us less than by way of a torch.cuda.Stream object)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())

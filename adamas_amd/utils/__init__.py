@@ -136,8 +136,7 @@ def append_kvh(k: torch.Tensor, v: torch.Tensor, h: Optional[torch.Tensor],
     if nh != c.num_kv_heads or d != c.head_dim:
         raise RuntimeError("k does not match the controller's num_kv_heads/head_dim")
     nq = c.num_heads   # query heads (= nh unless grouped-query attention)
-    kv = c.pool.kv[layer_idx]
-    codes = c.pool.codes[layer_idx]
+    kv, codes = c.pool.kv_address(layer_idx), c.pool.codes_address(layer_idx)
     stream = _lib.current_stream()
     # decode: h stacks Hadamard(q) on Hadamard(k) (twice the rows of k), or q is given for the fused kernel
     is_decode = q is not None or (h is not None and (
@@ -153,7 +152,7 @@ def append_kvh(k: torch.Tensor, v: torch.Tensor, h: Optional[torch.Tensor],
         if n > total:
             raise RuntimeError("prepare_hadamard must reserve the tokens before append_kvh")
         rc = lib.adamas_append_prefill(k.data_ptr(), v.data_ptr(), _lib.ptr(h), n, total - n,
-                                       kv.data_ptr(), codes.data_ptr(), c.seqs.table_ptr(seq_idx),
+                                       kv, codes, c.seqs.table_ptr(seq_idx),
                                        c.seqs.max_pages, nh, d, c.page_size, c.hadamard_scale,
                                        c.code_flags, stream)
         _lib.check(rc, "adamas_append_prefill")
@@ -173,7 +172,7 @@ def append_kvh(k: torch.Tensor, v: torch.Tensor, h: Optional[torch.Tensor],
         raise RuntimeError("prepare_hadamard must reserve the token before append_kvh")
     o = torch.empty((n, nq, d // 8), dtype=torch.int16, device=k.device)
     rc = lib.adamas_append_decode(_lib.ptr(q), k.data_ptr(), v.data_ptr(), _lib.ptr(h), o.data_ptr(),
-                                  kv.data_ptr(), codes.data_ptr(), c.seqs.table_dev.data_ptr(),
+                                  kv, codes, c.seqs.table_dev.data_ptr(),
                                   c.seqs.indptr_dev.data_ptr(), c.seqs.seq_lens_dev.data_ptr(), n,
                                   nq, nh, d, c.page_size, c.hadamard_scale, c.code_flags, stream)
     _lib.check(rc, "adamas_append_decode")
@@ -197,7 +196,7 @@ def decode_estimate(q: torch.Tensor, iController: InferenceController, layer_idx
         raise RuntimeError("decode_estimate needs at least one past token")
     stride = (lmax - 1 + 7) // 8 * 8
     buf = torch.empty((c.batch_size, c.num_heads, stride), dtype=torch.float16, device=q.device)
-    rc = _lib.load().adamas_estimate(q.data_ptr(), c.pool.codes[layer_idx].data_ptr(),
+    rc = _lib.load().adamas_estimate(q.data_ptr(), c.pool.codes_address(layer_idx),
                                      c.seqs.table_dev.data_ptr(), c.seqs.indptr_dev.data_ptr(),
                                      c.seqs.seq_lens_dev.data_ptr(), buf.data_ptr(),
                                      c.num_heads * stride, stride, _lib.DIST_FP16, c.batch_size,
@@ -291,7 +290,7 @@ def decode_sparse_attn(q: torch.Tensor, iController: InferenceController, layer_
         sel_ptr, stride, n_sel = topk_indices.data_ptr(), topk_indices.stride(0), topk_indices.shape[1]
     ws = c.workspace(c.inference_page_budget or 1)
     rc = _lib.load().adamas_sparse_decode_f(
-        q.data_ptr(), c.pool.kv[layer_idx].data_ptr(), c.seqs.table_dev.data_ptr(),
+        q.data_ptr(), c.pool.kv_address(layer_idx), c.seqs.table_dev.data_ptr(),
         c.seqs.indptr_dev.data_ptr(), c.seqs.seq_lens_dev.data_ptr(), sel_ptr, stride, n_sel,
         o.data_ptr(), ws.data_ptr(), ws.numel(), c.batch_size, c.num_heads, c.num_kv_heads,
         c.head_dim, c.page_size, 1.0 / math.sqrt(c.head_dim), c.max_len_now, c.kv_flags,
@@ -424,8 +423,8 @@ def decode_step(q: torch.Tensor, q_code: torch.Tensor, iController: InferenceCon
     ws = c.workspace(budget)
     sel = c.topk_dindices_buffer if return_indices else None
     rc = _lib.load().adamas_decode_step_f(
-        q.data_ptr(), q_code.data_ptr(), c.pool.kv[layer_idx].data_ptr(),
-        c.pool.codes[layer_idx].data_ptr(), c.seqs.table_dev.data_ptr(),
+        q.data_ptr(), q_code.data_ptr(), c.pool.kv_address(layer_idx),
+        c.pool.codes_address(layer_idx), c.seqs.table_dev.data_ptr(),
         c.seqs.indptr_dev.data_ptr(), c.seqs.seq_lens_dev.data_ptr(), budget, o.data_ptr(),
         _lib.ptr(sel), ws.data_ptr(), ws.numel(), c.batch_size, c.num_heads, c.num_kv_heads,
         c.head_dim, c.page_size, 1.0 / math.sqrt(c.head_dim), c.max_len_now, c.seqs.max_pages,
@@ -519,6 +518,8 @@ def prefill_forward(q: torch.Tensor, iController: InferenceController, layer_idx
 def _prefill(q: torch.Tensor, c: InferenceController, layer_idx: int, length: int,
              device: int) -> torch.Tensor:
     """The kernel behind prefill_forward, on q's device, which is the current one."""
+    if layer_idx < 0:   # (as KvCache.buf_layer)
+        raise IndexError("layer index out of range")
     n = q.shape[0]
     if q.data_ptr() % 16:   # a view into the middle of something: the kernel reads 128 bits at a time
         q = q.clone()
@@ -666,7 +667,7 @@ def rope_append_decode(qkv: torch.Tensor, cos_table: torch.Tensor, sin_table: to
     q_code = torch.empty((n, nq, 16), dtype=torch.int16, device=qkv.device)
     rc = _lib.load().adamas_rope_append_decode(
         qkv.data_ptr(), cos_table.data_ptr(), sin_table.data_ptr(), q.data_ptr(), q_code.data_ptr(),
-        c.pool.kv[layer_idx].data_ptr(), c.pool.codes[layer_idx].data_ptr(),
+        c.pool.kv_address(layer_idx), c.pool.codes_address(layer_idx),
         c.seqs.table_dev.data_ptr(), c.seqs.indptr_dev.data_ptr(), c.seqs.seq_lens_dev.data_ptr(), n,
         nq, nkv, 128, c.page_size, c.hadamard_scale, c.code_flags, _lib.current_stream())
     _lib.check(rc, "adamas_rope_append_decode")
@@ -762,8 +763,8 @@ def decode_layer_step(qkv: torch.Tensor, cos_table: torch.Tensor, sin_table: tor
     ws = c.workspace(budget)
     sel = c.topk_dindices_buffer if return_indices else None
     rc = _lib.load().adamas_decode_layer_step(
-        qkv.data_ptr(), cos_table.data_ptr(), sin_table.data_ptr(), c.pool.kv[layer_idx].data_ptr(),
-        c.pool.codes[layer_idx].data_ptr(), c.seqs.table_dev.data_ptr(), c.seqs.indptr_dev.data_ptr(),
+        qkv.data_ptr(), cos_table.data_ptr(), sin_table.data_ptr(), c.pool.kv_address(layer_idx),
+        c.pool.codes_address(layer_idx), c.seqs.table_dev.data_ptr(), c.seqs.indptr_dev.data_ptr(),
         c.seqs.seq_lens_dev.data_ptr(), budget, o.data_ptr(), _lib.ptr(sel), ws.data_ptr(), ws.numel(),
         n, nq, nkv, 128, c.page_size, 1.0 / math.sqrt(c.head_dim), c.max_len_now, c.seqs.max_pages,
         c.hadamard_scale, c.code_flags | c.codes_hint, _lib.current_stream())

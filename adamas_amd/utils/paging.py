@@ -32,6 +32,14 @@ class TensorLayout:
     FORMAT2STR = {0: "NHD", 1: "HND"}
 
 
+def _row_address(t: torch.Tensor, i: int) -> int:
+    """t[i].data_ptr() without making the view."""
+    n = t.shape[0]
+    if not -n <= i < n:
+        raise IndexError(f"index {i} is out of bounds for dimension 0 with size {n}")
+    return t.data_ptr() + (i + n if i < 0 else i) * t.stride(0) * t.element_size()
+
+
 class PagePool:
     """Physical pages of every layer.
 
@@ -61,6 +69,14 @@ class PagePool:
             raise ValueError("page_order must be a permutation of range(num_pages)")
         self._free: List[int] = order[::-1]  # pop() hands pages out in `order`
         self._busy = set()
+
+    def kv_address(self, layer: int) -> int:
+        """Address of kv[layer] (1 us less than through a view of it)."""
+        return _row_address(self.kv, layer)
+
+    def codes_address(self, layer: int) -> int:
+        """Address of codes[layer]."""
+        return _row_address(self.codes, layer)
 
     @property
     def num_free_pages(self) -> int:

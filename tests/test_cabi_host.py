@@ -373,3 +373,16 @@ def test_codes_cached_hint():
     assert lib.adamas_decode_step_f(*step, 2 * _lib.F_CODES_CACHED, None) == -1
     assert lib.adamas_sparse_decode_f(*[16] * 5, None, 0, 0, 16, None, 0, 1, 32, 32, 64, 16, 1.0, 100,
                                       _lib.F_CODES_CACHED, None) == -1
+
+
+def test_layer_addresses():
+    """The addresses handed to the library are those of the layers' views, for the same indices."""
+    c = _ctrl(num_layers=3)
+    for layer in range(-3, 3):
+        assert c.pool.kv_address(layer) == c.pool.kv[layer].data_ptr()
+        assert c.pool.codes_address(layer) == c.pool.codes[layer].data_ptr()
+    for layer in (-4, 3):
+        with pytest.raises(IndexError):
+            c.pool.kv_address(layer)
+        with pytest.raises(IndexError):
+            c.pool.codes_address(layer)

@@ -201,3 +201,11 @@ def test_module_call_order_prefill_then_decode(gpu_device, budget):
         assert np.abs(qd.astype(np.float64) - rq[t]).max() <= 8e-3
         step = O.decode_step(qd, kc, vc, min(budget, t + 1))
         assert np.abs(T.np16(o[0]).astype(np.float64) - step["out"]).max() <= ATTN_TOL_ABS, t
+
+
+def test_operators_launch_on_the_current_stream(gpu_device):
+    from adamas_amd import _lib
+    side = torch.cuda.Stream(gpu_device)
+    for stream in (torch.cuda.current_stream(), side):
+        with torch.cuda.stream(stream):
+            assert _lib.current_stream() == torch.cuda.current_stream().cuda_stream == stream.cuda_stream
