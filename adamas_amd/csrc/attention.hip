@@ -21,11 +21,12 @@ constexpr int kTile = 8;             // rows per group per tile, at most
 // single workgroup per head takes 25 us for 1024 rows), a group finishes sooner the fewer rows it
 // has to ask for, and publishing a partial result costs about a microsecond.  Hence: up to 64 rows
 // 16 groups of 4, up to 128 rows 32 groups of 4 (one split, no merge, no workspace); up to 512 rows
-// splits of 64 rows (32 groups of 2, at most 8 splits); up to 2048 rows splits of 128 (64 groups of
-// 2, at most 16); beyond that splits of 256 (64 groups of 4).  Measured at 32 heads, rows = 128 /
+// splits of 64 rows (32 groups of 2, at most 8 splits); up to 1408 rows splits of 128 (64 groups of
+// 2, at most 11); beyond that, and where more workgroups than run at once would come of it, four rows in flight
+// (row_launch).  Measured at 32 heads, rows = 128 /
 // 256 / 512 / 1024 / 2048 / 4096, in us: 5.8 / 6.5 / 7.4 / 9.3 / 13.5 / 18.8 (with 16 groups of 8
 // rows and splits of 128 rows up to 1024 rows, 32 groups of 8 beyond: 7.5 / 9.5 / 10.1 / 12.4 / 15.8
-// / 20.6).
+// / 20.6); 2048 rows four in flight 12.5.
 constexpr uint32_t kDeferredMergeSplits = 24;  // splits from which the partials get a merge launch
 // (measured at 32768 tokens, 32 heads: 16 splits 14.7 us merged inside the launch, 15.8 us with a merge
 // launch; 32 splits 26.6 against 22.5 us)
@@ -71,14 +72,20 @@ __global__ __launch_bounds__(kThreads) void sparse_decode_kernel(
   kv.seq_len = seq_len;
 
   SoftmaxState st;
-  // (token positions through the page table: branching around unused entries measured faster
-  // here than loading always, 7.9 against 8.0 us at 128 rows)
-  attend_rows<kGroups, kTileRows, false, kBf16>(kv, qf, g, row_begin, row_end,
-                              [&](uint32_t r) __attribute__((always_inline)) -> int32_t {
-                                if (dense) return static_cast<int32_t>(r);
-                                return (r < n_sel) ? sel[r] : seq_len - 1;
-                              },
-                              st);
+  // (token positions through the page table: branching around unused entries measured faster for lists
+  // than loading always, 7.9 against 8.0 us at 128 rows, and for all positions with four rows per group, 16.5
+  // against 17.5 us at 4000; with two, loading always takes 3 % off: 1000 positions 8.8 -> 8.5 us)
+  if (kTileRows == 2 && dense)  // (uniform)
+    attend_rows<kGroups, kTileRows, false, kBf16, true>(
+        kv, qf, g, row_begin, row_end,
+        [&](uint32_t r) __attribute__((always_inline)) -> int32_t { return static_cast<int32_t>(r); }, st);
+  else
+    attend_rows<kGroups, kTileRows, false, kBf16>(kv, qf, g, row_begin, row_end,
+                                [&](uint32_t r) __attribute__((always_inline)) -> int32_t {
+                                  if (dense) return static_cast<int32_t>(r);
+                                  return (r < n_sel) ? sel[r] : seq_len - 1;
+                                },
+                                st);
 
   float M, L, O;
   merge_groups<kGroups>(st, g, c, tid, sh.merge, M, L, O);
@@ -974,6 +981,31 @@ extern "C" size_t adamas_workspace_bytes(uint32_t batch, uint32_t num_heads, uin
   return workspace_layout(batch, num_heads, max_seq_len, budget).total;
 }
 
+// Workgroups of sparse_decode_kernel for `n_rows` rows each of `heads` (sequence, query head) pairs: threads, rows
+// in flight per group of 16 lanes, rows per round and rounds' worth of workgroups (see the rule at kTile).  Two
+// rows in flight instead of four give twice the workgroups, half the rows each: better as long as they all
+// run at once and the merge of a head stays short.  Two / four, 32:32 heads, us a launch with its append:
+// 2000 positions 14.4 / 13.4, 1400 12.3 / 12.3, 1000 10.9 / 11.3; 3 sequences of 600 to 1500 21.6 / 17.9, 16 of 150 to
+// 250 21.9 / 17.3, 2 of 600 to 1000 13.2 / 13.4; 32:8 heads, 8 of 150 to 250 12.4 / 13.0.
+struct RowLaunch {
+  uint32_t threads, tile, rows_per_iter;
+  uint64_t workgroups;
+  bool one_round;  // all of them run at once: 2048 threads per CU
+};
+static RowLaunch row_launch(uint64_t heads, uint32_t n_rows) {
+  RowLaunch r;
+  r.threads = n_rows <= 64 ? 256u : n_rows <= 512 ? 512u : 1024u;
+  auto with_tile = [&](uint32_t tile) {
+    r.tile = tile;
+    r.rows_per_iter = r.threads / 16u * tile;
+    r.workgroups = heads * ((n_rows + r.rows_per_iter - 1) / r.rows_per_iter);
+    r.one_round = r.workgroups * r.threads <= 256u * 2048u;
+  };
+  with_tile(n_rows <= 128 || n_rows > 1408 ? 4u : 2u);
+  if (!r.one_round) with_tile(4u);
+  return r;
+}
+
 // Whether attention over all tokens goes through the kernel for row lists (sel_idx == nullptr: the rows are
 // the positions 0 .. seq_len - 1) instead of the dense kernels, which take eight heads at once and leave CUs
 // idle where there is little to do.  One sequence: up to 4096 tokens, 2048 where the row kernel would read a
@@ -984,7 +1016,9 @@ extern "C" size_t adamas_workspace_bytes(uint32_t batch, uint32_t num_heads, uin
 //     32:8 heads 5.3 / 6.4, 32 8.6 / 6.5; with two heads per group, or more than a matrix-core tile takes, 16
 //     of 128 9.9 / 10.4 and 7.6 / 9.2 (32:16, 32:2), 32 14.7 / 13.3 and 11.0 / 9.1.
 //   - Beyond, 32:32 heads: 32 sequences of 160 23.9 / 24.6, 64 50.3 / 36.6, 4 of 1000 19.6 / 20.5, 8 33.4 /
-//     30.1; 32:8 heads: 8 of 256 9.9 / 13.8, 16 18.6 / 15.2, 2 of 1000 10.0 / 13.6, 4 16.8 / 14.8.  A single
+//     30.1; 32:8 heads: 8 of 256 9.9 / 13.8, 16 18.6 / 15.2, 2 of 1000 10.0 / 13.6.  Groups of more than 256 tokens
+//     also as long as the row kernel's workgroups all run at once (launch with its append): 32:8 heads, 2 of 2000 14.9 /
+//     16.1, 4 of 1000 15.2 / 17.6, 8 of 500 15.3 / 17.6, but 3 of 1300 21.6 / 17.6, 12 of 340 20.0 / 17.6.  A single
 //     group of eight heads fills fewer workgroups: 32 of 1000 32.7 / 37.5 at 8:8, 64 70.9 / 63.3; 16 17.3 /
 //     18.6 at 8:4, 32 29.8 / 20.7.
 static bool dense_as_rows(uint32_t batch, uint32_t num_heads, uint32_t group, uint32_t max_seq_len) {
@@ -998,7 +1032,8 @@ static bool dense_as_rows(uint32_t batch, uint32_t num_heads, uint32_t group, ui
     limit = group == 1 ? 163840u : 81920u;
     if (num_heads == kDenseHeads && group <= 2) limit *= 2u;
   }
-  return static_cast<uint64_t>(batch) * max_seq_len * num_heads <= limit;
+  const uint64_t heads = static_cast<uint64_t>(batch) * num_heads;
+  return heads * max_seq_len <= limit || (group > 1 && max_seq_len > 256 && row_launch(heads, max_seq_len).one_round);
 }
 
 static int sparse_decode_impl(const void* q, const void* kv_data, const int32_t* page_indices,
@@ -1135,9 +1170,8 @@ static int sparse_decode_impl(const void* q, const void* kv_data, const int32_t*
   const uint32_t n_rows = sel_idx ? n_sel + 1u : max_seq_len;
   // one round of loads per split (see the rule at kTile; up to 128 rows that is a single
   // split, which needs no workspace), more where that would take more than kMaxSplits splits
-  const uint32_t threads = n_rows <= 64 ? 256u : n_rows <= 512 ? 512u : 1024u;
-  const uint32_t tile = n_rows <= 128 ? 4u : n_rows <= 2048 ? 2u : 4u;
-  const uint32_t rows_per_iter = threads / 16u * tile;
+  const RowLaunch rl = row_launch(static_cast<uint64_t>(batch) * num_heads, n_rows);
+  const uint32_t threads = rl.threads, tile = rl.tile, rows_per_iter = rl.rows_per_iter;
   uint32_t rows_per_split = rows_per_iter;
   uint32_t n_split = (n_rows + rows_per_split - 1) / rows_per_split;
   if (n_split > kMaxSplits) {

@@ -54,6 +54,20 @@ def test_dense_attention_of_ragged_batches(gpu_device, lens, kv_heads, page, dty
         assert bool(((o[b].double() - ref).abs() <= bound).all()), (b, n)
 
 
+@pytest.mark.parametrize("lens,kv_heads,page,dtype,layout", [
+    ([1408], 32, 16, torch.float16, 0),               # two rows in flight, the last length of them
+    ([1409], 8, 1, torch.bfloat16, 1),                # four
+    ([1000, 1, 999, 641], 8, 16, torch.float16, 0),   # four sequences whose workgroups just run at once
+    ([1025, 1, 999, 641], 8, 16, torch.float16, 0),   # and no longer
+    ([512, 500, 129, 3, 257, 511, 64, 65], 4, 16, torch.bfloat16, 0),
+    ([513, 500, 129, 3, 257, 511, 64, 65], 16, 32, torch.float16, 1),
+    ([256] * 8, 32, 16, torch.float16, 0),
+    ([250, 193] * 8, 32, 16, torch.bfloat16, 0),      # more than run at once: four rows in flight
+])
+def test_dense_attention_at_the_edges_of_the_row_kernel(gpu_device, lens, kv_heads, page, dtype, layout):
+    test_dense_attention_of_ragged_batches(gpu_device, lens, kv_heads, page, dtype, layout)
+
+
 @pytest.mark.parametrize("lens,kv_heads,dtype", [
     ([2000, 1777], 8, torch.float16), ([2000, 1777], 4, torch.float16), ([1900] * 4, 16, torch.float16),
     ([2000, 1777], 8, torch.bfloat16), ([9000], 8, torch.float16)])
