@@ -890,14 +890,21 @@ constexpr uint32_t kHsaMaxTokens = kHsaMaxSlab * 32;             // 32 slabs per
 // workgroup where the length allows it, and never more than 16 slabs for the sake of the rows
 // (beyond that the merge inside the launch costs more than the shorter gather saves).  Measured
 // against slabs of 4096 tokens throughout: 8192 tokens, budget 4096: 41.0 -> 24.8 us; 16384 / 1024:
-// 20.1 -> 18.4; 32768 / 1024: 23.3 -> 22.7; a target of 32 rows or a cap of 32 slabs is slower.
-inline int hsa_items(uint32_t max_seq_len, uint32_t budget) {
+// 20.1 -> 18.4; 32768 / 1024: 23.3 -> 22.7; a target of 32 rows or a cap of 32 slabs is slower.  In
+// batches slabs of 2048 tokens are taken where those of 1024 would not all run at once (seven fit the LDS of a
+// CU): each sums the chunk rows of its head once more.  1024 / 2048 / 4096 tokens, us a layer at 32:32 and 32:8
+// heads: 16 sequences of 2000 to 7500, budget 512, 57.5 / 55.2 / 55.5 and 49.4 / 46.9 / 47.2; 8 of 4000 to 15000, 3000,
+// 116.6 / 110.0 / 107.2 and 91.5 / 87.7 / 88.7; 10 of 5000 to 12000, 2000, 104.2 / 103.4 / 114.2 and 80.6 / 82.0 / 92.8;
+// with fewer workgroups, 2 of 3000 to 6000, 600, 20.4 / 22.4 / 22.8 and 20.0 / 21.9 / 22.6.
+constexpr uint64_t kHsaWorkgroups = 7 * 256;
+inline int hsa_items(uint32_t max_seq_len, uint32_t budget, uint64_t heads) {
   const uint32_t n = max_seq_len > 1 ? max_seq_len - 1 : 1;
   const uint32_t most =
       std::max((n + kHsaMaxSlab - 1) / kHsaMaxSlab, std::min(16u, (budget + 63u) / 64u));
   int items = kHsaMaxItems;
   while (items > 4 && (n + kHsaThreads * (items / 2) - 1) / (kHsaThreads * (items / 2)) <= most)
     items /= 2;
+  if (items == 4 && heads * ((n + kHsaThreads * 4 - 1) / (kHsaThreads * 4)) > kHsaWorkgroups) items = 8;
   return items;
 }
 
@@ -1578,7 +1585,7 @@ extern "C" int adamas_decode_step_f(const void* q, const void* q_code, const voi
     ADAMAS_RETURN_IF_LAUNCH_FAILED();
     // selection from the histograms and attention over the selected rows, one launch
     const bool bf16 = (flags & ADAMAS_F_BF16) != 0, hnd = (flags & ADAMAS_F_HND) != 0;
-    int items = hsa_items(max_seq_len, budget);
+    int items = hsa_items(max_seq_len, budget, static_cast<uint64_t>(batch) * num_heads);
     while (kHsaThreads * static_cast<uint32_t>(items) < chunk_tokens) items *= 2;  // slabs of whole chunks
     const uint32_t slab_tokens = kHsaThreads * static_cast<uint32_t>(items);
     const dim3 hgrid(batch * num_heads, (max_seq_len - 1 + slab_tokens - 1) / slab_tokens);

@@ -137,3 +137,10 @@ def test_step_of_narrow_workgroups_reads_codes_through_and_past_the_caches(gpu_d
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
     U.decode_topk(U.decode_estimate(q_code, ctrl, 0), ctrl)
     assert torch.equal(got[0][1].sort(dim=1).values, ctrl.topk_dindices_buffer.sort(dim=1).values)
+
+
+@pytest.mark.parametrize("longest,kv_heads,layout", [(3072, 32, 0), (3074, 8, 1), (4097, 32, 0)])
+def test_step_of_more_slabs_than_run_at_once(gpu_device, longest, kv_heads, layout):
+    """512 (sequence, head) pairs: slabs of 1024 tokens up to 3073, of 2048 beyond."""
+    lens = [longest] + [2 + (613 * i) % (longest - 2) for i in range(15)]
+    _check(gpu_device, lens, 600, 16, kv_heads, torch.float16, layout)
