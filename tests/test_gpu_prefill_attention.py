@@ -79,6 +79,10 @@ def test_prefill_attention_edges(gpu_device, n, past, kv_heads, page, dtype, lay
     (130, 70, 8, 4, torch.bfloat16, 1),       # the largest power of two below it
     (100, 301, 8, 24, torch.float16, 0),      # a multiple of eight that is no power of two
     (65, 190, 32, 128, torch.bfloat16, 1),    # a page of two tiles, the second tile not begun
+    (128, 300, 32, 16, torch.float16, 0),     # 128 stacked rows: the last call of eight waves
+    (129, 300, 32, 16, torch.bfloat16, 1),    # four waves, one row in the second workgroup
+    (50, 2510, 8, 16, torch.float16, 0),      # 2560 tokens: the longest call of four waves
+    (50, 2511, 8, 16, torch.bfloat16, 0),     # eight
     (4230, 0, 8, 16, torch.float16, 0),       # 67 tiles: the page ids a wave keeps are looked up again
     (4230, 0, 8, 1, torch.bfloat16, 0),
 ])
