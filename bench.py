@@ -113,7 +113,7 @@ def estimator_instance(_lib, page_size: int, heads: int, batch: int, max_seq_len
     share = 4 if grouped and (batch > 1 or p["heads"] == 8) else 1
     return (f"estimate_select_kernel<{16 if page_size == 16 else 0}, {p['passes']}, "
             f"{flag(p['partial'])}, false, {p['heads']}, false, {share}, "
-            f"{flag(p['heads'] == 8 and share == 1)}>")
+            f"{flag(share == 1)}>")
 
 
 def log(msg: str) -> None:
