@@ -868,35 +868,40 @@ __global__ __launch_bounds__(kAttThreads) void select_attend_kernel(
 // ---- budgets beyond the candidate lists: selection from the histograms and attention in one launch --
 // The estimator in histogram mode leaves, per head, the distances of all tokens, a 512-bin histogram
 // per chunk of 512 to 2048 tokens and, per sequence, the K row index of every token.  grid (sequence*heads,
-// slabs of 4096 tokens), 256 threads.  Every workgroup works the threshold out for itself from the
+// slabs of 1024, 2048 or 4096 tokens), 256 or 512 threads.  Every workgroup works the threshold out for itself from the
 // chunk rows (they are small and sit in L2; rows of one head are the fast grid dimension so that its
 // slabs share a die), adding up on the side the rows of the chunks BEFORE its slab: those give the
 // number of selected tokens that precede the slab, i.e. the tie quota left for it and where its
-// positions go.  Then it selects among its own 4096 distances (class masks and DPP prefix scans),
-// keeps the K rows of the selected tokens in LDS and attends them: 16 groups of 16 lanes, tiles of
+// positions go.  Then it selects among the slab's distances (class masks and DPP prefix scans),
+// keeps the K rows of the selected tokens in LDS and attends them: groups of 16 lanes, tiles of up to
 // 8 rows.  The slabs of a head are merged inside the launch (split_merge.h).  Against a launch that
 // writes the selection followed by the attention operator, this saves a launch, the list's trip
 // through memory and the wait for it.
 constexpr int kHsaThreads = 256;
-constexpr int kHsaWaves = kHsaThreads / kWave;
-constexpr int kHsaMaxItems = 16;                                 // distances per thread, at most
+constexpr int kHsaWideThreads = 512;
+constexpr int kHsaMaxItems = 16;                                 // distances per thread of 256, at most
 constexpr uint32_t kHsaMaxSlab = kHsaThreads * kHsaMaxItems;     // 4096 tokens per workgroup, at most
-constexpr int kHsaGroups = kHsaThreads / 16;
 constexpr uint32_t kHsaMaxTokens = kHsaMaxSlab * 32;             // 32 slabs per head at most
 
-// Tokens per thread of hist_select_attend_kernel (4, 8 or 16: slabs of 1024, 2048 or 4096 tokens).
+// Tokens per thread of 256 in hist_select_attend_kernel (4, 8 or 16: slabs of 1024, 2048 or 4096 tokens).
 // One CU gathers scattered rows slowly, so the slab is halved while that leaves at most
 // max(slabs of 4096 tokens, min(16, budget / 64)) slabs per head: about 64 selected rows per
 // workgroup where the length allows it, and never more than 16 slabs for the sake of the rows
 // (beyond that the merge inside the launch costs more than the shorter gather saves).  Measured
 // against slabs of 4096 tokens throughout: 8192 tokens, budget 4096: 41.0 -> 24.8 us; 16384 / 1024:
 // 20.1 -> 18.4; 32768 / 1024: 23.3 -> 22.7; a target of 32 rows or a cap of 32 slabs is slower.  In
-// batches slabs of 2048 tokens are taken where those of 1024 would not all run at once (seven fit the LDS of a
-// CU): each sums the chunk rows of its head once more.  1024 / 2048 / 4096 tokens, us a layer at 32:32 and 32:8
+// batches slabs of 2048 tokens are taken where those of 1024 are clearly more than run at once (six to a CU, by
+// their registers): each sums the chunk rows of its head once more.  1024 / 2048 / 4096 tokens, us a layer at 32:32 and 32:8
 // heads: 16 sequences of 2000 to 7500, budget 512, 57.5 / 55.2 / 55.5 and 49.4 / 46.9 / 47.2; 8 of 4000 to 15000, 3000,
 // 116.6 / 110.0 / 107.2 and 91.5 / 87.7 / 88.7; 10 of 5000 to 12000, 2000, 104.2 / 103.4 / 114.2 and 80.6 / 82.0 / 92.8;
 // with fewer workgroups, 2 of 3000 to 6000, 600, 20.4 / 22.4 / 22.8 and 20.0 / 21.9 / 22.6.
+// Above ten slabs of 1024 tokens those of 2048 are taken where 512 threads work on each (hsa_threads) and
+// more than 64 workgroups are left: half as many partials to merge.  1024 / 2048 tokens, 32:32 and 32:8 heads:
+// 12000 tokens, budget 1024 19.5 / 19.1 and 18.8 / 18.4; 16384, 1024 20.3 / 19.6 and 19.4 / 18.6; 2 sequences of
+// 12000 to 16000, 1024, 27.7 / 26.6 and 24.8 / 23.9; with ten slabs or few heads, 9000, 1024 18.8 / 19.5 and
+// 18.6 / 19.3; 12000, 1024, 8:8 heads 17.5 / 18.0.
 constexpr uint64_t kHsaWorkgroups = 7 * 256;
+constexpr uint64_t kHsaWideWorkgroups = 2 * 256;
 inline int hsa_items(uint32_t max_seq_len, uint32_t budget, uint64_t heads) {
   const uint32_t n = max_seq_len > 1 ? max_seq_len - 1 : 1;
   const uint32_t most =
@@ -905,7 +910,22 @@ inline int hsa_items(uint32_t max_seq_len, uint32_t budget, uint64_t heads) {
   while (items > 4 && (n + kHsaThreads * (items / 2) - 1) / (kHsaThreads * (items / 2)) <= most)
     items /= 2;
   if (items == 4 && heads * ((n + kHsaThreads * 4 - 1) / (kHsaThreads * 4)) > kHsaWorkgroups) items = 8;
+  if (items == 4 && n > 10u * kHsaThreads * 4) {
+    const uint64_t half = heads * ((n + kHsaThreads * 8 - 1) / (kHsaThreads * 8));
+    if (half > 64 && half <= kHsaWideWorkgroups) items = 8;
+  }
   return items;
+}
+
+// Threads per workgroup for slabs of 256 * items tokens.  While there are at most two workgroups of 512 to a CU
+// (three run at once), they take slabs of 2048 and 4096 tokens: their serial parts, the chunk rows
+// per part and the rows per group, are half as long, and a CU that has one or two workgroups has eight waves for
+// each.  In us a layer with 256 / 512 threads, 32:32 and 32:8 heads, one sequence: 12000 tokens, budget 300
+// 18.5 / 17.8 and 17.7 / 16.9; 24000, 512 21.4 / 21.0 and 20.5 / 20.0; 32768, 2048 27.9 / 26.1 and 25.6 / 22.7;
+// 60000, 2048 39.4 / 37.6 and 35.0 / 33.3; 3 sequences of 15000 to 20000, 500, 31.7 / 30.7 and 26.8 / 25.4.  With
+// more workgroups: 100000, 1024 47.0 / 48.7 and 39.0 / 40.7; 16 of 2000 to 7500, 512, 54.7 / 59.6 and 46.4 / 50.7.
+inline int hsa_threads(int items, uint64_t workgroups) {
+  return items >= 8 && workgroups <= kHsaWideWorkgroups ? kHsaWideThreads : kHsaThreads;
 }
 
 // Chunk rows a thread asks for at a time (four threads share a bin group).  More in flight help one
@@ -914,20 +934,21 @@ inline int hsa_items(uint32_t max_seq_len, uint32_t budget, uint64_t heads) {
 constexpr int kHsaRows = 4;
 typedef uint32_t fs_uint4 __attribute__((ext_vector_type(4)));
 
-template <int kItems>
+template <int kThreads, int kItems>
 struct HistSelectAttendShared {
-  alignas(16) uint32_t all[kHsaWaves][kHistBins];  // partial sums over all chunk rows
-  alignas(16) uint32_t pre[kHsaWaves][kHistBins];  // partial sums over the chunk rows before the slab
-  uint32_t wtot[kHsaWaves], wpre[kHsaWaves], wclass[kHsaWaves];
+  static constexpr int kWaves = kThreads / kWave;
+  alignas(16) uint32_t all[kWaves][kHistBins];  // partial sums over all chunk rows
+  alignas(16) uint32_t pre[kWaves][kHistBins];  // partial sums over the chunk rows before the slab
+  uint32_t wtot[kWaves], wpre[kWaves], wclass[kWaves];
   uint32_t pre_tied;   // tokens at the threshold distance in the chunks before the slab
   SelectPlan plan;
-  int32_t rows[kHsaThreads * kItems + 1];  // K rows of the slab's selected tokens (slab 0: then the current token)
-  MergeShared<kHsaGroups> merge;
+  int32_t rows[kThreads * kItems + 1];  // K rows of the slab's selected tokens (slab 0: then the current token)
+  MergeShared<kThreads / 16> merge;
   uint32_t is_last;
 };
 
-template <bool kBf16, bool kHnd, int kItems>
-__global__ __launch_bounds__(kHsaThreads) void hist_select_attend_kernel(
+template <bool kBf16, bool kHnd, int kThreads, int kItems>
+__global__ __launch_bounds__(kThreads) void hist_select_attend_kernel(
     const uint16_t* __restrict__ dist, const uint16_t* __restrict__ hist,
     const uint32_t* __restrict__ rowmap, const int32_t* __restrict__ seq_lens, int64_t dist_stride,
     uint32_t n_chunks, uint32_t num_heads, uint32_t chunk_tokens, uint32_t k,
@@ -936,10 +957,12 @@ __global__ __launch_bounds__(kHsaThreads) void hist_select_attend_kernel(
     __half* __restrict__ out, int32_t* __restrict__ sel_out, float* partial,
     uint32_t* __restrict__ counters, uint32_t num_kv_heads, uint32_t kv_inv16, uint32_t page_size,
     float scale_log2) {
-  static_assert(kHsaThreads * 2 == kHistBins, "two bins per thread in the prefix sum");
+  constexpr int kWaves = kThreads / kWave, kGroups = kThreads / 16;
+  constexpr int kBins = kHistBins / kThreads;              // bins per thread in the prefix sum
+  static_assert(kBins == 1 || kBins == 2, "256 or 512 threads");
   static_assert(kItems == 4 || kItems == 8 || kItems == 16, "whole histogram rows per slab");
-  constexpr uint32_t kSlab = kHsaThreads * kItems;         // tokens per workgroup
-  __shared__ HistSelectAttendShared<kItems> sh;
+  constexpr uint32_t kSlab = kThreads * kItems;         // tokens per workgroup
+  __shared__ HistSelectAttendShared<kThreads, kItems> sh;
   const uint32_t bh = blockIdx.x, slab = blockIdx.y;
   const uint32_t b = bh / num_heads, head = bh - b * num_heads;
   const uint32_t tid = threadIdx.x;
@@ -951,7 +974,7 @@ __global__ __launch_bounds__(kHsaThreads) void hist_select_attend_kernel(
   // ---- everything whose address does not depend on the sequence length is asked for first: thread t
   // holds the kItems consecutive tokens t*kItems .. of the slab (distances and K rows; past the row's
   // end some valid piece of it, masked below), thread (part, seg) bins 8*seg .. 8*seg+7 of the first
-  // chunk rows part, part+4, ... (16-bit counts; a row past the sequence holds zeros)
+  // chunk rows part, part + kWaves, ... (16-bit counts; a row past the sequence holds zeros)
   const uint32_t e0 = slab_base + tid * kItems;
   const uint32_t part = tid >> 6, seg = tid & 63u;
   const unsigned char* hb = reinterpret_cast<const unsigned char*>(hist) +
@@ -980,7 +1003,7 @@ __global__ __launch_bounds__(kHsaThreads) void hist_select_attend_kernel(
 #pragma unroll
     for (int u = 0; u < kHsaRows; ++u)
       hrow[u] = *reinterpret_cast<const fs_uint4*>(
-          hb + static_cast<size_t>(min(part + 4u * u, n_chunks - 1u)) * (2 * kHistBins));
+          hb + static_cast<size_t>(min(part + kWaves * u, n_chunks - 1u)) * (2 * kHistBins));
 #pragma unroll
     for (int j = 0; j < kItems / 4; ++j) {
       const uint4 v = *reinterpret_cast<const uint4*>(rm + min(e0 + 4u * j, end - 4u));
@@ -995,7 +1018,7 @@ __global__ __launch_bounds__(kHsaThreads) void hist_select_attend_kernel(
     if (slab == 0) {
       if (tid < kHeadDim) store_elem<kBf16>(out + static_cast<size_t>(bh) * kHeadDim + tid, 0.f);
       if (sdst)
-        for (uint32_t i = tid; i < k; i += kHsaThreads) sdst[i] = -1;
+        for (uint32_t i = tid; i < k; i += kThreads) sdst[i] = -1;
     }
     return;
   }
@@ -1022,16 +1045,16 @@ __global__ __launch_bounds__(kHsaThreads) void hist_select_attend_kernel(
     const uint32_t c_first = slab_base / chunk_tokens;  // chunks below it precede the slab (whole chunks)
     const uint32_t rows_used = min(n_chunks, (n + chunk_tokens - 1) / chunk_tokens);  // rows of this sequence
     uint32_t acc[8] = {0, 0, 0, 0, 0, 0, 0, 0}, pre[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    for (uint32_t c0 = part; c0 < rows_used; c0 += 4 * kHsaRows) {
+    for (uint32_t c0 = part; c0 < rows_used; c0 += kWaves * kHsaRows) {
       if (c0 != part) {
 #pragma unroll
         for (int u = 0; u < kHsaRows; ++u)
           hrow[u] = *reinterpret_cast<const fs_uint4*>(
-              hb + static_cast<size_t>(min(c0 + 4u * u, n_chunks - 1u)) * (2 * kHistBins));
+              hb + static_cast<size_t>(min(c0 + kWaves * u, n_chunks - 1u)) * (2 * kHistBins));
       }
 #pragma unroll
       for (int u = 0; u < kHsaRows; ++u) {
-        const uint32_t c = c0 + 4u * u;
+        const uint32_t c = c0 + kWaves * u;
         const uint32_t used = c < rows_used ? 0xffffffffu : 0u, m = c < c_first ? used : 0u;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -1051,42 +1074,39 @@ __global__ __launch_bounds__(kHsaThreads) void hist_select_attend_kernel(
     dp[1] = make_uint4(pre[4], pre[5], pre[6], pre[7]);
   }
   __syncthreads();
-  // ---- thread t owns bins 2t and 2t+1: prefix sum -> the plan
-  uint32_t ca0 = 0, ca1 = 0, cp0 = 0, cp1 = 0;
+  // ---- thread t owns bins kBins*t ..: prefix sum -> the plan
+  uint32_t ca[kBins] = {}, cp[kBins] = {};
 #pragma unroll
-  for (int p = 0; p < kHsaWaves; ++p) {
-    const uint2 x = *reinterpret_cast<const uint2*>(&sh.all[p][2 * tid]);
-    const uint2 y = *reinterpret_cast<const uint2*>(&sh.pre[p][2 * tid]);
-    ca0 += x.x;
-    ca1 += x.y;
-    cp0 += y.x;
-    cp1 += y.y;
+  for (int p = 0; p < kWaves; ++p) {
+#pragma unroll
+    for (int j = 0; j < kBins; ++j) {  // (neighbours: one 64-bit read where there are two)
+      ca[j] += sh.all[p][kBins * tid + j];
+      cp[j] += sh.pre[p][kBins * tid + j];
+    }
   }
-  const uint32_t incl = wave_inclusive_scan_dpp(ca0 + ca1);
+  const uint32_t incl = wave_inclusive_scan_dpp(kBins == 2 ? ca[0] + ca[kBins - 1] : ca[0]);
   if (lane == kWave - 1) sh.wtot[wave] = incl;
   __syncthreads();
-  uint32_t cum1 = incl;  // tokens with a distance <= bin 2t+1
-  for (int w = 0; w < wave; ++w) cum1 += sh.wtot[w];
-  const uint32_t cum0 = cum1 - ca1;  // <= bin 2t
-  if (cum0 >= k && cum0 - ca0 < k) {  // exactly one bin holds the k-th smallest distance
-    sh.plan.thr = 2 * tid;
-    sh.plan.n_below = cum0 - ca0;
-    sh.plan.quota = k - (cum0 - ca0);
-    sh.plan.n_take = k;
-    sh.pre_tied = cp0;
+  uint32_t cum = incl;  // tokens with a distance <= the thread's last bin
+  for (int w = 0; w < wave; ++w) cum += sh.wtot[w];
+  const uint32_t cum_all = cum;
+#pragma unroll
+  for (int j = kBins - 1; j >= 0; --j) {
+    const uint32_t less = cum - ca[j];  // with a smaller distance than bin kBins*t + j
+    if (cum >= k && less < k) {         // exactly one bin holds the k-th smallest distance
+      sh.plan.thr = kBins * tid + j;
+      sh.plan.n_below = less;
+      sh.plan.quota = k - less;
+      sh.plan.n_take = k;
+      sh.pre_tied = cp[j];
+    }
+    cum = less;
   }
-  if (cum1 >= k && cum0 < k) {
-    sh.plan.thr = 2 * tid + 1;
-    sh.plan.n_below = cum0;
-    sh.plan.quota = k - cum0;
-    sh.plan.n_take = k;
-    sh.pre_tied = cp1;
-  }
-  if (tid == kHsaThreads - 1 && cum1 < k) {  // fewer tokens than k: all of them are taken
+  if (tid == kThreads - 1 && cum_all < k) {  // fewer tokens than k: all of them are taken
     sh.plan.thr = kHistBins;
-    sh.plan.n_below = cum1;
+    sh.plan.n_below = cum_all;
     sh.plan.quota = 0;
-    sh.plan.n_take = cum1;
+    sh.plan.n_take = cum_all;
     sh.pre_tied = 0;
   }
   __syncthreads();
@@ -1094,7 +1114,9 @@ __global__ __launch_bounds__(kHsaThreads) void hist_select_attend_kernel(
   const uint32_t pre_tied = sh.pre_tied;
 
   // ---- selected tokens before the slab, class masks and ranks inside it
-  const uint32_t mine_pre = (2 * tid < plan.thr ? cp0 : 0u) + (2 * tid + 1 < plan.thr ? cp1 : 0u);
+  uint32_t mine_pre = 0;
+#pragma unroll
+  for (int j = 0; j < kBins; ++j) mine_pre += kBins * tid + j < plan.thr ? cp[j] : 0u;
   const uint32_t wave_pre = wave_sum(mine_pre);
   uint32_t below[kItems / 4], equal[kItems / 4];
   raw_class_masks<kItems>(keys, plan.thr, below, equal);
@@ -1107,7 +1129,7 @@ __global__ __launch_bounds__(kHsaThreads) void hist_select_attend_kernel(
   __syncthreads();
   uint32_t base_b = 0, before = 0, slab_all = 0;
 #pragma unroll
-  for (int w = 0; w < kHsaWaves; ++w) {
+  for (int w = 0; w < kWaves; ++w) {
     base_b += sh.wpre[w];
     before += w < wave ? sh.wclass[w] : 0u;
     slab_all += sh.wclass[w];
@@ -1133,7 +1155,7 @@ __global__ __launch_bounds__(kHsaThreads) void hist_select_attend_kernel(
     if (tid == 0) sh.rows[n_rows] = cur_row;
     ++n_rows;
     if (sdst)
-      for (uint32_t i = plan.n_take + tid; i < k; i += kHsaThreads) sdst[i] = -1;
+      for (uint32_t i = plan.n_take + tid; i < k; i += kThreads) sdst[i] = -1;
   }
   __syncthreads();
 
@@ -1147,14 +1169,14 @@ __global__ __launch_bounds__(kHsaThreads) void hist_select_attend_kernel(
   // (a group asks for 2, 4 or 8 rows at a time: slots past the end load the last row again, so the
   // round is no larger than the slab's rows need)
   auto row_of = [&](uint32_t r) __attribute__((always_inline)) -> int32_t { return sh.rows[r]; };
-  if (n_rows <= kHsaGroups * 2u)
-    attend_rows<kHsaGroups, 2, true, kBf16, true>(kv, qf, g, 0u, n_rows, row_of, st);
-  else if (n_rows <= kHsaGroups * 4u)
-    attend_rows<kHsaGroups, 4, true, kBf16, true>(kv, qf, g, 0u, n_rows, row_of, st);
+  if (n_rows <= kGroups * 2u)
+    attend_rows<kGroups, 2, true, kBf16, true>(kv, qf, g, 0u, n_rows, row_of, st);
+  else if (n_rows <= kGroups * 4u)
+    attend_rows<kGroups, 4, true, kBf16, true>(kv, qf, g, 0u, n_rows, row_of, st);
   else
-    attend_rows<kHsaGroups, 8, true, kBf16, true>(kv, qf, g, 0u, n_rows, row_of, st);
+    attend_rows<kGroups, 8, true, kBf16, true>(kv, qf, g, 0u, n_rows, row_of, st);
   float M, L, O;
-  merge_groups<kHsaGroups>(st, g, c16, tid, sh.merge, M, L, O);
+  merge_groups<kGroups>(st, g, c16, tid, sh.merge, M, L, O);
   if (n_split == 1) {
     if (tid < kHeadDim)
       store_elem<kBf16>(out + static_cast<size_t>(bh) * kHeadDim + tid, L > 0.f ? O / L : 0.f);
@@ -1589,9 +1611,10 @@ extern "C" int adamas_decode_step_f(const void* q, const void* q_code, const voi
     while (kHsaThreads * static_cast<uint32_t>(items) < chunk_tokens) items *= 2;  // slabs of whole chunks
     const uint32_t slab_tokens = kHsaThreads * static_cast<uint32_t>(items);
     const dim3 hgrid(batch * num_heads, (max_seq_len - 1 + slab_tokens - 1) / slab_tokens);
-#define ADAMAS_LAUNCH_HSA_I(BF, HND, ITEMS)                                                       \
-  hipLaunchKernelGGL((hist_select_attend_kernel<BF, HND, ITEMS>), hgrid, dim3(kHsaThreads), 0, s, \
-                     dist, reinterpret_cast<const uint16_t*>(hist), rowmap, seq_lens,             \
+    const bool wide_groups = hsa_threads(items, static_cast<uint64_t>(hgrid.x) * hgrid.y) == kHsaWideThreads;
+#define ADAMAS_LAUNCH_HSA_I(BF, HND, THREADS, ITEMS)                                              \
+  hipLaunchKernelGGL((hist_select_attend_kernel<BF, HND, THREADS, ITEMS>), hgrid, dim3(THREADS),  \
+                     0, s, dist, reinterpret_cast<const uint16_t*>(hist), rowmap, seq_lens,       \
                      w.dist_stride, n_chunks, num_heads, chunk_tokens, n_sel,                     \
                      static_cast<const __half*>(q), static_cast<const __half*>(kv_data),          \
                      page_indices, page_indptr, static_cast<__half*>(out), sel_out,               \
@@ -1601,11 +1624,15 @@ extern "C" int adamas_decode_step_f(const void* q, const void* q_code, const voi
                      sm_scale * 1.4426950408889634f)
 #define ADAMAS_LAUNCH_HSA(BF, HND)          \
   if (items == 4) {                         \
-    ADAMAS_LAUNCH_HSA_I(BF, HND, 4);        \
+    ADAMAS_LAUNCH_HSA_I(BF, HND, 256, 4);   \
+  } else if (wide_groups && items == 8) {   \
+    ADAMAS_LAUNCH_HSA_I(BF, HND, 512, 4);   \
+  } else if (wide_groups) {                 \
+    ADAMAS_LAUNCH_HSA_I(BF, HND, 512, 8);   \
   } else if (items == 8) {                  \
-    ADAMAS_LAUNCH_HSA_I(BF, HND, 8);        \
+    ADAMAS_LAUNCH_HSA_I(BF, HND, 256, 8);   \
   } else {                                  \
-    ADAMAS_LAUNCH_HSA_I(BF, HND, 16);       \
+    ADAMAS_LAUNCH_HSA_I(BF, HND, 256, 16);  \
   }
     if (bf16 && hnd) {
       ADAMAS_LAUNCH_HSA(true, true);

@@ -144,3 +144,16 @@ def test_step_of_more_slabs_than_run_at_once(gpu_device, longest, kv_heads, layo
     """512 (sequence, head) pairs: slabs of 1024 tokens up to 3073, of 2048 beyond."""
     lens = [longest] + [2 + (613 * i) % (longest - 2) for i in range(15)]
     _check(gpu_device, lens, 600, 16, kv_heads, torch.float16, layout)
+
+
+@pytest.mark.parametrize("lens,budget,page,kv_heads,dtype,layout", [
+    ([10241], 1024, 16, 32, torch.float16, 0),          # ten slabs of 1024: the last with 256 threads on each
+    ([10242], 1024, 16, 8, torch.bfloat16, 1),          # the first of 2048 with 512
+    ([10242], 9000, 1, 32, torch.float16, 0),           # nearly every token
+    ([24577], 512, 16, 8, torch.float16, 0),            # slabs of 4096, the last with one token
+    ([65537], 2000, 16, 8, torch.float16, 0),           # 512 workgroups: the last with 512 threads
+    ([65538], 2000, 16, 8, torch.float16, 1),           # the first with 256 again
+    ([16000, 900, 2, 4098], 300, 16, 4, torch.bfloat16, 0),
+])
+def test_step_of_workgroups_of_512(gpu_device, lens, budget, page, kv_heads, dtype, layout):
+    _check(gpu_device, lens, budget, page, kv_heads, dtype, layout)
