@@ -21,12 +21,12 @@ constexpr int kTile = 8;             // rows per group per tile, at most
 // single workgroup per head takes 25 us for 1024 rows), a group finishes sooner the fewer rows it
 // has to ask for, and publishing a partial result costs about a microsecond.  Hence: up to 64 rows
 // 16 groups of 4, up to 128 rows 32 groups of 4 (one split, no merge, no workspace); up to 512 rows
-// splits of 64 rows (32 groups of 2, at most 8 splits); up to 1408 rows splits of 128 (64 groups of
-// 2, at most 11); beyond that, and where more workgroups than run at once would come of it, four rows in flight
+// splits of 64 rows (32 groups of 2, at most 8 splits); up to 2048 rows splits of 128 (64 groups of
+// 2, at most 16); beyond that, and where more workgroups than run at once would come of it, four rows in flight
 // (row_launch).  Measured at 32 heads, rows = 128 /
 // 256 / 512 / 1024 / 2048 / 4096, in us: 5.8 / 6.5 / 7.4 / 9.3 / 13.5 / 18.8 (with 16 groups of 8
 // rows and splits of 128 rows up to 1024 rows, 32 groups of 8 beyond: 7.5 / 9.5 / 10.1 / 12.4 / 15.8
-// / 20.6); 2048 rows four in flight 12.5.
+// / 20.6).
 constexpr uint32_t kDeferredMergeSplits = 24;  // splits from which the partials get a merge launch
 // (measured at 32768 tokens, 32 heads: 16 splits 14.7 us merged inside the launch, 15.8 us with a merge
 // launch; 32 splits 26.6 against 22.5 us)
@@ -984,9 +984,11 @@ extern "C" size_t adamas_workspace_bytes(uint32_t batch, uint32_t num_heads, uin
 // Workgroups of sparse_decode_kernel for `n_rows` rows each of `heads` (sequence, query head) pairs: threads, rows
 // in flight per group of 16 lanes, rows per round and rounds' worth of workgroups (see the rule at kTile).  Two
 // rows in flight instead of four give twice the workgroups, half the rows each: better as long as they all
-// run at once and the merge of a head stays short.  Two / four, 32:32 heads, us a launch with its append:
-// 2000 positions 14.4 / 13.4, 1400 12.3 / 12.3, 1000 10.9 / 11.3; 3 sequences of 600 to 1500 21.6 / 17.9, 16 of 150 to
-// 250 21.9 / 17.3, 2 of 600 to 1000 13.2 / 13.4; 32:8 heads, 8 of 150 to 250 12.4 / 13.0.
+// run at once.  Two / four, 32:32 heads, us a launch with its append: 3 sequences of 600 to 1500 21.6 / 17.9, 16
+// of 150 to 250 21.9 / 17.3, 2 of 600 to 1000 13.2 / 13.4; 32:8 heads, 8 of 150 to 250 12.4 / 13.0; one sequence of 1000
+// 10.9 / 11.3, 1400 12.3 / 12.3, 2000 14.4 / 13.4.  That last microsecond is left: splits of 256 rows add up in another
+// order than those of 128, and the dense layers of a decoder hand that rounding on to every later code threshold
+// (three layers, a prompt of 2000 tokens: the logits moved by up to 5e-3).
 struct RowLaunch {
   uint32_t threads, tile, rows_per_iter;
   uint64_t workgroups;
@@ -1001,7 +1003,7 @@ static RowLaunch row_launch(uint64_t heads, uint32_t n_rows) {
     r.workgroups = heads * ((n_rows + r.rows_per_iter - 1) / r.rows_per_iter);
     r.one_round = r.workgroups * r.threads <= 256u * 2048u;
   };
-  with_tile(n_rows <= 128 || n_rows > 1408 ? 4u : 2u);
+  with_tile(n_rows <= 128 || n_rows > 2048 ? 4u : 2u);
   if (!r.one_round) with_tile(4u);
   return r;
 }

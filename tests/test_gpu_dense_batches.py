@@ -55,8 +55,10 @@ def test_dense_attention_of_ragged_batches(gpu_device, lens, kv_heads, page, dty
 
 
 @pytest.mark.parametrize("lens,kv_heads,page,dtype,layout", [
-    ([1408], 32, 16, torch.float16, 0),               # two rows in flight, the last length of them
-    ([1409], 8, 1, torch.bfloat16, 1),                # four
+    ([1408], 32, 16, torch.float16, 0),               # two rows in flight, the last split full
+    ([1409], 8, 1, torch.bfloat16, 1),                # and with one row
+    ([2048], 8, 1, torch.bfloat16, 1),                # the last length of them
+    ([2049], 32, 16, torch.float16, 0),               # four
     ([1000, 1, 999, 641], 8, 16, torch.float16, 0),   # four sequences whose workgroups just run at once
     ([1025, 1, 999, 641], 8, 16, torch.float16, 0),   # and no longer
     ([512, 500, 129, 3, 257, 511, 64, 65], 4, 16, torch.bfloat16, 0),
@@ -66,6 +68,28 @@ def test_dense_attention_of_ragged_batches(gpu_device, lens, kv_heads, page, dty
 ])
 def test_dense_attention_at_the_edges_of_the_row_kernel(gpu_device, lens, kv_heads, page, dtype, layout):
     test_dense_attention_of_ragged_batches(gpu_device, lens, kv_heads, page, dtype, layout)
+
+
+@pytest.mark.parametrize("n,dtype,as_list", [
+    (1409, torch.float16, False), (2048, torch.float16, False), (2000, torch.bfloat16, False),
+    (1500, torch.bfloat16, True), (2048, torch.float16, True)])
+def test_splits_of_one_sequence_are_of_128_rows(gpu_device, n, dtype, as_list):
+    """Rows 0 and 1 cancel inside their split; row 128 is far too small to survive beside either of them
+    and only counts because it is added up in another split."""
+    dev = gpu_device
+    big, small = (65504., 0.75 * 2.0 ** -9) if dtype == torch.float16 else (2.0 ** 60, 1.)
+    ctrl = U.InferenceController(1, 32, 128, 16, 1 << 20, n, dtype, dev)
+    ctrl.pool.kv.zero_()
+    ctrl.prepare_hadamard(n)
+    ctrl.begin_forward(1)
+    for pos, value in ((0, big), (1, -big), (128, small)):
+        ctrl.pool.kv[0][ctrl.seqs.pages[0][pos // 16], 1, pos % 16] = value
+    sel = U.ALL_PAST_TOKENS
+    if as_list:     # (the current token is the last row)
+        sel = torch.arange(n - 1, device=dev, dtype=torch.int32).expand(32, -1).contiguous()
+    o = U.decode_sparse_attn(torch.zeros(1, 32, 128, dtype=dtype, device=dev), ctrl, 0, sel)
+    # every weight is 1 / n; one rounding to 16 bits (half an ulp of 8 bits, or of fp16's denormals)
+    assert bool(((o.double() - small / n).abs() <= 2.0 ** -8 * small / n + 2.0 ** -25).all()), float(o.float().max())
 
 
 @pytest.mark.parametrize("lens,kv_heads,dtype", [
