@@ -331,7 +331,8 @@ def _prefill_plan_reference(n_new, past, heads, kv_heads):
 
 
 @pytest.mark.parametrize("heads,kv_heads", [(32, 32), (32, 8), (32, 1), (24, 8), (512, 512)])
-@pytest.mark.parametrize("n_new,past", [(1, 0), (64, 16000), (300, 900), (257, 63), (1000, 3000), (2000, 0)])
+@pytest.mark.parametrize("n_new,past", [(1, 0), (64, 16000), (300, 900), (257, 63), (1000, 3000), (2000, 0),
+                                        (300, 553), (500, 300)])    # (calls that may get workgroups of four waves)
 def test_prefill_plan(heads, kv_heads, n_new, past):
     n_split = _prefill_plan_reference(n_new, past, heads, kv_heads)
     want = 0 if n_split == 1 else n_split * n_new * heads * 132 * 4

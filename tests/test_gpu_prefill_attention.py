@@ -97,6 +97,20 @@ def test_prefill_attention_page_sizes(gpu_device, n, past, kv_heads, page, dtype
     assert bool(((U.prefill_forward(q, ctrl, 0).double() - ref).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("n,past,kv_heads,dtype", [
+    (1200, 0, 32, torch.float16), (850, 0, 8, torch.bfloat16),      # token ranges
+    (200, 1200, 32, torch.float16), (64, 1000, 8, torch.float16),
+    (700, 0, 32, torch.float16), (2000, 553, 8, torch.bfloat16),    # one range of all tiles
+])
+def test_prefill_attention_of_both_workgroups_is_the_same(gpu_device, n, past, kv_heads, dtype):
+    """Pages of 16 slots get workgroups of four waves, pages of 4 those of eight."""
+    ctrl, q, k, v = _cache(gpu_device, n, past, kv_heads, 16, dtype, 0, False, n)
+    other = U.InferenceController(1, 32, 128, 4, 64, n + past, dtype, gpu_device, num_kv_heads=kv_heads)
+    other.prepare_hadamard(n + past)
+    U.append_kvh(k, v, None, other, 0)
+    assert torch.equal(U.prefill_forward(q, ctrl, 0), U.prefill_forward(q, other, 0))
+
+
 def test_prefill_attention_of_a_misaligned_view(gpu_device):
     ctrl, q, k, v = _cache(gpu_device, 40, 0, 32, 16, torch.float16, 0, False, 3)
     flat = torch.empty(q.numel() + 1, dtype=q.dtype, device=gpu_device)
