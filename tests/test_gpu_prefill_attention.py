@@ -97,6 +97,22 @@ def test_prefill_attention_page_sizes(gpu_device, n, past, kv_heads, page, dtype
     assert bool(((U.prefill_forward(q, ctrl, 0).double() - ref).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("kv_heads,page,dtype,layout", [
+    (32, 1 << 19, torch.float16, 0),          # K and V of a page exactly 2^32 bytes apart
+    (32, (1 << 19) + 1, torch.float16, 0),    # and a little more, addresses made in every lane
+    (8, 1 << 21, torch.bfloat16, 1),
+    (8, (1 << 21) - 1, torch.float16, 0),     # a little less
+])
+def test_prefill_attention_of_a_whole_context_in_one_page(gpu_device, kv_heads, page, dtype, layout):
+    n, past = 70, 200
+    ctrl, q, k, v = _cache(gpu_device, n, past, kv_heads, page, dtype, layout, False, kv_heads)
+    ref, mag = _reference(q, k, v, past)
+    # as at the edges above
+    u = 2.0 ** (-11 if dtype == torch.float16 else -8)
+    bound = u * (mag + ref.abs()) + 2.0 ** -14 * mag + 2.0 ** -25 * v.double().abs().sum(0).max()
+    assert bool(((U.prefill_forward(q, ctrl, 0).double() - ref).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("n,past,kv_heads,dtype", [
     (1200, 0, 32, torch.float16), (850, 0, 8, torch.bfloat16),      # token ranges
     (200, 1200, 32, torch.float16), (64, 1000, 8, torch.float16),
