@@ -1664,7 +1664,8 @@ extern "C" int adamas_decode_step_f(const void* q, const void* q_code, const voi
   return adamas_sparse_decode_f(q, kv_data, page_indices, page_indptr, seq_lens, sel,
                                 static_cast<int64_t>(n_sel), (max_seq_len > 1) ? n_sel : 0u, out,
                                 workspace, workspace_bytes, batch, num_heads, num_kv_heads,
-                                head_dim, page_size, sm_scale, max_seq_len, flags, stream);
+                                head_dim, page_size, sm_scale, max_seq_len,
+                                flags & ~ADAMAS_F_CODES_CACHED, stream);  // (a hint for the step's own kernels)
 }
 
 extern "C" int adamas_decode_step(const void* q, const void* q_code, const void* kv_data,

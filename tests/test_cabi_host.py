@@ -376,6 +376,20 @@ def test_codes_cached_hint():
                                       _lib.F_CODES_CACHED, None) == -1
 
 
+@pytest.mark.parametrize("length", [2, 4096, 140000])
+def test_general_path_of_the_step_takes_the_codes_hint(length):
+    """The step hands a budget of one token to the attention operator, which does not know the hint; without
+    a device all that is left is the HIP runtime's error at the launch."""
+    if torch.cuda.is_available():
+        pytest.skip("would launch on addresses that are none")
+    lib = _lib.load()
+    need = lib.adamas_workspace_bytes(1, 32, length, 1)
+    for flags in (0, _lib.F_CODES_CACHED):
+        rc = lib.adamas_decode_step_f(*[256] * 7, 1, 256, None, 256, need, 1, 32, 32, 128, 16, 1.0, length,
+                                      -(-length // 16), flags, None)
+        assert rc > 0, (flags, rc)
+
+
 def test_layer_addresses():
     """The addresses handed to the library are those of the layers' views, for the same indices."""
     c = _ctrl(num_layers=3)

@@ -139,6 +139,21 @@ def test_step_of_narrow_workgroups_reads_codes_through_and_past_the_caches(gpu_d
     assert torch.equal(got[0][1].sort(dim=1).values, ctrl.topk_dindices_buffer.sort(dim=1).values)
 
 
+@pytest.mark.parametrize("lens,budget,kv_heads", [
+    ([4096], 1, 32), ([3000, 700], 1, 8),     # nothing is selected
+    ([140000], 300, 32), ([140000], 1000, 8), # longer than the histograms go
+])
+def test_step_on_the_general_path_takes_the_codes_hint(gpu_device, lens, budget, kv_heads, monkeypatch):
+    from adamas_amd.utils import controller as C
+    ctrl, q, q_code = _controller(gpu_device, lens, budget, 16, kv_heads, torch.float16, 0, 5)
+    got = []
+    for limit in (0, 1 << 40):
+        monkeypatch.setattr(C, "CODES_CACHED_BYTES", limit)
+        assert bool(ctrl.codes_hint) == bool(limit)
+        got.append(U.decode_step(q, q_code, ctrl, 0))
+    assert torch.equal(*got) and bool(got[0].any())
+
+
 @pytest.mark.parametrize("longest,kv_heads,layout", [(3072, 32, 0), (3074, 8, 1), (4097, 32, 0)])
 def test_step_of_more_slabs_than_run_at_once(gpu_device, longest, kv_heads, layout):
     """512 (sequence, head) pairs: slabs of 1024 tokens up to 3073, of 2048 beyond."""
