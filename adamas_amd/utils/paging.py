@@ -16,6 +16,7 @@ controller.py:30-39 with kv_cache.py:88 divides the capacity by page_size twice.
 """
 from __future__ import annotations
 
+from operator import index
 from typing import Iterable, List, Optional, Sequence
 
 import torch
@@ -33,7 +34,11 @@ class TensorLayout:
 
 
 def _row_address(t: torch.Tensor, i: int) -> int:
-    """t[i].data_ptr() without making the view."""
+    """t[i].data_ptr() without making the view, as a Python int whatever kind of integer i is."""
+    try:
+        i = index(i)
+    except TypeError:   # (a slice or the like)
+        return t[i].data_ptr()
     n = t.shape[0]
     if not -n <= i < n:
         raise IndexError(f"index {i} is out of bounds for dimension 0 with size {n}")

@@ -5,6 +5,7 @@ import ctypes
 import os
 import re
 
+import numpy as np
 import pytest
 import torch
 
@@ -396,6 +397,14 @@ def test_layer_addresses():
     for layer in range(-3, 3):
         assert c.pool.kv_address(layer) == c.pool.kv[layer].data_ptr()
         assert c.pool.codes_address(layer) == c.pool.codes[layer].data_ptr()
+    for layer in (1, -1):
+        for kind in (np.int64, np.int32, np.uint8, torch.tensor, lambda i: torch.tensor(i, dtype=torch.int32)):
+            if layer < 0 and kind is np.uint8:
+                continue
+            for address, views in ((c.pool.kv_address, c.pool.kv), (c.pool.codes_address, c.pool.codes)):
+                got = ctypes.c_void_p.from_param(address(kind(layer)))    # (what the library is called with)
+                assert got.value == views[layer].data_ptr()
+    assert c.pool.kv_address(slice(1, 2)) == c.pool.kv[1].data_ptr()
     for layer in (-4, 3):
         with pytest.raises(IndexError):
             c.pool.kv_address(layer)
