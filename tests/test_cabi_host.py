@@ -402,8 +402,9 @@ def test_layer_addresses():
             if layer < 0 and kind is np.uint8:
                 continue
             for address, views in ((c.pool.kv_address, c.pool.kv), (c.pool.codes_address, c.pool.codes)):
-                got = ctypes.c_void_p.from_param(address(kind(layer)))    # (what the library is called with)
-                assert got.value == views[layer].data_ptr()
+                got = address(kind(layer))
+                ctypes.c_void_p.from_param(got)      # (as a call into the library does)
+                assert got == views[layer].data_ptr()
     assert c.pool.kv_address(slice(1, 2)) == c.pool.kv[1].data_ptr()
     for layer in (-4, 3):
         with pytest.raises(IndexError):
