@@ -99,6 +99,7 @@ F_BF16 = 2
 F_HND = 4
 F_NO_MFMA = 8
 F_CODES_CACHED = 16
+F_CODES_STREAMED = 64
 STATIC_SCRATCH_BYTES = 24 << 20
 E_SCRATCH = -5
 DIST_FP16, DIST_U16 = 0, 1

@@ -1241,8 +1241,13 @@ static bool est_share(uint32_t batch, int est_heads, uint32_t num_heads, uint32_
 }
 
 // Whether the estimator reads the codes past the caches.  Where the caches cannot keep them until the next
-// step that saves what they evict; where they can (the last level holds 256 MB, the caller says so with
-// ADAMAS_F_CODES_CACHED), workgroups wait for memory each time.  In us per layer with the layers in turn,
+// step that saves what they evict; where they can (the last level holds 256 MB), workgroups wait for memory
+// each time.  The caller knows which (ADAMAS_F_CODES_CACHED, ADAMAS_F_CODES_STREAMED); without either flag the
+// wide workgroups of the selection do, and the others (narrow ones, histograms) where the codes of the call
+// alone are too many.  What a caller who says nothing about a few cached layers would lose otherwise, a step of 32:32
+// heads through / past: budget 600, 4096 tokens 14.2 / 14.6, 16000 16.1 / 16.8; 128, 4 sequences of 1500 to 7000 14.0 /
+// 14.4; 64, 4096 tokens 9.9 / 9.8, this launch alone and repeated 5.0 / 5.4; 128, 8192 tokens 11.0 / 10.5.
+// In us per layer with the layers in turn,
 // through / past the caches.  Selection: 32 heads, 16 sequences of 8192 to 32768 tokens, 1 layer (335 MB of codes)
 // 88.2 / 80.1, 2 layers 87.0 / 77.0; 8 of 1500 to 7000, 4 layers (139 MB) 22.8 / 23.0, 8 layers 24.0 / 21.9; one
 // sequence of 4096, 8 layers (34 MB) 12.8 / 12.8, 80 layers 14.0 / 12.9; 8 heads, 131072, 7 layers (235 MB) 23.2 / 25.7, 9
@@ -1251,9 +1256,12 @@ static bool est_share(uint32_t batch, int est_heads, uint32_t num_heads, uint32_
 // A full chip of wide workgroups loses nothing by it in a step (65536 tokens, 2 layers 20.2 / 19.3).  The
 // shared instances read 128 or 256 bytes per token, lines that other workgroups want too, and always
 // lose: 32:8 heads, 16 of 8192 to 32768, 2 layers 51.0 / 56.9.
-static bool est_stream(uint32_t flags, int est_heads, bool share, uint32_t workgroups) {
-  return !share && ((est_heads == kFusedHeads && workgroups >= kStepWorkgroups) ||
-                    !(flags & ADAMAS_F_CODES_CACHED));
+constexpr uint64_t kCodesCachedBytes = uint64_t{280} << 20;
+constexpr uint32_t kCodesFlags = ADAMAS_F_CODES_CACHED | ADAMAS_F_CODES_STREAMED;
+static bool est_stream(uint32_t flags, bool wide_selection, bool share, uint32_t workgroups, uint64_t codes) {
+  if (share) return false;
+  if (flags & ADAMAS_F_CODES_CACHED) return wide_selection && workgroups >= kStepWorkgroups;
+  return wide_selection || (flags & ADAMAS_F_CODES_STREAMED) || codes * (2 * kCodeWords) > kCodesCachedBytes;
 }
 
 static StepGeom geom_of(const StepPlan& p) {
@@ -1273,7 +1281,8 @@ static int step_candidates_impl(const void* q_code, const void* code_data,
                                 uint32_t num_kv_heads, uint32_t page_size, uint32_t max_seq_len,
                                 uint32_t page_table_stride, uint32_t flags,
                                 adamas_stream_t stream, const QkvSource* qsrc) {
-  if (flags & ~(ADAMAS_F_BF16 | ADAMAS_F_HND | ADAMAS_F_CODES_CACHED)) return ADAMAS_E_BADARG;
+  if (flags & ~(ADAMAS_F_BF16 | ADAMAS_F_HND | kCodesFlags)) return ADAMAS_E_BADARG;
+  if ((flags & kCodesFlags) == kCodesFlags) return ADAMAS_E_BADARG;
   if (qsrc) q_code = qsrc->qkv;  // any valid, aligned pointer: the kernel does not read it
   if (!q_code || !code_data || !page_indices || (!page_indptr && !page_table_stride) ||
       !seq_lens || !workspace ||
@@ -1295,7 +1304,8 @@ static int step_candidates_impl(const void* q_code, const void* code_data,
   const StepPlan& plan = w.plan;
   const int est_heads = static_cast<int>(plan.heads);
   const bool share = est_share(batch, est_heads, num_heads, num_kv_heads);
-  const bool stream_codes = est_stream(flags, est_heads, share, plan.chunks * (num_heads / kFusedHeads));
+  const bool stream_codes = est_stream(flags, est_heads == kFusedHeads, share, plan.chunks * (num_heads / kFusedHeads),
+                                       uint64_t{batch} * max_seq_len * num_kv_heads);
   const dim3 grid(plan.chunks, num_heads / est_heads, batch);
   hipStream_t s = static_cast<hipStream_t>(stream);
 #define ADAMAS_LAUNCH_ESTSEL_Q(PG, PASSES, PARTIAL, HEADS, FROMQKV, SHARE, STREAM)                   \
@@ -1396,7 +1406,8 @@ static int step_attend_impl(const void* q, void* kv_data, void* code_data,
                             uint32_t head_dim, uint32_t page_size, float sm_scale,
                             uint32_t max_seq_len, uint32_t page_table_stride, uint32_t flags,
                             adamas_stream_t stream, const QkvSource* qsrc) {
-  if (flags & ~(ADAMAS_F_BF16 | ADAMAS_F_HND | ADAMAS_F_CODES_CACHED)) return ADAMAS_E_BADARG;
+  if (flags & ~(ADAMAS_F_BF16 | ADAMAS_F_HND | kCodesFlags)) return ADAMAS_E_BADARG;
+  if ((flags & kCodesFlags) == kCodesFlags) return ADAMAS_E_BADARG;
   if (qsrc) q = qsrc->qkv;
   const bool bf16 = (flags & ADAMAS_F_BF16) != 0;
   const bool hnd = (flags & ADAMAS_F_HND) != 0;
@@ -1497,7 +1508,8 @@ extern "C" int adamas_decode_step_f(const void* q, const void* q_code, const voi
                                     float sm_scale, uint32_t max_seq_len,
                                     uint32_t page_table_stride, uint32_t flags,
                                     adamas_stream_t stream) {
-  if (flags & ~(ADAMAS_F_BF16 | ADAMAS_F_HND | ADAMAS_F_CODES_CACHED)) return ADAMAS_E_BADARG;
+  if (flags & ~(ADAMAS_F_BF16 | ADAMAS_F_HND | kCodesFlags)) return ADAMAS_E_BADARG;
+  if ((flags & kCodesFlags) == kCodesFlags) return ADAMAS_E_BADARG;
   if (!q || !q_code || !kv_data || !code_data || !page_indices || !page_indptr || !seq_lens ||
       !out || !workspace || budget == 0 || max_seq_len == 0 || batch == 0 || page_size == 0)
     return ADAMAS_E_BADARG;
@@ -1552,7 +1564,7 @@ extern "C" int adamas_decode_step_f(const void* q, const void* q_code, const voi
                                         2 * ((wide + kStepWorkgroups - 1) / kStepWorkgroups);
     const int est_heads = narrow ? 4 : kFusedHeads;
     const bool share = est_share(batch, est_heads, num_heads, num_kv_heads);
-    const bool stream_codes = !share && !(flags & ADAMAS_F_CODES_CACHED);  // (as in est_stream)
+    const bool stream_codes = est_stream(flags, false, share, 0u, uint64_t{batch} * max_seq_len * num_kv_heads);
     const dim3 grid(n_chunks, num_heads / est_heads, batch);
     StepGeom hist_geom;
     hist_geom.units_q = chunk_tokens / kStepUnit;
@@ -1665,7 +1677,7 @@ extern "C" int adamas_decode_step_f(const void* q, const void* q_code, const voi
                                 static_cast<int64_t>(n_sel), (max_seq_len > 1) ? n_sel : 0u, out,
                                 workspace, workspace_bytes, batch, num_heads, num_kv_heads,
                                 head_dim, page_size, sm_scale, max_seq_len,
-                                flags & ~ADAMAS_F_CODES_CACHED, stream);  // (a hint for the step's own kernels)
+                                flags & ~kCodesFlags, stream);  // (hints for the step's own kernels)
 }
 
 extern "C" int adamas_decode_step(const void* q, const void* q_code, const void* kv_data,
@@ -1693,8 +1705,8 @@ extern "C" int adamas_decode_layer_step(const void* qkv, const float* cos_table,
                                         float hadamard_scale, uint32_t flags,
                                         adamas_stream_t stream) {
   if (!qkv || !cos_table || !sin_table || !kv_data || !code_data) return ADAMAS_E_BADARG;
-  if (flags & ~(ADAMAS_F_CODE_FROM_FP32 | ADAMAS_F_BF16 | ADAMAS_F_HND | ADAMAS_F_CODES_CACHED))
-    return ADAMAS_E_BADARG;
+  if (flags & ~(ADAMAS_F_CODE_FROM_FP32 | ADAMAS_F_BF16 | ADAMAS_F_HND | kCodesFlags)) return ADAMAS_E_BADARG;
+  if ((flags & kCodesFlags) == kCodesFlags) return ADAMAS_E_BADARG;
   if ((reinterpret_cast<uintptr_t>(qkv) | reinterpret_cast<uintptr_t>(cos_table) |
        reinterpret_cast<uintptr_t>(sin_table)) & 15)
     return ADAMAS_E_ALIGN;
@@ -1704,8 +1716,8 @@ extern "C" int adamas_decode_layer_step(const void* qkv, const float* cos_table,
   src.sin_table = sin_table;
   src.scale = hadamard_scale;
   src.code_flags = flags;
-  // format and layout of the caches, and the hint about the codes
-  const uint32_t kv_flags = flags & (ADAMAS_F_BF16 | ADAMAS_F_HND | ADAMAS_F_CODES_CACHED);
+  // format and layout of the caches, and the hints about the codes
+  const uint32_t kv_flags = flags & (ADAMAS_F_BF16 | ADAMAS_F_HND | kCodesFlags);
   int rc = step_candidates_impl(nullptr, code_data, page_indices, page_indptr, seq_lens, budget,
                                 workspace, workspace_bytes, batch, num_heads, num_kv_heads,
                                 page_size, max_seq_len, page_table_stride, kv_flags, stream, &src);

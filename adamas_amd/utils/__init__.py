@@ -428,7 +428,7 @@ def decode_step(q: torch.Tensor, q_code: torch.Tensor, iController: InferenceCon
         c.seqs.indptr_dev.data_ptr(), c.seqs.seq_lens_dev.data_ptr(), budget, o.data_ptr(),
         _lib.ptr(sel), ws.data_ptr(), ws.numel(), c.batch_size, c.num_heads, c.num_kv_heads,
         c.head_dim, c.page_size, 1.0 / math.sqrt(c.head_dim), c.max_len_now, c.seqs.max_pages,
-        c.kv_flags | c.codes_hint, _lib.current_stream())
+        c.kv_flags | c.codes_flags, _lib.current_stream())
     _lib.check(rc, "adamas_decode_step")
     return (o, sel) if return_indices else o
 
@@ -767,7 +767,7 @@ def decode_layer_step(qkv: torch.Tensor, cos_table: torch.Tensor, sin_table: tor
         c.pool.codes_address(layer_idx), c.seqs.table_dev.data_ptr(), c.seqs.indptr_dev.data_ptr(),
         c.seqs.seq_lens_dev.data_ptr(), budget, o.data_ptr(), _lib.ptr(sel), ws.data_ptr(), ws.numel(),
         n, nq, nkv, 128, c.page_size, 1.0 / math.sqrt(c.head_dim), c.max_len_now, c.seqs.max_pages,
-        c.hadamard_scale, c.code_flags | c.codes_hint, _lib.current_stream())
+        c.hadamard_scale, c.code_flags | c.codes_flags, _lib.current_stream())
     _lib.check(rc, "adamas_decode_layer_step")
     return (o, sel) if return_indices else o
 

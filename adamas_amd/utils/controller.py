@@ -140,6 +140,12 @@ class InferenceController:
         nbytes = self.num_layers * (tokens * self.num_kv_heads * 2 * CODE_WORDS + rows * self.num_heads * 512)
         return _lib.F_CODES_CACHED if nbytes <= CODES_CACHED_BYTES else 0
 
+    @property
+    def codes_flags(self) -> int:
+        """The flag that says whether the codes stay cached or not, for the library (which without either
+        does not know of the other layers)."""
+        return self.codes_hint or _lib.F_CODES_STREAMED
+
     def workspace(self, budget: int, max_len: Optional[int] = None) -> torch.Tensor:
         """Workspace of the attention kernel and of the step for this token budget and the length
         bound the library is called with (`max_len`, by default max_len_now, which is what the

@@ -111,9 +111,10 @@ def estimator_instance(_lib, page_size: int, heads: int, batch: int, max_seq_len
     flag = lambda v: "true" if v else "false"
     grouped = heads // (kv_heads or heads) % 4 == 0
     share = 4 if grouped and (batch > 1 or p["heads"] == 8) else 1
+    codes = batch * max_seq_len * (kv_heads or heads) * 32   # bytes (no hint is given about the other layers)
     return (f"estimate_select_kernel<{16 if page_size == 16 else 0}, {p['passes']}, "
             f"{flag(p['partial'])}, false, {p['heads']}, false, {share}, "
-            f"{flag(share == 1)}>")
+            f"{flag(share == 1 and (p['heads'] == 8 or codes > 280 << 20))}>")
 
 
 def log(msg: str) -> None:

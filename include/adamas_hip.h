@@ -66,6 +66,11 @@ typedef void* adamas_stream_t;
                                       steps of a layer (every layer, every sequence) stay in the
                                       last-level cache, so the codes are not read past it.  A hint:
                                       the results are the same with and without                       */
+#define ADAMAS_F_CODES_STREAMED 64u /* the opposite, for the same calls: they do not stay there, so the codes
+                                      are read past it wherever that helps.  With neither flag that is done
+                                      in the kernel of eight heads per workgroup, and in the others where
+                                      the codes of the call alone are more than the cache holds.  Both
+                                      together are refused (ADAMAS_E_BADARG)                          */
 
 /* output formats of adamas_estimate / key modes of adamas_topk */
 #define ADAMAS_DIST_FP16 0u /* integer distance stored as fp16 (the reference's output dtype) */
@@ -95,7 +100,8 @@ int adamas_hadamard(const void* x, void* out, uint64_t n_rows, float scale, adam
  *                   the KV cache, the attention output); codes, distances, selections and all
  *                   arithmetic (fp32) are unchanged;
  *   ADAMAS_F_HND  : the other page layout of the KV cache (see the flag);
- *   ADAMAS_F_CODES_CACHED : a hint for the decode step, its two halves and the layer step (see the flag).
+ *   ADAMAS_F_CODES_CACHED, ADAMAS_F_CODES_STREAMED : hints for the decode step, its two halves and the layer
+ *                   step (see the flags).
  * The un-suffixed entry points are flags = 0; the append entry points have taken flags all along;
  * estimate and top-k see neither float data nor KV pages.  Flags an entry point does not know give
  * ADAMAS_E_BADARG.  The reference dispatches fp16 only

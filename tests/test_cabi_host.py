@@ -377,6 +377,25 @@ def test_codes_cached_hint():
                                       _lib.F_CODES_CACHED, None) == -1
 
 
+def test_hints_about_the_codes():
+    """Either of them for the step, its halves and the layer step, not both; neither for the operators."""
+    lib = _lib.load()
+    cached, streamed = _lib.F_CODES_CACHED, _lib.F_CODES_STREAMED
+    for hint, want in ((cached, -2), (streamed, -2), (cached | streamed, -1)):    # (head_dim 64, 4 heads: refused later)
+        tail = (hint, None)
+        assert lib.adamas_decode_step_f(*[16] * 7, 8, 16, None, 256, 1 << 40, 1, 32, 32, 64, 16, 1.0, 100, 8, *tail) == want
+        assert lib.adamas_step_candidates_f(*[16] * 5, 8, 256, 1 << 40, 1, 4, 4, 16, 100, 8, *tail) == want
+        assert lib.adamas_step_attend_f(*[16] * 6, 8, 16, None, 256, 1 << 40, 1, 32, 32, 64, 16, 1.0, 100, 8, *tail) == want
+        assert lib.adamas_decode_layer_step(*[16] * 8, 8, 16, None, 256, 1 << 40, 1, 4, 4, 128, 16, 1.0, 100, 8, 1.0,
+                                            *tail) == want
+        assert lib.adamas_sparse_decode_f(*[16] * 5, None, 0, 0, 16, None, 0, 1, 32, 32, 64, 16, 1.0, 100, *tail) == -1
+    c = _ctrl(num_layers=3)
+    c._len_bound = 1 << 20
+    assert c.codes_flags == streamed
+    c._len_bound = 1
+    assert c.codes_flags == cached
+
+
 @pytest.mark.parametrize("length", [2, 4096, 140000])
 def test_general_path_of_the_step_takes_the_codes_hint(length):
     """The step hands a budget of one token to the attention operator, which does not know the hint; without

@@ -139,6 +139,36 @@ def test_step_of_narrow_workgroups_reads_codes_through_and_past_the_caches(gpu_d
     assert torch.equal(got[0][1].sort(dim=1).values, ctrl.topk_dindices_buffer.sort(dim=1).values)
 
 
+@pytest.mark.parametrize("lens,budget,cached,unknown", [
+    ([4096], 64, False, False), ([700, 5000, 513], 100, False, False),    # selection, narrow workgroups
+    ([32768], 128, True, True),                                           # wide ones on the whole chip
+    ([4096], 600, False, False), ([700, 5000, 513], 600, False, False),   # histograms
+    ([19000] + [600] * 15, 100, False, True),                             # 16 * 19000 tokens: 311 MB of codes at most
+])
+def test_step_reads_codes_past_the_caches_when_told_so(gpu_device, lens, budget, cached, unknown):
+    """The last template argument of the estimator that is launched, for each hint and for none."""
+    from torch.profiler import ProfilerActivity, profile
+    from adamas_amd import _lib
+    c, q, q_code = _controller(gpu_device, lens, budget, 16, 32, torch.float16, 0, 7)
+    o, ws = torch.empty_like(q), c.workspace(budget)
+
+    def launched(flags):
+        with profile(activities=[ProfilerActivity.CUDA]) as p:
+            rc = _lib.load().adamas_decode_step_f(
+                q.data_ptr(), q_code.data_ptr(), c.pool.kv.data_ptr(), c.pool.codes.data_ptr(),
+                c.seqs.table_dev.data_ptr(), c.seqs.indptr_dev.data_ptr(), c.seqs.seq_lens_dev.data_ptr(), budget,
+                o.data_ptr(), None, ws.data_ptr(), ws.numel(), len(lens), 32, 32, 128, 16, 128 ** -0.5, max(lens),
+                c.seqs.max_pages, flags, _lib.current_stream())
+            assert rc == 0
+            torch.cuda.synchronize()
+        name = next(e.name for e in p.events() if "estimate_select_kernel" in e.name)
+        return {"true": True, "false": False}[name.split("<")[1].split(">")[0].split(", ")[-1]]
+
+    assert launched(_lib.F_CODES_STREAMED)
+    assert launched(_lib.F_CODES_CACHED) == cached
+    assert launched(0) == unknown
+
+
 @pytest.mark.parametrize("lens,budget,kv_heads", [
     ([4096], 1, 32), ([3000, 700], 1, 8),     # nothing is selected
     ([140000], 300, 32), ([140000], 1000, 8), # longer than the histograms go
