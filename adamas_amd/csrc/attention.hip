@@ -985,10 +985,11 @@ extern "C" size_t adamas_workspace_bytes(uint32_t batch, uint32_t num_heads, uin
 // in flight per group of 16 lanes, rows per round and rounds' worth of workgroups (see the rule at kTile).  Two
 // rows in flight instead of four give twice the workgroups, half the rows each: better as long as they all
 // run at once.  Two / four, 32:32 heads, us a launch with its append: 3 sequences of 600 to 1500 21.6 / 17.9, 16
-// of 150 to 250 21.9 / 17.3, 2 of 600 to 1000 13.2 / 13.4; 32:8 heads, 8 of 150 to 250 12.4 / 13.0; one sequence of 1000
-// 10.9 / 11.3, 1400 12.3 / 12.3, 2000 14.4 / 13.4.  That last microsecond is left: splits of 256 rows add up in another
-// order than those of 128, and the dense layers of a decoder hand that rounding on to every later code threshold
-// (three layers, a prompt of 2000 tokens: the logits moved by up to 5e-3).
+// of 150 to 250 21.9 / 17.3, 2 of 600 to 1000 13.2 / 13.4; 32:8 heads, 8 of 150 to 250 12.4 / 13.0.  One sequence, alone: 32:32
+// heads 1409 positions 10.6 / 10.5, 2000 12.4 / 11.7, 32:8 1500 9.9 / 10.3, 2000 10.8 / 9.2, 16:2 1700 8.9 / 10.0, 8:8 2000
+// 7.9 / 8.7.  It keeps two up to 2048 rows, also where four are a little faster: splits of 256 rows add up in
+// another order than those of 128, and the dense layers of a decoder hand that rounding on to every later code
+// threshold (three layers, a prompt of 2000 tokens: the logits moved by up to 5e-3).
 struct RowLaunch {
   uint32_t threads, tile, rows_per_iter;
   uint64_t workgroups;
@@ -1020,7 +1021,9 @@ static RowLaunch row_launch(uint64_t heads, uint32_t n_rows) {
 //   - Beyond, 32:32 heads: 32 sequences of 160 23.9 / 24.6, 64 50.3 / 36.6, 4 of 1000 19.6 / 20.5, 8 33.4 /
 //     30.1; 32:8 heads: 8 of 256 9.9 / 13.8, 16 18.6 / 15.2, 2 of 1000 10.0 / 13.6.  Groups of more than 256 tokens
 //     also as long as the row kernel's workgroups all run at once (launch with its append): 32:8 heads, 2 of 2000 14.9 /
-//     16.1, 4 of 1000 15.2 / 17.6, 8 of 500 15.3 / 17.6, but 3 of 1300 21.6 / 17.6, 12 of 340 20.0 / 17.6.  A single
+//     16.1, 4 of 1000 15.2 / 17.6, 8 of 500 15.3 / 17.6, but 3 of 1300 21.6 / 17.6, 12 of 340 20.0 / 17.6; other groups
+//     (alone): 2 of 1000 to 2000 12.0 / 13.8, 11.1 / 13.7, 11.5 / 11.9 and 11.0 / 12.4 at 32:16, 32:4, 32:2 and 24:8, 16.4 /
+//     15.9 at 40:8; 2 of 600 to 1000 11.1 / 15.2 at 64:8, 10.8 / 13.1 at 48:8; 16 of 100 to 512 10.8 / 14.8 at 16:2.  A single
 //     group of eight heads fills fewer workgroups: 32 of 1000 32.7 / 37.5 at 8:8, 64 70.9 / 63.3; 16 17.3 /
 //     18.6 at 8:4, 32 29.8 / 20.7.
 static bool dense_as_rows(uint32_t batch, uint32_t num_heads, uint32_t group, uint32_t max_seq_len) {

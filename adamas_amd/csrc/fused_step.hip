@@ -890,11 +890,14 @@ constexpr uint32_t kHsaMaxTokens = kHsaMaxSlab * 32;             // 32 slabs per
 // (beyond that the merge inside the launch costs more than the shorter gather saves).  Measured
 // against slabs of 4096 tokens throughout: 8192 tokens, budget 4096: 41.0 -> 24.8 us; 16384 / 1024:
 // 20.1 -> 18.4; 32768 / 1024: 23.3 -> 22.7; a target of 32 rows or a cap of 32 slabs is slower.  In
-// batches slabs of 2048 tokens are taken where those of 1024 are clearly more than run at once (six to a CU, by
-// their registers): each sums the chunk rows of its head once more.  1024 / 2048 / 4096 tokens, us a layer at 32:32 and 32:8
+// batches slabs of 2048 tokens are taken where those of 1024 are clearly more than run at once (six to a CU in
+// fp16, by their registers): each sums the chunk rows of its head once more.  1024 / 2048 / 4096 tokens, us a layer at 32:32 and 32:8
 // heads: 16 sequences of 2000 to 7500, budget 512, 57.5 / 55.2 / 55.5 and 49.4 / 46.9 / 47.2; 8 of 4000 to 15000, 3000,
 // 116.6 / 110.0 / 107.2 and 91.5 / 87.7 / 88.7; 10 of 5000 to 12000, 2000, 104.2 / 103.4 / 114.2 and 80.6 / 82.0 / 92.8;
-// with fewer workgroups, 2 of 3000 to 6000, 600, 20.4 / 22.4 / 22.8 and 20.0 / 21.9 / 22.6.
+// with fewer workgroups, 2 of 3000 to 6000, 600, 20.4 / 22.4 / 22.8 and 20.0 / 21.9 / 22.6.  In bf16 (96 to 100
+// registers, four or five to a CU) the line would lie lower: with 1280 to 1792 workgroups of 1024 / 2048 tokens 8 of 5500
+// to 6100, 512, 36.9 / 35.7 and 32.8 / 31.8, 16 of 1000 to 3000, 600, 49.7 / 47.3 and 45.2 / 43.5, 5 of 6000 to 8100, 600,
+// 31.1 / 31.2 and 27.9 / 29.8; fp16 34.1 / 35.4 and 31.1 / 32.1, 48.1 / 48.0 and 43.6 / 43.6, 30.4 / 31.2 and 28.1 / 29.1.
 // Above ten slabs of 1024 tokens those of 2048 are taken where 512 threads work on each (hsa_threads) and
 // more than 64 workgroups are left: half as many partials to merge.  1024 / 2048 tokens, 32:32 and 32:8 heads:
 // 12000 tokens, budget 1024 19.5 / 19.1 and 18.8 / 18.4; 16384, 1024 20.3 / 19.6 and 19.4 / 18.6; 2 sequences of
@@ -918,7 +921,7 @@ inline int hsa_items(uint32_t max_seq_len, uint32_t budget, uint64_t heads) {
 }
 
 // Threads per workgroup for slabs of 256 * items tokens.  While there are at most two workgroups of 512 to a CU
-// (three run at once), they take slabs of 2048 and 4096 tokens: their serial parts, the chunk rows
+// (in fp16 three run at once, in bf16 two), they take slabs of 2048 and 4096 tokens: their serial parts, the chunk rows
 // per part and the rows per group, are half as long, and a CU that has one or two workgroups has eight waves for
 // each.  In us a layer with 256 / 512 threads, 32:32 and 32:8 heads, one sequence: 12000 tokens, budget 300
 // 18.5 / 17.8 and 17.7 / 16.9; 24000, 512 21.4 / 21.0 and 20.5 / 20.0; 32768, 2048 27.9 / 26.1 and 25.6 / 22.7;
@@ -1247,9 +1250,8 @@ static bool est_share(uint32_t batch, int est_heads, uint32_t num_heads, uint32_
 // alone are too many.  What a caller who says nothing about a few cached layers would lose otherwise, a step of 32:32
 // heads through / past: budget 600, 4096 tokens 14.2 / 14.6, 16000 16.1 / 16.8; 128, 4 sequences of 1500 to 7000 14.0 /
 // 14.4; 64, 4096 tokens 9.9 / 9.8, this launch alone and repeated 5.0 / 5.4; 128, 8192 tokens 11.0 / 10.5.
-// In us per layer with the layers in turn,
-// through / past the caches.  Selection: 32 heads, 16 sequences of 8192 to 32768 tokens, 1 layer (335 MB of codes)
-// 88.2 / 80.1, 2 layers 87.0 / 77.0; 8 of 1500 to 7000, 4 layers (139 MB) 22.8 / 23.0, 8 layers 24.0 / 21.9; one
+// In us per layer with the layers in turn, through / past the caches.  Selection: 32 heads, 16 sequences of 8192 to 32768
+// tokens, 1 layer (335 MB of codes) 88.2 / 80.1, 2 layers 87.0 / 77.0; 8 of 1500 to 7000, 4 layers (139 MB) 22.8 / 23.0, 8 layers 24.0 / 21.9; one
 // sequence of 4096, 8 layers (34 MB) 12.8 / 12.8, 80 layers 14.0 / 12.9; 8 heads, 131072, 7 layers (235 MB) 23.2 / 25.7, 9
 // layers 27.2 / 25.6.  Histograms, budget 512: 16 of 4000 to 16000, 1 layer (164 MB) 82.6 / 81.9, 2 layers
 // 88.8 / 81.6; 65536 tokens, 4 layers (268 MB) 31.9 / 32.7, 8 layers 32.6 / 31.7.

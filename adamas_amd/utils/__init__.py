@@ -518,8 +518,6 @@ def prefill_forward(q: torch.Tensor, iController: InferenceController, layer_idx
 def _prefill(q: torch.Tensor, c: InferenceController, layer_idx: int, length: int,
              device: int) -> torch.Tensor:
     """The kernel behind prefill_forward, on q's device, which is the current one."""
-    if layer_idx < 0:   # (as KvCache.buf_layer)
-        raise IndexError("layer index out of range")
     n = q.shape[0]
     if q.data_ptr() % 16:   # a view into the middle of something: the kernel reads 128 bits at a time
         q = q.clone()
