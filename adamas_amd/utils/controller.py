@@ -134,7 +134,8 @@ class InferenceController:
 
     @property
     def codes_hint(self) -> int:
-        """F_CODES_CACHED for the decode step where the codes of all layers stay cached between tokens."""
+        """F_CODES_CACHED for the decode step where the codes of all layers stay cached between tokens (the rows
+        that a full budget selects are counted, also for sequences that are shorter)."""
         tokens = sum(self.seqs.lengths) if self._len_bound is None else self.batch_size * self._len_bound
         rows = self.batch_size * (self.inference_page_budget or 0)
         nbytes = self.num_layers * (tokens * self.num_kv_heads * 2 * CODE_WORDS + rows * self.num_heads * 512)

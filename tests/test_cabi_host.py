@@ -360,7 +360,8 @@ def test_prefill_plan_is_quick(args):
 
 
 def test_codes_cached_hint():
-    """The controller's hint goes by the codes of all layers and sequences: 32 bytes per token and head."""
+    """The controller's hint goes by what a token reads in all layers and sequences: codes, 32 bytes per token
+    and key/value head, and here no selected rows."""
     from adamas_amd.utils.controller import CODES_CACHED_BYTES
     c = _ctrl(num_layers=3, batch_size=2)
     c.seqs.lengths[:] = [5, 7]
@@ -375,6 +376,24 @@ def test_codes_cached_hint():
     assert lib.adamas_decode_step_f(*step, 2 * _lib.F_CODES_CACHED, None) == -1
     assert lib.adamas_sparse_decode_f(*[16] * 5, None, 0, 0, 16, None, 0, 1, 32, 32, 64, 16, 1.0, 100,
                                       _lib.F_CODES_CACHED, None) == -1
+
+
+@pytest.mark.parametrize("kv_heads", [32, 8])
+def test_codes_cached_hint_of_a_ragged_batch_with_a_budget(kv_heads):
+    """Eager steps count the tokens that are there, and with them the selected K and V rows of every query head."""
+    from adamas_amd.utils.controller import CODES_CACHED_BYTES
+    layers, budget = 40, 100
+    c = _ctrl(num_layers=layers, batch_size=3, num_kv_heads=kv_heads)
+    rows = layers * 3 * budget * 32 * 2 * 256
+    edge = (CODES_CACHED_BYTES - rows) // (layers * kv_heads * 32)     # tokens
+    c.inference_page_budget = budget
+    for tokens, want in ((edge, _lib.F_CODES_CACHED), (edge + 1, 0)):
+        c.seqs.lengths[:] = [tokens - 900, 700, 200]
+        assert c._len_bound is None and c.codes_hint == want
+    c.inference_page_budget = None
+    assert c.codes_hint == _lib.F_CODES_CACHED
+    c.seqs.lengths[0] = CODES_CACHED_BYTES // (layers * kv_heads * 32) - 899
+    assert c.codes_hint == 0
 
 
 def test_hints_about_the_codes():
