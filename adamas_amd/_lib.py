@@ -162,4 +162,7 @@ def ptr(t) -> int | None:
 
 def current_stream() -> int:
     """The current stream of the current device (2.7 us less than by way of a torch.cuda.Stream object)."""
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    try:
+        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    except AttributeError:   # (not public names: another torch may lack them)
+        return torch.cuda.current_stream().cuda_stream

@@ -396,6 +396,15 @@ def test_codes_cached_hint_of_a_ragged_batch_with_a_budget(kv_heads):
     assert c.codes_hint == 0
 
 
+def test_current_stream_without_the_private_names(monkeypatch):
+    """Falls back to the stream object where torch lacks them."""
+    class Stream:
+        cuda_stream = 77
+    monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream")
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: Stream)
+    assert _lib.current_stream() == 77
+
+
 def test_hints_about_the_codes():
     """Either of them for the step, its halves and the layer step, not both; neither for the operators."""
     lib = _lib.load()
