@@ -216,40 +216,42 @@ struct MergeShared {
   static constexpr int kWavesM = kGroups / 4;
   float m[kWavesM];
   float l[kWavesM];
-  float o[kWavesM][kHeadDim];
+  alignas(16) float o[kWavesM][kHeadDim];
 };
 
-// Folds the state of the lane `delta` lanes away into this lane's state (both hold the same channels).
-__device__ __forceinline__ void fold_state(SoftmaxState& st, int delta) {
-  const float m_o = __shfl_xor(st.m, delta);
-  const float l_o = __shfl_xor(st.l, delta);
-  const float m_n = fmaxf(st.m, m_o);
-  const float a = exp2_raw(st.m - m_n), b = exp2_raw(m_o - m_n);
-  st.l = st.l * a + l_o * b;
+// Folds the states of two 16-lane groups of a wave, the groups kDelta / 16 apart, channel by channel: both end up
+// with the result of the lower group.  Lane swaps of the vector unit, no trip through the LDS crossbar: a layer of a step
+// over 4096 tokens, budget 64, 12.35 -> 12.20 us.
+template <int kDelta>
+__device__ __forceinline__ void fold_state(SoftmaxState& st) {
+  static_assert(kDelta == 16 || kDelta == 32, "groups of one wave");
+  // lo: the lower group's value in both groups, hi: the upper group's
+  auto both = [](float x, float& lo, float& hi) __attribute__((always_inline)) {
+    const uint32_t u = __float_as_uint(x);
+    const auto r = kDelta == 16 ? __builtin_amdgcn_permlane16_swap(u, u, false, false)
+                                : __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    lo = __uint_as_float(r[0]);
+    hi = __uint_as_float(r[1]);
+  };
+  float m0, m1, l0, l1;
+  both(st.m, m0, m1);
+  both(st.l, l0, l1);
+  st.m = fmaxf(m0, m1);
+  const float a = exp2_raw(m0 - st.m), b = exp2_raw(m1 - st.m);
+  st.l = l0 * a + l1 * b;
 #pragma unroll
-  for (int j = 0; j < 8; ++j) st.o[j] = st.o[j] * a + __shfl_xor(st.o[j], delta) * b;
-  st.m = m_n;
+  for (int j = 0; j < 8; ++j) {
+    float o0, o1;
+    both(st.o[j], o0, o1);
+    st.o[j] = o0 * a + o1 * b;
+  }
 }
 
-// Merges the kGroups group states of a workgroup (kGroups / 4 waves).  After the call the threads
-// tid < 128 hold, for channel tid, the merged maximum M, denominator L and numerator O.
+// Merges the states of the waves that lie in LDS, for channel tid < 128 (see merge_groups).
 template <int kGroups>
-__device__ __forceinline__ void merge_groups(SoftmaxState st, uint32_t g, uint32_t c,
-                                             uint32_t tid, MergeShared<kGroups>& sh, float& M,
-                                             float& L, float& O) {
+__device__ __forceinline__ void merge_waves(uint32_t tid, const MergeShared<kGroups>& sh, float& M, float& L,
+                                            float& O) {
   constexpr int kWavesM = kGroups / 4;
-  fold_state(st, 16);
-  fold_state(st, 32);  // every lane now holds the state of its wave for channels 8c .. 8c+7
-  const uint32_t w = g >> 2;
-  if ((g & 3u) == 0) {
-    if (c == 0) {
-      sh.m[w] = st.m;
-      sh.l[w] = st.l;
-    }
-#pragma unroll
-    for (int j = 0; j < 8; ++j) sh.o[w][8 * c + j] = st.o[j];
-  }
-  __syncthreads();
   M = kNegBig;
   L = 0.f;
   O = 0.f;
@@ -263,6 +265,27 @@ __device__ __forceinline__ void merge_groups(SoftmaxState st, uint32_t g, uint32
       O += sh.o[i][tid] * wgt;
     }
   }
+}
+
+// Merges the kGroups group states of a workgroup (kGroups / 4 waves).  After the call the threads
+// tid < 128 hold, for channel tid, the merged maximum M, denominator L and numerator O.
+template <int kGroups>
+__device__ __forceinline__ void merge_groups(SoftmaxState st, uint32_t g, uint32_t c,
+                                             uint32_t tid, MergeShared<kGroups>& sh, float& M,
+                                             float& L, float& O) {
+  fold_state<16>(st);
+  fold_state<32>(st);  // every lane now holds the state of its wave for channels 8c .. 8c+7
+  const uint32_t w = g >> 2;
+  if ((g & 3u) == 0) {
+    if (c == 0) {
+      sh.m[w] = st.m;
+      sh.l[w] = st.l;
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) sh.o[w][8 * c + j] = st.o[j];
+  }
+  __syncthreads();
+  merge_waves(tid, sh, M, L, O);
 }
 
 // query fragment of a lane: 8 channels, pre-multiplied by sm_scale * log2(e)

@@ -44,6 +44,24 @@ __device__ __forceinline__ uint32_t wave_inclusive_scan_dpp(uint32_t v) {
   return static_cast<uint32_t>(x);
 }
 
+// inclusive prefix sum over the first kLanes (4 or 8) lanes of every row of 16
+template <int kLanes>
+__device__ __forceinline__ uint32_t row_inclusive_scan(uint32_t v) {
+  static_assert(kLanes == 4 || kLanes == 8, "two or three steps");
+  int x = static_cast<int>(v);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, false);  // row_shr:1
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, false);  // row_shr:2
+  if (kLanes == 8) x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, false);  // row_shr:4
+  return static_cast<uint32_t>(x);
+}
+
+// sum over the first kLanes lanes of the wave, uniform
+template <int kLanes>
+__device__ __forceinline__ uint32_t sum_of_first(uint32_t v) {
+  return static_cast<uint32_t>(
+      __builtin_amdgcn_readlane(static_cast<int>(row_inclusive_scan<kLanes>(v)), kLanes - 1));
+}
+
 // Per-lane exclusive prefix (below | tied << 16) over the lower lanes of the wave, for class masks
 // spread over kRegs registers per lane (4 items each, item order = register order); `total` gets the
 // wave totals.
@@ -215,11 +233,9 @@ struct WavePlan {
   uint32_t n_take;   // k, or the number of keys if that is smaller
 };
 
-__device__ __forceinline__ WavePlan wave_plan_from_hist(const uint32_t* hist_lds, uint32_t k) {
+// counts of bins 8*lane .. 8*lane+7
+__device__ __forceinline__ WavePlan wave_plan_from_counts(const uint32_t (&c)[8], uint32_t k) {
   const int lane = lane_id();
-  const uint4 hv0 = *reinterpret_cast<const uint4*>(&hist_lds[8 * lane]);
-  const uint4 hv1 = *reinterpret_cast<const uint4*>(&hist_lds[8 * lane + 4]);
-  const uint32_t c[8] = {hv0.x, hv0.y, hv0.z, hv0.w, hv1.x, hv1.y, hv1.z, hv1.w};
   uint32_t lane_sum = 0;
 #pragma unroll
   for (int j = 0; j < 8; ++j) lane_sum += c[j];
@@ -233,14 +249,14 @@ __device__ __forceinline__ WavePlan wave_plan_from_hist(const uint32_t* hist_lds
     p.n_take = total;
     return p;
   }
-  // exactly one bin holds the k-th smallest key; its lane finds it among its 8 bins
-  uint32_t run = incl - lane_sum, t_l = 0, nb_l = 0;
+  // exactly one bin holds the k-th smallest key; its lane finds it among its 8 bins: behind those whose
+  // running count stays below k
+  uint32_t run = incl - lane_sum, t_l = 8u * static_cast<uint32_t>(lane), nb_l = run;
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
-    const bool here = run < k && run + c[j] >= k;
-    t_l = here ? 8u * static_cast<uint32_t>(lane) + j : t_l;
-    nb_l = here ? run : nb_l;
     run += c[j];
+    t_l += run < k ? 1u : 0u;
+    nb_l = run < k ? run : nb_l;
   }
   const uint64_t cross = __ballot(incl - lane_sum < k && incl >= k);
   const int src = __builtin_amdgcn_readfirstlane(__ffsll(static_cast<long long>(cross)) - 1);
@@ -249,6 +265,14 @@ __device__ __forceinline__ WavePlan wave_plan_from_hist(const uint32_t* hist_lds
   p.quota = k - p.n_below;
   p.n_take = k;
   return p;
+}
+
+__device__ __forceinline__ WavePlan wave_plan_from_hist(const uint32_t* hist_lds, uint32_t k) {
+  const int lane = lane_id();
+  const uint4 hv0 = *reinterpret_cast<const uint4*>(&hist_lds[8 * lane]);
+  const uint4 hv1 = *reinterpret_cast<const uint4*>(&hist_lds[8 * lane + 4]);
+  const uint32_t c[8] = {hv0.x, hv0.y, hv0.z, hv0.w, hv1.x, hv1.y, hv1.z, hv1.w};
+  return wave_plan_from_counts(c, k);
 }
 
 // One wave: the kc smallest of its 64 x kItems keys (lane l holds items kItems*l .. kItems*l +

@@ -33,6 +33,12 @@ __device__ __forceinline__ void wait_own_stores() {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
+// A word of memory that nothing writes during the launch, at an address that is the same in the whole wave: a
+// scalar load wherever the compiler stands.
+__device__ __forceinline__ int32_t load_scalar(const int32_t* p) {
+  return *(const __attribute__((address_space(4))) int32_t*)(reinterpret_cast<uintptr_t>(p));
+}
+
 __device__ __forceinline__ int lane_id() { return static_cast<int>(threadIdx.x) & 63; }
 
 // 4-level bucket of a Hadamard output value: (v > -10) + (v > 0) + (v > 10).
@@ -95,6 +101,23 @@ __device__ __forceinline__ void store_elem(__half* p, float x) {
 inline uint32_t group_inv16(uint32_t group) { return (65536u + group - 1u) / group; }
 __device__ __forceinline__ uint32_t kv_head_of(uint32_t head, uint32_t inv16) {
   return (head * inv16) >> 16;
+}
+
+// Query head of workgroup x of a launch with one workgroup per query head (times whatever else): the workgroups
+// of the query heads that share a key/value head lie num_kv_heads apart, i.e. on one die where that is a multiple
+// of the eight dies or the other way round, and find each other's rows in its L2.  order16 is the 16-bit
+// reciprocal of num_kv_heads, or 0 to take the heads as they come (one query head per key/value head, or
+// head counts beyond what the reciprocal divides exactly).
+inline uint32_t head_order16(uint32_t num_heads, uint32_t num_kv_heads) {
+  const bool grouped = num_heads != num_kv_heads && static_cast<uint64_t>(num_heads) * num_kv_heads < 65536u;
+  return grouped ? group_inv16(num_kv_heads) : 0u;
+}
+__device__ __forceinline__ uint32_t head_of_block(uint32_t x, uint32_t num_heads, uint32_t num_kv_heads,
+                                                  uint32_t order16) {
+  if (order16 == 0u) return x;
+  const uint32_t i = (x * order16) >> 16;  // x / num_kv_heads: which of its group
+  const uint32_t kv = x - i * num_kv_heads;
+  return kv * ((num_heads * order16) >> 16) + i;
 }
 
 // Physical location of logical token t of a sequence whose page table starts at `table`.

@@ -931,72 +931,97 @@ inline int hsa_threads(int items, uint64_t workgroups) {
   return items >= 8 && workgroups <= kHsaWideWorkgroups ? kHsaWideThreads : kHsaThreads;
 }
 
-// Chunk rows a thread asks for at a time (four threads share a bin group).  More in flight help one
-// sequence a little (23989 tokens, 32:8 heads: 19.7 us with 4, 18.9 with 12) but cost the registers that
-// keep more workgroups on a CU in batches (8 sequences of up to 7000: 30.4 us with 4, 32.5 with 12).
-constexpr int kHsaRows = 4;
+// Chunk rows a wave asks for at a time.  Workgroups of 512 threads, few to a CU, ask for all rows of a
+// sequence at once (at most 64); in batches the registers are worth more as workgroups.
+template <int kThreads>
+constexpr int kHsaRows = kThreads == kHsaWideThreads ? 8 : 4;
 typedef uint32_t fs_uint4 __attribute__((ext_vector_type(4)));
 
 template <int kThreads, int kItems>
 struct HistSelectAttendShared {
   static constexpr int kWaves = kThreads / kWave;
-  alignas(16) uint32_t all[kWaves][kHistBins];  // partial sums over all chunk rows
-  alignas(16) uint32_t pre[kWaves][kHistBins];  // partial sums over the chunk rows before the slab
-  uint32_t wtot[kWaves], wpre[kWaves], wclass[kWaves];
-  uint32_t pre_tied;   // tokens at the threshold distance in the chunks before the slab
-  SelectPlan plan;
+  // the sum of the chunk rows each wave has read, two 16-bit bins per word: a wave reads at most 16 rows of
+  // 2048 tokens (static_assert in the kernel), so no bin exceeds 32768
+  alignas(16) uint32_t hist[kWaves][kHistBins / 2];
+  alignas(16) uint4 plan;            // WavePlan
+  // per wave: its keys below | at the threshold << 16, tokens before the slab in its rows at it and below it
+  alignas(16) uint4 wcount[kWaves];
   int32_t rows[kThreads * kItems + 1];  // K rows of the slab's selected tokens (slab 0: then the current token)
   MergeShared<kThreads / 16> merge;
   uint32_t is_last;
 };
 
+// Bound by the chain of memory round trips and barriers and, with several workgroups to a CU, by the instructions in
+// front of the gather.  So the chunk rows are added as they are, two bins to a word; one wave reads the threshold off
+// the sum while the others leave it the issue slots; only the one bin that decides the ties is counted before the slab
+// (the bins below it too where the caller wants positions); nothing waits for the current token's page; and all waves
+// of the last workgroup of a head read its partials.  In batches the workgroups of the heads that share a key/value
+// head lie on one die (head_of_block; 1.3 %, one sequence loses 0.6 %: it is not bound by its bytes).  us a layer of
+// a step before / now: 23989 tokens, 32:8 heads, bf16, budget 1024 20.9 / 20.2; 8 sequences of 1500 to 7000, 32:8
+// heads, 512, 31.5 / 30.3.  Where the time goes in the first of these, 9.5 us from the first workgroup's start to the
+// last one's end: loads 1.3, sum and threshold 0.7, selection 0.7, rows and softmax 2.0 to 2.7, merge of the waves
+// 1.0, partial out and counter 1.2, merge of the slabs 1.2, the rest is workgroups that share a CU.
 template <bool kBf16, bool kHnd, int kThreads, int kItems>
 __global__ __launch_bounds__(kThreads) void hist_select_attend_kernel(
-    const uint16_t* __restrict__ dist, const uint16_t* __restrict__ hist,
-    const uint32_t* __restrict__ rowmap, const int32_t* __restrict__ seq_lens, int64_t dist_stride,
-    uint32_t n_chunks, uint32_t num_heads, uint32_t chunk_tokens, uint32_t k,
-    const __half* __restrict__ q, const __half* __restrict__ kv_data,
-    const int32_t* __restrict__ page_indices, const int32_t* __restrict__ page_indptr,
-    __half* __restrict__ out, int32_t* __restrict__ sel_out, float* partial,
-    uint32_t* __restrict__ counters, uint32_t num_kv_heads, uint32_t kv_inv16, uint32_t page_size,
-    float scale_log2) {
-  constexpr int kWaves = kThreads / kWave, kGroups = kThreads / 16;
-  constexpr int kBins = kHistBins / kThreads;              // bins per thread in the prefix sum
-  static_assert(kBins == 1 || kBins == 2, "256 or 512 threads");
+    const unsigned char* hist, const uint16_t* dist, const uint32_t* rowmap,
+    const int32_t* __restrict__ seq_lens, uint32_t dist_stride, uint32_t n_chunks, uint32_t num_heads, uint32_t chunk_log2, uint32_t k,
+    uint32_t batch, const __half* __restrict__ q, const __half* __restrict__ kv_data,
+    const int32_t* __restrict__ page_indices, const int32_t* __restrict__ page_indptr, __half* __restrict__ out,
+    int32_t* __restrict__ sel_out, float* partial, uint32_t* __restrict__ counters, uint32_t num_kv_heads,
+    uint32_t kv_inv16, uint32_t order16, uint32_t page_size, uint32_t table_stride, float scale_log2) {
+  constexpr int kWaves = kThreads / kWave, kGroups = kThreads / 16, kRows = kHsaRows<kThreads>;
   static_assert(kItems == 4 || kItems == 8 || kItems == 16, "whole histogram rows per slab");
+  // what a bin of a wave's sum can hold: the tokens of its share of the at most 64 chunks
+  constexpr int kBinMost = kStepMaxChunks / kWaves * (kFusedBlock * kFusedMaxPasses);
+  static_assert(kBinMost < 65536, "16-bit sums");
   constexpr uint32_t kSlab = kThreads * kItems;         // tokens per workgroup
   __shared__ HistSelectAttendShared<kThreads, kItems> sh;
-  const uint32_t bh = blockIdx.x, slab = blockIdx.y;
-  const uint32_t b = bh / num_heads, head = bh - b * num_heads;
+  const uint32_t head = head_of_block(blockIdx.x, num_heads, num_kv_heads, order16), b = blockIdx.y, slab = blockIdx.z;
+  const uint32_t bh = b * num_heads + head;
   const uint32_t tid = threadIdx.x;
   const int lane = lane_id();
-  const int wave = wave_id_uniform();
+  const uint32_t wave = static_cast<uint32_t>(wave_id_uniform());
   const uint32_t g = tid >> 4, c16 = tid & 15;
-  int32_t* sdst = sel_out ? sel_out + static_cast<size_t>(bh) * k : nullptr;
   const uint32_t slab_base = slab * kSlab;
-  // ---- everything whose address does not depend on the sequence length is asked for first: thread t
-  // holds the kItems consecutive tokens t*kItems .. of the slab (distances and K rows; past the row's
-  // end some valid piece of it, masked below), thread (part, seg) bins 8*seg .. 8*seg+7 of the first
-  // chunk rows part, part + kWaves, ... (16-bit counts; a row past the sequence holds zeros)
+  const int32_t seq_len = seq_lens[b];
+  auto slabs_of = [&](int32_t len) __attribute__((always_inline)) -> uint32_t {  // slabs that hold past tokens, or one
+    return len > 1 ? (static_cast<uint32_t>(len) - 2u) / kSlab + 1u : 1u;
+  };
+  // a batch has many slabs past the end of a shorter sequence: they leave before they read anything.  One
+  // sequence has few, and does not wait for its length here.
+  if (batch > 1u) {
+    int32_t len = seq_len;
+    asm volatile("" : "+s"(len));  // (the wait stays inside the branch)
+    if (slab >= slabs_of(len)) return;
+  }
+
+  // ---- thread t holds the kItems consecutive tokens t*kItems .. of the slab (distances and K rows; past the
+  // row's end some valid piece of it, masked below), lane l of wave w bins 8*l .. 8*l+7 of the chunk rows
+  // w, w + kWaves, ... (16-bit counts; a row past the sequence holds zeros)
   const uint32_t e0 = slab_base + tid * kItems;
-  const uint32_t part = tid >> 6, seg = tid & 63u;
-  const unsigned char* hb = reinterpret_cast<const unsigned char*>(hist) +
-                            static_cast<size_t>(bh) * n_chunks * (2 * kHistBins) + seg * 16u;
+  const unsigned char* hb = hist + static_cast<size_t>(bh) * n_chunks * (2 * kHistBins);
+  const uint32_t lane16 = static_cast<uint32_t>(lane) * 16u;
   uint32_t keys[kItems], trow[kItems];
-  fs_uint4 hrow[kHsaRows];
+  fs_uint4 hrow[kRows];
   uint32_t kw[kItems / 2];  // two distances per word
+  auto ask_rows = [&](uint32_t c0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < kRows; ++u)
+      hrow[u] = *reinterpret_cast<const fs_uint4*>(
+          hb + static_cast<size_t>(min(c0 + kWaves * u, n_chunks - 1u)) * (2 * kHistBins) + lane16);
+  };
+  ask_rows(wave);
   {
-    const uint16_t* drow = dist + static_cast<int64_t>(bh) * dist_stride;   // 16-byte aligned
-    const uint32_t* rm = rowmap + static_cast<int64_t>(b) * dist_stride;
-    const uint32_t end = static_cast<uint32_t>(dist_stride);                // a multiple of 8
+    const uint16_t* drow = dist + static_cast<size_t>(bh) * dist_stride;   // 16-byte aligned
+    const uint32_t* rm = rowmap + static_cast<size_t>(b) * dist_stride;
     if (kItems == 4) {
-      const uint2 v = *reinterpret_cast<const uint2*>(drow + min(e0, end - 4u));
+      const uint2 v = *reinterpret_cast<const uint2*>(drow + min(e0, dist_stride - 4u));  // (a multiple of 8)
       kw[0] = v.x;
       kw[1] = v.y;
     } else {
 #pragma unroll
       for (int j = 0; j < kItems / 8; ++j) {
-        const uint4 v = *reinterpret_cast<const uint4*>(drow + min(e0 + 8u * j, end - 8u));
+        const uint4 v = *reinterpret_cast<const uint4*>(drow + min(e0 + 8u * j, dist_stride - 8u));
         kw[4 * j] = v.x;
         kw[4 * j + 1] = v.y;
         kw[4 * j + 2] = v.z;
@@ -1004,158 +1029,160 @@ __global__ __launch_bounds__(kThreads) void hist_select_attend_kernel(
       }
     }
 #pragma unroll
-    for (int u = 0; u < kHsaRows; ++u)
-      hrow[u] = *reinterpret_cast<const fs_uint4*>(
-          hb + static_cast<size_t>(min(part + kWaves * u, n_chunks - 1u)) * (2 * kHistBins));
-#pragma unroll
     for (int j = 0; j < kItems / 4; ++j) {
-      const uint4 v = *reinterpret_cast<const uint4*>(rm + min(e0 + 4u * j, end - 4u));
+      const uint4 v = *reinterpret_cast<const uint4*>(rm + min(e0 + 4u * j, dist_stride - 4u));
       trow[4 * j] = v.x;
       trow[4 * j + 1] = v.y;
       trow[4 * j + 2] = v.z;
       trow[4 * j + 3] = v.w;
     }
   }
-  const int32_t seq_len = seq_lens[b];
-  if (seq_len <= 0) {  // a sequence without tokens: zeros and an empty selection
-    if (slab == 0) {
-      if (tid < kHeadDim) store_elem<kBf16>(out + static_cast<size_t>(bh) * kHeadDim + tid, 0.f);
-      if (sdst)
-        for (uint32_t i = tid; i < k; i += kThreads) sdst[i] = -1;
+  const uint32_t n = seq_len > 1 ? static_cast<uint32_t>(seq_len) - 1u : 0u;  // past tokens
+  const uint32_t n_split = slabs_of(seq_len);
+  float qf[8];
+  load_query<kBf16>(q + static_cast<size_t>(bh) * kHeadDim, c16, scale_log2, qf);
+  // the current token is attended with the first slab
+  const uint32_t cur_lp = n / page_size;
+  int32_t cur_page = 0;
+  if (slab == 0 && seq_len > 0)
+    cur_page = load_scalar(page_indices + (table_stride ? static_cast<size_t>(b) * table_stride
+                                                        : static_cast<size_t>(load_scalar(page_indptr + b))) +
+                           cur_lp);
+
+  // ---- chunk rows summed up: all of them, and those before the slab
+  const uint32_t c_first = slab_base >> chunk_log2;  // chunks below it precede the slab (whole chunks)
+  uint32_t acc[4] = {0u, 0u, 0u, 0u}, pre[4] = {0u, 0u, 0u, 0u};
+  auto add_rows = [&](uint32_t c0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < kRows; ++u) {
+      const uint32_t c = c0 + kWaves * u;   // (uniform, as are the conditions)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        acc[j] += c < n_chunks ? hrow[u][j] : 0u;
+        pre[j] = c < c_first ? acc[j] : pre[j];
+      }
     }
+  };
+  add_rows(wave);
+  for (uint32_t c0 = wave + kWaves * kRows; c0 < n_chunks; c0 += kWaves * kRows) {
+    ask_rows(c0);
+    add_rows(c0);
+  }
+  *reinterpret_cast<uint4*>(&sh.hist[wave][4 * lane]) = make_uint4(acc[0], acc[1], acc[2], acc[3]);
+  __syncthreads();
+  asm volatile("" : "+s"(cur_page));  // (not waited for before the barrier)
+  int32_t* sdst = sel_out ? sel_out + static_cast<size_t>(bh) * k : nullptr;
+  if (slab >= n_split) return;
+  if (seq_len <= 0) {  // a sequence without tokens (its one slab): zeros and an empty selection
+    if (tid < kHeadDim) store_elem<kBf16>(out + static_cast<size_t>(bh) * kHeadDim + tid, 0.f);
+    if (sdst)
+      for (uint32_t i = tid; i < k; i += kThreads) sdst[i] = -1;
     return;
   }
-  const uint32_t n = static_cast<uint32_t>(seq_len) - 1u;                 // past tokens
-  const uint32_t n_split = n ? (n + kSlab - 1) / kSlab : 1u;              // slabs that hold tokens
-  if (slab >= n_split) return;
 #pragma unroll
   for (int i = 0; i < kItems; ++i) {
     const uint32_t v = (kw[i >> 1] >> (16 * (i & 1))) & 0xffffu;
     keys[i] = e0 + i < n ? v : 0xffffu;  // past the end: above every threshold
   }
-  float qf[8];
-  load_query<kBf16>(q + static_cast<size_t>(bh) * kHeadDim, c16, scale_log2, qf);
-  const int32_t* table = page_indices + page_indptr[b];
-  const uint32_t rows_per_page = kHnd ? 2u * page_size * num_kv_heads : 2u * page_size;
-  int32_t cur_row = 0;
-  if (slab == 0) {  // the current token is attended with the first slab
-    const uint32_t lp = n / page_size;
-    cur_row = static_cast<int32_t>(static_cast<uint32_t>(table[lp]) * rows_per_page + (n - lp * page_size));
-  }
 
-  // ---- chunk rows summed up: all of them, and those before the slab
-  {
-    const uint32_t c_first = slab_base / chunk_tokens;  // chunks below it precede the slab (whole chunks)
-    const uint32_t rows_used = min(n_chunks, (n + chunk_tokens - 1) / chunk_tokens);  // rows of this sequence
-    uint32_t acc[8] = {0, 0, 0, 0, 0, 0, 0, 0}, pre[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    for (uint32_t c0 = part; c0 < rows_used; c0 += kWaves * kHsaRows) {
-      if (c0 != part) {
+  // ---- the first wave: the sums of all waves -> the plan (the others leave it the issue slots)
+  if (wave == 0u) {
+    uint4 part[kWaves];
 #pragma unroll
-        for (int u = 0; u < kHsaRows; ++u)
-          hrow[u] = *reinterpret_cast<const fs_uint4*>(
-              hb + static_cast<size_t>(min(c0 + kWaves * u, n_chunks - 1u)) * (2 * kHistBins));
-      }
+    for (int p = 0; p < kWaves; ++p) part[p] = *reinterpret_cast<const uint4*>(&sh.hist[p][4 * lane]);
+    __builtin_amdgcn_sched_barrier(0);
+    constexpr int kPacked = 65535 / kBinMost;  // waves whose counts add up in 16 bits: 1 of 4, 3 of 8
+    uint32_t cnt[8] = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};
 #pragma unroll
-      for (int u = 0; u < kHsaRows; ++u) {
-        const uint32_t c = c0 + kWaves * u;
-        const uint32_t used = c < rows_used ? 0xffffffffu : 0u, m = c < c_first ? used : 0u;
+    for (int p = 0; p < kWaves; p += kPacked) {
+      uint32_t w[4] = {part[p].x, part[p].y, part[p].z, part[p].w};
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const uint32_t w = hrow[u][j] & used, wm = hrow[u][j] & m;
-          acc[2 * j] += w & 0xffffu;
-          acc[2 * j + 1] += w >> 16;
-          pre[2 * j] += wm & 0xffffu;
-          pre[2 * j + 1] += wm >> 16;
+      for (int i = 1; i < kPacked; ++i)
+        if (p + i < kWaves) {
+          w[0] += part[p + i].x;
+          w[1] += part[p + i].y;
+          w[2] += part[p + i].z;
+          w[3] += part[p + i].w;
         }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        cnt[2 * j] += w[j] & 0xffffu;
+        cnt[2 * j + 1] += w[j] >> 16;
       }
     }
-    uint4* da = reinterpret_cast<uint4*>(&sh.all[part][seg * 8u]);
-    da[0] = make_uint4(acc[0], acc[1], acc[2], acc[3]);
-    da[1] = make_uint4(acc[4], acc[5], acc[6], acc[7]);
-    uint4* dp = reinterpret_cast<uint4*>(&sh.pre[part][seg * 8u]);
-    dp[0] = make_uint4(pre[0], pre[1], pre[2], pre[3]);
-    dp[1] = make_uint4(pre[4], pre[5], pre[6], pre[7]);
+    const WavePlan p = wave_plan_from_counts(cnt, k);
+    if (lane == 0) sh.plan = make_uint4(p.thr, p.n_below, p.quota, p.n_take);
   }
   __syncthreads();
-  // ---- thread t owns bins kBins*t ..: prefix sum -> the plan
-  uint32_t ca[kBins] = {}, cp[kBins] = {};
-#pragma unroll
-  for (int p = 0; p < kWaves; ++p) {
-#pragma unroll
-    for (int j = 0; j < kBins; ++j) {  // (neighbours: one 64-bit read where there are two)
-      ca[j] += sh.all[p][kBins * tid + j];
-      cp[j] += sh.pre[p][kBins * tid + j];
-    }
+  WavePlan plan;
+  {
+    const uint4 p = sh.plan;
+    plan.thr = __builtin_amdgcn_readfirstlane(p.x);
+    plan.n_below = __builtin_amdgcn_readfirstlane(p.y);
+    plan.quota = __builtin_amdgcn_readfirstlane(p.z);
+    plan.n_take = __builtin_amdgcn_readfirstlane(p.w);
   }
-  const uint32_t incl = wave_inclusive_scan_dpp(kBins == 2 ? ca[0] + ca[kBins - 1] : ca[0]);
-  if (lane == kWave - 1) sh.wtot[wave] = incl;
-  __syncthreads();
-  uint32_t cum = incl;  // tokens with a distance <= the thread's last bin
-  for (int w = 0; w < wave; ++w) cum += sh.wtot[w];
-  const uint32_t cum_all = cum;
-#pragma unroll
-  for (int j = kBins - 1; j >= 0; --j) {
-    const uint32_t less = cum - ca[j];  // with a smaller distance than bin kBins*t + j
-    if (cum >= k && less < k) {         // exactly one bin holds the k-th smallest distance
-      sh.plan.thr = kBins * tid + j;
-      sh.plan.n_below = less;
-      sh.plan.quota = k - less;
-      sh.plan.n_take = k;
-      sh.pre_tied = cp[j];
-    }
-    cum = less;
-  }
-  if (tid == kThreads - 1 && cum_all < k) {  // fewer tokens than k: all of them are taken
-    sh.plan.thr = kHistBins;
-    sh.plan.n_below = cum_all;
-    sh.plan.quota = 0;
-    sh.plan.n_take = cum_all;
-    sh.pre_tied = 0;
-  }
-  __syncthreads();
-  const SelectPlan plan = sh.plan;
-  const uint32_t pre_tied = sh.pre_tied;
 
   // ---- selected tokens before the slab, class masks and ranks inside it
-  uint32_t mine_pre = 0;
+  // tied tokens in the wave's rows before the slab: one bin (with a threshold behind the last bin the quota is zero
+  // and the number is not used)
+  const uint32_t thr_word = (plan.thr >> 1) & 3u;
+  const uint32_t pre_word = thr_word == 0u ? pre[0] : thr_word == 1u ? pre[1] : thr_word == 2u ? pre[2] : pre[3];
+  const uint32_t wave_tied =
+      (static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(pre_word), (plan.thr >> 3) & 63u)) >>
+       (16u * (plan.thr & 1u))) & 0xffffu;
+  // and those below the threshold, which only the positions in the whole selection need
+  uint32_t wave_below = 0;
+  if (sdst) {
 #pragma unroll
-  for (int j = 0; j < kBins; ++j) mine_pre += kBins * tid + j < plan.thr ? cp[j] : 0u;
-  const uint32_t wave_pre = wave_sum(mine_pre);
+    for (int j = 0; j < 8; ++j) {
+      const uint32_t v = j & 1 ? pre[j >> 1] >> 16 : pre[j >> 1] & 0xffffu;
+      wave_below += 8u * static_cast<uint32_t>(lane) + j < plan.thr ? v : 0u;
+    }
+    wave_below = wave_sum(wave_below);
+  }
   uint32_t below[kItems / 4], equal[kItems / 4];
   raw_class_masks<kItems>(keys, plan.thr, below, equal);
   uint32_t total;
   const uint32_t excl = lane_scan<kItems / 4>(below, equal, total);  // below | tied << 16
-  if (lane == 0) {
-    sh.wpre[wave] = wave_pre;
-    sh.wclass[wave] = total;
-  }
+  if (lane == 0) sh.wcount[wave] = make_uint4(total, wave_tied, wave_below, 0u);
   __syncthreads();
-  uint32_t base_b = 0, before = 0, slab_all = 0;
-#pragma unroll
-  for (int w = 0; w < kWaves; ++w) {
-    base_b += sh.wpre[w];
-    before += w < wave ? sh.wclass[w] : 0u;
-    slab_all += sh.wclass[w];
-  }
+  const uint4 wc = sh.wcount[lane & (kWaves - 1)];
+  const uint32_t incl = row_inclusive_scan<kWaves>(wc.x);
+  const uint32_t before = __builtin_amdgcn_readlane(incl - wc.x, wave);   // in the waves before
+  const uint32_t slab_all = __builtin_amdgcn_readlane(incl, kWaves - 1);
+  const uint32_t pre_tied = sum_of_first<kWaves>(wc.y);
   const uint32_t slab_below = slab_all & 0xffffu, slab_tied = slab_all >> 16;
   // tied tokens of this slab that are inside the quota (ties go to the lowest index: the chunks
   // before the slab come first)
   const uint32_t tied_left = plan.quota > pre_tied ? plan.quota - pre_tied : 0u;
   const uint32_t slab_tied_taken = min(slab_tied, tied_left);
-  // positions in the whole selection: the tokens below the threshold in index order, then the ties
-  lane_emit<kItems / 4>(below, equal, plan.n_below, plan.quota,
-                           base_b + (before & 0xffffu) + (excl & 0xffffu),
-                           pre_tied + (before >> 16) + (excl >> 16),
-                           [&](uint32_t pos, int i) __attribute__((always_inline)) {
-                             const bool is_b = keys[i] < plan.thr;
-                             const uint32_t local = is_b ? pos - base_b
-                                                         : slab_below + (pos - plan.n_below - pre_tied);
-                             sh.rows[local] = static_cast<int32_t>(trow[i]);
-                             if (sdst) sdst[pos] = static_cast<int32_t>(e0 + i);
-                           });
+  {
+    // the slab's list: the tokens below the threshold in index order, then its ties
+    uint32_t pb = (before & 0xffffu) + (excl & 0xffffu), pe = (before >> 16) + (excl >> 16);
+#pragma unroll
+    for (int i = 0; i < kItems; ++i) {
+      const bool is_b = keys[i] < plan.thr, is_e = keys[i] == plan.thr;
+      if (is_b || (is_e && pe < tied_left)) sh.rows[is_b ? pb : slab_below + pe] = static_cast<int32_t>(trow[i]);
+      pb += is_b ? 1u : 0u;
+      pe += is_e ? 1u : 0u;
+    }
+  }
+  if (sdst) {  // positions in the whole selection: the same over all slabs
+    const uint32_t base_b = sum_of_first<kWaves>(wc.z);
+    lane_emit<kItems / 4>(below, equal, plan.n_below, plan.quota, base_b + (before & 0xffffu) + (excl & 0xffffu),
+                          pre_tied + (before >> 16) + (excl >> 16),
+                          [&](uint32_t pos, int i) __attribute__((always_inline)) {
+                            sdst[pos] = static_cast<int32_t>(e0 + i);
+                          });
+  }
   uint32_t n_rows = slab_below + slab_tied_taken;
   if (slab == 0) {
-    if (tid == 0) sh.rows[n_rows] = cur_row;
+    if (tid == 0) {
+      const uint32_t rows_per_page = kHnd ? 2u * page_size * num_kv_heads : 2u * page_size;
+      sh.rows[n_rows] = static_cast<int32_t>(static_cast<uint32_t>(cur_page) * rows_per_page +
+                                             (n - cur_lp * page_size));
+    }
     ++n_rows;
     if (sdst)
       for (uint32_t i = plan.n_take + tid; i < k; i += kThreads) sdst[i] = -1;
@@ -1195,12 +1222,10 @@ __global__ __launch_bounds__(kThreads) void hist_select_attend_kernel(
     __hip_atomic_store(mine + 2 + tid, O, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   if (!split_arrive_is_last(&counters[bh], n_split, sh.is_last, tid)) return;
-  if (tid < kHeadDim) {
-    float LL, OO[1];
-    merge_partials<1>(partial + static_cast<size_t>(bh) * kMaxSplits * kPartialFloats, n_split, tid,
-                      LL, OO);
-    store_elem<kBf16>(out + static_cast<size_t>(bh) * kHeadDim + tid, LL > 0.f ? OO[0] / LL : 0.f);
-  }
+  merge_partials_waves<kWaves>(partial + static_cast<size_t>(bh) * kMaxSplits * kPartialFloats, n_split, wave,
+                               lane, tid, sh.merge, M, L, O);
+  if (tid < kHeadDim)
+    store_elem<kBf16>(out + static_cast<size_t>(bh) * kHeadDim + tid, L > 0.f ? O / L : 0.f);
   if (tid == 0) counters[bh] = 0;  // ready for the next launch on this stream
 }
 
@@ -1624,17 +1649,21 @@ extern "C" int adamas_decode_step_f(const void* q, const void* q_code, const voi
     int items = hsa_items(max_seq_len, budget, static_cast<uint64_t>(batch) * num_heads);
     while (kHsaThreads * static_cast<uint32_t>(items) < chunk_tokens) items *= 2;  // slabs of whole chunks
     const uint32_t slab_tokens = kHsaThreads * static_cast<uint32_t>(items);
-    const dim3 hgrid(batch * num_heads, (max_seq_len - 1 + slab_tokens - 1) / slab_tokens);
-    const bool wide_groups = hsa_threads(items, static_cast<uint64_t>(hgrid.x) * hgrid.y) == kHsaWideThreads;
+    const dim3 hgrid(num_heads, batch, (max_seq_len - 1 + slab_tokens - 1) / slab_tokens);
+    const bool wide_groups =
+        hsa_threads(items, static_cast<uint64_t>(num_heads) * batch * hgrid.z) == kHsaWideThreads;
+    uint32_t chunk_log2 = 0;
+    while ((1u << chunk_log2) < chunk_tokens) ++chunk_log2;
 #define ADAMAS_LAUNCH_HSA_I(BF, HND, THREADS, ITEMS)                                              \
   hipLaunchKernelGGL((hist_select_attend_kernel<BF, HND, THREADS, ITEMS>), hgrid, dim3(THREADS),  \
-                     0, s, dist, reinterpret_cast<const uint16_t*>(hist), rowmap, seq_lens,       \
-                     w.dist_stride, n_chunks, num_heads, chunk_tokens, n_sel,                     \
+                     0, s, hist, dist, rowmap, seq_lens, static_cast<uint32_t>(w.dist_stride),    \
+                     n_chunks, num_heads, chunk_log2, n_sel, batch,                               \
                      static_cast<const __half*>(q), static_cast<const __half*>(kv_data),          \
                      page_indices, page_indptr, static_cast<__half*>(out), sel_out,               \
                      reinterpret_cast<float*>(ws + w.partial_off),                                \
                      reinterpret_cast<uint32_t*>(ws + w.counters_off), num_kv_heads,              \
-                     group_inv16(num_heads / num_kv_heads), page_size,                            \
+                     group_inv16(num_heads / num_kv_heads), batch > 1 ? head_order16(num_heads, num_kv_heads) : 0u, \
+                     page_size, page_table_stride,                                                \
                      sm_scale * 1.4426950408889634f)
 #define ADAMAS_LAUNCH_HSA(BF, HND)          \
   if (items == 4) {                         \

@@ -127,4 +127,53 @@ __device__ __forceinline__ void merge_partial_pairs(const float* base, uint32_t 
   }
 }
 
+// The same by all kWaves waves of the last workgroup: wave w folds the partials w, w + kWaves, ... (lane l
+// channels 2l and 2l+1), the waves meet in LDS; threads tid < 128 return channel tid.  With up to 4 * kWaves
+// partials all loads of a wave are one memory round trip, and a lane issues a handful instead of three per
+// partial.
+template <int kWaves, int kGroups>
+__device__ __forceinline__ void merge_partials_waves(const float* base, uint32_t n_split, uint32_t wave, int lane,
+                                                     uint32_t tid, MergeShared<kGroups>& sh, float& M, float& L,
+                                                     float& O) {
+  static_assert(kGroups == 4 * kWaves, "one state per wave");
+  constexpr int kBatch = 4;
+  float m_w = kNegBig, l_w = 0.f, a_w[2] = {0.f, 0.f};
+  for (uint32_t s0 = wave; s0 < n_split; s0 += kBatch * kWaves) {
+    uint64_t ml[kBatch], aa[kBatch];
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      const uint32_t s2 = min(s0 + u * kWaves, n_split - 1);  // past the end: a duplicate, left out below
+      const uint64_t* p = reinterpret_cast<const uint64_t*>(base + static_cast<size_t>(s2) * kPartialFloats);
+      ml[u] = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      aa[u] = __hip_atomic_load(p + 1 + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    float m_new = m_w;
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u)
+      m_new = fmaxf(m_new, s0 + u * kWaves < n_split ? __uint_as_float(static_cast<uint32_t>(ml[u])) : kNegBig);
+    const float keep = exp2_raw(m_w - m_new);
+    l_w *= keep;
+    a_w[0] *= keep;
+    a_w[1] *= keep;
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      const bool used = s0 + u * kWaves < n_split;
+      const float wgt = used ? exp2_raw(__uint_as_float(static_cast<uint32_t>(ml[u])) - m_new) : 0.f;
+      if (!used) aa[u] = 0;  // (zero times an infinity is NaN)
+      l_w += __uint_as_float(static_cast<uint32_t>(ml[u] >> 32)) * wgt;
+      a_w[0] += __uint_as_float(static_cast<uint32_t>(aa[u])) * wgt;
+      a_w[1] += __uint_as_float(static_cast<uint32_t>(aa[u] >> 32)) * wgt;
+    }
+    m_w = m_new;
+  }
+  // (every thread is behind the barriers of split_arrive_is_last: nobody reads the group states any more)
+  if (lane == 0) {
+    sh.m[wave] = m_w;
+    sh.l[wave] = l_w;
+  }
+  *reinterpret_cast<float2*>(&sh.o[wave][2 * lane]) = make_float2(a_w[0], a_w[1]);
+  __syncthreads();
+  merge_waves(tid, sh, M, L, O);
+}
+
 }  // namespace adamas

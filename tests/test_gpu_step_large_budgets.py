@@ -202,3 +202,28 @@ def test_step_of_more_slabs_than_run_at_once(gpu_device, longest, kv_heads, layo
 ])
 def test_step_of_workgroups_of_512(gpu_device, lens, budget, page, kv_heads, dtype, layout):
     _check(gpu_device, lens, budget, page, kv_heads, dtype, layout)
+
+
+@pytest.mark.parametrize("lens,budget,kv_heads", [
+    ([131073], 2000, 8),             # a wave's rows hold 32768 tokens, all in one bin
+    ([65537], 2000, 32),             # the same for the eight waves of the wide workgroup
+    ([4097, 900, 33000], 300, 16),
+])
+def test_step_of_equal_distances_takes_the_first_tokens(gpu_device, lens, budget, kv_heads):
+    ctrl, q, q_code = _controller(gpu_device, lens, budget, 16, kv_heads, torch.float16, 0, 3)
+    ctrl.pool.codes.fill_(0x1b1b)
+    _, sel = U.decode_step(q, q_code, ctrl, 0, return_indices=True)
+    pos = torch.arange(budget - 1, device=gpu_device, dtype=torch.int32)
+    for b, n in enumerate(lens):
+        rows = sel[32 * b:32 * (b + 1)].sort(dim=1).values
+        assert torch.equal(rows, pos.expand(32, -1)), b
+    o, _ = U.decode_step(q, q_code, ctrl, 0, return_indices=True)
+    assert torch.equal(o, U.decode_step(q, q_code, ctrl, 0))
+    o2 = U.decode_sparse_attn(q, ctrl, 0, sel.contiguous())
+    assert bool(((o.float() - o2.float()).abs() <= 2.0 ** -10 * o2.float().abs() + 1e-5).all())
+
+
+@pytest.mark.parametrize("kv_heads", [1, 2, 16])
+def test_step_in_the_order_of_key_value_heads(gpu_device, kv_heads):
+    """The workgroups of the heads that share a key/value head lie together."""
+    _check(gpu_device, [5000, 700], 400, 16, kv_heads, torch.float16, 0)
