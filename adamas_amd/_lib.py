@@ -6,12 +6,14 @@ or an entry point fails, an exception is raised.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 from ctypes import c_char_p, c_float, c_int, c_int32, c_int64, c_size_t, c_uint32, c_uint64, c_void_p
 from pathlib import Path
 
 import torch  # noqa: F401  (loads the HIP runtime this library binds to, before the library itself)
 
 LIB_PATH = Path(__file__).resolve().parent / "lib" / "libadamas_hip.so"
+HOST_PATH = LIB_PATH.with_name("adamas_host.so")   # the operators' native host side (csrc/host_ops.cpp)
 
 # name -> (restype, argtypes); order and types mirror include/adamas_hip.h
 _SIGNATURES = {
@@ -124,6 +126,17 @@ def load() -> ctypes.CDLL:
         fn.argtypes = argtypes
     _lib = lib
     return lib
+
+
+def load_host():
+    """The extension module that calls the library for the operators of a decode token.  Raises if it is not built."""
+    load()
+    if not HOST_PATH.exists():
+        raise RuntimeError(f"{HOST_PATH} is missing: build it with `python -m adamas_amd.build`")
+    spec = importlib.util.spec_from_file_location("adamas_host", HOST_PATH)
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    return module
 
 
 def step_plan(batch: int, num_heads: int, max_seq_len: int, budget: int) -> dict:

@@ -1,4 +1,5 @@
-"""Builds libadamas_hip.so (hand-written HIP kernels + the C ABI) for gfx950 with hipcc.
+"""Builds libadamas_hip.so (hand-written HIP kernels + the C ABI) for gfx950 with hipcc, and adamas_host.so (the native
+host side of the operators of a decode token) with g++.
 
 The library is built in-tree (adamas_amd/lib/) so that it travels with the source tree; nothing is
 installed into site-packages and nothing is compiled at import time.
@@ -14,6 +15,7 @@ PKG_DIR = Path(__file__).resolve().parent
 CSRC_DIR = PKG_DIR / "csrc"
 LIB_DIR = PKG_DIR / "lib"
 LIB_PATH = LIB_DIR / "libadamas_hip.so"
+HOST_PATH = LIB_DIR / "adamas_host.so"
 
 SOURCES = ["hadamard.hip", "estimate.hip", "topk.hip", "attention.hip", "fused_step.hip",
            "prefill.hip", "decoder_ops.hip"]
@@ -48,7 +50,7 @@ def _run(cmd, verbose):
         print(proc.stdout)
         print(proc.stderr)
     if proc.returncode != 0:
-        raise RuntimeError(f"hipcc failed with exit code {proc.returncode}")
+        raise RuntimeError(f"{cmd[0]} failed with exit code {proc.returncode}")
 
 
 def build_library(verbose: bool = False, jobs: int = 0) -> Path:
@@ -67,7 +69,26 @@ def build_library(verbose: bool = False, jobs: int = 0) -> Path:
                                        str(so[1])], verbose), zip(SOURCES, objects)))
     _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", *[str(o) for o in objects], "-o",
           str(LIB_PATH)], verbose)
+    _run(host_command(), verbose)
     return LIB_PATH
+
+
+def host_command() -> list:
+    """g++ for the extension module of csrc/host_ops.cpp: no device code, torch's headers and libraries (which the
+    process has loaded by the time the module is), the HIP library beside it."""
+    import sysconfig
+
+    import torch
+
+    root = Path(torch.__file__).resolve().parent
+    rocm = Path(find_hipcc()).resolve().parents[1]
+    includes = [root / "include", root / "include" / "torch" / "csrc" / "api" / "include", rocm / "include",
+                sysconfig.get_paths()["include"]]
+    return ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+            *[f"-I{d}" for d in includes], str(CSRC_DIR / "host_ops.cpp"), "-o", str(HOST_PATH),
+            f"-L{root / 'lib'}", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip",
+            f"-L{LIB_DIR}", f"-l:{LIB_PATH.name}", "-Wl,-rpath,$ORIGIN"]
 
 
 if __name__ == "__main__":

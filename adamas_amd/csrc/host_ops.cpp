@@ -1,0 +1,449 @@
+// The host side of one decode token's operators, for CPython and torch tensors.
+//
+// A decode step is three to six launches of a few microseconds each, and an operator that checks its tensors, reads
+// its controller and calls the library through ctypes costs 6 to 12 us of host time: eager steps over short contexts
+// waited for Python.  Each function here does the same checks and the same call in one native function.  It serves
+// the ordinary call only: plain tensors on the current device, in the shapes, types and order that the operator
+// asks for, a controller of the package's own class, nothing to allocate but the result.  For anything else it
+// returns None before it has done anything, and the operator in utils/__init__.py goes its general way, which is
+// also the one that says what is wrong.  Nothing is kept between calls: every call reads the controller anew.
+#include <Python.h>
+
+#include <ATen/ATen.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/Dtype.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <cmath>
+
+#include "../../include/adamas_hip.h"
+
+namespace {
+
+// ---- names, classes and constants of the package, set once by setup() ----------------------------------------------
+PyTypeObject* g_controller_type = nullptr;
+PyObject* g_controller_module = nullptr;  // holds CODES_CACHED_BYTES
+PyObject* g_all_past = nullptr;           // ALL_PAST_TOKENS
+
+#define ADAMAS_NAMES(X)                                                                                             \
+  X(dtype) X(batch_size) X(num_layers) X(num_heads) X(num_kv_heads) X(head_dim) X(page_size) X(max_seq_len)         \
+  X(hadamard_scale) X(kv_flags) X(code_flags) X(pool) X(seqs) X(kv) X(codes) X(table_dev) X(indptr_dev)             \
+  X(seq_lens_dev) X(lengths) X(max_pages) X(inference_page_budget) X(topk_dout_buffer) X(topk_dindices_buffer)      \
+  X(topk_buf) X(_workspace) X(_len_bound) X(_estimate_buf) X(_estimate_version) X(CODES_CACHED_BYTES)
+#define ADAMAS_DECLARE(n) PyObject* s_##n = nullptr;
+ADAMAS_NAMES(ADAMAS_DECLARE)
+#undef ADAMAS_DECLARE
+
+// What makes a call fall back to the general way: not an error.
+struct General {};
+
+struct Ref {  // an owned reference
+  PyObject* p = nullptr;
+  Ref() = default;
+  explicit Ref(PyObject* q) : p(q) {}
+  Ref(const Ref&) = delete;
+  Ref& operator=(const Ref&) = delete;
+  ~Ref() { Py_XDECREF(p); }
+};
+
+PyObject* attr(PyObject* o, PyObject* name) {
+  PyObject* v = PyObject_GetAttr(o, name);
+  if (!v) {
+    PyErr_Clear();
+    throw General{};
+  }
+  return v;
+}
+
+long as_long(PyObject* v) {
+  if (!PyLong_CheckExact(v)) throw General{};
+  int over = 0;
+  const long x = PyLong_AsLongAndOverflow(v, &over);
+  if (over) throw General{};
+  return x;
+}
+
+long attr_long(PyObject* o, PyObject* name) {
+  const Ref v(attr(o, name));
+  return as_long(v.p);
+}
+
+uint32_t attr_u32(PyObject* o, PyObject* name) {
+  const long x = attr_long(o, name);
+  if (x < 0 || x > 0x7fffffffL) throw General{};
+  return static_cast<uint32_t>(x);
+}
+
+// A plain tensor on the current device: no subclass, no wrapper of a transform, no lazy bits.
+const at::Tensor& plain(PyObject* o) {
+  if (!THPVariable_CheckExact(o)) throw General{};
+  const at::Tensor& t = THPVariable_Unpack(o);
+  static const c10::DispatchKeySet usual({c10::DispatchKey::CUDA, c10::DispatchKey::AutogradCUDA,
+                                          c10::DispatchKey::ADInplaceOrView, c10::DispatchKey::AutocastCUDA});
+  if (!t.defined() || !t.has_storage() || (t.key_set().raw_repr() & ~usual.raw_repr()) != 0 || !t.is_cuda())
+    throw General{};
+  return t;
+}
+
+struct Owned {  // a tensor attribute, kept alive for the call
+  Ref ref;
+  const at::Tensor& t;
+  Owned(PyObject* o, PyObject* name) : ref(attr(o, name)), t(plain(ref.p)) {}
+  char* data() const { return static_cast<char*>(t.data_ptr()); }
+};
+
+// The controller's numbers and device-side state.
+struct Controller {
+  PyObject* c;
+  long batch, heads, kv_heads, page, max_len, min_len, sum_len;
+  bool bounded = false;  // lengths stand in for a bound while a graph is in use
+  at::ScalarType dtype;
+  Ref pool, seqs;
+
+  explicit Controller(PyObject* obj) : c(obj) {
+    if (Py_TYPE(obj) != g_controller_type) throw General{};
+    if (c10::impl::TorchDispatchModeTLS::any_modes_set()) throw General{};
+    const Ref d(attr(c, s_dtype));
+    if (!THPDtype_Check(d.p)) throw General{};
+    dtype = reinterpret_cast<THPDtype*>(d.p)->scalar_type;
+    batch = attr_u32(c, s_batch_size);
+    heads = attr_u32(c, s_num_heads);
+    kv_heads = attr_u32(c, s_num_kv_heads);
+    page = attr_u32(c, s_page_size);
+    if (attr_long(c, s_head_dim) != ADAMAS_HEAD_DIM) throw General{};
+    pool.p = attr(c, s_pool);
+    seqs.p = attr(c, s_seqs);
+    const Ref lens(attr(seqs.p, s_lengths));
+    if (!PyList_CheckExact(lens.p) || PyList_GET_SIZE(lens.p) == 0) throw General{};
+    max_len = min_len = as_long(PyList_GET_ITEM(lens.p, 0));
+    sum_len = 0;
+    for (Py_ssize_t i = 0; i < PyList_GET_SIZE(lens.p); ++i) {
+      const long n = as_long(PyList_GET_ITEM(lens.p, i));
+      max_len = std::max(max_len, n);
+      min_len = std::min(min_len, n);
+      sum_len += n;
+    }
+    const Ref bound(attr(c, s__len_bound));
+    if (bound.p != Py_None) {
+      max_len = as_long(bound.p);
+      bounded = true;
+    }
+    if (max_len < 0 || max_len > 0x7fffffffL) throw General{};
+  }
+
+  // the budget of the coming layers, none = General
+  uint32_t budget() const {
+    const long b = attr_long(c, s_inference_page_budget);
+    if (b < 1 || b > 0x7fffffffL) throw General{};
+    return static_cast<uint32_t>(b);
+  }
+
+  // address of one layer of a pool tensor
+  char* layer(const Owned& pool_tensor, PyObject* index) const {
+    const long i = as_long(index), n = pool_tensor.t.size(0);
+    if (i < -n || i >= n) throw General{};
+    return pool_tensor.data() + (i < 0 ? i + n : i) * pool_tensor.t.stride(0) * pool_tensor.t.element_size();
+  }
+
+  // the flag that InferenceController.codes_flags gives
+  uint32_t codes_flags(uint32_t budget_now) const {
+    const long tokens = bounded ? batch * max_len : sum_len;
+    const long bytes = static_cast<long>(attr_u32(c, s_num_layers)) *
+                       (tokens * kv_heads * 2 * ADAMAS_CODE_WORDS + batch * static_cast<long>(budget_now) * heads * 512);
+    return bytes <= attr_long(g_controller_module, s_CODES_CACHED_BYTES) ? ADAMAS_F_CODES_CACHED
+                                                                         : ADAMAS_F_CODES_STREAMED;
+  }
+
+  void check_workspace(const Owned& ws, uint32_t budget_now) const {
+    const long most = attr_u32(c, s_max_seq_len);
+    const uint32_t b = static_cast<uint32_t>(std::max(1L, std::min(static_cast<long>(budget_now), most)));
+    const uint32_t len = static_cast<uint32_t>(std::max(1L, std::min(max_len, most)));
+    if (static_cast<size_t>(ws.t.numel()) <
+        adamas_workspace_bytes(static_cast<uint32_t>(batch), static_cast<uint32_t>(heads), len, b))
+      throw General{};
+  }
+};
+
+// the current stream, if t lies on the current device
+adamas_stream_t stream_of(const at::Tensor& t) {
+  const auto s = c10::hip::getCurrentHIPStream();
+  if (s.device_index() != t.get_device()) throw General{};
+  return s.stream();
+}
+
+void need(bool ok) {
+  if (!ok) throw General{};
+}
+
+void need_rows(const at::Tensor& t, at::ScalarType dtype, long n, long heads, long d) {
+  need(t.scalar_type() == dtype && t.dim() == 3 && t.size(0) == n && t.size(1) == heads && t.size(2) == d &&
+       t.is_contiguous());
+}
+
+PyObject* failed(const char* what, int code) {
+  PyErr_Format(PyExc_RuntimeError, "%s failed with error code %d: %s", what, code, adamas_error_string(code));
+  return nullptr;
+}
+
+template <typename F>
+int released(F&& f) {  // a launch can wait for room in the queue: other threads go on meanwhile
+  int rc;
+  Py_BEGIN_ALLOW_THREADS
+  rc = f();
+  Py_END_ALLOW_THREADS
+  return rc;
+}
+
+// ---- the operators ---------------------------------------------------------------------------------------------------
+PyObject* hadamard(PyObject* const* a, Py_ssize_t) {  // x, inplace, scale
+  const at::Tensor& x = plain(a[0]);
+  need(a[1] == Py_False && PyFloat_CheckExact(a[2]) && !c10::impl::TorchDispatchModeTLS::any_modes_set());
+  need((x.scalar_type() == at::kHalf || x.scalar_type() == at::kBFloat16) && x.dim() > 0 &&
+       x.size(-1) == ADAMAS_HEAD_DIM && x.is_contiguous());
+  adamas_stream_t s = stream_of(x);
+  at::Tensor out = at::empty_like(x);
+  const float scale = static_cast<float>(PyFloat_AS_DOUBLE(a[2]));
+  const uint32_t flags = x.scalar_type() == at::kBFloat16 ? ADAMAS_F_BF16 : 0u;
+  const void* xp = x.data_ptr();
+  void* op = out.data_ptr();
+  const uint64_t rows = static_cast<uint64_t>(x.numel()) / ADAMAS_HEAD_DIM;
+  const int rc = released([&] { return adamas_hadamard_f(xp, op, rows, scale, flags, s); });
+  if (rc) return failed("adamas_hadamard", rc);
+  return THPVariable_Wrap(out);
+}
+
+PyObject* append_decode(PyObject* const* a, Py_ssize_t) {  // k, v, h, q, controller, layer
+  const bool from_h = a[2] != Py_None;
+  need(from_h != (a[3] != Py_None));
+  const Controller c(a[4]);
+  const at::Tensor &k = plain(a[0]), &v = plain(a[1]), &x = plain(from_h ? a[2] : a[3]);
+  const long n = c.batch;
+  need_rows(k, c.dtype, n, c.kv_heads, ADAMAS_HEAD_DIM);
+  need_rows(v, c.dtype, n, c.kv_heads, ADAMAS_HEAD_DIM);
+  if (!from_h) {
+    need_rows(x, c.dtype, n, c.heads, ADAMAS_HEAD_DIM);
+  } else if (c.heads == c.kv_heads) {
+    need_rows(x, c.dtype, 2 * n, c.heads, ADAMAS_HEAD_DIM);
+  } else {
+    need(x.scalar_type() == c.dtype && x.dim() == 2 && x.size(0) == n * (c.heads + c.kv_heads) &&
+         x.size(1) == ADAMAS_HEAD_DIM && x.is_contiguous());
+  }
+  need(c.min_len >= 1);
+  const Owned kv(c.pool.p, s_kv), codes(c.pool.p, s_codes), table(c.seqs.p, s_table_dev),
+      indptr(c.seqs.p, s_indptr_dev), lens(c.seqs.p, s_seq_lens_dev);
+  const Ref scale(attr(c.c, s_hadamard_scale));
+  need(PyFloat_CheckExact(scale.p));
+  const uint32_t flags = attr_u32(c.c, s_code_flags);
+  char *kv_p = c.layer(kv, a[5]), *codes_p = c.layer(codes, a[5]);
+  adamas_stream_t s = stream_of(k);
+  at::Tensor o = at::empty({n, c.heads, ADAMAS_CODE_WORDS}, k.options().dtype(at::kShort));
+  const void *kp = k.data_ptr(), *vp = v.data_ptr(), *xp = x.data_ptr();
+  void* op = o.data_ptr();
+  const int rc = released([&] {
+    return adamas_append_decode(from_h ? nullptr : xp, kp, vp, from_h ? xp : nullptr, static_cast<uint16_t*>(op), kv_p,
+                                codes_p, reinterpret_cast<int32_t*>(table.data()),
+                                reinterpret_cast<int32_t*>(indptr.data()), reinterpret_cast<int32_t*>(lens.data()),
+                                static_cast<uint32_t>(n), static_cast<uint32_t>(c.heads),
+                                static_cast<uint32_t>(c.kv_heads), ADAMAS_HEAD_DIM, static_cast<uint32_t>(c.page),
+                                static_cast<float>(PyFloat_AS_DOUBLE(scale.p)), flags, s);
+  });
+  if (rc) return failed("adamas_append_decode", rc);
+  return THPVariable_Wrap(o);
+}
+
+PyObject* estimate(PyObject* const* a, Py_ssize_t) {  // q_code, controller, layer
+  const Controller c(a[1]);
+  const at::Tensor& q = plain(a[0]);
+  need(q.element_size() == 2 && q.dim() == 3 && q.size(0) == c.batch && q.size(1) == c.heads &&
+       q.size(2) == ADAMAS_CODE_WORDS && q.is_contiguous() && c.max_len >= 2);
+  const Owned codes(c.pool.p, s_codes), table(c.seqs.p, s_table_dev), indptr(c.seqs.p, s_indptr_dev),
+      lens(c.seqs.p, s_seq_lens_dev);
+  char* codes_p = c.layer(codes, a[2]);
+  adamas_stream_t s = stream_of(q);
+  const long n = c.max_len - 1, stride = (n + 7) / 8 * 8;
+  at::Tensor buf = at::empty({c.batch, c.heads, stride}, q.options().dtype(at::kHalf));
+  const void* qp = q.data_ptr();
+  void* bp = buf.data_ptr();
+  const int rc = released([&] {
+    return adamas_estimate(static_cast<const uint16_t*>(qp), codes_p, reinterpret_cast<int32_t*>(table.data()),
+                           reinterpret_cast<int32_t*>(indptr.data()), reinterpret_cast<int32_t*>(lens.data()), bp,
+                           c.heads * stride, stride, ADAMAS_DIST_FP16, static_cast<uint32_t>(c.batch),
+                           static_cast<uint32_t>(c.heads), static_cast<uint32_t>(c.kv_heads),
+                           static_cast<uint32_t>(c.page), static_cast<uint32_t>(c.max_len), s);
+  });
+  if (rc) return failed("adamas_estimate", rc);
+  at::Tensor out = c.batch == 1 ? buf.as_strided({c.heads, n}, {stride, 1})
+                                : buf.as_strided({c.batch, c.heads, n}, {c.heads * stride, stride, 1});
+  const Ref version(PyLong_FromLongLong(buf._version())), held(THPVariable_Wrap(buf));
+  if (!version.p || !held.p || PyObject_SetAttr(c.c, s__estimate_buf, held.p) < 0 ||
+      PyObject_SetAttr(c.c, s__estimate_version, version.p) < 0)
+    return nullptr;
+  return THPVariable_Wrap(out);
+}
+
+PyObject* topk(PyObject* const* a, Py_ssize_t) {  // estimate, controller, integer_keys; True when done
+  const Controller c(a[1]);
+  const at::Tensor& est = plain(a[0]);
+  const long rows = c.batch * c.heads;
+  need(est.scalar_type() == at::kHalf && (est.dim() == 2 || est.dim() == 3) && est.stride(-1) == 1);
+  long row_stride = est.stride(0);
+  if (est.dim() == 3) {
+    need(est.size(0) == c.batch && est.size(1) == c.heads && est.stride(0) == est.stride(1) * est.size(1));
+    row_stride = est.stride(1);
+  } else {
+    need(est.size(0) == rows);
+  }
+  const uint32_t k = c.budget() - 1u;
+  const long n = est.size(-1);
+  need(n > 0 && (n >= static_cast<long>(k) || c.batch > 1));
+  const Owned idx(c.c, s_topk_dindices_buffer), val(c.c, s_topk_dout_buffer), scratch(c.c, s_topk_buf),
+      lens(c.seqs.p, s_seq_lens_dev);
+  const long most = attr_u32(c.c, s_max_seq_len);
+  need(static_cast<size_t>(scratch.t.numel()) >=
+       adamas_topk_workspace_bytes(static_cast<uint32_t>(rows), static_cast<uint32_t>(std::max(n, most)), k));
+  bool integer = a[2] == Py_True;
+  if (a[2] == Py_None) {
+    // views of the buffer that the last estimate filled and that nobody has edited since
+    const Ref held(PyObject_GetAttr(c.c, s__estimate_buf));
+    if (!held.p) {
+      PyErr_Clear();
+    } else if (held.p != Py_None) {
+      const at::Tensor& buf = plain(held.p);
+      const char* base = static_cast<const char*>(buf.storage().data());
+      const char* p = static_cast<const char*>(est.data_ptr());
+      integer = static_cast<long>(buf._version()) == attr_long(c.c, s__estimate_version) && base <= p &&
+                p < base + buf.storage().nbytes();
+    }
+  } else {
+    need(integer || a[2] == Py_False);
+  }
+  adamas_stream_t s = stream_of(est);
+  const void* ep = est.data_ptr();
+  const int rc = released([&] {
+    return adamas_topk(ep, row_stride, static_cast<uint32_t>(n),
+                       c.batch > 1 ? reinterpret_cast<int32_t*>(lens.data()) : nullptr, static_cast<uint32_t>(c.heads),
+                       -1, nullptr, 0, static_cast<uint32_t>(rows), k, reinterpret_cast<int32_t*>(idx.data()),
+                       val.data(), k, integer ? ADAMAS_KEY_FP16_INT : ADAMAS_KEY_FP16_GENERIC, scratch.data(),
+                       static_cast<size_t>(scratch.t.numel()), s);
+  });
+  if (rc) return failed("adamas_topk", rc);
+  Py_RETURN_TRUE;
+}
+
+PyObject* sparse_attn(PyObject* const* a, Py_ssize_t) {  // q, controller, layer, indices
+  const Controller c(a[1]);
+  const at::Tensor& q = plain(a[0]);
+  need_rows(q, c.dtype, c.batch, c.heads, ADAMAS_HEAD_DIM);
+  const int32_t* sel = nullptr;
+  long stride = 0, n_sel = 0;
+  if (a[3] != Py_None && a[3] != g_all_past) {
+    const at::Tensor& t = plain(a[3]);
+    need(t.scalar_type() == at::kInt && t.dim() == 2 && t.is_contiguous() && t.size(0) == c.batch * c.heads);
+    sel = static_cast<const int32_t*>(t.data_ptr());
+    stride = t.stride(0);
+    n_sel = t.size(1);
+  }
+  const Ref b(attr(c.c, s_inference_page_budget));
+  const uint32_t budget = b.p == Py_None ? 1u : std::max(c.budget(), 1u);
+  const Owned kv(c.pool.p, s_kv), table(c.seqs.p, s_table_dev), indptr(c.seqs.p, s_indptr_dev),
+      lens(c.seqs.p, s_seq_lens_dev), ws(c.c, s__workspace);
+  c.check_workspace(ws, budget);
+  const uint32_t flags = attr_u32(c.c, s_kv_flags);
+  char* kv_p = c.layer(kv, a[2]);
+  adamas_stream_t s = stream_of(q);
+  at::Tensor o = at::empty_like(q);
+  const void* qp = q.data_ptr();
+  void* op = o.data_ptr();
+  const int rc = released([&] {
+    return adamas_sparse_decode_f(qp, kv_p, reinterpret_cast<int32_t*>(table.data()),
+                                  reinterpret_cast<int32_t*>(indptr.data()), reinterpret_cast<int32_t*>(lens.data()),
+                                  sel, stride, static_cast<uint32_t>(n_sel), op, ws.data(),
+                                  static_cast<size_t>(ws.t.numel()), static_cast<uint32_t>(c.batch),
+                                  static_cast<uint32_t>(c.heads), static_cast<uint32_t>(c.kv_heads), ADAMAS_HEAD_DIM,
+                                  static_cast<uint32_t>(c.page), static_cast<float>(1.0 / std::sqrt(128.0)),
+                                  static_cast<uint32_t>(c.max_len), flags, s);
+  });
+  if (rc) return failed("adamas_sparse_decode", rc);
+  return THPVariable_Wrap(o);
+}
+
+PyObject* step(PyObject* const* a, Py_ssize_t) {  // q, q_code, controller, layer (no positions asked for)
+  const Controller c(a[2]);
+  const at::Tensor &q = plain(a[0]), &code = plain(a[1]);
+  need(q.scalar_type() == c.dtype && q.dim() == 3 && q.is_contiguous() && code.dim() == 3 && code.is_contiguous());
+  const uint32_t budget = c.budget();
+  const Owned kv(c.pool.p, s_kv), codes(c.pool.p, s_codes), table(c.seqs.p, s_table_dev),
+      indptr(c.seqs.p, s_indptr_dev), lens(c.seqs.p, s_seq_lens_dev), ws(c.c, s__workspace);
+  c.check_workspace(ws, budget);
+  const uint32_t flags = attr_u32(c.c, s_kv_flags) | c.codes_flags(budget), pages = attr_u32(c.seqs.p, s_max_pages);
+  char *kv_p = c.layer(kv, a[3]), *codes_p = c.layer(codes, a[3]);
+  adamas_stream_t s = stream_of(q);
+  at::Tensor o = at::empty_like(q);
+  const void *qp = q.data_ptr(), *cp = code.data_ptr();
+  void* op = o.data_ptr();
+  const int rc = released([&] {
+    return adamas_decode_step_f(qp, cp, kv_p, codes_p, reinterpret_cast<int32_t*>(table.data()),
+                                reinterpret_cast<int32_t*>(indptr.data()), reinterpret_cast<int32_t*>(lens.data()),
+                                budget, op, nullptr, ws.data(), static_cast<size_t>(ws.t.numel()),
+                                static_cast<uint32_t>(c.batch), static_cast<uint32_t>(c.heads),
+                                static_cast<uint32_t>(c.kv_heads), ADAMAS_HEAD_DIM, static_cast<uint32_t>(c.page),
+                                static_cast<float>(1.0 / std::sqrt(128.0)), static_cast<uint32_t>(c.max_len), pages,
+                                flags, s);
+  });
+  if (rc) return failed("adamas_decode_step", rc);
+  return THPVariable_Wrap(o);
+}
+
+template <PyObject* (*F)(PyObject* const*, Py_ssize_t), int kArgs>
+PyObject* entry(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != kArgs) {
+    PyErr_Format(PyExc_TypeError, "%d arguments expected, got %zd", kArgs, n);
+    return nullptr;
+  }
+  try {
+    return F(args, n);
+  } catch (const General&) {
+    Py_RETURN_NONE;
+  }
+  END_HANDLE_TH_ERRORS
+}
+
+PyObject* setup(PyObject*, PyObject* const* args, Py_ssize_t n) {  // InferenceController, its module, ALL_PAST_TOKENS
+  if (n != 3 || !PyType_Check(args[0])) {
+    PyErr_SetString(PyExc_TypeError, "setup(controller class, its module, marker) expected");
+    return nullptr;
+  }
+  for (Py_ssize_t i = 0; i < n; ++i) Py_INCREF(args[i]);
+  g_controller_type = reinterpret_cast<PyTypeObject*>(args[0]);
+  g_controller_module = args[1];
+  g_all_past = args[2];
+  Py_RETURN_NONE;
+}
+
+#define ADAMAS_ENTRY(name, f, n) \
+  {name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&entry<f, n>)), METH_FASTCALL, nullptr}
+PyMethodDef g_methods[] = {
+    ADAMAS_ENTRY("hadamard", hadamard, 3),
+    ADAMAS_ENTRY("append_decode", append_decode, 6),
+    ADAMAS_ENTRY("estimate", estimate, 3),
+    ADAMAS_ENTRY("topk", topk, 3),
+    ADAMAS_ENTRY("sparse_attn", sparse_attn, 4),
+    ADAMAS_ENTRY("step", step, 4),
+    {"setup", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&setup)), METH_FASTCALL, nullptr},
+    {nullptr, nullptr, 0, nullptr}};
+
+PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "adamas_host", nullptr, -1, g_methods,
+                        nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit_adamas_host(void) {
+#define ADAMAS_INTERN(n) \
+  if (!(s_##n = PyUnicode_InternFromString(#n))) return nullptr;
+  ADAMAS_NAMES(ADAMAS_INTERN)
+#undef ADAMAS_INTERN
+  return PyModule_Create(&g_module);
+}

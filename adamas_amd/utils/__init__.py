@@ -3,7 +3,7 @@
 Same function names, argument order and return values as adamas/utils/__init__.py of the reference
 (append_kvh :94-157, decode_estimate :203-237, decode_topk :239-269, decode_sparse_attn :271-308,
 pack_2bit :55-76), apply_rope_in_place :26-53, prefill_forward :159-201, rms_norm_forward :79-92), so the reference's
-attention module (adamas/models/Adamas.py:68-225) can drive it unchanged.  Every function allocates its output with torch, checks shapes and dtypes in Python
+attention module (adamas/models/Adamas.py:68-225) can drive it unchanged.  Every function allocates its output with torch, checks shapes and dtypes
 (RuntimeError on violation, like TORCH_CHECK in the reference bindings) and calls one entry point of
 libadamas_hip.so on the current stream.  There is no fallback path: without the library the calls raise.
 
@@ -20,6 +20,7 @@ from typing import Optional
 import torch
 
 from .. import _lib
+from . import controller as _controller_module
 from .controller import ALL_PAST_TOKENS, ORTHONORMAL_SCALE, RAW_SCALE, InferenceController
 from .paging import CODE_WORDS, KvCache, PagePool, PagedSequences, TensorLayout
 
@@ -59,6 +60,20 @@ __all__ = [
 
 _FLOAT_DTYPES = (torch.float16, torch.bfloat16)
 
+# The operators of a decode token try a native function first (csrc/host_ops.cpp), which serves the ordinary call and
+# returns None for any other before it has done anything; what follows the try serves every call and names what is
+# wrong with one.  Host time of a call without / with it, us (a launch is 2 to 2.5 of it): hadamard_transform 5.5 / 3.8,
+# append_kvh 9.5 / 4.3, decode_estimate 9.8 / 4.5, decode_topk 8.6 / 5.4, decode_sparse_attn 9.0 / 4.5, decode_step
+# 12.1 / 7.5; the six operators of the attention module, 16384 tokens, two layers 116 / 73.
+_host = None
+
+
+def _load_host():
+    global _host
+    _host = _lib.load_host()
+    _host.setup(InferenceController, _controller_module, ALL_PAST_TOKENS)
+    return _host
+
 
 def _check_cuda_contig(t: torch.Tensor, name: str, dtype=None, ndim=None):
     if not isinstance(t, torch.Tensor):
@@ -82,6 +97,9 @@ def hadamard_transform(x: torch.Tensor, inplace: bool = False,
     transform (128**-0.5) that module's published source computes; `scale` 1.0 is the raw +-1
     butterfly.
     """
+    out = (_host or _load_host()).hadamard(x, inplace, scale)
+    if out is not None:
+        return out
     _check_cuda_contig(x, "x", _FLOAT_DTYPES)
     if x.shape[-1] != 128:
         raise RuntimeError("hadamard_transform supports a last dimension of 128 only")
@@ -126,6 +144,9 @@ def append_kvh(k: torch.Tensor, v: torch.Tensor, h: Optional[torch.Tensor],
     [B*num_heads + B*num_kv_heads, D] of Hadamard(q) rows followed by Hadamard(k) rows.
     Reference: adamas/utils/__init__.py:94-157.
     """
+    o = (_host or _load_host()).append_decode(k, v, h, q, iController, layer_idx)
+    if o is not None:
+        return o
     lib = _lib.load()
     c = iController
     _check_cuda_contig(k, "k", c.dtype, 3)
@@ -187,6 +208,9 @@ def decode_estimate(q: torch.Tensor, iController: InferenceController, layer_idx
     entries are exact integers in [0, 384].  The current token is excluded.
     Reference: adamas/utils/__init__.py:203-237.
     """
+    out = (_host or _load_host()).estimate(q, iController, layer_idx)
+    if out is not None:
+        return out
     c = iController
     _check_cuda_contig(q, "q", None, 3)
     if q.element_size() != 2 or q.shape != (c.batch_size, c.num_heads, CODE_WORDS):
@@ -228,6 +252,8 @@ def decode_topk(estimated_attn_score: torch.Tensor, iController: InferenceContro
     place since (the controller holds the buffer, so its memory cannot be reused by another tensor
     meanwhile); a copy of it, or any other tensor, is treated as arbitrary keys.
     """
+    if (_host or _load_host()).topk(estimated_attn_score, iController, integer_keys):
+        return
     c = iController
     est = estimated_attn_score
     if est.dtype != torch.float16 or not est.is_cuda or est.stride(-1) != 1:
@@ -276,6 +302,9 @@ def decode_sparse_attn(q: torch.Tensor, iController: InferenceController, layer_
     rope_scale / rope_theta are accepted and ignored, as in the reference (RotaryMode::kNone,
     adamas/ops/csrc/approx_attn.cu:135).  Reference: adamas/utils/__init__.py:271-308.
     """
+    o = (_host or _load_host()).sparse_attn(q, iController, layer_idx, topk_indices)
+    if o is not None:
+        return o
     c = iController
     _check_cuda_contig(q, "q", c.dtype, 3)
     if q.shape != (c.batch_size, c.num_heads, c.head_dim):
@@ -413,6 +442,10 @@ def decode_step(q: torch.Tensor, q_code: torch.Tensor, iController: InferenceCon
     """estimate -> top-k -> sparse attention for one layer behind a single call (the sequence
     Adamas.py:176-201 of the reference).  Returns o [B, H, D] and, on request, the selected
     positions [B*H, budget-1]."""
+    if not return_indices:
+        o = (_host or _load_host()).step(q, q_code, iController, layer_idx)
+        if o is not None:
+            return o
     c = iController
     _check_cuda_contig(q, "q", c.dtype, 3)
     _check_cuda_contig(q_code, "q_code", None, 3)
