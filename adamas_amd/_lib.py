@@ -33,6 +33,7 @@ _SIGNATURES = {
     "adamas_topk": (c_int, [c_void_p, c_int64, c_uint32, c_void_p, c_uint32, c_int32, c_void_p,
                              c_int64, c_uint32, c_uint32, c_void_p, c_void_p, c_int64, c_uint32,
                              c_void_p, c_size_t, c_void_p]),
+    "adamas_write_words": (c_int, [c_void_p, c_void_p, c_uint32, c_void_p]),
     "adamas_read_probe": (c_int, [c_void_p, c_size_t, c_void_p, c_void_p]),
     "adamas_topk_workspace_bytes": (c_size_t, [c_uint32, c_uint32, c_uint32]),
     "adamas_workspace_bytes": (c_size_t, [c_uint32, c_uint32, c_uint32, c_uint32]),
@@ -102,6 +103,7 @@ F_HND = 4
 F_NO_MFMA = 8
 F_CODES_CACHED = 16
 F_CODES_STREAMED = 64
+MAX_WORDS = 1024          # of adamas_write_words
 STATIC_SCRATCH_BYTES = 24 << 20
 E_SCRATCH = -5
 DIST_FP16, DIST_U16 = 0, 1
@@ -159,6 +161,13 @@ def check(code: int, what: str) -> None:
         raise RuntimeError(f"{what} failed with error code {code}: {error_string(code)}")
 
 
+def write_words(address: int, values, stream: int) -> None:
+    """values (at most MAX_WORDS 32-bit integers) to device memory, as arguments of a launch: nothing is staged and
+    the host does not wait."""
+    n = len(values)
+    check(load().adamas_write_words(address, (c_int32 * n)(*values), n, stream), "adamas_write_words")
+
+
 def dtype_flags(dtype) -> int:
     """The `flags` bit of the append entry points for this dtype."""
     if dtype == torch.float16:
@@ -173,9 +182,10 @@ def ptr(t) -> int | None:
     return None if t is None else t.data_ptr()
 
 
-def current_stream() -> int:
-    """The current stream of the current device (2.7 us less than by way of a torch.cuda.Stream object)."""
+def current_stream(device: int | None = None) -> int:
+    """The current stream of a device, by default the current one (2.7 us less than by way of a torch.cuda.Stream
+    object)."""
     try:
-        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice() if device is None else device)
     except AttributeError:   # (not public names: another torch may lack them)
-        return torch.cuda.current_stream().cuda_stream
+        return (torch.cuda.current_stream() if device is None else torch.cuda.current_stream(device)).cuda_stream

@@ -8,6 +8,8 @@
 // A wave takes 16 consecutive tokens (16 loads in flight), adds the two halves of a head with one
 // DPP lane swap, and stores 8 distances per lane as one 128-bit store into out[head][t..t+8).
 // The distance arithmetic on the packed codes is in codes.h.
+#include <algorithm>
+
 #include "codes.h"
 
 namespace adamas {
@@ -132,9 +134,34 @@ __global__ __launch_bounds__(512) void read_probe_kernel(const uint4* __restrict
   if (acc == 0x9e3779b9u && sink) *sink = acc;
 }
 
+// A few words of host memory as arguments of a launch.
+constexpr uint32_t kWordsPerLaunch = 256;  // 1 KB of arguments
+struct Words {
+  int32_t v[kWordsPerLaunch];
+};
+
+__global__ __launch_bounds__(kWordsPerLaunch) void write_words_kernel(int32_t* __restrict__ dst, uint32_t n,
+                                                                      const Words words) {
+  if (threadIdx.x < n) dst[threadIdx.x] = words.v[threadIdx.x];
+}
+
 }  // namespace adamas
 
 using namespace adamas;
+
+extern "C" int adamas_write_words(int32_t* dst, const int32_t* words, uint32_t n, adamas_stream_t stream) {
+  if (!dst || !words || n == 0 || n > ADAMAS_MAX_WORDS) return ADAMAS_E_BADARG;
+  if (reinterpret_cast<uintptr_t>(dst) & 3) return ADAMAS_E_ALIGN;
+  for (uint32_t at = 0; at < n; at += kWordsPerLaunch) {
+    const uint32_t count = std::min(n - at, kWordsPerLaunch);
+    Words w = {};
+    std::copy(words + at, words + at + count, w.v);
+    hipLaunchKernelGGL(write_words_kernel, dim3(1), dim3(kWordsPerLaunch), 0, static_cast<hipStream_t>(stream),
+                       dst + at, count, w);
+    ADAMAS_RETURN_IF_LAUNCH_FAILED();
+  }
+  return 0;
+}
 
 extern "C" int adamas_read_probe(const void* data, size_t bytes, void* sink,
                                  adamas_stream_t stream) {

@@ -11,6 +11,7 @@
 
 #include <ATen/ATen.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/Exceptions.h>
@@ -29,8 +30,8 @@ PyObject* g_all_past = nullptr;           // ALL_PAST_TOKENS
 
 #define ADAMAS_NAMES(X)                                                                                             \
   X(dtype) X(batch_size) X(num_layers) X(num_heads) X(num_kv_heads) X(head_dim) X(page_size) X(max_seq_len)         \
-  X(hadamard_scale) X(kv_flags) X(code_flags) X(pool) X(seqs) X(kv) X(codes) X(table_dev) X(indptr_dev)             \
-  X(seq_lens_dev) X(lengths) X(max_pages) X(inference_page_budget) X(topk_dout_buffer) X(topk_dindices_buffer)      \
+  X(hadamard_scale) X(kv_flags) X(code_flags) X(pool) X(seqs) X(kv) X(codes) X(_table_dev) X(indptr_dev)             \
+  X(_seq_lens_dev) X(_host_waits) X(_writer) X(lengths) X(max_pages) X(inference_page_budget) X(topk_dout_buffer) X(topk_dindices_buffer)      \
   X(topk_buf) X(_workspace) X(_len_bound) X(_estimate_buf) X(_estimate_version) X(CODES_CACHED_BYTES)
 #define ADAMAS_DECLARE(n) PyObject* s_##n = nullptr;
 ADAMAS_NAMES(ADAMAS_DECLARE)
@@ -94,6 +95,13 @@ struct Owned {  // a tensor attribute, kept alive for the call
   char* data() const { return static_cast<char*>(t.data_ptr()); }
 };
 
+// the current stream, if t lies on the current device
+adamas_stream_t stream_of(const at::Tensor& t) {
+  const auto s = c10::hip::getCurrentHIPStream();
+  if (s.device_index() != t.get_device()) throw General{};
+  return s.stream();
+}
+
 // The controller's numbers and device-side state.
 struct Controller {
   PyObject* c;
@@ -156,6 +164,19 @@ struct Controller {
                                                                          : ADAMAS_F_CODES_STREAMED;
   }
 
+  // The current stream, if it is t's device's and lengths and pages need no wait there: those are read from the
+  // tensors behind PagedSequences.table_dev and .seq_lens_dev, whose getters see to the other streams and graphs.
+  adamas_stream_t stream(const at::Tensor& t) const {
+    adamas_stream_t s = stream_of(t);
+    const Ref waits(attr(seqs.p, s__host_waits));
+    if (waits.p == Py_True) return s;
+    const Ref writer(attr(seqs.p, s__writer));
+    if (waits.p != Py_False || (writer.p != Py_None && as_long(writer.p) != reinterpret_cast<long>(s)) ||
+        c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None)
+      throw General{};
+    return s;
+  }
+
   void check_workspace(const Owned& ws, uint32_t budget_now) const {
     const long most = attr_u32(c, s_max_seq_len);
     const uint32_t b = static_cast<uint32_t>(std::max(1L, std::min(static_cast<long>(budget_now), most)));
@@ -165,13 +186,6 @@ struct Controller {
       throw General{};
   }
 };
-
-// the current stream, if t lies on the current device
-adamas_stream_t stream_of(const at::Tensor& t) {
-  const auto s = c10::hip::getCurrentHIPStream();
-  if (s.device_index() != t.get_device()) throw General{};
-  return s.stream();
-}
 
 void need(bool ok) {
   if (!ok) throw General{};
@@ -231,13 +245,13 @@ PyObject* append_decode(PyObject* const* a, Py_ssize_t) {  // k, v, h, q, contro
          x.size(1) == ADAMAS_HEAD_DIM && x.is_contiguous());
   }
   need(c.min_len >= 1);
-  const Owned kv(c.pool.p, s_kv), codes(c.pool.p, s_codes), table(c.seqs.p, s_table_dev),
-      indptr(c.seqs.p, s_indptr_dev), lens(c.seqs.p, s_seq_lens_dev);
+  const Owned kv(c.pool.p, s_kv), codes(c.pool.p, s_codes), table(c.seqs.p, s__table_dev),
+      indptr(c.seqs.p, s_indptr_dev), lens(c.seqs.p, s__seq_lens_dev);
   const Ref scale(attr(c.c, s_hadamard_scale));
   need(PyFloat_CheckExact(scale.p));
   const uint32_t flags = attr_u32(c.c, s_code_flags);
   char *kv_p = c.layer(kv, a[5]), *codes_p = c.layer(codes, a[5]);
-  adamas_stream_t s = stream_of(k);
+  adamas_stream_t s = c.stream(k);
   at::Tensor o = at::empty({n, c.heads, ADAMAS_CODE_WORDS}, k.options().dtype(at::kShort));
   const void *kp = k.data_ptr(), *vp = v.data_ptr(), *xp = x.data_ptr();
   void* op = o.data_ptr();
@@ -258,10 +272,10 @@ PyObject* estimate(PyObject* const* a, Py_ssize_t) {  // q_code, controller, lay
   const at::Tensor& q = plain(a[0]);
   need(q.element_size() == 2 && q.dim() == 3 && q.size(0) == c.batch && q.size(1) == c.heads &&
        q.size(2) == ADAMAS_CODE_WORDS && q.is_contiguous() && c.max_len >= 2);
-  const Owned codes(c.pool.p, s_codes), table(c.seqs.p, s_table_dev), indptr(c.seqs.p, s_indptr_dev),
-      lens(c.seqs.p, s_seq_lens_dev);
+  const Owned codes(c.pool.p, s_codes), table(c.seqs.p, s__table_dev), indptr(c.seqs.p, s_indptr_dev),
+      lens(c.seqs.p, s__seq_lens_dev);
   char* codes_p = c.layer(codes, a[2]);
-  adamas_stream_t s = stream_of(q);
+  adamas_stream_t s = c.stream(q);
   const long n = c.max_len - 1, stride = (n + 7) / 8 * 8;
   at::Tensor buf = at::empty({c.batch, c.heads, stride}, q.options().dtype(at::kHalf));
   const void* qp = q.data_ptr();
@@ -299,7 +313,7 @@ PyObject* topk(PyObject* const* a, Py_ssize_t) {  // estimate, controller, integ
   const long n = est.size(-1);
   need(n > 0 && (n >= static_cast<long>(k) || c.batch > 1));
   const Owned idx(c.c, s_topk_dindices_buffer), val(c.c, s_topk_dout_buffer), scratch(c.c, s_topk_buf),
-      lens(c.seqs.p, s_seq_lens_dev);
+      lens(c.seqs.p, s__seq_lens_dev);
   const long most = attr_u32(c.c, s_max_seq_len);
   need(static_cast<size_t>(scratch.t.numel()) >=
        adamas_topk_workspace_bytes(static_cast<uint32_t>(rows), static_cast<uint32_t>(std::max(n, most)), k));
@@ -319,7 +333,7 @@ PyObject* topk(PyObject* const* a, Py_ssize_t) {  // estimate, controller, integ
   } else {
     need(integer || a[2] == Py_False);
   }
-  adamas_stream_t s = stream_of(est);
+  adamas_stream_t s = c.stream(est);
   const void* ep = est.data_ptr();
   const int rc = released([&] {
     return adamas_topk(ep, row_stride, static_cast<uint32_t>(n),
@@ -347,12 +361,12 @@ PyObject* sparse_attn(PyObject* const* a, Py_ssize_t) {  // q, controller, layer
   }
   const Ref b(attr(c.c, s_inference_page_budget));
   const uint32_t budget = b.p == Py_None ? 1u : std::max(c.budget(), 1u);
-  const Owned kv(c.pool.p, s_kv), table(c.seqs.p, s_table_dev), indptr(c.seqs.p, s_indptr_dev),
-      lens(c.seqs.p, s_seq_lens_dev), ws(c.c, s__workspace);
+  const Owned kv(c.pool.p, s_kv), table(c.seqs.p, s__table_dev), indptr(c.seqs.p, s_indptr_dev),
+      lens(c.seqs.p, s__seq_lens_dev), ws(c.c, s__workspace);
   c.check_workspace(ws, budget);
   const uint32_t flags = attr_u32(c.c, s_kv_flags);
   char* kv_p = c.layer(kv, a[2]);
-  adamas_stream_t s = stream_of(q);
+  adamas_stream_t s = c.stream(q);
   at::Tensor o = at::empty_like(q);
   const void* qp = q.data_ptr();
   void* op = o.data_ptr();
@@ -374,12 +388,12 @@ PyObject* step(PyObject* const* a, Py_ssize_t) {  // q, q_code, controller, laye
   const at::Tensor &q = plain(a[0]), &code = plain(a[1]);
   need(q.scalar_type() == c.dtype && q.dim() == 3 && q.is_contiguous() && code.dim() == 3 && code.is_contiguous());
   const uint32_t budget = c.budget();
-  const Owned kv(c.pool.p, s_kv), codes(c.pool.p, s_codes), table(c.seqs.p, s_table_dev),
-      indptr(c.seqs.p, s_indptr_dev), lens(c.seqs.p, s_seq_lens_dev), ws(c.c, s__workspace);
+  const Owned kv(c.pool.p, s_kv), codes(c.pool.p, s_codes), table(c.seqs.p, s__table_dev),
+      indptr(c.seqs.p, s_indptr_dev), lens(c.seqs.p, s__seq_lens_dev), ws(c.c, s__workspace);
   c.check_workspace(ws, budget);
   const uint32_t flags = attr_u32(c.c, s_kv_flags) | c.codes_flags(budget), pages = attr_u32(c.seqs.p, s_max_pages);
   char *kv_p = c.layer(kv, a[3]), *codes_p = c.layer(codes, a[3]);
-  adamas_stream_t s = stream_of(q);
+  adamas_stream_t s = c.stream(q);
   at::Tensor o = at::empty_like(q);
   const void *qp = q.data_ptr(), *cp = code.data_ptr();
   void* op = o.data_ptr();

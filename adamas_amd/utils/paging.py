@@ -21,6 +21,8 @@ from typing import Iterable, List, Optional, Sequence
 
 import torch
 
+from .. import _lib
+
 CODE_WORDS = 16  # uint16 words of packed 2-bit code per (token, head) at head_dim 128
 
 
@@ -115,9 +117,50 @@ class PagedSequences:
         self.lengths: List[int] = [0] * batch
         self.device = device
         # fixed stride per sequence => the indptr never changes
-        self.table_dev = torch.zeros(batch * self.max_pages, dtype=torch.int32, device=device)
+        self._table_dev = torch.zeros(batch * self.max_pages, dtype=torch.int32, device=device)
         self.indptr_dev = (torch.arange(batch + 1, dtype=torch.int32) * self.max_pages).to(device)
-        self.seq_lens_dev = torch.zeros(batch, dtype=torch.int32, device=device)
+        self._seq_lens_dev = torch.zeros(batch, dtype=torch.int32, device=device)
+        # Lengths and page ids are written by a launch that the host does not wait for, while everything that
+        # reads them is launched on the stream of that launch.  The first use on another stream, or in a graph
+        # (which is replayed on whatever stream), waits for what is written and ends that: from then on the host
+        # waits for every write, and no stream can be too early.
+        self._host_waits = not self._table_dev.is_cuda
+        self._writer: Optional[int] = None    # stream of the last write that the host did not wait for
+
+    @property
+    def table_dev(self) -> torch.Tensor:
+        if not self._host_waits:
+            self._note_use()
+        return self._table_dev
+
+    @property
+    def seq_lens_dev(self) -> torch.Tensor:
+        if not self._host_waits:
+            self._note_use()
+        return self._seq_lens_dev
+
+    def _note_use(self) -> None:
+        if torch.cuda.is_current_stream_capturing():
+            self._host_waits = True   # (nothing to wait for: capture does not execute)
+        elif self._writer is not None and _lib.current_stream(self._table_dev.get_device()) != self._writer:
+            torch.cuda.synchronize(self._table_dev.device)
+            self._host_waits = True
+
+    def _write(self, dst: torch.Tensor, start: int, values: List[int]) -> None:
+        """dst[start:] = values, without waiting for it where that is safe (see __init__): a decode loop that
+        waits for the copy of one length after every token leaves the GPU idle while the host catches up
+        (2000 + 24 tokens through three layers 11.47 -> 10.76 ms)."""
+        n = len(values)
+        if (self._host_waits or n > _lib.MAX_WORDS or dst.get_device() != torch.cuda.current_device()
+                or torch.cuda.is_current_stream_capturing()):
+            dst[start:start + n] = torch.tensor(values, dtype=torch.int32)
+            return
+        stream = _lib.current_stream()
+        if self._writer is not None and stream != self._writer:
+            self._note_use()
+            return self._write(dst, start, values)
+        _lib.write_words(dst.data_ptr() + 4 * start, values, stream)
+        self._writer = stream
 
     def reserve(self, new_tokens: Sequence[int]) -> List[int]:
         """Grow sequence b by new_tokens[b] tokens; returns the number of new pages per sequence."""
@@ -135,11 +178,11 @@ class PagedSequences:
             fresh = [self.pool.take() for _ in range(need)]
             if fresh:
                 start = b * self.max_pages + len(self.pages[b])
-                self.table_dev[start:start + need] = torch.tensor(fresh, dtype=torch.int32)
+                self._write(self._table_dev, start, fresh)
                 self.pages[b].extend(fresh)
             self.lengths[b] = target
             added.append(need)
-        self.seq_lens_dev.copy_(torch.tensor(self.lengths, dtype=torch.int32))
+        self._write(self._seq_lens_dev, 0, self.lengths)
         return added
 
     def reserve_pages_ahead(self, extra_tokens: int) -> None:
@@ -155,7 +198,7 @@ class PagedSequences:
             if need > 0:
                 fresh = [self.pool.take() for _ in range(need)]
                 start = b * self.max_pages + len(self.pages[b])
-                self.table_dev[start:start + need] = torch.tensor(fresh, dtype=torch.int32)
+                self._write(self._table_dev, start, fresh)
                 self.pages[b].extend(fresh)
 
     def advance_on_device(self) -> None:

@@ -213,6 +213,16 @@ int adamas_topk(const void* values, int64_t row_stride, uint32_t n_max, const in
  */
 int adamas_read_probe(const void* data, size_t bytes, void* sink, adamas_stream_t stream);
 
+/* Most words of adamas_write_words. */
+#define ADAMAS_MAX_WORDS 1024u
+
+/*
+ * dst[0 .. n) = words: up to 1024 32-bit words of host memory (sequence lengths, page ids) to device memory, as
+ * arguments of a launch (one for every 256 words).  `words` is read before the call returns and nothing waits;
+ * other reads and writes of dst are ordered by the stream.
+ */
+int adamas_write_words(int32_t* dst, const int32_t* words, uint32_t n, adamas_stream_t stream);
+
 /* Bytes of workspace adamas_topk needs for these sizes (see adamas_topk). */
 size_t adamas_topk_workspace_bytes(uint32_t num_rows, uint32_t n_max, uint32_t k);
 

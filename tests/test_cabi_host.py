@@ -458,3 +458,13 @@ def test_layer_addresses():
             c.pool.kv_address(layer)
         with pytest.raises(IndexError):
             c.pool.codes_address(layer)
+
+
+def test_write_words_arguments():
+    lib = _lib.load()
+    words = (_lib.c_int32 * 4)()
+    assert lib.adamas_write_words(None, words, 4, None) == -1
+    assert lib.adamas_write_words(16, None, 4, None) == -1
+    assert lib.adamas_write_words(16, words, 0, None) == -1
+    assert lib.adamas_write_words(16, words, _lib.MAX_WORDS + 1, None) == -1
+    assert lib.adamas_write_words(18, words, 4, None) == -4

@@ -1,0 +1,131 @@
+"""Lengths and page ids reach the device without the host waiting for them, and every reader finds them: on the
+stream that wrote them, on others, in graphs that are replayed."""
+import pytest
+import torch
+
+import adamas_amd.utils as U
+from adamas_amd import _lib
+from adamas_amd.utils.paging import PagedSequences, PagePool
+
+pytestmark = pytest.mark.gpu
+
+
+def _seqs(dev, batch, capacity, page=1):
+    pool = PagePool(1, 8, 128, page, batch * -(-capacity // page), torch.float16, dev,
+                    page_order=list(range(batch * -(-capacity // page)))[::-1])
+    return PagedSequences(pool, batch, capacity, dev)
+
+
+@pytest.mark.parametrize("n", [1, 2, 255, 256, 257, _lib.MAX_WORDS, _lib.MAX_WORDS + 1])
+def test_pages_and_lengths_arrive(gpu_device, n):
+    s = _seqs(gpu_device, 2, n + 3)
+    s.reserve([n, 1])
+    s.reserve([2, 0])
+    assert not s._host_waits
+    assert s.seq_lens_dev.tolist() == [n + 2, 1]
+    table = s.table_dev.view(2, -1).tolist()
+    assert table[0][:n + 2] == s.pages[0] and table[1][:1] == s.pages[1]
+    assert not any(table[0][n + 2:]) and not any(table[1][1:])
+
+
+def test_many_writes_behind_a_busy_stream_keep_their_order(gpu_device):
+    s = _seqs(gpu_device, 1, 64)
+    x = torch.randn(4096, 4096, device=gpu_device)
+    seen = []
+    for _ in range(20):
+        x = x @ x * 1e-3      # the host is far ahead of the device
+        s.reserve([1])
+        seen.append(s.seq_lens_dev.clone())
+    assert torch.cat(seen).tolist() == list(range(1, 21))
+
+
+def test_another_stream_waits(gpu_device):
+    s = _seqs(gpu_device, 1, 64)
+    x = torch.randn(8192, 8192, device=gpu_device)
+    torch.cuda.synchronize()
+    for _ in range(5):
+        x = x @ x * 1e-4
+    s.reserve([7])                                   # behind the products
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):                    # (no event between the streams)
+        got = s.seq_lens_dev.clone()
+        side.synchronize()
+    assert got.tolist() == [7] and s._host_waits
+    s.reserve([3])                                   # the host waits from now on
+    with torch.cuda.stream(side):
+        got = s.seq_lens_dev.clone()
+    side.synchronize()
+    assert got.tolist() == [10]
+
+
+def test_a_captured_use_ends_writes_without_waiting(gpu_device):
+    s = _seqs(gpu_device, 1, 64)
+    s.reserve([2])
+    out = torch.zeros(1, dtype=torch.int32, device=gpu_device)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out.copy_(s.seq_lens_dev)
+    assert s._host_waits
+    side = torch.cuda.Stream()
+    for n in range(3, 8):
+        s.reserve([1])
+        with torch.cuda.stream(side):
+            graph.replay()
+        side.synchronize()
+        assert out.item() == n
+
+
+def test_eager_decoding_of_a_controller_on_one_stream(gpu_device):
+    """Token by token with and without the wait: the same selections and outputs."""
+    got = []
+    for waits in (False, True):
+        g = torch.Generator(device=gpu_device).manual_seed(1)
+        c = U.InferenceController(1, 32, 128, 16, 64, 400, torch.float16, gpu_device)
+        c.seqs._host_waits = waits
+        k, v = (torch.randn(330, 32, 128, generator=g, device=gpu_device).half() for _ in range(2))
+        c.prepare_hadamard(330)
+        U.append_kvh(k, v, None, c, 0)
+        out = []
+        for _ in range(40):
+            c.prepare_hadamard(1)
+            c.begin_forward(1)
+            q, k, v = (torch.randn(1, 32, 128, generator=g, device=gpu_device).half() for _ in range(3))
+            out.append(U.decode_step(q, U.append_kvh(k, v, None, c, 0, q=q), c, 0))
+        assert c.seqs._host_waits == waits
+        got.append(torch.cat(out))
+    assert torch.equal(*got)
+
+
+def test_operators_see_to_other_streams_and_graphs(gpu_device):
+    """The native host side leaves such calls to the getters of the tables."""
+    c = U.InferenceController(1, 32, 128, 16, 64, 400, torch.float16, gpu_device)
+    g = torch.Generator(device=gpu_device).manual_seed(2)
+    k, v = (torch.randn(330, 32, 128, generator=g, device=gpu_device).half() for _ in range(2))
+    q, kn, vn = (torch.randn(1, 32, 128, generator=g, device=gpu_device).half() for _ in range(3))
+    want = []
+    for use in ("same", "side", "graph"):
+        c.clean_states()
+        c.seqs._host_waits, c.seqs._writer = False, None
+        c.prepare_hadamard(329)
+        U.append_kvh(k[:329].contiguous(), v[:329].contiguous(), None, c, 0)
+        c.prepare_hadamard(1)
+        c.begin_forward(1)
+        c.workspace(64)
+        torch.cuda.synchronize()
+        if use == "same":
+            out = U.decode_step(q, U.append_kvh(kn, vn, None, c, 0, q=q), c, 0)
+            assert not c.seqs._host_waits
+        elif use == "side":
+            side = torch.cuda.Stream()
+            with torch.cuda.stream(side):
+                out = U.decode_step(q, U.append_kvh(kn, vn, None, c, 0, q=q), c, 0)
+            side.synchronize()
+            assert c.seqs._host_waits
+        else:
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph):
+                out = U.decode_step(q, U.append_kvh(kn, vn, None, c, 0, q=q), c, 0)
+            assert c.seqs._host_waits
+            graph.replay()
+        want.append(out.clone())
+    assert torch.equal(want[0], want[1]) and torch.equal(want[0], want[2])
