@@ -37,14 +37,17 @@ struct AttnShared {
   uint32_t is_last;
 };
 
-template <bool kBf16, bool kHnd, int kThreads = 256, int kTileRows = kTile>
+// group_inv: 2^32 / group of query heads, rounded up (head / group by one multiplication: exact for heads below
+// 2^16), 0 for one query head per key/value head; page_shift: log2 of the page size, 32 where it is none.
+// kAll: all positions of the sequence (no list).
+template <bool kBf16, bool kHnd, int kThreads, int kTileRows, bool kAll>
 __global__ __launch_bounds__(kThreads) void sparse_decode_kernel(
     const __half* __restrict__ q, const __half* __restrict__ kv_data,
     const int32_t* __restrict__ page_indices, const int32_t* __restrict__ page_indptr,
     const int32_t* __restrict__ seq_lens, const int32_t* __restrict__ sel_idx, int64_t sel_stride,
     uint32_t n_sel, __half* __restrict__ out, float* partial,
-    uint32_t* __restrict__ counters, uint32_t num_heads, uint32_t num_kv_heads, uint32_t page_size,
-    float scale_log2, uint32_t rows_per_split, uint32_t deferred_merge) {
+    uint32_t* __restrict__ counters, uint32_t num_heads, uint32_t num_kv_heads, uint32_t group_inv,
+    uint32_t page_size, uint32_t page_shift, float scale_log2, uint32_t rows_per_split, uint32_t deferred_merge) {
   constexpr int kGroups = kThreads / 16;  // rows in flight per load instruction of the workgroup
   __shared__ AttnShared<kGroups> sh;
   const uint32_t split = blockIdx.x, n_split = gridDim.x;
@@ -56,9 +59,8 @@ __global__ __launch_bounds__(kThreads) void sparse_decode_kernel(
   const uint32_t bh = b * num_heads + head;
 
   const int32_t seq_len = seq_lens[b];
-  const bool dense = sel_idx == nullptr;
-  const uint32_t n_rows = dense ? static_cast<uint32_t>(seq_len) : n_sel + 1u;
-  const int32_t* sel = dense ? nullptr : sel_idx + static_cast<int64_t>(bh) * sel_stride;
+  const uint32_t n_rows = kAll ? static_cast<uint32_t>(seq_len) : n_sel + 1u;
+  const int32_t* sel = kAll ? nullptr : sel_idx + static_cast<int64_t>(bh) * sel_stride;
   const uint32_t row_begin = split * rows_per_split;
   const uint32_t row_end = min(n_rows, row_begin + rows_per_split);
 
@@ -68,21 +70,16 @@ __global__ __launch_bounds__(kThreads) void sparse_decode_kernel(
   kv.kv_data = kv_data;
   kv.table = page_indices + page_indptr[b];
   // grouped-query attention: query head h reads the K/V rows of key head h / group
-  set_kv_layout_static<kHnd>(kv, head / (num_heads / num_kv_heads), c, num_kv_heads, page_size);
+  set_kv_layout_static<kHnd>(kv, group_inv ? __umulhi(head, group_inv) : head, c, num_kv_heads, page_size);
   kv.seq_len = seq_len;
 
   SoftmaxState st;
-  // (token positions through the page table: branching around unused entries measured faster for lists
-  // than loading always, 7.9 against 8.0 us at 128 rows, and for all positions with four rows per group, 16.5
-  // against 17.5 us at 4000; with two, loading always takes 3 % off: 1000 positions 8.8 -> 8.5 us)
-  if (kTileRows == 2 && dense)  // (uniform)
-    attend_rows<kGroups, kTileRows, false, kBf16, true>(
-        kv, qf, g, row_begin, row_end,
-        [&](uint32_t r) __attribute__((always_inline)) -> int32_t { return static_cast<int32_t>(r); }, st);
+  if (kTileRows == 2 || (kThreads <= 512 && !kAll))  // (the rule stands at attend_positions)
+    attend_positions<kGroups, kTileRows, kBf16, kAll>(kv, qf, g, row_begin, row_end, sel, n_sel, page_shift, st);
   else
     attend_rows<kGroups, kTileRows, false, kBf16>(kv, qf, g, row_begin, row_end,
                                 [&](uint32_t r) __attribute__((always_inline)) -> int32_t {
-                                  if (dense) return static_cast<int32_t>(r);
+                                  if (kAll) return static_cast<int32_t>(r);
                                   return (r < n_sel) ? sel[r] : seq_len - 1;
                                 },
                                 st);
@@ -1194,13 +1191,22 @@ static int sparse_decode_impl(const void* q, const void* kv_data, const int32_t*
   }
   // from kDeferredMergeSplits splits on, the merge is a second short launch
   const uint32_t deferred = n_split >= kDeferredMergeSplits ? 1u : 0u;
-#define ADAMAS_LAUNCH_SPARSE_T(BF, HND, T, TILE)                                                \
-  hipLaunchKernelGGL((sparse_decode_kernel<BF, HND, T, TILE>), dim3(n_split, num_heads, batch), \
-                     dim3(T), 0, static_cast<hipStream_t>(stream),                              \
-                     static_cast<const __half*>(q), static_cast<const __half*>(kv_data),        \
-                     page_indices, page_indptr, seq_lens, sel_idx, sel_stride, n_sel,           \
-                     static_cast<__half*>(out), partial, counters, num_heads, num_kv_heads,     \
-                     page_size, scale_log2, rows_per_split, deferred)
+  const uint32_t group_inv = gq == 1 ? 0u : static_cast<uint32_t>(((uint64_t{1} << 32) + gq - 1) / gq);
+  uint32_t page_shift = 0;
+  while (page_shift < 32u && (uint64_t{1} << page_shift) != page_size) ++page_shift;
+#define ADAMAS_LAUNCH_SPARSE_A(BF, HND, T, TILE, ALL)                                                \
+  hipLaunchKernelGGL((sparse_decode_kernel<BF, HND, T, TILE, ALL>), dim3(n_split, num_heads, batch), \
+                     dim3(T), 0, static_cast<hipStream_t>(stream),                                   \
+                     static_cast<const __half*>(q), static_cast<const __half*>(kv_data),             \
+                     page_indices, page_indptr, seq_lens, sel_idx, sel_stride, n_sel,                \
+                     static_cast<__half*>(out), partial, counters, num_heads, num_kv_heads,          \
+                     group_inv, page_size, page_shift, scale_log2, rows_per_split, deferred)
+#define ADAMAS_LAUNCH_SPARSE_T(BF, HND, T, TILE)          \
+  if (sel_idx) {                                          \
+    ADAMAS_LAUNCH_SPARSE_A(BF, HND, T, TILE, false);      \
+  } else {                                                \
+    ADAMAS_LAUNCH_SPARSE_A(BF, HND, T, TILE, true);       \
+  }
 #define ADAMAS_LAUNCH_SPARSE_L(BF, HND)          \
   if (threads == 256) {                          \
     ADAMAS_LAUNCH_SPARSE_T(BF, HND, 256, 4);     \
@@ -1227,6 +1233,7 @@ static int sparse_decode_impl(const void* q, const void* kv_data, const int32_t*
 #undef ADAMAS_LAUNCH_SPARSE
 #undef ADAMAS_LAUNCH_SPARSE_L
 #undef ADAMAS_LAUNCH_SPARSE_T
+#undef ADAMAS_LAUNCH_SPARSE_A
   ADAMAS_RETURN_IF_LAUNCH_FAILED();
   if (deferred) {
     if (bf16)
