@@ -937,6 +937,19 @@ template <int kThreads>
 constexpr int kHsaRows = kThreads == kHsaWideThreads ? 8 : 4;
 typedef uint32_t fs_uint4 __attribute__((ext_vector_type(4)));
 
+// v[i] of registers, i from the lane
+template <int kItems>
+__device__ __forceinline__ uint32_t pick(const uint32_t (&v)[kItems], uint32_t i) {
+  uint32_t t[kItems];
+#pragma unroll
+  for (int j = 0; j < kItems; ++j) t[j] = v[j];
+#pragma unroll
+  for (int bit = 1, n = kItems; n > 1; bit *= 2, n /= 2)
+#pragma unroll
+    for (int j = 0; j < n / 2; ++j) t[j] = i & bit ? t[2 * j + 1] : t[2 * j];
+  return t[0];
+}
+
 template <int kThreads, int kItems>
 struct HistSelectAttendShared {
   static constexpr int kWaves = kThreads / kWave;
@@ -958,7 +971,7 @@ struct HistSelectAttendShared {
 // of the last workgroup of a head read its partials.  In batches the workgroups of the heads that share a key/value
 // head lie on one die (head_of_block; 1.3 %, one sequence loses 0.6 %: it is not bound by its bytes).  us a layer of
 // a step before / now: 23989 tokens, 32:8 heads, bf16, budget 1024 20.9 / 20.2; 8 sequences of 1500 to 7000, 32:8
-// heads, 512, 31.5 / 30.3.  Where the time goes in the first of these, 9.5 us from the first workgroup's start to the
+// heads, 512, 31.5 / 30.3; 8 of 4000 to 15000, 3000, 112.5 / 113.2 and, 32:8 heads, 88.5 / 77.7.  Where the time goes in the first of these, 9.5 us from the first workgroup's start to the
 // last one's end: loads 1.3, sum and threshold 0.7, selection 0.7, rows and softmax 2.0 to 2.7, merge of the waves
 // 1.0, partial out and counter 1.2, merge of the slabs 1.2, the rest is workgroups that share a CU.
 template <bool kBf16, bool kHnd, int kThreads, int kItems>
@@ -1051,6 +1064,7 @@ __global__ __launch_bounds__(kThreads) void hist_select_attend_kernel(
 
   // ---- chunk rows summed up: all of them, and those before the slab
   const uint32_t c_first = slab_base >> chunk_log2;  // chunks below it precede the slab (whole chunks)
+  const uint32_t rows_used = min(n_chunks, (n + (1u << chunk_log2) - 1u) >> chunk_log2);  // those of this sequence
   uint32_t acc[4] = {0u, 0u, 0u, 0u}, pre[4] = {0u, 0u, 0u, 0u};
   auto add_rows = [&](uint32_t c0) __attribute__((always_inline)) {
 #pragma unroll
@@ -1058,13 +1072,13 @@ __global__ __launch_bounds__(kThreads) void hist_select_attend_kernel(
       const uint32_t c = c0 + kWaves * u;   // (uniform, as are the conditions)
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        acc[j] += c < n_chunks ? hrow[u][j] : 0u;
+        acc[j] += c < rows_used ? hrow[u][j] : 0u;
         pre[j] = c < c_first ? acc[j] : pre[j];
       }
     }
   };
   add_rows(wave);
-  for (uint32_t c0 = wave + kWaves * kRows; c0 < n_chunks; c0 += kWaves * kRows) {
+  for (uint32_t c0 = wave + kWaves * kRows; c0 < rows_used; c0 += kWaves * kRows) {
     ask_rows(c0);
     add_rows(c0);
   }
@@ -1141,10 +1155,16 @@ __global__ __launch_bounds__(kThreads) void hist_select_attend_kernel(
     }
     wave_below = wave_sum(wave_below);
   }
-  uint32_t below[kItems / 4], equal[kItems / 4];
-  raw_class_masks<kItems>(keys, plan.thr, below, equal);
-  uint32_t total;
-  const uint32_t excl = lane_scan<kItems / 4>(below, equal, total);  // below | tied << 16
+  uint32_t below = 0, equal = 0;  // bit i: item i
+#pragma unroll
+  for (int i = 0; i < kItems; ++i) {
+    below |= keys[i] < plan.thr ? 1u << i : 0u;
+    equal |= keys[i] == plan.thr ? 1u << i : 0u;
+  }
+  const uint32_t own = __popc(below) | (__popc(equal) << 16);
+  const uint32_t upto = wave_inclusive_scan_dpp(own);
+  const uint32_t excl = upto - own;  // below | tied << 16 in lower lanes
+  const uint32_t total = __builtin_amdgcn_readlane(upto, kWave - 1);
   if (lane == 0) sh.wcount[wave] = make_uint4(total, wave_tied, wave_below, 0u);
   __syncthreads();
   const uint4 wc = sh.wcount[lane & (kWaves - 1)];
@@ -1160,21 +1180,36 @@ __global__ __launch_bounds__(kThreads) void hist_select_attend_kernel(
   {
     // the slab's list: the tokens below the threshold in index order, then its ties
     uint32_t pb = (before & 0xffffu) + (excl & 0xffffu), pe = (before >> 16) + (excl >> 16);
+    if (kItems <= 8) {
 #pragma unroll
-    for (int i = 0; i < kItems; ++i) {
-      const bool is_b = keys[i] < plan.thr, is_e = keys[i] == plan.thr;
-      if (is_b || (is_e && pe < tied_left)) sh.rows[is_b ? pb : slab_below + pe] = static_cast<int32_t>(trow[i]);
-      pb += is_b ? 1u : 0u;
-      pe += is_e ? 1u : 0u;
+      for (int i = 0; i < kItems; ++i) {
+        const bool is_b = keys[i] < plan.thr, is_e = keys[i] == plan.thr;
+        if (is_b || (is_e && pe < tied_left)) sh.rows[is_b ? pb : slab_below + pe] = static_cast<int32_t>(trow[i]);
+        pb += is_b ? 1u : 0u;
+        pe += is_e ? 1u : 0u;
+      }
+    } else {
+      // a few of many: the set bits are walked (us a layer, item by item / so: 100000 tokens, budget 1024, 42.4 / 42.1
+      // and, 32:8 heads, bf16, 31.6 / 31.2; 60000, 2048, 33.0 / 32.8; with eight items the same)
+      for (uint32_t m = below | equal; m; m &= m - 1u) {
+        const uint32_t i = __ffs(m) - 1;
+        const bool is_b = (below >> i) & 1u;
+        if (is_b || pe < tied_left) sh.rows[is_b ? pb : slab_below + pe] = static_cast<int32_t>(pick<kItems>(trow, i));
+        pb += is_b ? 1u : 0u;
+        pe += is_b ? 0u : 1u;
+      }
     }
   }
   if (sdst) {  // positions in the whole selection: the same over all slabs
-    const uint32_t base_b = sum_of_first<kWaves>(wc.z);
-    lane_emit<kItems / 4>(below, equal, plan.n_below, plan.quota, base_b + (before & 0xffffu) + (excl & 0xffffu),
-                          pre_tied + (before >> 16) + (excl >> 16),
-                          [&](uint32_t pos, int i) __attribute__((always_inline)) {
-                            sdst[pos] = static_cast<int32_t>(e0 + i);
-                          });
+    uint32_t pb = sum_of_first<kWaves>(wc.z) + (before & 0xffffu) + (excl & 0xffffu);
+    uint32_t pe = pre_tied + (before >> 16) + (excl >> 16);
+    for (uint32_t m = below | equal; m; m &= m - 1u) {
+      const uint32_t i = __ffs(m) - 1;
+      const bool is_b = (below >> i) & 1u;
+      if (is_b || pe < plan.quota) sdst[is_b ? pb : plan.n_below + pe] = static_cast<int32_t>(e0 + i);
+      pb += is_b ? 1u : 0u;
+      pe += is_b ? 0u : 1u;
+    }
   }
   uint32_t n_rows = slab_below + slab_tied_taken;
   if (slab == 0) {
