@@ -292,20 +292,23 @@ __device__ __forceinline__ WavePlan wave_plan_from_hist(const uint32_t* hist_lds
 // kSkipInvalid: items that are no keys are left out of the counting by a branch (worth it where many
 // lanes hold none: they would all add to one spare word); otherwise they count into a spare word
 // without a branch.
-template <int kItems, bool kSkipInvalid, typename KeyOf, typename Payload>
+// kCounted: hist_lds holds the counts already.
+template <int kItems, bool kSkipInvalid, bool kCounted = false, typename KeyOf, typename Payload>
 __device__ __forceinline__ void chunk_select_capped(const uint32_t (&keys)[kItems], uint32_t kc,
                                                     uint64_t* dst, uint32_t* hist_lds,
                                                     KeyOf&& key_of, Payload&& payload) {
   static_assert(kItems <= 32, "one class bit per item");
   const int lane = lane_id();
-  *reinterpret_cast<uint4*>(&hist_lds[8 * lane]) = make_uint4(0u, 0u, 0u, 0u);
-  *reinterpret_cast<uint4*>(&hist_lds[8 * lane + 4]) = make_uint4(0u, 0u, 0u, 0u);
+  if (!kCounted) {
+    *reinterpret_cast<uint4*>(&hist_lds[8 * lane]) = make_uint4(0u, 0u, 0u, 0u);
+    *reinterpret_cast<uint4*>(&hist_lds[8 * lane + 4]) = make_uint4(0u, 0u, 0u, 0u);
 #pragma unroll
-  for (int i = 0; i < kItems; ++i) {
-    if (kSkipInvalid) {
-      if (keys[i] < static_cast<uint32_t>(kHistBins)) atomicAdd(&hist_lds[keys[i]], 1u);
-    } else {
-      atomicAdd(&hist_lds[min(keys[i], static_cast<uint32_t>(kHistBins))], 1u);
+    for (int i = 0; i < kItems; ++i) {
+      if (kSkipInvalid) {
+        if (keys[i] < static_cast<uint32_t>(kHistBins)) atomicAdd(&hist_lds[keys[i]], 1u);
+      } else {
+        atomicAdd(&hist_lds[min(keys[i], static_cast<uint32_t>(kHistBins))], 1u);
+      }
     }
   }
   // the LDS operations of one wave are carried out in order: the counts are complete here

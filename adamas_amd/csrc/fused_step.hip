@@ -163,6 +163,13 @@ __global__ __launch_bounds__(kHeads * kWave) void estimate_select_kernel(
     uint32_t* __restrict__ rowmap_out = nullptr, QkvSource src = QkvSource()) {
   static_assert(!kHist || !kPartial, "the histogram mode works on chunks of 512, 1024 or 2048 tokens");
   constexpr int kItems = 8 * kPasses;                 // tokens per lane in the selection phase
+  // With several passes the narrow and the shared instances count the distances as they come, under the loads of the
+  // next pass, instead of 16 or 32 to a lane when all loads have ended (us a layer of a step, at the end / as they come,
+  // 100000 tokens, 32:8 heads, budget 200, 20.4 / 19.8; 50000, 128, 16.3 / 15.7; 3 sequences of 40000 to 50000, 32:32,
+  // 41.4 / 39.8).  The wide one, eight heads apart in a wave and a full chip of it waiting for memory, gains nothing
+  // (131072 tokens 38.3 / 38.5), nor does a single pass, whose last loads' counts are waited for either way (32768
+  // tokens, this launch 10.3 / 10.7).
+  constexpr bool kCountEarly = !kHist && kPasses >= 2 && (kShare == 4 || kHeads == 4);
   static_assert(kHeads == 8 || kHeads == 4, "a token's codes are read by 2 * kHeads lanes");
   static_assert(kShare == 1 || kShare == 4, "a lane serves one head, or four that share a key/value head");
   constexpr uint32_t kLoadTokens = 32 / kHeads * kShare;    // tokens per load instruction: 4 or 8 (16 or 32)
@@ -354,6 +361,7 @@ __global__ __launch_bounds__(kHeads * kWave) void estimate_select_kernel(
             v += swap_adjacent(v);
             const uint32_t d = half ? (v >> 16) : (v & 0xffffu);
             sh.dist[hl + h][tok] = mine ? static_cast<uint16_t>(d) : 0xffffu;
+            if (kCountEarly && mine) atomicAdd(&sh.hist[hl + h][d], 1u);
           }
         }
         return;
@@ -376,11 +384,18 @@ __global__ __launch_bounds__(kHeads * kWave) void estimate_select_kernel(
           const uint32_t tok = tok_u + (2 * i2 + half) * kLoadTokens + sub;
           const uint32_t d = half ? (v >> 16) : (v & 0xffffu);
           sh.dist[hl][tok] = (chunk_base + tok < n) ? static_cast<uint16_t>(d) : 0xffffu;
+          if (kCountEarly && chunk_base + tok < n) atomicAdd(&sh.hist[hl][d], 1u);
         }
       }
     };
     uint4 buf0[kLoads], buf1[kLoads];
     issue(0, buf0);
+    if (kCountEarly) {
+      *reinterpret_cast<uint4*>(&sh.hist[wave][8 * lane]) = make_uint4(0u, 0u, 0u, 0u);
+      *reinterpret_cast<uint4*>(&sh.hist[wave][8 * lane + 4]) = make_uint4(0u, 0u, 0u, 0u);
+      // (waits for LDS only, as below; with kFromQkv the barrier there does)
+      if (!kFromQkv) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    }
     // the query codes for the second launch (behind the code loads: the store waits for the query
     // code, which must not hold the code loads back)
     if (!kFromQkv && !kHist && chunk == 0 && sub == 0) {
@@ -468,7 +483,7 @@ __global__ __launch_bounds__(kHeads * kWave) void estimate_select_kernel(
     }
   }
   // the K row of a listed token is read when it is written out (a handful per wave)
-  chunk_select_capped<kItems, kPartial>(
+  chunk_select_capped<kItems, kPartial, kCountEarly>(
       keys, geom.kc, dst, sh.hist[wave],
       [&](uint32_t tok) __attribute__((always_inline)) -> uint32_t { return sh.dist[wave][tok]; },
       [&](uint32_t tok) __attribute__((always_inline)) -> uint32_t { return sh.krow[tok]; });

@@ -227,3 +227,12 @@ def test_step_of_equal_distances_takes_the_first_tokens(gpu_device, lens, budget
 def test_step_in_the_order_of_key_value_heads(gpu_device, kv_heads):
     """The workgroups of the heads that share a key/value head lie together."""
     _check(gpu_device, [5000, 700], 400, 16, kv_heads, torch.float16, 0)
+
+
+@pytest.mark.parametrize("lens,budget,page,kv_heads,layout", [
+    ([70001, 1030, 2], 128, 16, 32, 0),     # narrow workgroups, four passes, the last one ragged
+    ([33000, 600], 64, 1, 32, 1),           # two passes
+    ([66000, 65537], 200, 16, 8, 0),        # four heads to a lane
+])
+def test_step_of_several_passes_counts_as_it_goes(gpu_device, lens, budget, page, kv_heads, layout):
+    _check(gpu_device, lens, budget, page, kv_heads, torch.float16, layout)
