@@ -23,10 +23,10 @@ constexpr int kTile = 8;             // rows per group per tile, at most
 // 16 groups of 4, up to 128 rows 32 groups of 4 (one split, no merge, no workspace); up to 512 rows
 // splits of 64 rows (32 groups of 2, at most 8 splits); up to 2048 rows splits of 128 (64 groups of
 // 2, at most 16); beyond that, and where more workgroups than run at once would come of it, four rows in flight
-// (row_launch).  Measured at 32 heads, rows = 128 /
-// 256 / 512 / 1024 / 2048 / 4096, in us: 5.8 / 6.5 / 7.4 / 9.3 / 13.5 / 18.8 (with 16 groups of 8
-// rows and splits of 128 rows up to 1024 rows, 32 groups of 8 beyond: 7.5 / 9.5 / 10.1 / 12.4 / 15.8
-// / 20.6).
+// (row_launch).  Lists at 32 heads, rows = 128 / 256 / 1000 / 2048 / 4096, in us: 4.2 / 5.9 / 8.4 / 12.1 / 19.2,
+// 512 at 32:8 heads 7.2.  The lines were drawn with rows fetched one by one, rows = 128 / 256 / 512 / 1024 / 2048 /
+// 4096: 5.8 / 6.5 / 7.4 / 9.3 / 13.5 / 18.8 (with 16 groups of 8 rows and splits of 128 rows up to 1024 rows, 32
+// groups of 8 beyond: 7.5 / 9.5 / 10.1 / 12.4 / 15.8 / 20.6).
 constexpr uint32_t kDeferredMergeSplits = 24;  // splits from which the partials get a merge launch
 // (measured at 32768 tokens, 32 heads: 16 splits 14.7 us merged inside the launch, 15.8 us with a merge
 // launch; 32 splits 26.6 against 22.5 us)

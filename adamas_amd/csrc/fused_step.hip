@@ -986,8 +986,8 @@ struct HistSelectAttendShared {
 // of the last workgroup of a head read its partials.  In batches the workgroups of the heads that share a key/value
 // head lie on one die (head_of_block; 1.3 %, one sequence loses 0.6 %: it is not bound by its bytes).  us a layer of
 // a step before / now: 23989 tokens, 32:8 heads, bf16, budget 1024 20.9 / 20.2; 8 sequences of 1500 to 7000, 32:8
-// heads, 512, 31.5 / 30.3; 8 of 4000 to 15000, 3000, 112.5 / 113.2 and, 32:8 heads, 88.5 / 77.7.  Where the time goes in the first of these, 9.5 us from the first workgroup's start to the
-// last one's end: loads 1.3, sum and threshold 0.7, selection 0.7, rows and softmax 2.0 to 2.7, merge of the waves
+// heads, 512, 31.5 / 30.2; 8 of 4000 to 15000, 3000, 112.5 / 113.2 and, 32:8 heads, 88.5 / 77.7.  Where the time
+// goes in the first of these, 9.5 us from the first workgroup's start to the last one's end: loads 1.3, sum and threshold 0.7, selection 0.7, rows and softmax 2.0 to 2.7, merge of the waves
 // 1.0, partial out and counter 1.2, merge of the slabs 1.2, the rest is workgroups that share a CU.
 template <bool kBf16, bool kHnd, int kThreads, int kItems>
 __global__ __launch_bounds__(kThreads) void hist_select_attend_kernel(
