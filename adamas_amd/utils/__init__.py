@@ -144,9 +144,10 @@ def append_kvh(k: torch.Tensor, v: torch.Tensor, h: Optional[torch.Tensor],
     [B*num_heads + B*num_kv_heads, D] of Hadamard(q) rows followed by Hadamard(k) rows.
     Reference: adamas/utils/__init__.py:94-157.
     """
-    o = (_host or _load_host()).append_decode(k, v, h, q, iController, layer_idx)
-    if o is not None:
-        return o
+    if h is not None or q is not None:   # (neither: a prompt)
+        o = (_host or _load_host()).append_decode(k, v, h, q, iController, layer_idx)
+        if o is not None:
+            return o
     lib = _lib.load()
     c = iController
     _check_cuda_contig(k, "k", c.dtype, 3)

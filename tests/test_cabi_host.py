@@ -468,3 +468,31 @@ def test_write_words_arguments():
     assert lib.adamas_write_words(16, words, 0, None) == -1
     assert lib.adamas_write_words(16, words, _lib.MAX_WORDS + 1, None) == -1
     assert lib.adamas_write_words(18, words, 4, None) == -4
+
+
+def test_a_call_that_the_native_host_side_leaves_costs_little():
+    """Every operator asks the native function first, so one that declines (here: tensors on the CPU, neither h nor q,
+    a controller that is none) must cost next to nothing: at most a few calls of an empty library function (0.9 of it
+    measured; 15 where each decline was an exception)."""
+    import time
+    host, version = U._load_host(), _lib.load().adamas_version
+    c = U.InferenceController(1, 8, 128, 16, 64, 64, torch.float16, "cpu")
+    x = torch.zeros(1, 8, 128).half()
+    declined = [lambda: host.hadamard(x, False, 1.0), lambda: host.hadamard(x, True, 1.0),
+                lambda: host.append_decode(x, x, None, None, c, 0), lambda: host.append_decode(x, x, None, x, c, 0),
+                lambda: host.estimate(x, c, 0), lambda: host.topk(x, c, None), lambda: host.sparse_attn(x, c, 0, None),
+                lambda: host.step(x, x, c, 0), lambda: host.step(x, x, None, 0)]
+
+    def best(call, n=2000):
+        times = []
+        for _ in range(20):
+            t0 = time.perf_counter()
+            for _ in range(n):
+                call()
+            times.append(time.perf_counter() - t0)
+        return min(times)
+
+    unit = best(version)
+    for i, call in enumerate(declined):
+        assert call() is None
+        assert best(call) < 6 * unit, i

@@ -115,7 +115,8 @@ def test_calls_that_go_the_general_way(gpu_device, monkeypatch):
 
     x = torch.randn(4, 128, device=dev).half()
     y = U.hadamard_transform(x)
-    assert torch.equal(general(lambda: U.hadamard_transform(x, True)), y) and torch.equal(x, y)
+    host.served.clear()
+    assert U.hadamard_transform(x, True) is x and torch.equal(x, y) and host.served == [True]
     assert torch.equal(general(lambda: U.hadamard_transform(x, scale=1)), U.hadamard_transform(x, scale=1.0))
     est = U.decode_estimate(code, c, 0)
     est.mul_(1)                                                        # edited: arbitrary keys from now on
