@@ -174,7 +174,7 @@ struct Controller {
   }
 
   // The current stream, if it is t's device's and lengths and pages need no wait there: those are read from the
-  // tensors behind PagedSequences.table_dev and .seq_lens_dev, whose getters see to the other streams and graphs.
+  // tensors as they are, and PagedSequences.launch_addresses sees to the other streams and graphs.
   bool stream(const at::Tensor& t, adamas_stream_t& s) const {
     Ref waits, writer;
     if (!stream_of(t, s) || !waits.read(seqs.p, s__host_waits)) return false;

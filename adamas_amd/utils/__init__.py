@@ -174,7 +174,7 @@ def append_kvh(k: torch.Tensor, v: torch.Tensor, h: Optional[torch.Tensor],
         if n > total:
             raise RuntimeError("prepare_hadamard must reserve the tokens before append_kvh")
         rc = lib.adamas_append_prefill(k.data_ptr(), v.data_ptr(), _lib.ptr(h), n, total - n,
-                                       kv, codes, c.seqs.table_ptr(seq_idx),
+                                       kv, codes, c.seqs.launch_addresses(seq_idx)[0],
                                        c.seqs.max_pages, nh, d, c.page_size, c.hadamard_scale,
                                        c.code_flags, stream)
         _lib.check(rc, "adamas_append_prefill")
@@ -194,9 +194,8 @@ def append_kvh(k: torch.Tensor, v: torch.Tensor, h: Optional[torch.Tensor],
         raise RuntimeError("prepare_hadamard must reserve the token before append_kvh")
     o = torch.empty((n, nq, d // 8), dtype=torch.int16, device=k.device)
     rc = lib.adamas_append_decode(_lib.ptr(q), k.data_ptr(), v.data_ptr(), _lib.ptr(h), o.data_ptr(),
-                                  kv, codes, c.seqs.table_dev.data_ptr(),
-                                  c.seqs.indptr_dev.data_ptr(), c.seqs.seq_lens_dev.data_ptr(), n,
-                                  nq, nh, d, c.page_size, c.hadamard_scale, c.code_flags, stream)
+                                  kv, codes, *c.seqs.launch_addresses(), n, nq, nh, d, c.page_size,
+                                  c.hadamard_scale, c.code_flags, stream)
     _lib.check(rc, "adamas_append_decode")
     return o
 
@@ -222,8 +221,7 @@ def decode_estimate(q: torch.Tensor, iController: InferenceController, layer_idx
     stride = (lmax - 1 + 7) // 8 * 8
     buf = torch.empty((c.batch_size, c.num_heads, stride), dtype=torch.float16, device=q.device)
     rc = _lib.load().adamas_estimate(q.data_ptr(), c.pool.codes_address(layer_idx),
-                                     c.seqs.table_dev.data_ptr(), c.seqs.indptr_dev.data_ptr(),
-                                     c.seqs.seq_lens_dev.data_ptr(), buf.data_ptr(),
+                                     *c.seqs.launch_addresses(), buf.data_ptr(),
                                      c.num_heads * stride, stride, _lib.DIST_FP16, c.batch_size,
                                      c.num_heads, c.num_kv_heads, c.page_size, lmax,
                                      _lib.current_stream())
@@ -285,7 +283,7 @@ def decode_topk(estimated_attn_score: torch.Tensor, iController: InferenceContro
     ragged = c.batch_size > 1
     buf = c.topk_workspace(n, k)
     rc = _lib.load().adamas_topk(est2.data_ptr(), est2.stride(0), n,
-                                 c.seqs.seq_lens_dev.data_ptr() if ragged else None,
+                                 c.seqs.launch_addresses()[2] if ragged else None,
                                  c.num_heads, -1, None, 0, rows, k,
                                  c.topk_dindices_buffer.data_ptr(), c.topk_dout_buffer.data_ptr(), k,
                                  mode, buf.data_ptr(), buf.numel(), _lib.current_stream())
@@ -320,8 +318,7 @@ def decode_sparse_attn(q: torch.Tensor, iController: InferenceController, layer_
         sel_ptr, stride, n_sel = topk_indices.data_ptr(), topk_indices.stride(0), topk_indices.shape[1]
     ws = c.workspace(c.inference_page_budget or 1)
     rc = _lib.load().adamas_sparse_decode_f(
-        q.data_ptr(), c.pool.kv_address(layer_idx), c.seqs.table_dev.data_ptr(),
-        c.seqs.indptr_dev.data_ptr(), c.seqs.seq_lens_dev.data_ptr(), sel_ptr, stride, n_sel,
+        q.data_ptr(), c.pool.kv_address(layer_idx), *c.seqs.launch_addresses(), sel_ptr, stride, n_sel,
         o.data_ptr(), ws.data_ptr(), ws.numel(), c.batch_size, c.num_heads, c.num_kv_heads,
         c.head_dim, c.page_size, 1.0 / math.sqrt(c.head_dim), c.max_len_now, c.kv_flags,
         _lib.current_stream())
@@ -458,8 +455,7 @@ def decode_step(q: torch.Tensor, q_code: torch.Tensor, iController: InferenceCon
     sel = c.topk_dindices_buffer if return_indices else None
     rc = _lib.load().adamas_decode_step_f(
         q.data_ptr(), q_code.data_ptr(), c.pool.kv_address(layer_idx),
-        c.pool.codes_address(layer_idx), c.seqs.table_dev.data_ptr(),
-        c.seqs.indptr_dev.data_ptr(), c.seqs.seq_lens_dev.data_ptr(), budget, o.data_ptr(),
+        c.pool.codes_address(layer_idx), *c.seqs.launch_addresses(), budget, o.data_ptr(),
         _lib.ptr(sel), ws.data_ptr(), ws.numel(), c.batch_size, c.num_heads, c.num_kv_heads,
         c.head_dim, c.page_size, 1.0 / math.sqrt(c.head_dim), c.max_len_now, c.seqs.max_pages,
         c.kv_flags | c.codes_flags, _lib.current_stream())
@@ -507,7 +503,7 @@ def _prefill_with_torch_operators(q: torch.Tensor, c: InferenceController, layer
     """prefill_forward out of torch operators in float32, blocks of 4096 query rows."""
     n, p = q.shape[0], c.page_size
     n_pages = (length + p - 1) // p
-    kv = c.kv_cache.buf_layer(layer_idx).index_select(0, c.seqs.table_dev[:n_pages].long())
+    kv = c.kv_cache.buf_layer(layer_idx).index_select(0, c.seqs.launch_table()[:n_pages].long())
     kv = kv.permute(1, 3, 0, 2, 4) if c.layout == TensorLayout.NHD else kv.permute(1, 2, 0, 3, 4)
     keys, values = kv.reshape(2, c.num_kv_heads, n_pages * p, c.head_dim)[:, :, :length].float()
     group, past = c.num_heads // c.num_kv_heads, length - n
@@ -560,7 +556,7 @@ def _prefill(q: torch.Tensor, c: InferenceController, layer_idx: int, length: in
     need = lib.adamas_prefill_workspace_bytes(n, length - n, c.num_heads, c.num_kv_heads)
     ws = torch.empty(need, dtype=torch.uint8, device=q.device) if need else None
     rc = lib.adamas_prefill_attention(q.data_ptr(), c.kv_cache.buf_layer(layer_idx).data_ptr(),
-                                      c.seqs.table_ptr(0), o.data_ptr(), _lib.ptr(ws), need, n,
+                                      c.seqs.launch_addresses()[0], o.data_ptr(), _lib.ptr(ws), need, n,
                                       length - n, c.num_heads, c.num_kv_heads, c.head_dim, c.page_size,
                                       1.0 / math.sqrt(c.head_dim), c.kv_flags,
                                       torch._C._cuda_getCurrentRawStream(device))
@@ -699,9 +695,7 @@ def rope_append_decode(qkv: torch.Tensor, cos_table: torch.Tensor, sin_table: to
     q_code = torch.empty((n, nq, 16), dtype=torch.int16, device=qkv.device)
     rc = _lib.load().adamas_rope_append_decode(
         qkv.data_ptr(), cos_table.data_ptr(), sin_table.data_ptr(), q.data_ptr(), q_code.data_ptr(),
-        c.pool.kv_address(layer_idx), c.pool.codes_address(layer_idx),
-        c.seqs.table_dev.data_ptr(), c.seqs.indptr_dev.data_ptr(), c.seqs.seq_lens_dev.data_ptr(), n,
-        nq, nkv, 128, c.page_size, c.hadamard_scale, c.code_flags, _lib.current_stream())
+        c.pool.kv_address(layer_idx), c.pool.codes_address(layer_idx), *c.seqs.launch_addresses(), n, nq, nkv, 128, c.page_size, c.hadamard_scale, c.code_flags, _lib.current_stream())
     _lib.check(rc, "adamas_rope_append_decode")
     return q, q_code
 
@@ -796,8 +790,8 @@ def decode_layer_step(qkv: torch.Tensor, cos_table: torch.Tensor, sin_table: tor
     sel = c.topk_dindices_buffer if return_indices else None
     rc = _lib.load().adamas_decode_layer_step(
         qkv.data_ptr(), cos_table.data_ptr(), sin_table.data_ptr(), c.pool.kv_address(layer_idx),
-        c.pool.codes_address(layer_idx), c.seqs.table_dev.data_ptr(), c.seqs.indptr_dev.data_ptr(),
-        c.seqs.seq_lens_dev.data_ptr(), budget, o.data_ptr(), _lib.ptr(sel), ws.data_ptr(), ws.numel(),
+        c.pool.codes_address(layer_idx), *c.seqs.launch_addresses(), budget, o.data_ptr(), _lib.ptr(sel),
+        ws.data_ptr(), ws.numel(),
         n, nq, nkv, 128, c.page_size, 1.0 / math.sqrt(c.head_dim), c.max_len_now, c.seqs.max_pages,
         c.hadamard_scale, c.code_flags | c.codes_flags, _lib.current_stream())
     _lib.check(rc, "adamas_decode_layer_step")

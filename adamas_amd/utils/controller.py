@@ -107,7 +107,8 @@ class InferenceController:
         self._workspace_need = {}
         self._len_bound: Optional[int] = None
 
-    # --- device-side views used by the operator functions -----------------------------------------
+    # --- device-side views for callers (the first look makes the host wait for later writes to them, see
+    # PagedSequences.table_dev; the operators do not come this way) -----------------------------------
     @property
     def kv_indices_with_last(self) -> torch.Tensor:
         return self.seqs.table_dev

@@ -121,30 +121,52 @@ class PagedSequences:
         self.indptr_dev = (torch.arange(batch + 1, dtype=torch.int32) * self.max_pages).to(device)
         self._seq_lens_dev = torch.zeros(batch, dtype=torch.int32, device=device)
         # Lengths and page ids are written by a launch that the host does not wait for, while everything that
-        # reads them is launched on the stream of that launch.  The first use on another stream, or in a graph
-        # (which is replayed on whatever stream), waits for what is written and ends that: from then on the host
-        # waits for every write, and no stream can be too early.
+        # reads them is launched by this package's operators on the stream of that launch.  The first operator on
+        # another stream or in a graph (which is replayed on whatever stream), and the first look from outside (a
+        # tensor or an address once handed out is used at any time on any stream), wait for what is written and end
+        # that for good: from then on the host waits for every write, and no stream can be too early.
         self._host_waits = not self._table_dev.is_cuda
         self._writer: Optional[int] = None    # stream of the last write that the host did not wait for
 
     @property
     def table_dev(self) -> torch.Tensor:
-        if not self._host_waits:
-            self._note_use()
+        """The page table [batch * max_pages] int32.  From the first look at it or at seq_lens_dev on, the host waits
+        for every write, so that who holds them may read them on any stream, as soon as the call that grew a
+        sequence has returned."""
+        self._end_writes_without_waiting()
         return self._table_dev
 
     @property
     def seq_lens_dev(self) -> torch.Tensor:
-        if not self._host_waits:
-            self._note_use()
+        """The lengths [batch] int32 (see table_dev)."""
+        self._end_writes_without_waiting()
         return self._seq_lens_dev
 
-    def _note_use(self) -> None:
-        if torch.cuda.is_current_stream_capturing():
-            self._host_waits = True   # (nothing to wait for: capture does not execute)
-        elif self._writer is not None and _lib.current_stream(self._table_dev.get_device()) != self._writer:
+    def launch_addresses(self, b: int = 0):
+        """(page table of sequence b, indptr, lengths) on the device, for a launch on the current stream now; not to
+        be kept."""
+        if not self._host_waits:
+            self._note_use()
+        return (self._table_dev.data_ptr() + 4 * b * self.max_pages, self.indptr_dev.data_ptr(),
+                self._seq_lens_dev.data_ptr())
+
+    def launch_table(self) -> torch.Tensor:
+        """table_dev for operators launched on the current stream now; not to be kept."""
+        if not self._host_waits:
+            self._note_use()
+        return self._table_dev
+
+    def _end_writes_without_waiting(self) -> None:
+        if self._host_waits:
+            return
+        if self._writer is not None and not torch.cuda.is_current_stream_capturing():
             torch.cuda.synchronize(self._table_dev.device)
-            self._host_waits = True
+        self._host_waits = True
+
+    def _note_use(self) -> None:
+        if torch.cuda.is_current_stream_capturing() or (
+                self._writer is not None and _lib.current_stream(self._table_dev.get_device()) != self._writer):
+            self._end_writes_without_waiting()
 
     def _write(self, dst: torch.Tensor, start: int, values: List[int]) -> None:
         """dst[start:] = values, without waiting for it where that is safe (see __init__): a decode loop that
@@ -203,7 +225,9 @@ class PagedSequences:
 
     def advance_on_device(self) -> None:
         """One more token for every sequence, on the device only (graph-capturable)."""
-        self.seq_lens_dev.add_(1)
+        if not self._host_waits:
+            self._note_use()
+        self._seq_lens_dev.add_(1)
 
     def note_advanced(self, n_tokens: int) -> None:
         """Bring the host-side lengths in line after `n_tokens` device-side advances."""
@@ -217,10 +241,12 @@ class PagedSequences:
             self.pool.give_back(self.pages[b])
             self.pages[b] = []
             self.lengths[b] = 0
-        self.seq_lens_dev.zero_()
+        if not self._host_waits:
+            self._note_use()
+        self._seq_lens_dev.zero_()
 
     def table_ptr(self, b: int) -> int:
-        """Device address of the first page-table entry of sequence b."""
+        """Device address of the first page-table entry of sequence b (see table_dev)."""
         return self.table_dev.data_ptr() + 4 * b * self.max_pages
 
 

@@ -5,6 +5,7 @@ import torch
 
 import adamas_amd.utils as U
 from adamas_amd import _lib
+from adamas_amd.decoder import DecoderConfig, LlamaShapedDecoder
 from adamas_amd.utils.paging import PagedSequences, PagePool
 
 pytestmark = pytest.mark.gpu
@@ -35,7 +36,8 @@ def test_many_writes_behind_a_busy_stream_keep_their_order(gpu_device):
     for _ in range(20):
         x = x @ x * 1e-3      # the host is far ahead of the device
         s.reserve([1])
-        seen.append(s.seq_lens_dev.clone())
+        seen.append(s._seq_lens_dev.clone())     # as an operator's launch reads them
+    assert not s._host_waits
     assert torch.cat(seen).tolist() == list(range(1, 21))
 
 
@@ -129,3 +131,44 @@ def test_operators_see_to_other_streams_and_graphs(gpu_device):
             graph.replay()
         want.append(out.clone())
     assert torch.equal(want[0], want[1]) and torch.equal(want[0], want[2])
+
+
+@pytest.mark.parametrize("held", ["lengths", "table", "address"])
+def test_what_has_been_handed_out_is_written_when_the_call_returns(gpu_device, held):
+    """A tensor or an address taken once is right on any stream after every reserve."""
+    c = U.InferenceController(1, 32, 128, 16, 64, 400, torch.float16, gpu_device, page_order=list(range(25))[::-1])
+    c.prepare_hadamard(5)
+    assert not c.seqs._host_waits
+    if held == "lengths":
+        view = c.seq_lens
+    elif held == "table":
+        view = c.kv_indices_with_last
+    else:
+        assert c.seqs.table_ptr(0) == c.seqs._table_dev.data_ptr()
+        view = c.seqs._table_dev
+    assert c.seqs._host_waits
+    x = torch.randn(8192, 8192, device=gpu_device)
+    torch.cuda.synchronize()
+    for _ in range(5):
+        x = x @ x * 1e-4
+    c.prepare_hadamard(30)                           # behind the products
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):                    # (no event between the streams)
+        got = view.clone()
+        side.synchronize()
+    assert got[:3].tolist() == ([35] if held == "lengths" else [24, 23, 22])
+
+
+def test_a_request_waits_for_no_write(gpu_device):
+    """Prompt and eager steps of a decoder take nothing that would make the host wait."""
+    cfg = DecoderConfig(num_layers=2, hidden=256, num_heads=8, intermediate=512, vocab=64, dense_layers=1)
+    model = LlamaShapedDecoder(cfg, gpu_device)
+    model.init_cache(16, 128, 32)
+    ids = torch.arange(60, device=gpu_device)
+    for _ in range(2):
+        model.clear()
+        model.prefill(ids[:50])
+        for i in range(50, 60):
+            model.decode_step_eager(ids[i:i + 1])
+    assert not model.ctrl.seqs._host_waits
+    assert model.ctrl.seq_lens.tolist() == [60]
