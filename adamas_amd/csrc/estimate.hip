@@ -163,6 +163,17 @@ extern "C" int adamas_write_words(int32_t* dst, const int32_t* words, uint32_t n
   return 0;
 }
 
+extern "C" int adamas_wait_event(void* event) {
+  if (!event) return ADAMAS_E_BADARG;
+  // a capture forbids the capturing thread to wait, for fear of what it has captured; this event is none of that
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  hipError_t err = hipThreadExchangeStreamCaptureMode(&mode);
+  if (err != hipSuccess) return static_cast<int>(err);
+  err = hipEventSynchronize(static_cast<hipEvent_t>(event));
+  const hipError_t back = hipThreadExchangeStreamCaptureMode(&mode);
+  return static_cast<int>(err != hipSuccess ? err : back);
+}
+
 extern "C" int adamas_read_probe(const void* data, size_t bytes, void* sink,
                                  adamas_stream_t stream) {
   if (!data || bytes == 0) return ADAMAS_E_BADARG;

@@ -1,5 +1,7 @@
 """Lengths and page ids reach the device without the host waiting for them, and every reader finds them: on the
 stream that wrote them, on others, in graphs that are replayed."""
+import copy
+
 import pytest
 import torch
 
@@ -172,3 +174,47 @@ def test_a_request_waits_for_no_write(gpu_device):
             model.decode_step_eager(ids[i:i + 1])
     assert not model.ctrl.seqs._host_waits
     assert model.ctrl.seq_lens.tolist() == [60]
+
+
+@pytest.mark.parametrize("default", [True, False])
+def test_a_capture_waits_for_what_is_still_to_be_written(gpu_device, default):
+    """Written on the default stream and captured on another one, without the synchronization that torch.cuda.graph
+    begins with; or all on one other stream, where the host waits for every write.  Replayed on a third stream."""
+    writer = torch.cuda.default_stream() if default else torch.cuda.Stream()
+    other, third = torch.cuda.Stream(), torch.cuda.Stream()
+    x = torch.randn(8192, 8192, device=gpu_device)
+    lens, pages = (torch.zeros(1, dtype=torch.int32, device=gpu_device) for _ in range(2))
+    torch.cuda.synchronize()
+    with torch.cuda.stream(writer):
+        s = _seqs(gpu_device, 1, 64)
+        x = x @ x * 1e-4
+        torch.cuda.synchronize()
+        for _ in range(5):
+            x = x @ x * 1e-4
+        s.reserve([7])                               # behind the products
+        assert s._host_waits != default
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(other if default else writer):
+        graph.capture_begin()
+        s.launch_addresses()                         # as an operator asks for them
+        lens.copy_(s._seq_lens_dev)
+        pages.copy_(s._table_dev[:1])
+        graph.capture_end()
+    assert s._host_waits and s._writer is None
+    for _ in range(2):
+        with torch.cuda.stream(third):
+            graph.replay()
+        third.synchronize()
+        assert lens.tolist() == [7] and pages.tolist() == [63]
+        with torch.cuda.stream(third):
+            lens.zero_()
+            pages.zero_()
+
+
+def test_a_copy_waits_for_its_own_writes(gpu_device):
+    s = _seqs(gpu_device, 1, 64)
+    s.reserve([7])
+    t = copy.deepcopy(s)
+    assert t._host_waits and not s._host_waits
+    t.reserve([1])
+    assert t.seq_lens_dev.tolist() == [8] and s.seq_lens_dev.tolist() == [7]
