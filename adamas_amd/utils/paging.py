@@ -178,13 +178,12 @@ class PagedSequences:
         waits for the copy of one length after every token leaves the GPU idle while the host catches up
         (2000 + 24 tokens through three layers 11.47 -> 10.76 ms)."""
         n = len(values)
-        if (self._host_waits or n > _lib.MAX_WORDS or dst.get_device() != torch.cuda.current_device()
-                or torch.cuda.is_current_stream_capturing()):
+        if not self._host_waits and (_lib.current_stream(dst.get_device()) != 0
+                                     or torch.cuda.is_current_stream_capturing()):
+            self._end_writes_without_waiting()   # (ahead of any write from another stream)
+        if self._host_waits or n > _lib.MAX_WORDS or dst.get_device() != torch.cuda.current_device():
             dst[start:start + n] = torch.tensor(values, dtype=torch.int32)
             return
-        if _lib.current_stream() != 0:
-            self._end_writes_without_waiting()
-            return self._write(dst, start, values)
         _lib.write_words(dst.data_ptr() + 4 * start, values, 0)
         self._note_write()
 

@@ -218,3 +218,21 @@ def test_a_copy_waits_for_its_own_writes(gpu_device):
     assert t._host_waits and not s._host_waits
     t.reserve([1])
     assert t.seq_lens_dev.tolist() == [8] and s.seq_lens_dev.tolist() == [7]
+
+
+@pytest.mark.parametrize("pages", [1, _lib.MAX_WORDS, _lib.MAX_WORDS + 1])
+def test_a_write_from_another_stream_comes_behind_those_before(gpu_device, pages):
+    """Whatever its size, and so by whatever way it goes."""
+    s = _seqs(gpu_device, 1, pages + 8)
+    x = torch.randn(8192, 8192, device=gpu_device)
+    x = x @ x * 1e-4
+    torch.cuda.synchronize()
+    for _ in range(5):
+        x = x @ x * 1e-4
+    s.reserve([7])                                   # behind the products
+    event = s._written
+    with torch.cuda.stream(torch.cuda.Stream()):
+        assert not event.query()
+        s.reserve_pages_ahead(pages)
+        assert event.query() and s._host_waits and s._writer is None
+    assert s.table_dev.tolist() == s.pages[0] + [0] * (s.max_pages - 7 - pages) and s.seq_lens_dev.tolist() == [7]
