@@ -146,6 +146,16 @@ class PagedSequences:
         self._end_writes_without_waiting()
         return self._seq_lens_dev
 
+    @table_dev.setter
+    def table_dev(self, table: torch.Tensor) -> None:
+        self._end_writes_without_waiting()
+        self._table_dev = table
+
+    @seq_lens_dev.setter
+    def seq_lens_dev(self, lengths: torch.Tensor) -> None:
+        self._end_writes_without_waiting()
+        self._seq_lens_dev = lengths
+
     def launch_addresses(self, b: int = 0):
         """(page table of sequence b, indptr, lengths) on the device, for a launch on the current stream now; not to
         be kept."""

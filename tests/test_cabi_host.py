@@ -497,3 +497,14 @@ def test_a_call_that_the_native_host_side_leaves_costs_little():
     for i, call in enumerate(declined):
         assert call() is None
         assert best(call) < 6 * unit, i
+
+
+def test_tables_can_be_assigned():
+    """As the plain attributes that they were: operators and later growth use the tensors given."""
+    c = U.InferenceController(1, 32, 128, 16, 64, 64, torch.float16, "cpu")
+    lengths, table = torch.zeros(1, dtype=torch.int32), torch.zeros(4, dtype=torch.int32)
+    c.seqs.seq_lens_dev, c.seqs.table_dev = lengths, table
+    c.prepare_hadamard(20)
+    assert lengths.tolist() == [20] and table[:2].tolist() == c.seqs.pages[0]
+    assert c.seq_lens is lengths and c.kv_indices_with_last is table
+    assert c.seqs.launch_addresses() == (table.data_ptr(), c.seqs.indptr_dev.data_ptr(), lengths.data_ptr())
