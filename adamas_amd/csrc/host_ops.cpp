@@ -11,7 +11,6 @@
 
 #include <ATen/ATen.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
-#include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/Exceptions.h>
@@ -32,7 +31,7 @@ PyObject* g_all_past = nullptr;           // ALL_PAST_TOKENS
 #define ADAMAS_NAMES(X)                                                                                             \
   X(dtype) X(batch_size) X(num_layers) X(num_heads) X(num_kv_heads) X(head_dim) X(page_size) X(max_seq_len)         \
   X(hadamard_scale) X(kv_flags) X(code_flags) X(pool) X(seqs) X(kv) X(codes) X(_table_dev) X(indptr_dev)             \
-  X(_seq_lens_dev) X(_host_waits) X(_writer) X(lengths) X(max_pages) X(inference_page_budget)                        \
+  X(_seq_lens_dev) X(_host_waits) X(lengths) X(max_pages) X(inference_page_budget)                                   \
   X(topk_dout_buffer) X(topk_dindices_buffer) X(topk_buf) X(_workspace) X(_len_bound) X(_estimate_buf)               \
   X(_estimate_version) X(CODES_CACHED_BYTES)
 #define ADAMAS_DECLARE(n) PyObject* s_##n = nullptr;
@@ -173,16 +172,12 @@ struct Controller {
     return true;
   }
 
-  // The current stream, if it is t's device's and lengths and pages need no wait there: those are read from the
-  // tensors as they are, and PagedSequences.launch_addresses sees to the other streams and graphs.
+  // The current stream, if it is t's device's and lengths and pages need no wait there (PagedSequences.__init__):
+  // PagedSequences.launch_addresses sees to the others.
   bool stream(const at::Tensor& t, adamas_stream_t& s) const {
-    Ref waits, writer;
-    if (!stream_of(t, s) || !waits.read(seqs.p, s__host_waits)) return false;
-    if (waits.p == Py_True) return true;
-    long w;
-    return waits.p == Py_False && writer.read(seqs.p, s__writer) &&
-           (writer.p == Py_None || (as_long(writer.p, w) && w == reinterpret_cast<long>(s))) &&
-           c10::hip::currentStreamCaptureStatusMayInitCtx() == c10::hip::CaptureStatus::None;
+    Ref waits;
+    return stream_of(t, s) && waits.read(seqs.p, s__host_waits) &&
+           (waits.p == Py_True || (waits.p == Py_False && s == nullptr));
   }
 
   bool workspace(Owned& ws, uint32_t budget_now) const {  // the controller's, if it is large enough

@@ -179,8 +179,7 @@ class PagedSequences:
         self._host_waits = True
 
     def _note_use(self) -> None:
-        if torch.cuda.is_current_stream_capturing() or (
-                self._writer is not None and _lib.current_stream(self._table_dev.get_device()) != self._writer):
+        if _lib.current_stream(self._table_dev.get_device()) != 0:   # (no capture is on the default stream)
             self._end_writes_without_waiting()
 
     def _write(self, dst: torch.Tensor, start: int, values: List[int]) -> None:
@@ -188,9 +187,8 @@ class PagedSequences:
         waits for the copy of one length after every token leaves the GPU idle while the host catches up
         (2000 + 24 tokens through three layers 11.47 -> 10.76 ms)."""
         n = len(values)
-        if not self._host_waits and (_lib.current_stream(dst.get_device()) != 0
-                                     or torch.cuda.is_current_stream_capturing()):
-            self._end_writes_without_waiting()   # (ahead of any write from another stream)
+        if not self._host_waits:
+            self._note_use()   # (ahead of any write from another stream)
         if self._host_waits or n > _lib.MAX_WORDS or dst.get_device() != torch.cuda.current_device():
             dst[start:start + n] = torch.tensor(values, dtype=torch.int32)
             return
