@@ -219,11 +219,12 @@ __device__ __forceinline__ void attend_rows(const HeadKV& kv, const float (&qf)[
 // The same for a list of positions in memory, or all positions (kAll): row r < n_sel is position sel[r]
 // (outside [0, seq_len): an unused entry), row n_sel the newest token.  Positions, page ids and rows are three
 // memory round trips that depend on each other, so each is asked for by all rows of a tile before the next; row
-// by row, with branches around unused entries (attend_rows), a tile is three round trips per row.  Row by row / so,
-// us a launch, 32:32 heads: lists of 63 positions 4.5 / 3.8, 127 5.2 / 4.3, 255 6.6 / 6.0, 511 at 32:8 heads 7.6 / 7.2,
-// 999 8.9 / 8.4, 16 sequences of 127 10.5 / 9.2.  Where the rows themselves are the time it is the other way
-// round, more of them in flight make a gather no faster: 4095 positions with 1024 threads 19.1 / 20.1, and all
-// positions with four rows a group: 4000 18.3 / 19.0, 16 sequences of 150 to 250 16.3 / 17.6 (with two rows the same).
+// by row, with branches around unused entries (attend_rows), a tile is three round trips per row.  A tile in which
+// the wave has no used entry (most of a short sequence's list) ends with its positions.  Row by row / so, us a
+// launch, 32:32 heads: lists of 63 positions 4.3 / 3.4, 127 4.8 / 3.9, 255 6.0 / 5.6, 511 at 32:8 heads 6.9 / 6.5, 999
+// 7.8 / 7.4, 16 sequences of 127 8.1 / 7.1, of 999 52.3 / 49.4, 2 of 2047 15.9 / 15.6; 16 lists of 511 at 32:8 heads 28.4 /
+// 24.4, with 40 entries used in 15 of them 18.4 / 16.3 (23.0 with every tile asked for).
+// All positions with four rows a group stay with attend_rows: 4000 18.3 / 19.0, 16 sequences of 150 to 250 16.3 / 17.6.
 template <int kGroups, int kTile, bool kBf16, bool kAll>
 __device__ __forceinline__ void attend_positions(const HeadKV& kv, const float (&qf)[8], uint32_t g,
                                                  uint32_t row_begin, uint32_t row_end, const int32_t* sel,
@@ -250,6 +251,13 @@ __device__ __forceinline__ void attend_positions(const HeadKV& kv, const float (
     for (int i = 0; i < kTile; ++i) {
       valid[i] = base + i * kGroups + g < row_end && pos[i] >= 0 && pos[i] < kv.seq_len;
       slot[i] = static_cast<uint32_t>(min(max(pos[i], 0), kv.seq_len - 1));
+    }
+    if (!kAll) {
+      bool some = false;
+#pragma unroll
+      for (int i = 0; i < kTile; ++i) some = some || valid[i];
+      // (the hint keeps the loads below in line: 127 positions 3.92 us without it, 3.85 with)
+      if (__builtin_expect(__ballot(some) == 0, 0)) continue;
     }
     if (page_shift < 32u) {  // (uniform) pages of a power of two slots
 #pragma unroll

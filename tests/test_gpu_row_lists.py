@@ -78,6 +78,32 @@ def test_lists_of_positions(gpu_device, lens, rows, page, heads, kv_heads, dtype
         assert bool(((got[b].double() - want).abs() <= ulp * want.abs() + 2e-5).all()), b
 
 
+@pytest.mark.parametrize("rows,used,batch,kv_heads", [
+    (63, 5, 3, 32), (127, 1, 4, 8), (128, 33, 4, 32), (511, 40, 8, 32), (512, 0, 20, 8), (999, 65, 3, 32),
+    (999, 130, 20, 8), (2047, 257, 8, 32), (2500, 3, 2, 8),
+])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_lists_mostly_unused(gpu_device, rows, used, batch, kv_heads, dtype):
+    """Whole tiles without an entry, for lists of every kind of workgroup: the first sequence's list is full, the others
+    have `used` entries, in front or (every other sequence) at the end."""
+    lens = [2600] + [max(used, 1) + 2] * (batch - 1)
+    c, q, kv, g = _setup(gpu_device, lens, 16, 32, kv_heads, dtype, 0)
+    sel = torch.full((batch, 32, rows), -1, dtype=torch.int32, device=gpu_device)
+    for b, n in enumerate(lens):
+        kv[b][1][0] = torch.inf      # (what a clamped position reads, attended by nobody)
+        m = rows if b == 0 else used
+        for h in range(32):
+            some = torch.randperm(n - 2, generator=g, device=gpu_device)[:m].int() + 1
+            sel[b, h, (slice(0, m) if b % 2 == 0 else slice(rows - m, rows))] = some
+    _append(c, kv)
+    got = U.decode_sparse_attn(q, c, 0, sel.view(batch * 32, rows))
+    ulp = 2.0 ** (-10 if dtype == torch.float16 else -7)
+    for b in range(batch):
+        want = _want(q[b], *kv[b], sel[b])
+        # one rounding of the result, and fp32 sums of up to 2501 terms of size 1
+        assert bool(((got[b].double() - want).abs() <= ulp * want.abs() + 2e-5).all()), b
+
+
 @pytest.mark.parametrize("lens,page,heads,kv_heads", [
     ([64], 16, 32, 32), ([129], 5, 32, 8), ([1000], 24, 32, 32), ([1409], 16, 24, 8), ([4096], 48, 32, 32),
     ([150, 250, 3], 16, 32, 32), ([600, 1000], 7, 32, 8),
