@@ -224,6 +224,7 @@ __device__ __forceinline__ void attend_rows(const HeadKV& kv, const float (&qf)[
 // launch, 32:32 heads: lists of 63 positions 4.3 / 3.4, 127 4.8 / 3.9, 255 6.0 / 5.6, 511 at 32:8 heads 6.9 / 6.5, 999
 // 7.8 / 7.4, 16 sequences of 127 8.1 / 7.1, of 999 52.3 / 49.4, 2 of 2047 15.9 / 15.6; 16 lists of 511 at 32:8 heads 28.4 /
 // 24.4, with 40 entries used in 15 of them 18.4 / 16.3 (23.0 with every tile asked for).
+// One list of 4095 of 8192 tokens loses (16.6 / 17.3; of 16384 16.8 / 16.2).
 // All positions with four rows a group stay with attend_rows: 4000 18.3 / 19.0, 16 sequences of 150 to 250 16.3 / 17.6.
 template <int kGroups, int kTile, bool kBf16, bool kAll>
 __device__ __forceinline__ void attend_positions(const HeadKV& kv, const float (&qf)[8], uint32_t g,
@@ -295,12 +296,23 @@ struct MergeShared {
   alignas(16) float o[kWavesM][kHeadDim];
 };
 
-// Folds the states of two 16-lane groups of a wave, the groups kDelta / 16 apart, channel by channel: both end up
-// with the result of the lower group.  Lane swaps of the vector unit, no trip through the LDS crossbar: a layer of a step
-// over 4096 tokens, budget 64, 12.35 -> 12.20 us.
-template <int kDelta>
+// Folds the states of two 16-lane groups of a wave, the groups kDelta / 16 apart, channel by channel: the lower group
+// ends up with the result.  Lane swaps of the vector unit are the shorter way (a layer of a step over 4096 tokens,
+// budget 64, 12.35 -> 12.20 us); kCrossbar goes through the LDS crossbar and leaves the vector unit to other waves,
+// which is faster where there are many on a CU (sparse_decode_kernel).
+template <int kDelta, bool kCrossbar = false>
 __device__ __forceinline__ void fold_state(SoftmaxState& st) {
   static_assert(kDelta == 16 || kDelta == 32, "groups of one wave");
+  if (kCrossbar) {
+    const float m_o = __shfl_xor(st.m, kDelta), l_o = __shfl_xor(st.l, kDelta);
+    const float m_n = fmaxf(st.m, m_o);
+    const float a = exp2_raw(st.m - m_n), b = exp2_raw(m_o - m_n);
+    st.l = st.l * a + l_o * b;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) st.o[j] = st.o[j] * a + __shfl_xor(st.o[j], kDelta) * b;
+    st.m = m_n;
+    return;
+  }
   // lo: the lower group's value in both groups, hi: the upper group's
   auto both = [](float x, float& lo, float& hi) __attribute__((always_inline)) {
     const uint32_t u = __float_as_uint(x);
@@ -345,12 +357,12 @@ __device__ __forceinline__ void merge_waves(uint32_t tid, const MergeShared<kGro
 
 // Merges the kGroups group states of a workgroup (kGroups / 4 waves).  After the call the threads
 // tid < 128 hold, for channel tid, the merged maximum M, denominator L and numerator O.
-template <int kGroups>
+template <int kGroups, bool kCrossbar = false>
 __device__ __forceinline__ void merge_groups(SoftmaxState st, uint32_t g, uint32_t c,
                                              uint32_t tid, MergeShared<kGroups>& sh, float& M,
                                              float& L, float& O) {
-  fold_state<16>(st);
-  fold_state<32>(st);  // every lane now holds the state of its wave for channels 8c .. 8c+7
+  fold_state<16, kCrossbar>(st);
+  fold_state<32, kCrossbar>(st);  // the lowest group now holds the state of its wave, lane c channels 8c .. 8c+7
   const uint32_t w = g >> 2;
   if ((g & 3u) == 0) {
     if (c == 0) {

@@ -39,12 +39,13 @@ struct AttnShared {
 
 // group_inv: 2^32 / group of query heads, rounded up (head / group by one multiplication: exact for heads below
 // 2^16), 0 for one query head per key/value head; page_shift: log2 of the page size, 32 where it is none.
-// kAll: all positions of the sequence (no list).
+// kAll: all positions of the sequence (no list).  kCrossbar: how the groups of a wave are folded (fold_state, the rule stands at
+// the launch).
 // Lists with four rows a group in flight would take 78 to 86 registers, and five or six waves a SIMD instead of eight:
 // held to 64, without spills, 16 lists of 511 entries, 32:8 heads, bf16, take 24.4 us instead of 25.4, with 40 entries
 // used in 15 of them 16.3 instead of 18.8; two workgroups of 1024 threads fit a CU (16 lists of 999 49.4, row by row
 // 52.3).
-template <bool kBf16, bool kHnd, int kThreads, int kTileRows, bool kAll>
+template <bool kBf16, bool kHnd, int kThreads, int kTileRows, bool kAll, bool kCrossbar>
 __global__ __launch_bounds__(kThreads, !kAll && kTileRows == 4 ? 8 : 1) void sparse_decode_kernel(
     const __half* __restrict__ q, const __half* __restrict__ kv_data,
     const int32_t* __restrict__ page_indices, const int32_t* __restrict__ page_indptr,
@@ -86,7 +87,7 @@ __global__ __launch_bounds__(kThreads, !kAll && kTileRows == 4 ? 8 : 1) void spa
         [&](uint32_t r) __attribute__((always_inline)) -> int32_t { return static_cast<int32_t>(r); }, st);
 
   float M, L, O;
-  merge_groups<kGroups>(st, g, c, tid, sh.merge, M, L, O);
+  merge_groups<kGroups, kCrossbar>(st, g, c, tid, sh.merge, M, L, O);
   if (n_split == 1) {
     // an empty row list (a sequence without tokens) gives zeros, not 0/0
     if (tid < kHeadDim)
@@ -1193,32 +1194,44 @@ static int sparse_decode_impl(const void* q, const void* kv_data, const int32_t*
   // from kDeferredMergeSplits splits on, the merge is a second short launch
   const uint32_t deferred = n_split >= kDeferredMergeSplits ? 1u : 0u;
   const uint32_t group_inv = gq == 1 ? 0u : static_cast<uint32_t>(((uint64_t{1} << 32) + gq - 1) / gq);
+  // Groups are folded through the LDS crossbar where more than 16 waves come to a CU, and in workgroups of 1024
+  // threads, which are 16; by lane swaps where there are fewer.  Lane swaps / crossbar, us a launch: all positions, 1300
+  // at 32:8 heads 9.6 / 8.0, 2000 10.3 / 9.6, 1000 7.05 / 6.95, 8 of 500 15.8 / 15.2, 64 of 60 13.4 / 12.9, 64 3.49 / 3.62;
+  // lists, 4 of 300 7.6 / 7.1, one of 999 7.37 / 7.28 (with 40 used 6.3 / 6.6), of 511 with 32 used 5.7 / 5.9, of 63 3.42 /
+  // 3.58.  (Decided in the kernel: 1300 8.7, 1000 7.3.)
+  const bool crossbar = static_cast<uint64_t>(n_split) * num_heads * batch * threads > 256u * 1024u;
   uint32_t page_shift = 0;
   while (page_shift < 32u && (uint64_t{1} << page_shift) != page_size) ++page_shift;
-#define ADAMAS_LAUNCH_SPARSE_A(BF, HND, T, TILE, ALL)                                                \
-  hipLaunchKernelGGL((sparse_decode_kernel<BF, HND, T, TILE, ALL>), dim3(n_split, num_heads, batch), \
-                     dim3(T), 0, static_cast<hipStream_t>(stream),                                   \
-                     static_cast<const __half*>(q), static_cast<const __half*>(kv_data),             \
-                     page_indices, page_indptr, seq_lens, sel_idx, sel_stride, n_sel,                \
-                     static_cast<__half*>(out), partial, counters, num_heads, num_kv_heads,          \
+#define ADAMAS_LAUNCH_SPARSE_A(BF, HND, T, TILE, ALL, XBAR)                                                \
+  hipLaunchKernelGGL((sparse_decode_kernel<BF, HND, T, TILE, ALL, XBAR>), dim3(n_split, num_heads, batch), \
+                     dim3(T), 0, static_cast<hipStream_t>(stream),                                         \
+                     static_cast<const __half*>(q), static_cast<const __half*>(kv_data),                   \
+                     page_indices, page_indptr, seq_lens, sel_idx, sel_stride, n_sel,                      \
+                     static_cast<__half*>(out), partial, counters, num_heads, num_kv_heads,                \
                      group_inv, page_size, page_shift, scale_log2, rows_per_split, deferred)
-#define ADAMAS_LAUNCH_SPARSE_T(BF, HND, T, TILE)          \
+#define ADAMAS_LAUNCH_SPARSE_X(BF, HND, T, TILE, XBAR)    \
   if (sel_idx) {                                          \
-    ADAMAS_LAUNCH_SPARSE_A(BF, HND, T, TILE, false);      \
+    ADAMAS_LAUNCH_SPARSE_A(BF, HND, T, TILE, false, XBAR);\
   } else {                                                \
-    ADAMAS_LAUNCH_SPARSE_A(BF, HND, T, TILE, true);       \
+    ADAMAS_LAUNCH_SPARSE_A(BF, HND, T, TILE, true, XBAR); \
   }
-#define ADAMAS_LAUNCH_SPARSE_L(BF, HND)          \
-  if (threads == 256) {                          \
-    ADAMAS_LAUNCH_SPARSE_T(BF, HND, 256, 4);     \
-  } else if (threads == 512 && tile == 4) {      \
-    ADAMAS_LAUNCH_SPARSE_T(BF, HND, 512, 4);     \
-  } else if (threads == 512) {                   \
-    ADAMAS_LAUNCH_SPARSE_T(BF, HND, 512, 2);     \
-  } else if (tile == 2) {                        \
-    ADAMAS_LAUNCH_SPARSE_T(BF, HND, 1024, 2);    \
-  } else {                                       \
-    ADAMAS_LAUNCH_SPARSE_T(BF, HND, 1024, 4);    \
+#define ADAMAS_LAUNCH_SPARSE_T(BF, HND, T, TILE)      \
+  if (crossbar) {                                     \
+    ADAMAS_LAUNCH_SPARSE_X(BF, HND, T, TILE, true);   \
+  } else {                                            \
+    ADAMAS_LAUNCH_SPARSE_X(BF, HND, T, TILE, false);  \
+  }
+#define ADAMAS_LAUNCH_SPARSE_L(BF, HND)               \
+  if (threads == 256) {                               \
+    ADAMAS_LAUNCH_SPARSE_T(BF, HND, 256, 4);          \
+  } else if (threads == 512 && tile == 4) {           \
+    ADAMAS_LAUNCH_SPARSE_T(BF, HND, 512, 4);          \
+  } else if (threads == 512) {                        \
+    ADAMAS_LAUNCH_SPARSE_T(BF, HND, 512, 2);          \
+  } else if (tile == 2) {                             \
+    ADAMAS_LAUNCH_SPARSE_X(BF, HND, 1024, 2, true);   \
+  } else {                                            \
+    ADAMAS_LAUNCH_SPARSE_X(BF, HND, 1024, 4, true);   \
   }
 #define ADAMAS_LAUNCH_SPARSE(BF)        \
   if (flags & ADAMAS_F_HND) {           \
@@ -1234,6 +1247,7 @@ static int sparse_decode_impl(const void* q, const void* kv_data, const int32_t*
 #undef ADAMAS_LAUNCH_SPARSE
 #undef ADAMAS_LAUNCH_SPARSE_L
 #undef ADAMAS_LAUNCH_SPARSE_T
+#undef ADAMAS_LAUNCH_SPARSE_X
 #undef ADAMAS_LAUNCH_SPARSE_A
   ADAMAS_RETURN_IF_LAUNCH_FAILED();
   if (deferred) {
