@@ -222,8 +222,8 @@ __device__ __forceinline__ void attend_rows(const HeadKV& kv, const float (&qf)[
 // by row, with branches around unused entries (attend_rows), a tile is three round trips per row.  A tile in which
 // the wave has no used entry (most of a short sequence's list) ends with its positions.  Row by row / so, us a
 // launch, 32:32 heads: lists of 63 positions 4.3 / 3.4, 127 4.8 / 3.9, 255 6.0 / 5.6, 511 at 32:8 heads 6.9 / 6.5, 999
-// 7.8 / 7.4, 16 sequences of 127 8.1 / 7.1, of 999 52.3 / 49.4, 2 of 2047 15.9 / 15.6; 16 lists of 511 at 32:8 heads 28.4 /
-// 24.4, with 40 entries used in 15 of them 18.4 / 16.3 (23.0 with every tile asked for).
+// 7.8 / 7.4, 16 sequences of 127 8.1 / 7.1, of 999 52.3 / 49.4, 2 of 2047 15.9 / 15.6; 16 lists of 511 at 32:8 heads
+// 28.4 / 24.4, with 40 entries used in 15 of them 18.4 / 16.3 (23.0 with every tile asked for).
 // One list of 4095 of 8192 tokens loses (16.6 / 17.3; of 16384 16.8 / 16.2).
 // All positions with four rows a group stay with attend_rows: 4000 18.3 / 19.0, 16 sequences of 150 to 250 16.3 / 17.6.
 template <int kGroups, int kTile, bool kBf16, bool kAll>

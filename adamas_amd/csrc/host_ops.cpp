@@ -194,6 +194,12 @@ bool is_rows(const at::Tensor& t, at::ScalarType dtype, long n, long heads) {
          t.size(2) == ADAMAS_HEAD_DIM && t.is_contiguous();
 }
 
+// the packed code of a query
+bool is_code(const at::Tensor& t, const Controller& c) {
+  return t.element_size() == 2 && t.dim() == 3 && t.size(0) == c.batch && t.size(1) == c.heads &&
+         t.size(2) == ADAMAS_CODE_WORDS && t.is_contiguous();
+}
+
 PyObject* failed(const char* what, int code) {
   PyErr_Format(PyExc_RuntimeError, "%s failed with error code %d: %s", what, code, adamas_error_string(code));
   return nullptr;
@@ -272,8 +278,7 @@ PyObject* estimate(PyObject* const* a, Py_ssize_t) {  // q_code, controller, lay
   const at::Tensor* q = plain(a[0]);
   Controller c;
   ADAMAS_NEED(q && c.read(a[1]));
-  ADAMAS_NEED(q->element_size() == 2 && q->dim() == 3 && q->size(0) == c.batch && q->size(1) == c.heads &&
-              q->size(2) == ADAMAS_CODE_WORDS && q->is_contiguous() && c.max_len >= 2);
+  ADAMAS_NEED(is_code(*q, c) && c.max_len >= 2);
   Owned codes, table, indptr, lens;
   char* codes_p;
   adamas_stream_t s;
@@ -395,8 +400,7 @@ PyObject* step(PyObject* const* a, Py_ssize_t) {  // q, q_code, controller, laye
   const at::Tensor *q = plain(a[0]), *code = plain(a[1]);
   Controller c;
   ADAMAS_NEED(q && code && c.read(a[2]));
-  ADAMAS_NEED(q->scalar_type() == c.dtype && q->dim() == 3 && q->is_contiguous() && code->dim() == 3 &&
-              code->is_contiguous());
+  ADAMAS_NEED(is_rows(*q, c.dtype, c.batch, c.heads) && is_code(*code, c));
   uint32_t budget, flags, cached, pages;
   Owned kv, codes, table, indptr, lens, ws;
   char *kv_p, *codes_p;

@@ -447,6 +447,9 @@ def decode_step(q: torch.Tensor, q_code: torch.Tensor, iController: InferenceCon
     c = iController
     _check_cuda_contig(q, "q", c.dtype, 3)
     _check_cuda_contig(q_code, "q_code", None, 3)
+    rows = c.batch_size * c.num_heads
+    if q.numel() != rows * c.head_dim or q_code.numel() * q_code.element_size() != rows * 2 * CODE_WORDS:
+        raise RuntimeError("q must be [B, H, D] and q_code the packed query code [B, H, 16] of 16-bit words")
     if c.inference_page_budget is None:
         raise RuntimeError("begin_forward must be called before decode_step")
     budget = c.inference_page_budget

@@ -125,6 +125,11 @@ def test_calls_that_go_the_general_way(gpu_device, monkeypatch):
     for call, what in ((lambda: U.decode_step(q.cpu(), code, c, 0), "must be a CUDA"),
                        (lambda: U.decode_step(q.float(), code, c, 0), "must have dtype"),
                        (lambda: U.decode_step(torch.cat((q, q), 2)[:, :, :128], code, c, 0), "must be contiguous"),
+                       (lambda: U.decode_step(q[:, :8].contiguous(), code, c, 0), r"q must be \[B, H, D\]"),
+                       (lambda: U.decode_step(torch.cat((q, q)), code, c, 0), r"q must be \[B, H, D\]"),
+                       (lambda: U.decode_step(q, code[:, :8].contiguous(), c, 0), "packed query code"),
+                       (lambda: U.decode_step(q, code.long(), c, 0), "packed query code"),
+                       (lambda: U.decode_step(q[:, :8].contiguous(), code, c, 0, return_indices=True), "q must be"),
                        (lambda: U.append_kvh(k, v[:, :8].contiguous(), None, c, 0, q=q), "same shape"),
                        (lambda: U.append_kvh(k, v, None, c, 0, q=q[:, :8].contiguous()), "q must be"),
                        (lambda: U.decode_estimate(code.long(), c, 0), "packed query code"),
@@ -136,6 +141,7 @@ def test_calls_that_go_the_general_way(gpu_device, monkeypatch):
             call()
     with pytest.raises(IndexError):
         U.decode_step(q, code, c, 2)
+    assert torch.equal(general(lambda: U.decode_step(q.view(8, 4, 128), code, c, 1)).view_as(want), want)
     batched = torch.func.vmap(lambda t: t * 1)(q)
     assert torch.equal(U.decode_step(batched, code, c, 1), want)
     with pytest.raises(RuntimeError):
