@@ -157,19 +157,48 @@ def test_results_of_the_library_are_errors_with_its_text(gpu_device):
         U.decode_step(odd, code, c, 0)
 
 
-def test_on_the_current_stream(gpu_device):
+@pytest.mark.parametrize("op", ["hadamard", "hadamard in place", "append", "estimate", "topk", "sparse_attn", "step"])
+def test_on_the_current_stream(gpu_device, monkeypatch, op):
+    """The native function launches behind what its stream holds: on a side stream the input gets its values behind
+    matrix products that outlast the call, and nothing waits in between."""
     c, (q, k, v) = _controller(gpu_device, [700], 64, 32, torch.float16)
     code = U.append_kvh(k, v, None, c, 0, q=q)
-    want = U.decode_step(q, code, c, 0)
+    est = U.decode_estimate(code, c, 0)
+    U.decode_topk(est, c)
+    sel = c.topk_dindices_buffer.clone()
+    U.decode_step(q, code, c, 0)
+    assert c.seq_lens.tolist() == [700]     # (looked at: the lengths are there for every stream)
+
+    def topk(x):
+        U.decode_topk(x, c, True)
+        return c.topk_dindices_buffer.clone()
+
+    value, call = {"hadamard": (q, U.hadamard_transform),
+                   "hadamard in place": (q, lambda x: U.hadamard_transform(x, True)),
+                   "append": (q, lambda x: U.append_kvh(k, v, None, c, 0, q=x)),
+                   "estimate": (code, lambda x: U.decode_estimate(x, c, 0)),
+                   "topk": (est, topk),
+                   "sparse_attn": (q, lambda x: U.decode_sparse_attn(x, c, 0, sel)),
+                   "step": (q, lambda x: U.decode_step(x, code, c, 0))}[op]
+    want = call(value.clone())
+    early = call(torch.zeros_like(value)).clone()
+    assert not torch.equal(early, want)     # what a launch ahead of the values would give
+    want, x = want.clone(), torch.zeros_like(value)
+    a = torch.randn(8192, 8192, device=gpu_device)
+    a @ a
+    host = _Counting(U._load_host())
+    monkeypatch.setattr(U, "_host", host)
     torch.cuda.synchronize()
     side = torch.cuda.Stream()
-    x = torch.randn(4096, 4096, device=gpu_device)
     with torch.cuda.stream(side):
-        q2 = q
-        for _ in range(4):
-            x = x @ x * 1e-3
-        q2 = (q.float() + 0 * x[0, 0].nan_to_num()).half()    # behind the products, on this stream alone
-        got = U.decode_step(q2, code, c, 0)
+        for _ in range(3):
+            a = a @ a * 1e-4
+        busy = torch.cuda.Event()
+        busy.record()
+        x.copy_(value)
+        got = call(x)
+        assert not busy.query()             # (the products are still running: nobody has waited)
         got = got.clone()
     side.synchronize()
+    assert host.served == [True]
     assert torch.equal(got, want)
