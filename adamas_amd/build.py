@@ -86,6 +86,7 @@ def host_command() -> list:
                 sysconfig.get_paths()["include"]]
     return ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
             f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+            f'-DADAMAS_TORCH_VERSION="{torch.__version__}"',
             *[f"-I{d}" for d in includes], str(CSRC_DIR / "host_ops.cpp"), "-o", str(HOST_PATH),
             f"-L{root / 'lib'}", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip",
             f"-L{LIB_DIR}", f"-l:{LIB_PATH.name}", "-Wl,-rpath,$ORIGIN"]

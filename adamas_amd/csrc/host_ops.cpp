@@ -18,6 +18,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 
 #include "../../include/adamas_hip.h"
 
@@ -466,6 +467,18 @@ PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "adamas_host", nullptr, -1, g_met
 }  // namespace
 
 PyMODINIT_FUNC PyInit_adamas_host(void) {
+  // private headers: only the torch that this was built with
+  const Ref torch(PyImport_ImportModule("torch"));
+  if (!torch.p) return nullptr;
+  const Ref version(PyObject_GetAttrString(torch.p, "__version__"));
+  if (!version.p) return nullptr;
+  const Ref text(PyObject_Str(version.p));
+  const char* now = text.p ? PyUnicode_AsUTF8(text.p) : nullptr;
+  if (!now) return nullptr;
+  if (std::strcmp(now, ADAMAS_TORCH_VERSION) != 0) {
+    PyErr_Format(PyExc_ImportError, "it was built for torch %s, this is %s", ADAMAS_TORCH_VERSION, now);
+    return nullptr;
+  }
 #define ADAMAS_INTERN(n) \
   if (!(s_##n = PyUnicode_InternFromString(#n))) return nullptr;
   ADAMAS_NAMES(ADAMAS_INTERN)

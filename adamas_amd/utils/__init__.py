@@ -68,10 +68,21 @@ _FLOAT_DTYPES = (torch.float16, torch.bfloat16)
 _host = None
 
 
+class _GeneralWay:
+    """Stands for the native functions where there are none: serves no call."""
+
+    def _none(self, *args):
+        return None
+
+    hadamard = append_decode = estimate = topk = sparse_attn = step = _none
+
+
 def _load_host():
     global _host
-    _host = _lib.load_host()
-    _host.setup(InferenceController, _controller_module, ALL_PAST_TOKENS)
+    host = _lib.load_host()
+    if host is not None:
+        host.setup(InferenceController, _controller_module, ALL_PAST_TOKENS)
+    _host = host or _GeneralWay()
     return _host
 
 

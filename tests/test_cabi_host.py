@@ -508,3 +508,34 @@ def test_tables_can_be_assigned():
     assert lengths.tolist() == [20] and table[:2].tolist() == c.seqs.pages[0]
     assert c.seq_lens is lengths and c.kv_indices_with_last is table
     assert c.seqs.launch_addresses() == (table.data_ptr(), c.seqs.indptr_dev.data_ptr(), lengths.data_ptr())
+
+
+@pytest.mark.parametrize("missing", [True, False])
+def test_operators_work_without_their_native_host_side(missing):
+    """Without adamas_host.so, or with another torch than it was built for, a warning and the general way."""
+    import subprocess
+    import sys
+    program = f"""
+import warnings, torch
+if {missing}:
+    from adamas_amd import _lib
+    _lib.HOST_PATH = _lib.HOST_PATH.with_name("absent.so")
+else:
+    torch.__version__ = "0.1"
+import adamas_amd.utils as U
+x = torch.zeros(1, 8, 128).half()
+c = U.InferenceController(1, 8, 128, 16, 64, 64, torch.float16, "cpu")
+calls = [lambda: U.hadamard_transform(x), lambda: U.append_kvh(x, x, None, c, 0, q=x),
+         lambda: U.decode_estimate(x, c, 0), lambda: U.decode_topk(x, c), lambda: U.decode_sparse_attn(x, c, 0, None),
+         lambda: U.decode_step(x, x, c, 0)]
+with warnings.catch_warnings(record=True) as seen:
+    warnings.simplefilter("always")
+    for call in calls:
+        try:
+            call()
+        except RuntimeError as e:
+            print("CUDA" in str(e))
+print(len(seen), {"'it is not built'" if missing else "'built for torch'"} in str(seen[0].message))
+"""
+    run = subprocess.run([sys.executable, "-c", program], cwd=ROOT, capture_output=True, text=True, timeout=300)
+    assert run.stdout.split() == ["True"] * 6 + ["1", "True"], run.stdout + run.stderr
