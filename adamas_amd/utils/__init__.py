@@ -3,9 +3,10 @@
 Same function names, argument order and return values as adamas/utils/__init__.py of the reference
 (append_kvh :94-157, decode_estimate :203-237, decode_topk :239-269, decode_sparse_attn :271-308,
 pack_2bit :55-76), apply_rope_in_place :26-53, prefill_forward :159-201, rms_norm_forward :79-92), so the reference's
-attention module (adamas/models/Adamas.py:68-225) can drive it unchanged.  Every function allocates its output with torch, checks shapes and dtypes
-(RuntimeError on violation, like TORCH_CHECK in the reference bindings) and calls one entry point of
-libadamas_hip.so on the current stream.  There is no fallback path: without the library the calls raise.
+attention module (adamas/models/Adamas.py:68-225) can drive it unchanged.  Every function allocates its output
+with torch, checks shapes and dtypes (RuntimeError on violation, like TORCH_CHECK in the reference bindings) and
+calls one entry point of libadamas_hip.so on the current stream.  There is no fallback path: without the library
+the calls raise.
 
 Additions that have no counterpart in the reference:
   hadamard_transform   the transform itself (the reference imports a third-party CUDA module);
@@ -185,7 +186,7 @@ def append_kvh(k: torch.Tensor, v: torch.Tensor, h: Optional[torch.Tensor],
         if n > total:
             raise RuntimeError("prepare_hadamard must reserve the tokens before append_kvh")
         rc = lib.adamas_append_prefill(k.data_ptr(), v.data_ptr(), _lib.ptr(h), n, total - n,
-                                       kv, codes, c.seqs.launch_addresses(seq_idx)[0],
+                                       kv, codes, c.seqs.launch_table_address(stream, seq_idx),
                                        c.seqs.max_pages, nh, d, c.page_size, c.hadamard_scale,
                                        c.code_flags, stream)
         _lib.check(rc, "adamas_append_prefill")
@@ -205,7 +206,7 @@ def append_kvh(k: torch.Tensor, v: torch.Tensor, h: Optional[torch.Tensor],
         raise RuntimeError("prepare_hadamard must reserve the token before append_kvh")
     o = torch.empty((n, nq, d // 8), dtype=torch.int16, device=k.device)
     rc = lib.adamas_append_decode(_lib.ptr(q), k.data_ptr(), v.data_ptr(), _lib.ptr(h), o.data_ptr(),
-                                  kv, codes, *c.seqs.launch_addresses(), n, nq, nh, d, c.page_size,
+                                  kv, codes, *c.seqs.launch_addresses(stream), n, nq, nh, d, c.page_size,
                                   c.hadamard_scale, c.code_flags, stream)
     _lib.check(rc, "adamas_append_decode")
     return o
@@ -231,11 +232,11 @@ def decode_estimate(q: torch.Tensor, iController: InferenceController, layer_idx
         raise RuntimeError("decode_estimate needs at least one past token")
     stride = (lmax - 1 + 7) // 8 * 8
     buf = torch.empty((c.batch_size, c.num_heads, stride), dtype=torch.float16, device=q.device)
+    stream = _lib.current_stream()
     rc = _lib.load().adamas_estimate(q.data_ptr(), c.pool.codes_address(layer_idx),
-                                     *c.seqs.launch_addresses(), buf.data_ptr(),
+                                     *c.seqs.launch_addresses(stream), buf.data_ptr(),
                                      c.num_heads * stride, stride, _lib.DIST_FP16, c.batch_size,
-                                     c.num_heads, c.num_kv_heads, c.page_size, lmax,
-                                     _lib.current_stream())
+                                     c.num_heads, c.num_kv_heads, c.page_size, lmax, stream)
     _lib.check(rc, "adamas_estimate")
     out = buf[:, :, :lmax - 1]
     if c.batch_size == 1:
@@ -293,11 +294,12 @@ def decode_topk(estimated_attn_score: torch.Tensor, iController: InferenceContro
     mode = _lib.KEY_FP16_INT if integer_keys else _lib.KEY_FP16_GENERIC
     ragged = c.batch_size > 1
     buf = c.topk_workspace(n, k)
+    stream = _lib.current_stream()
     rc = _lib.load().adamas_topk(est2.data_ptr(), est2.stride(0), n,
-                                 c.seqs.launch_addresses()[2] if ragged else None,
+                                 c.seqs.launch_addresses(stream)[2] if ragged else None,
                                  c.num_heads, -1, None, 0, rows, k,
                                  c.topk_dindices_buffer.data_ptr(), c.topk_dout_buffer.data_ptr(), k,
-                                 mode, buf.data_ptr(), buf.numel(), _lib.current_stream())
+                                 mode, buf.data_ptr(), buf.numel(), stream)
     _lib.check(rc, "adamas_topk")
 
 
@@ -321,18 +323,18 @@ def decode_sparse_attn(q: torch.Tensor, iController: InferenceController, layer_
         raise RuntimeError("q must be [B, H, D]")
     o = torch.empty_like(q)
     if topk_indices is ALL_PAST_TOKENS or topk_indices is None:
-        sel_ptr, stride, n_sel = None, 0, 0
+        sel_ptr, stride_sel, n_sel = None, 0, 0
     else:
         _check_cuda_contig(topk_indices, "topk_indices", torch.int32, 2)
         if topk_indices.shape[0] != c.batch_size * c.num_heads:
             raise RuntimeError("topk_indices must have one row per (sequence, head)")
-        sel_ptr, stride, n_sel = topk_indices.data_ptr(), topk_indices.stride(0), topk_indices.shape[1]
+        sel_ptr, stride_sel, n_sel = topk_indices.data_ptr(), topk_indices.stride(0), topk_indices.shape[1]
     ws = c.workspace(c.inference_page_budget or 1)
+    stream = _lib.current_stream()
     rc = _lib.load().adamas_sparse_decode_f(
-        q.data_ptr(), c.pool.kv_address(layer_idx), *c.seqs.launch_addresses(), sel_ptr, stride, n_sel,
+        q.data_ptr(), c.pool.kv_address(layer_idx), *c.seqs.launch_addresses(stream), sel_ptr, stride_sel, n_sel,
         o.data_ptr(), ws.data_ptr(), ws.numel(), c.batch_size, c.num_heads, c.num_kv_heads,
-        c.head_dim, c.page_size, 1.0 / math.sqrt(c.head_dim), c.max_len_now, c.kv_flags,
-        _lib.current_stream())
+        c.head_dim, c.page_size, 1.0 / math.sqrt(c.head_dim), c.max_len_now, c.kv_flags, stream)
     _lib.check(rc, "adamas_sparse_decode")
     return o
 
@@ -467,12 +469,13 @@ def decode_step(q: torch.Tensor, q_code: torch.Tensor, iController: InferenceCon
     o = torch.empty_like(q)
     ws = c.workspace(budget)
     sel = c.topk_dindices_buffer if return_indices else None
+    stream = _lib.current_stream()
     rc = _lib.load().adamas_decode_step_f(
         q.data_ptr(), q_code.data_ptr(), c.pool.kv_address(layer_idx),
-        c.pool.codes_address(layer_idx), *c.seqs.launch_addresses(), budget, o.data_ptr(),
+        c.pool.codes_address(layer_idx), *c.seqs.launch_addresses(stream), budget, o.data_ptr(),
         _lib.ptr(sel), ws.data_ptr(), ws.numel(), c.batch_size, c.num_heads, c.num_kv_heads,
         c.head_dim, c.page_size, 1.0 / math.sqrt(c.head_dim), c.max_len_now, c.seqs.max_pages,
-        c.kv_flags | c.codes_flags, _lib.current_stream())
+        c.kv_flags | c.codes_flags, stream)
     _lib.check(rc, "adamas_decode_step")
     return (o, sel) if return_indices else o
 
@@ -569,11 +572,11 @@ def _prefill(q: torch.Tensor, c: InferenceController, layer_idx: int, length: in
     o = torch.empty_like(q)
     need = lib.adamas_prefill_workspace_bytes(n, length - n, c.num_heads, c.num_kv_heads)
     ws = torch.empty(need, dtype=torch.uint8, device=q.device) if need else None
+    stream = torch._C._cuda_getCurrentRawStream(device)
     rc = lib.adamas_prefill_attention(q.data_ptr(), c.kv_cache.buf_layer(layer_idx).data_ptr(),
-                                      c.seqs.launch_addresses()[0], o.data_ptr(), _lib.ptr(ws), need, n,
+                                      c.seqs.launch_table_address(stream), o.data_ptr(), _lib.ptr(ws), need, n,
                                       length - n, c.num_heads, c.num_kv_heads, c.head_dim, c.page_size,
-                                      1.0 / math.sqrt(c.head_dim), c.kv_flags,
-                                      torch._C._cuda_getCurrentRawStream(device))
+                                      1.0 / math.sqrt(c.head_dim), c.kv_flags, stream)
     _lib.check(rc, "adamas_prefill_attention")
     return o
 
@@ -707,9 +710,11 @@ def rope_append_decode(qkv: torch.Tensor, cos_table: torch.Tensor, sin_table: to
         raise RuntimeError("prepare_hadamard must reserve the token before the append")
     q = torch.empty((n, nq, 128), dtype=c.dtype, device=qkv.device)
     q_code = torch.empty((n, nq, 16), dtype=torch.int16, device=qkv.device)
+    stream = _lib.current_stream()
     rc = _lib.load().adamas_rope_append_decode(
         qkv.data_ptr(), cos_table.data_ptr(), sin_table.data_ptr(), q.data_ptr(), q_code.data_ptr(),
-        c.pool.kv_address(layer_idx), c.pool.codes_address(layer_idx), *c.seqs.launch_addresses(), n, nq, nkv, 128, c.page_size, c.hadamard_scale, c.code_flags, _lib.current_stream())
+        c.pool.kv_address(layer_idx), c.pool.codes_address(layer_idx), *c.seqs.launch_addresses(stream), n,
+        nq, nkv, 128, c.page_size, c.hadamard_scale, c.code_flags, stream)
     _lib.check(rc, "adamas_rope_append_decode")
     return q, q_code
 
@@ -802,12 +807,13 @@ def decode_layer_step(qkv: torch.Tensor, cos_table: torch.Tensor, sin_table: tor
     o = torch.empty((n, nq, 128), dtype=c.dtype, device=qkv.device)
     ws = c.workspace(budget)
     sel = c.topk_dindices_buffer if return_indices else None
+    stream = _lib.current_stream()
     rc = _lib.load().adamas_decode_layer_step(
         qkv.data_ptr(), cos_table.data_ptr(), sin_table.data_ptr(), c.pool.kv_address(layer_idx),
-        c.pool.codes_address(layer_idx), *c.seqs.launch_addresses(), budget, o.data_ptr(), _lib.ptr(sel),
+        c.pool.codes_address(layer_idx), *c.seqs.launch_addresses(stream), budget, o.data_ptr(), _lib.ptr(sel),
         ws.data_ptr(), ws.numel(),
         n, nq, nkv, 128, c.page_size, 1.0 / math.sqrt(c.head_dim), c.max_len_now, c.seqs.max_pages,
-        c.hadamard_scale, c.code_flags | c.codes_flags, _lib.current_stream())
+        c.hadamard_scale, c.code_flags | c.codes_flags, stream)
     _lib.check(rc, "adamas_decode_layer_step")
     return (o, sel) if return_indices else o
 

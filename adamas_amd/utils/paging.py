@@ -156,13 +156,17 @@ class PagedSequences:
         self._end_writes_without_waiting()
         self._seq_lens_dev = lengths
 
-    def launch_addresses(self, b: int = 0):
-        """(page table of sequence b, indptr, lengths) on the device, for a launch on the current stream now; not to
-        be kept."""
-        if not self._host_waits:
-            self._note_use()
-        return (self._table_dev.data_ptr() + 4 * b * self.max_pages, self.indptr_dev.data_ptr(),
-                self._seq_lens_dev.data_ptr())
+    def launch_addresses(self, stream: int):
+        """(page table, indptr, lengths) on the device, for a launch on `stream` now; not to be kept."""
+        if stream and not self._host_waits:   # (no capture is on the default stream)
+            self._end_writes_without_waiting()
+        return self._table_dev.data_ptr(), self.indptr_dev.data_ptr(), self._seq_lens_dev.data_ptr()
+
+    def launch_table_address(self, stream: int, b: int = 0) -> int:
+        """The page table of sequence b alone."""
+        if stream and not self._host_waits:
+            self._end_writes_without_waiting()
+        return self._table_dev.data_ptr() + 4 * b * self.max_pages
 
     def launch_table(self) -> torch.Tensor:
         """table_dev for operators launched on the current stream now; not to be kept."""
@@ -179,7 +183,7 @@ class PagedSequences:
         self._host_waits = True
 
     def _note_use(self) -> None:
-        if _lib.current_stream(self._table_dev.get_device()) != 0:   # (no capture is on the default stream)
+        if _lib.current_stream(self._table_dev.get_device()) != 0:
             self._end_writes_without_waiting()
 
     def _write(self, dst: torch.Tensor, start: int, values: List[int]) -> None:

@@ -507,7 +507,8 @@ def test_tables_can_be_assigned():
     c.prepare_hadamard(20)
     assert lengths.tolist() == [20] and table[:2].tolist() == c.seqs.pages[0]
     assert c.seq_lens is lengths and c.kv_indices_with_last is table
-    assert c.seqs.launch_addresses() == (table.data_ptr(), c.seqs.indptr_dev.data_ptr(), lengths.data_ptr())
+    assert c.seqs.launch_table_address(0) == table.data_ptr()
+    assert c.seqs.launch_addresses(0) == (table.data_ptr(), c.seqs.indptr_dev.data_ptr(), lengths.data_ptr())
 
 
 @pytest.mark.parametrize("missing", [True, False])

@@ -196,7 +196,7 @@ def test_a_capture_waits_for_what_is_still_to_be_written(gpu_device, default):
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.stream(other if default else writer):
         graph.capture_begin()
-        s.launch_addresses()                         # as an operator asks for them
+        s.launch_addresses(_lib.current_stream())    # as an operator asks for them
         lens.copy_(s._seq_lens_dev)
         pages.copy_(s._table_dev[:1])
         graph.capture_end()
