@@ -35,7 +35,7 @@ _SIGNATURES = {
                              c_int64, c_uint32, c_uint32, c_void_p, c_void_p, c_int64, c_uint32,
                              c_void_p, c_size_t, c_void_p]),
     "adamas_write_words": (c_int, [c_void_p, c_void_p, c_uint32, c_void_p]),
-    "adamas_wait_event": (c_int, [c_void_p]),
+    "adamas_wait_default_stream": (c_int, [c_int32]),
     "adamas_read_probe": (c_int, [c_void_p, c_size_t, c_void_p, c_void_p]),
     "adamas_topk_workspace_bytes": (c_size_t, [c_uint32, c_uint32, c_uint32]),
     "adamas_workspace_bytes": (c_size_t, [c_uint32, c_uint32, c_uint32, c_uint32]),
@@ -177,10 +177,9 @@ def write_words(address: int, values, stream: int) -> None:
     check(load().adamas_write_words(address, (c_int32 * n)(*values), n, stream), "adamas_write_words")
 
 
-def wait_event(event: int) -> None:
-    """The host waits for an event, also while this thread captures a stream into a graph (the event must have been
-    recorded outside of the capture)."""
-    check(load().adamas_wait_event(event), "adamas_wait_event")
+def wait_default_stream(device: int) -> None:
+    """The host waits for the default stream of a device, also while this thread captures another one into a graph."""
+    check(load().adamas_wait_default_stream(device), "adamas_wait_default_stream")
 
 
 def dtype_flags(dtype) -> int:

@@ -23,8 +23,8 @@ constexpr int kTile = 8;             // rows per group per tile, at most
 // 16 groups of 4, up to 128 rows 32 groups of 4 (one split, no merge, no workspace); up to 512 rows
 // splits of 64 rows (32 groups of 2, at most 8 splits); up to 2048 rows splits of 128 (64 groups of
 // 2, at most 16); beyond that, and where more workgroups than run at once would come of it, four rows in flight
-// (row_launch).  Lists at 32 heads, rows = 128 / 256 / 1000 / 2048 / 4096, in us: 4.2 / 5.9 / 8.4 / 12.1 / 19.2,
-// 512 at 32:8 heads 7.2.  The lines were drawn with rows fetched one by one, rows = 128 / 256 / 512 / 1024 / 2048 /
+// (row_launch).  Lists at 32 heads, rows = 128 / 256 / 512 / 1024 / 2048 / 4096, in us: 4.1 / 5.8 / 6.8 / 8.4 / 12.6 /
+// 18.3.  The lines were drawn with rows fetched one by one, rows = 128 / 256 / 512 / 1024 / 2048 /
 // 4096: 5.8 / 6.5 / 7.4 / 9.3 / 13.5 / 18.8 (with 16 groups of 8 rows and splits of 128 rows up to 1024 rows, 32
 // groups of 8 beyond: 7.5 / 9.5 / 10.1 / 12.4 / 15.8 / 20.6).
 constexpr uint32_t kDeferredMergeSplits = 24;  // splits from which the partials get a merge launch
@@ -39,8 +39,8 @@ struct AttnShared {
 
 // group_inv: 2^32 / group of query heads, rounded up (head / group by one multiplication: exact for heads below
 // 2^16), 0 for one query head per key/value head; page_shift: log2 of the page size, 32 where it is none.
-// kAll: all positions of the sequence (no list).  kCrossbar: how the groups of a wave are folded (fold_state, the rule stands at
-// the launch).
+// kAll: all positions of the sequence (no list).  kCrossbar: how the groups of a wave are folded (fold_state; the rule
+// stands at the launch).
 // Lists with four rows a group in flight would take 78 to 86 registers, and five or six waves a SIMD instead of eight:
 // held to 64, without spills, 16 lists of 511 entries, 32:8 heads, bf16, take 24.4 us instead of 25.4, with 40 entries
 // used in 15 of them 16.3 instead of 18.8; two workgroups of 1024 threads fit a CU (16 lists of 999 49.4, row by row
@@ -1195,10 +1195,10 @@ static int sparse_decode_impl(const void* q, const void* kv_data, const int32_t*
   const uint32_t deferred = n_split >= kDeferredMergeSplits ? 1u : 0u;
   const uint32_t group_inv = gq == 1 ? 0u : static_cast<uint32_t>(((uint64_t{1} << 32) + gq - 1) / gq);
   // Groups are folded through the LDS crossbar where more than 16 waves come to a CU, and in workgroups of 1024
-  // threads, which are 16; by lane swaps where there are fewer.  Lane swaps / crossbar, us a launch: all positions, 1300
-  // at 32:8 heads 9.6 / 8.0, 2000 10.3 / 9.6, 1000 7.05 / 6.95, 8 of 500 15.8 / 15.2, 64 of 60 13.4 / 12.9, 64 3.49 / 3.62;
-  // lists, 4 of 300 7.6 / 7.1, one of 999 7.37 / 7.28 (with 40 used 6.3 / 6.6), of 511 with 32 used 5.7 / 5.9, of 63 3.42 /
-  // 3.58.  (Decided in the kernel: 1300 8.7, 1000 7.3.)
+  // threads, which are 16; by lane swaps where there are fewer.  Lane swaps / crossbar, us a launch: all positions,
+  // 1300 at 32:8 heads 9.6 / 8.0, 2000 10.3 / 9.6, 1000 7.05 / 6.95, 8 of 500 15.8 / 15.2, 64 of 60 13.4 / 12.9, 64
+  // 3.49 / 3.62; lists, 4 of 300 7.6 / 7.1, one of 999 7.37 / 7.28 (with 40 used 6.3 / 6.6), of 511 with 32 used 5.7 /
+  // 5.9, of 63 3.42 / 3.58.  (Decided in the kernel: 1300 8.7, 1000 7.3.)
   const bool crossbar = static_cast<uint64_t>(n_split) * num_heads * batch * threads > 256u * 1024u;
   uint32_t page_shift = 0;
   while (page_shift < 32u && (uint64_t{1} << page_shift) != page_size) ++page_shift;

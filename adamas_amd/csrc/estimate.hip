@@ -163,15 +163,24 @@ extern "C" int adamas_write_words(int32_t* dst, const int32_t* words, uint32_t n
   return 0;
 }
 
-extern "C" int adamas_wait_event(void* event) {
-  if (!event) return ADAMAS_E_BADARG;
-  // a capture forbids the capturing thread to wait, for fear of what it has captured; this event is none of that
-  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-  hipError_t err = hipThreadExchangeStreamCaptureMode(&mode);
+extern "C" int adamas_wait_default_stream(int32_t device) {
+  int before = 0;
+  hipError_t err = hipGetDevice(&before);
   if (err != hipSuccess) return static_cast<int>(err);
-  err = hipEventSynchronize(static_cast<hipEvent_t>(event));
-  const hipError_t back = hipThreadExchangeStreamCaptureMode(&mode);
-  return static_cast<int>(err != hipSuccess ? err : back);
+  if (device != before && (err = hipSetDevice(device)) != hipSuccess) return static_cast<int>(err);
+  // a capture forbids the capturing thread to wait, for fear of what it has captured; the default stream has none of it
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  err = hipThreadExchangeStreamCaptureMode(&mode);
+  if (err == hipSuccess) {
+    err = hipStreamSynchronize(nullptr);
+    const hipError_t back = hipThreadExchangeStreamCaptureMode(&mode);
+    if (err == hipSuccess) err = back;
+  }
+  if (device != before) {
+    const hipError_t back = hipSetDevice(before);
+    if (err == hipSuccess) err = back;
+  }
+  return static_cast<int>(err);
 }
 
 extern "C" int adamas_read_probe(const void* data, size_t bytes, void* sink,

@@ -164,11 +164,11 @@ __global__ __launch_bounds__(kHeads * kWave) void estimate_select_kernel(
   static_assert(!kHist || !kPartial, "the histogram mode works on chunks of 512, 1024 or 2048 tokens");
   constexpr int kItems = 8 * kPasses;                 // tokens per lane in the selection phase
   // With several passes the narrow and the shared instances count the distances as they come, under the loads of the
-  // next pass, instead of 16 or 32 to a lane when all loads have ended (us a layer of a step, at the end / as they come,
-  // 100000 tokens, 32:8 heads, budget 200, 20.4 / 19.8; 50000, 128, 16.3 / 15.7; 3 sequences of 40000 to 50000, 32:32,
-  // 41.4 / 39.8).  The wide one, eight heads apart in a wave and a full chip of it waiting for memory, gains nothing
-  // (131072 tokens 38.3 / 38.5), nor does a single pass, whose last loads' counts are waited for either way (32768
-  // tokens, this launch 10.3 / 10.7).
+  // next pass, instead of 16 or 32 to a lane when all loads have ended (us a layer of a step, at the end / as they
+  // come, 100000 tokens, 32:8 heads, budget 200, 20.4 / 19.8; 50000, 128, 16.3 / 15.7; 3 sequences of 40000 to 50000,
+  // 32:32, 41.4 / 39.8).  The wide one, eight heads apart in a wave and a full chip of it waiting for memory, gains
+  // nothing (131072 tokens 38.3 / 38.5), nor does a single pass, whose last loads' counts are waited for either way
+  // (32768 tokens, this launch 10.3 / 10.7).
   constexpr bool kCountEarly = !kHist && kPasses >= 2 && (kShare == 4 || kHeads == 4);
   static_assert(kHeads == 8 || kHeads == 4, "a token's codes are read by 2 * kHeads lanes");
   static_assert(kShare == 1 || kShare == 4, "a lane serves one head, or four that share a key/value head");
@@ -984,16 +984,19 @@ struct HistSelectAttendShared {
 // the sum while the others leave it the issue slots; only the one bin that decides the ties is counted before the slab
 // (the bins below it too where the caller wants positions); nothing waits for the current token's page; and all waves
 // of the last workgroup of a head read its partials.  In batches the workgroups of the heads that share a key/value
-// head lie on one die (head_of_block; 1.3 %, one sequence loses 0.6 %: it is not bound by its bytes).  us a layer of
-// a step before / now: 23989 tokens, 32:8 heads, bf16, budget 1024 20.9 / 20.2; 8 sequences of 1500 to 7000, 32:8
-// heads, 512, 31.5 / 30.2; 8 of 4000 to 15000, 3000, 112.5 / 113.2 and, 32:8 heads, 88.5 / 77.7.  Where the time
-// goes in the first of these, 9.5 us from the first workgroup's start to the last one's end: loads 1.3, sum and threshold 0.7, selection 0.7, rows and softmax 2.0 to 2.7, merge of the waves
-// 1.0, partial out and counter 1.2, merge of the slabs 1.2, the rest is workgroups that share a CU.
+// head lie on one die (head_of_block; one sequence loses 0.6 %: it is not bound by its bytes).  That gives most where
+// the heads' rows overlap: heads as they come / so, us a layer, 32:8 heads, 8 sequences of 1500 to 7000, budget 512,
+// 29.7 / 27.9, 12 of 2000 to 8000, bf16, 300, 33.4 / 32.8, 8 of 4000 to 15000, 3000, 89.1 / 71.1.  us a layer of a step
+// without all of this / with it: 23989 tokens, 32:8 heads, bf16, budget 1024 20.0 / 19.5; the three batches above 30.4
+// / 27.9, 34.0 / 32.8 and 90.4 / 71.1, the last at 32:32 heads 113.7 / 114.4.  Where the time goes in the first of
+// these, 9.5 us from the first workgroup's start to the last one's end: loads 1.3, sum and threshold 0.7, selection
+// 0.7, rows and softmax 2.0 to 2.7, merge of the waves 1.0, partial out and counter 1.2, merge of the slabs 1.2, the
+// rest is workgroups that share a CU.
 template <bool kBf16, bool kHnd, int kThreads, int kItems>
 __global__ __launch_bounds__(kThreads) void hist_select_attend_kernel(
     const unsigned char* hist, const uint16_t* dist, const uint32_t* rowmap,
-    const int32_t* __restrict__ seq_lens, uint32_t dist_stride, uint32_t n_chunks, uint32_t num_heads, uint32_t chunk_log2, uint32_t k,
-    uint32_t batch, const __half* __restrict__ q, const __half* __restrict__ kv_data,
+    const int32_t* __restrict__ seq_lens, uint32_t dist_stride, uint32_t n_chunks, uint32_t num_heads,
+    uint32_t chunk_log2, uint32_t k, uint32_t batch, const __half* __restrict__ q, const __half* __restrict__ kv_data,
     const int32_t* __restrict__ page_indices, const int32_t* __restrict__ page_indptr, __half* __restrict__ out,
     int32_t* __restrict__ sel_out, float* partial, uint32_t* __restrict__ counters, uint32_t num_kv_heads,
     uint32_t kv_inv16, uint32_t order16, uint32_t page_size, uint32_t table_stride, float scale_log2) {

@@ -120,17 +120,16 @@ class PagedSequences:
         self._table_dev = torch.zeros(batch * self.max_pages, dtype=torch.int32, device=device)
         self.indptr_dev = (torch.arange(batch + 1, dtype=torch.int32) * self.max_pages).to(device)
         self._seq_lens_dev = torch.zeros(batch, dtype=torch.int32, device=device)
-        # Lengths and page ids are written by a launch that the host does not wait for, while everything that
-        # reads them is launched by this package's operators on the stream of that launch.  That is the default
-        # stream, and the tables must have been allocated there: it cannot be captured, so the host can wait for what
-        # was written there at any time (HIP refuses to wait for an event of a stream that is being captured), and
-        # the tables' memory is not handed to another before a write to it is done.  The first operator on another
-        # stream or in a graph (which is replayed on whatever stream), and the first look from outside (a tensor or an
-        # address once handed out is used at any time on any stream), wait for what is written and end that for good:
-        # from then on the host waits for every write, and no stream can be too early.
+        # Lengths and page ids are written by a launch that the host does not wait for, while everything that reads them
+        # is launched by this package's operators on the stream of that launch.  That is the default stream, and the
+        # tables must have been allocated there: it cannot be captured, so the host can wait for what was written there
+        # at any time (HIP refuses to wait for a stream that is being captured), and the tables' memory is not handed to
+        # another before a write to it is done.  The first operator on another stream or in a graph (which is replayed
+        # on whatever stream), and the first look from outside (a tensor or an address once handed out is used at any
+        # time on any stream), wait for what is written and end that for good: from then on the host waits for every
+        # write, and no stream can be too early.
         self._host_waits = not (self._table_dev.is_cuda and _lib.current_stream(self._table_dev.get_device()) == 0)
         self._writer: Optional[int] = None    # the default stream once it has a write that the host did not wait for
-        self._written: Optional[torch.cuda.Event] = None    # recorded behind that write
 
     @property
     def table_dev(self) -> torch.Tensor:
@@ -178,7 +177,7 @@ class PagedSequences:
         if self._host_waits:
             return
         if self._writer is not None:
-            _lib.wait_event(self._written.cuda_event)   # (also while a stream is captured)
+            _lib.wait_default_stream(self._table_dev.get_device())   # (also while another stream is captured)
             self._writer = None
         self._host_waits = True
 
@@ -197,20 +196,12 @@ class PagedSequences:
             dst[start:start + n] = torch.tensor(values, dtype=torch.int32)
             return
         _lib.write_words(dst.data_ptr() + 4 * start, values, 0)
-        self._note_write()
-
-    def _note_write(self) -> None:
-        """Behind a write on the default stream."""
-        if self._written is None:
-            self._written = torch.cuda.Event()
-        self._written.record()
         self._writer = 0
 
-    def __getstate__(self):   # (for a copy or another process, without the event)
-        state = dict(self.__dict__, _written=None, _writer=None, _host_waits=True)
+    def __getstate__(self):   # (for a copy or another process)
         if self._writer is not None:
-            _lib.wait_event(self._written.cuda_event)
-        return state
+            _lib.wait_default_stream(self._table_dev.get_device())
+        return dict(self.__dict__, _writer=None, _host_waits=True)
 
     def reserve(self, new_tokens: Sequence[int]) -> List[int]:
         """Grow sequence b by new_tokens[b] tokens; returns the number of new pages per sequence."""

@@ -224,10 +224,10 @@ int adamas_read_probe(const void* data, size_t bytes, void* sink, adamas_stream_
 int adamas_write_words(int32_t* dst, const int32_t* words, uint32_t n, adamas_stream_t stream);
 
 /*
- * Returns when `event` (hipEvent_t, recorded outside of any capture) is done; allowed while the calling thread captures
- * a stream, whose graph it leaves as it is.
+ * Returns when what has been launched on the default stream of `device` is done; allowed while the calling thread
+ * captures another stream, whose graph it leaves as it is.
  */
-int adamas_wait_event(void* event);
+int adamas_wait_default_stream(int32_t device);
 
 /* Bytes of workspace adamas_topk needs for these sizes (see adamas_topk). */
 size_t adamas_topk_workspace_bytes(uint32_t num_rows, uint32_t n_max, uint32_t k);

@@ -468,7 +468,6 @@ def test_write_words_arguments():
     assert lib.adamas_write_words(16, words, 0, None) == -1
     assert lib.adamas_write_words(16, words, _lib.MAX_WORDS + 1, None) == -1
     assert lib.adamas_write_words(18, words, 4, None) == -4
-    assert lib.adamas_wait_event(None) == -1
 
 
 def test_a_call_that_the_native_host_side_leaves_costs_little():

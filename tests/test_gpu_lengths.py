@@ -230,7 +230,8 @@ def test_a_write_from_another_stream_comes_behind_those_before(gpu_device, pages
     for _ in range(5):
         x = x @ x * 1e-4
     s.reserve([7])                                   # behind the products
-    event = s._written
+    event = torch.cuda.Event()
+    event.record()
     with torch.cuda.stream(torch.cuda.Stream()):
         assert not event.query()
         s.reserve_pages_ahead(pages)
