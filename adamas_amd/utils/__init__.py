@@ -63,9 +63,10 @@ _FLOAT_DTYPES = (torch.float16, torch.bfloat16)
 
 # The operators of a decode token try a native function first (csrc/host_ops.cpp), which serves the ordinary call and
 # returns None for any other before it has done anything; what follows the try serves every call and names what is
-# wrong with one.  Host time of a call without / with it, us (a launch is 2 to 2.5 of it): hadamard_transform 5.5 / 3.8,
-# append_kvh 9.5 / 4.3, decode_estimate 9.8 / 4.5, decode_topk 8.6 / 5.4, decode_sparse_attn 9.0 / 4.5, decode_step
-# 12.1 / 7.5; the six operators of the attention module, 16384 tokens, two layers 116 / 73.
+# wrong with one.  Host time of a call without / with it, us (a launch is 2 to 2.5 of it): hadamard_transform 5.7 / 3.9, in
+# place 4.3 / 2.9, append_kvh 9.4 / 4.6, decode_estimate 9.9 / 4.9, decode_topk 8.6 / 5.4, decode_sparse_attn 8.0 / 4.8,
+# decode_step 12.0 / 7.8; the six operators of the attention module, 16384 tokens, two layers 116 / 75; a call that is
+# not served costs 0.1 to 1.5 more than without.
 _host = None
 
 

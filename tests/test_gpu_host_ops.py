@@ -191,7 +191,7 @@ def test_on_the_current_stream(gpu_device, monkeypatch, op):
     torch.cuda.synchronize()
     side = torch.cuda.Stream()
     with torch.cuda.stream(side):
-        for _ in range(3):
+        for _ in range(6):
             a = a @ a * 1e-4
         busy = torch.cuda.Event()
         busy.record()
